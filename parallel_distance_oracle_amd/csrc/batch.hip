@@ -494,13 +494,17 @@ __global__ void k_zero_u64(unsigned long long *p, uint64_t count)
 
 // Level masks (see bp_mask_scan) and nonempty-set masks (bp_nz_filter) of
 // every vertex: one 128-byte row per vertex.
-__global__ __launch_bounds__(256) void k_bp_masks(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                                  unsigned long long *lmask)
+__global__ __launch_bounds__(256) void k_bp_masks(uint32_t n, const uint8_t *bpd, unsigned long long *lmask)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
-        uint32_t d[13];
-        load_dline(bpd, (uint32_t)v, d);
+        uint32_t d[kBpdStride / 4];
+        const uint4 *line = reinterpret_cast<const uint4 *>(bpd + v * kBpdStride);
+#pragma unroll
+        for (int q = 0; q < (int)kBpdStride / 16; ++q) {
+            const uint4 x = line[q];
+            d[4 * q] = x.x, d[4 * q + 1] = x.y, d[4 * q + 2] = x.z, d[4 * q + 3] = x.w;
+        }
         unsigned long long m[kLmWords] = {};
 #pragma unroll
         for (int i = 0; i < (int)kBP; ++i) {
@@ -508,9 +512,10 @@ __global__ __launch_bounds__(256) void k_bp_masks(uint32_t n, const uint8_t *bpd
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 if (x == (uint32_t)k) m[k] |= 1ull << i;
-            const ulonglong2 st = bps[v * kBP + i];
-            if (st.x) m[8] |= 1ull << i;
-            if (st.y) m[9] |= 1ull << i;
+            const int nzb = (int)kBpNzByte + i / 4;
+            const uint32_t nz = d[nzb >> 2] >> (8 * (nzb & 3) + (i & 3));
+            m[kLmNz1] |= (unsigned long long)(nz & 1u) << i;
+            m[kLmNz0] |= (unsigned long long)((nz >> 4) & 1u) << i;
         }
         uint4 *dst = reinterpret_cast<uint4 *>(lmask + v * kLmWords);
 #pragma unroll
@@ -1875,8 +1880,7 @@ static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index
                        (uint64_t)dc_rows * kBatch * sizeof(DT) / 4, ~0u);
     hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.ind.p, (uint64_t)n * kWords);
     hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.cand.p, (uint64_t)n * kWords);
-    hipLaunchKernelGGL(k_bp_masks, dim3(fg), dim3(256), 0, st, n, idx->bpd.p, (const ulonglong2 *)idx->bps.p,
-                       B.lmask.p);
+    hipLaunchKernelGGL(k_bp_masks, dim3(fg), dim3(256), 0, st, n, idx->bpd.p, B.lmask.p);
     hipLaunchKernelGGL(k_hub_info_init, dim3(fg), dim3(256), 0, st, B.hinfo.p, (uint64_t)n);
     hipLaunchKernelGGL(k_fill_u32, dim3(fg), dim3(256), 0, st, B.d1len.p, (uint64_t)n, 0u);
     hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, reinterpret_cast<unsigned long long *>(B.lrec.p),

@@ -251,6 +251,7 @@ pado_gpu_status build_bp(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<uint8_t>
         hipLaunchKernelGGL(k_bp_store, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, i, lvl.p, s1.p, s0.p,
                            idx->bpd.p, (unsigned long long *)idx->bps.p);
     }
+    launch_bp_finish(n, false, idx->bps.p, idx->bpd.p, st);
     PADO_HIP(hipStreamSynchronize(st));
     idx->bp_max_level = max_level;
     return PADO_GPU_OK;

@@ -15,7 +15,7 @@
 //   k_ms_child : slots where v is at d and u is unvisited -> u joins level d+1
 //                there (nm), bp_dist = d+1, S^-1/S^0 of v pushed into u's slot
 //   k_ms_update: vis |= nm for the new frontier; fm cleared for the old one
-// Finally S^0 is masked with ~S^-1 (PARA:829-835).  The set unions are 64-bit
+// Finally S^0 is masked with ~S^-1 (PARA:829-835, k_bp_finish).  The set unions are 64-bit
 // atomicOr, order-free, so the records are deterministic.
 #include "internal.hpp"
 
@@ -138,17 +138,6 @@ __global__ __launch_bounds__(256) void k_ms_update(const uint32_t *old_list, con
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < no; i += stride) fm_old[old_list[i]] = 0ull;
 }
 
-__global__ void k_ms_finish(uint32_t n, ulonglong2 *bps)
-{
-    const uint64_t total = (uint64_t)n * kBP;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        ulonglong2 s = bps[i];
-        s.y &= ~s.x;
-        bps[i] = s;
-    }
-}
-
 __global__ void k_ms_fill(uint8_t *bpd, uint64_t nbpd, u64 *z0, uint64_t nz0)
 {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -159,6 +148,36 @@ __global__ void k_ms_fill(uint8_t *bpd, uint64_t nbpd, u64 *z0, uint64_t nz0)
 __global__ void k_ms_zero_counts(uint32_t *c) { c[threadIdx.x] = 0; }
 
 }  // namespace
+
+// Sixteen lanes per vertex: lane l < 13 masks the sets of slots 4l..4l+3 and
+// writes their byte of nonempty-set bits, so one pass over the sets (800 B per
+// vertex) does both.
+__global__ __launch_bounds__(256) void k_bp_finish(uint32_t n, int mask, ulonglong2 *bps, uint8_t *bpd)
+{
+    const uint32_t l = threadIdx.x & 15u;
+    const uint32_t stride = (gridDim.x * blockDim.x) / 16;
+    if (l > (kBP - 1) / 4) return;
+    for (uint32_t v = (blockIdx.x * blockDim.x + threadIdx.x) / 16; v < n; v += stride) {
+        ulonglong2 *row = bps + (uint64_t)v * kBP + 4 * l;
+        const uint32_t cnt = min(4u, kBP - 4 * l);
+        uint32_t nz = 0;
+        for (uint32_t j = 0; j < cnt; ++j) {
+            ulonglong2 s = row[j];
+            if (mask && (s.x & s.y)) {
+                s.y &= ~s.x;
+                row[j] = s;
+            }
+            nz |= (s.x ? 1u << j : 0u) | (s.y ? 16u << j : 0u);
+        }
+        bpd[(uint64_t)v * kBpdStride + kBpNzByte + l] = (uint8_t)nz;
+    }
+}
+
+void launch_bp_finish(uint32_t n, bool mask, uint64_t *bps, uint8_t *bpd, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_bp_finish, dim3(grid_for((uint64_t)n * 16, 256, 16384)), dim3(256), 0, st, n, mask ? 1 : 0,
+                       (ulonglong2 *)bps, bpd);
+}
 
 void select_bp_roots(uint32_t n, const uint64_t *off, const uint32_t *adj, std::vector<uint8_t> &used,
                      uint32_t *roots, BpSeeds &seeds, const uint32_t *map)
@@ -312,7 +331,7 @@ pado_gpu_status build_bp_seeded(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<u
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    hipLaunchKernelGGL(k_ms_finish, dim3(8192), dim3(256), 0, st, n, bps);
+    launch_bp_finish(n, true, idx->bps.p, idx->bpd.p, st);
     PADO_HIP(hipStreamSynchronize(st));
     idx->bp_max_level = max_level;
     return PADO_GPU_OK;

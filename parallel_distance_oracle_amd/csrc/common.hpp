@@ -15,7 +15,11 @@
 namespace pado {
 
 constexpr uint32_t kBP = 50;          // BITPARALLEL_SIZE (PARA:45)
-constexpr uint32_t kBpdStride = 64;   // bytes per vertex in the bp_dist array (50 used)
+constexpr uint32_t kBpdStride = 64;   // bytes per vertex in the bp_dist array (50 distances, kBpNzByte on: below)
+// Bytes 51..63 of a vertex's distance line: byte kBpNzByte + l tells which of
+// the slots 4l..4l+3 have a nonempty S^-1 (bits 0..3) and S^0 (bits 4..7).
+// The queries read the line anyway and skip the sets that it rules out.
+constexpr uint32_t kBpNzByte = 51;
 constexpr uint32_t kBatch = 1024;     // BATCH_SIZE (PARA:42)
 constexpr uint32_t kWords = kBatch / 64;  // 64-bit words per 1024-root bitmap row
 constexpr uint8_t kInf8 = 255;        // SMALLI_MAX (GLB:40)
@@ -87,7 +91,9 @@ inline std::recursive_mutex &capture_mutex()
     return m;
 }
 
-// Device buffer owned by a handle.
+// Device buffer owned by a handle.  kBufSlack bytes past its end are its own
+// too: a 16-byte read that starts inside it may run over the end (query.hip).
+constexpr size_t kBufSlack = 16;
 template <class T>
 struct DevBuf {
     T *p = nullptr;
@@ -97,7 +103,7 @@ struct DevBuf {
         release();
         if (count == 0) count = 1;
         std::lock_guard<std::recursive_mutex> g(capture_mutex());
-        hipError_t e = hipMalloc((void **)&p, count * sizeof(T));
+        hipError_t e = hipMalloc((void **)&p, count * sizeof(T) + kBufSlack);
         if (e != hipSuccess) {
             p = nullptr;
             set_error("hipMalloc(" + std::to_string(count * sizeof(T)) + " B): " + hipGetErrorString(e));
@@ -224,7 +230,8 @@ struct pado_gpu_index {
     uint32_t wide = 0;  // labels in the wide hop domain (Hop<true>)
     uint32_t bp_pass_through = 0;  // wide build whose bit-parallel BFS was cut at level 254:
                                    // its bit-parallel vertices were labeled as ordinary hubs
-    // Bit-parallel labels, rank space: bpd[v*64 + i], bps[(v*50 + i)*2 + {0,1}].
+    // Bit-parallel labels, rank space: bpd[v*64 + i], bps[(v*50 + i)*2 + {0,1}];
+    // the rest of a bpd line holds the nonempty-set bits (kBpNzByte).
     pado::DevBuf<uint8_t> bpd;
     pado::DevBuf<uint64_t> bps;
     // Canonical labels, rank space: CSR of packed (hub << 8) | dist, hubs ascending.

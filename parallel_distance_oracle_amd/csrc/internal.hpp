@@ -14,6 +14,11 @@ pado_gpu_status build_bp(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<uint8_t>
 pado_gpu_status build_bp_multi(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<uint8_t> &d_used,
                                std::vector<uint8_t> &h_used);
 
+// Writes the nonempty-set bits (kBpNzByte) of every vertex's distance line from
+// its sets; whatever fills bpd / bps ends with it.  With `mask` the sets are
+// first made disjoint, S^0 \ S^-1 (PARA:829-835).
+void launch_bp_finish(uint32_t n, bool mask, uint64_t *bps, uint8_t *bpd, hipStream_t st);
+
 // Seeds of the multi-source sweep: slot roots (j = 255) and their selected
 // neighbours (j = neighbour index), as vertex ids of the graph being labeled.
 struct BpSeeds {

@@ -539,6 +539,7 @@ pado_gpu_status pado_gpu_index_import(pado_gpu_ctx *ctx, uint32_t n, const uint8
         set_error("index import copy failed");
         return PADO_GPU_ERR_HIP;
     }
+    launch_bp_finish(n, false, idx->bps.p, idx->bpd.p, st);
     if (total)
         hipLaunchKernelGGL(k_pack_labels, dim3(grid_for(total, 256, 8192)), dim3(256), 0, st, total, dh.p, dd.p,
                            idx->lab.p);

@@ -13,36 +13,50 @@
 // reproduces the reference's answers bit for bit.  Either way the slot order
 // does not matter: the result is a minimum over slots.
 //
-// Mapping: one wave per pair.  Lanes 0..49 take one bit-parallel slot each:
-// first the distance bytes only, then, after a wave minimum m of the slot
-// sums, the set pairs of just the slots that could still go below m (sum
-// <= m + 1).  The wave intersects the two hub-sorted label lists: the longer
-// list is copied into the wave's LDS (up to kQLds labels) and lanes take 64
-// labels of the shorter list at a time and binary-search them there, so the
-// search's dependent steps are LDS reads instead of global ones.  A wave of
-// the batch kernels answers pairs i, i + W, i + 2W, ... (W = waves in the
-// grid) as a software pipeline: while pair i is answered, pair i + W's label
-// offsets and pair i + 2W's ids are already in flight (1.37 -> 1.45 G
-// queries/s on R-MAT 20 uniform pairs; loading the next pair's bit-parallel
-// bytes early as well measured slower).  Within a pair, every read that needs
-// only the label offsets is issued first (distance bytes, the shorter list's
-// first 64 labels, the longer list's first 256), the set pairs are requested
-// next and the label search runs while they are in flight.  k_query is held
-// to 64 VGPRs (8 waves per SIMD instead of 7): 1.45 -> 1.98 G queries/s for
-// both changes (without the cap, 128 early labels per wave measured best).
+// Mapping: four pairs per wave, sixteen lanes (one DPP row) each; a wave
+// holds up to 64 consecutive pairs (lane j: pair j's ids and label offsets,
+// loaded together) and answers them four at a time.
+//   Bit-parallel slots: a lane takes four slots as bytes of one word of the
+// distance line.  With m the smallest slot sum, only slots at m or m + 1 can
+// lower it, and only where the sets that decide are nonempty; the line's
+// spare bytes say which are (bp_nz_byte), so most set pairs are never read.
+//   Labels: the longer list goes through the group's LDS tile (kQTile labels,
+// padded with all-ones to a power of two), and each lane searches four labels
+// of the shorter list in it at once, branch-free.  The reads that need only
+// the offsets go out together: distance words, the longer list's first 128
+// labels, the shorter list's first 64; the set pairs are requested next and
+// the search runs while they are in flight.
+//
+// What bounds it: instruction issue.  One wave per pair spent 234 vector
+// instructions a pair (73% of the SIMDs' issue slots on R-MAT 20) and read
+// all set pairs within one of the smallest sum (46 slots a pair; the
+// nonempty-set bits leave 2.3).  One million pairs, half of them Zipf, on the
+// R-MAT 14 index: 264 -> 122 us; 2 million on the weighted R-MAT 18 index:
+// 744 -> 555 us; 6 million in host arrays, R-MAT 18: 3.66 -> 2.76 ms; 10
+// million uniform pairs on R-MAT 20: 4.99 -> 4.47 ms.
 #include "internal.hpp"
 
 namespace pado {
 namespace {
 
-__device__ inline uint32_t wave_min_u32(uint32_t x)
-{
-    for (int o = 32; o > 0; o >>= 1) {
-        uint32_t y = __shfl_xor(x, o);
-        x = y < x ? y : x;
-    }
-    return x;
-}
+constexpr uint32_t kQWaves = 4;               // waves per query block
+constexpr uint32_t kQLanes = 16;              // lanes per pair: one DPP row
+constexpr uint32_t kQGroups = 64 / kQLanes;   // pairs a wave answers at once
+constexpr uint32_t kQTile = 256;              // labels of the longer list held in LDS
+constexpr uint32_t kQStep = 4 * kQLanes;      // labels a group moves per load: four per lane
+constexpr uint32_t kQPre = 2;                 // such loads of the longer list issued with the first reads
+// Groups' tiles start at different LDS banks: the first search steps of all
+// groups read the same tile position.
+constexpr uint32_t kQStride = kQTile + 8;
+constexpr uint32_t kQBuf = kQGroups * kQStride;  // LDS words per wave
+// Waves per SIMD the query kernels are compiled for: five is what their
+// registers take without spilling (at eight, 22 spilled registers made the
+// small-index batch below 171 us).
+constexpr int kQOcc = 5;
+constexpr uint32_t kNoSlot = 0x7FFFu;         // sum of a slot that does not count
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));  // four words at any word address
 
 // Orders LDS writes of some lanes of a wave before reads by other lanes.
 __device__ inline void q_lds_sync()
@@ -52,286 +66,349 @@ __device__ inline void q_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-constexpr uint32_t kQLds = 1024;   // labels of the longer list staged in LDS per wave
-constexpr uint32_t kServeLds = 768;  // the same in the resident serving kernel
-constexpr uint32_t kQWaves = 4;    // waves per query block
-constexpr uint32_t kQPre = 4;      // longer-list loads per lane issued with the pair's first reads
-constexpr uint32_t kWPre = 4;      // the same for weighted pairs (8 measured slower)
-
-}  // namespace
-
-// Index of the first entry of the sorted list L[0..len) whose hub is >= key
-// (labels compared by hub, the bits above the distance field).
-template <bool W>
-__device__ inline uint32_t lower_hub(const uint32_t *L, uint32_t len, uint32_t key)
+template <int N>
+__device__ inline uint32_t row_ror(uint32_t x)
 {
-    uint32_t lo = 0, hi = len;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if ((L[mid] >> Hop<W>::kBits) < key)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x120 + N, 0xF, 0xF, false);
 }
 
-// One pair whose label offsets (oa, la), (ob, lb) are already loaded.
-// sbuf: the wave's kQLds-entry LDS buffer.  Hop<false>: the reference's
-// answers (255 for unreachable or >= 253); Hop<true>: exact hops, 0xFFFF for
-// unreachable, using only bit-parallel slots reached on both sides.
-template <bool W, uint32_t LDS = kQLds>
-__device__ inline uint32_t pair_distance_at(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                            const uint32_t *lab, uint32_t a, uint32_t b, uint64_t oa, uint32_t la,
-                                            uint64_t ob, uint32_t lb, bool ref_compat, uint32_t *sbuf)
+// The least value of the sixteen lanes of a group, in all of them.
+__device__ inline uint32_t group_min(uint32_t x)
+{
+    x = min(x, row_ror<8>(x));
+    x = min(x, row_ror<4>(x));
+    x = min(x, row_ror<2>(x));
+    return min(x, row_ror<1>(x));
+}
+
+// The largest of the values that the four lanes r0 .. r0 + 3 hold, as a scalar.
+__device__ inline uint32_t quad_max(uint32_t x, uint32_t r0)
+{
+    const uint32_t a = __builtin_amdgcn_readlane(x, r0), b = __builtin_amdgcn_readlane(x, r0 + 1);
+    const uint32_t c = __builtin_amdgcn_readlane(x, r0 + 2), d = __builtin_amdgcn_readlane(x, r0 + 3);
+    return max(max(a, b), max(c, d));
+}
+
+// Four list entries from position j (any words where j is past the list; see
+// mask4).  A read that starts inside the list may run up to three words past
+// its end: device buffers have that much slack (DevBuf).
+__device__ inline u32x4 load4(const uint32_t *p, uint32_t j, uint32_t len)
+{
+    u32x4 v = {~0u, ~0u, ~0u, ~0u};
+    if (j < len) v = *reinterpret_cast<const u32x4_at4 *>(p + j);
+    return v;
+}
+
+// The entries of load4 past the list as all-ones, which no hub is.  Apart from
+// the load, so that a pair's loads are all in flight before the first is
+// waited for.
+__device__ inline u32x4 mask4(u32x4 v, uint32_t j, uint32_t len)
+{
+    v.x = j < len ? v.x : ~0u;
+    v.y = j + 1 < len ? v.y : ~0u;
+    v.z = j + 2 < len ? v.z : ~0u;
+    v.w = j + 3 < len ? v.w : ~0u;
+    return v;
+}
+
+// Lower bounds of four keys in a tile of `size` ascending words (a power of
+// two, at least 1): pos[q] = the tile position of the first word >= key[q],
+// or the last position.
+__device__ inline void search4(const uint32_t *tile, uint32_t size, const u32x4 &key, uint32_t (&pos)[4])
+{
+#pragma unroll
+    for (int q = 0; q < 4; ++q) pos[q] = 0;
+    for (uint32_t half = size >> 1; half; half >>= 1) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pos[q] += tile[pos[q] + half - 1] < key[q] ? half : 0u;
+    }
+}
+
+// A lane's pair: ids and the two label lists, the shorter first.  `in` is
+// false for a lane without a pair or with an id past the index.
+struct QPair {
+    uint32_t a, b;
+    uint64_t os, ot;
+    uint32_t ls, lt;
+    bool in;
+};
+
+__device__ inline QPair load_pair(bool has, uint32_t n, const uint64_t *loff, uint32_t a, uint32_t b)
+{
+    QPair p{0, 0, 0, 0, 0, 0, has && a < n && b < n};
+    if (p.in) {
+        const uint64_t oa = loff[a], ob = loff[b];
+        const uint32_t la = (uint32_t)(loff[a + 1] - oa), lb = (uint32_t)(loff[b + 1] - ob);
+        const bool sw = la > lb;
+        p.a = a;
+        p.b = b;
+        p.os = sw ? ob : oa;
+        p.ot = sw ? oa : ob;
+        p.ls = sw ? lb : la;
+        p.lt = sw ? la : lb;
+    }
+    return p;
+}
+
+__device__ inline uint64_t shfl64(uint64_t x, uint32_t src)
+{
+    const uint32_t lo = __shfl((uint32_t)x, src), hi = __shfl((uint32_t)(x >> 32), src);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// The power of two at or above x (x in [1, kQTile]; 1 for 0).
+__device__ inline uint32_t tile_size(uint32_t x) { return x <= 1u ? 1u : 1u << (32 - __builtin_clz(x - 1u)); }
+
+// Answers the wave's pairs, lane j holding pair j < len: returns lane j's
+// answer.  Hop<false>: the reference's answers (255 for unreachable or >=
+// 253); Hop<true>: exact hops, 0xFFFF for unreachable, using only
+// bit-parallel slots reached on both sides.  sbuf: the wave's kQBuf words.
+template <bool W>
+__device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bps, const uint32_t *lab,
+                                        const QPair &p, uint32_t len, bool ref_compat, uint32_t *sbuf)
 {
     constexpr uint32_t B = Hop<W>::kBits, MASK = Hop<W>::kInf;
     constexpr uint32_t UNREACHED = W ? 0xFFFFu : 255u;
-    const uint32_t lane = threadIdx.x & 63;
-    if (a >= n || b >= n) return a == b ? 0u : UNREACHED;
-    // Every load that needs only the offsets goes out first: the slots'
-    // distance bytes, the shorter list's first 64 labels and the longer
-    // list's first kQPre * 64 labels (into registers; written to LDS after
-    // the set pairs are requested), so the pair's chain of dependent global
-    // reads is bytes -> set pairs, with the label search in between.
-    uint32_t da = 0, db = 0;
-    if (lane < kBP) {
-        da = bpd[(uint64_t)a * kBpdStride + lane];
-        db = bpd[(uint64_t)b * kBpdStride + lane];
-    }
-    const uint32_t *S = lab + (la <= lb ? oa : ob);
-    const uint32_t *T = lab + (la <= lb ? ob : oa);
-    const uint32_t ls = la <= lb ? la : lb, lt = la <= lb ? lb : la;
-    const bool staged = lt <= LDS;
-    const uint32_t s0 = lane < ls ? S[lane] : 0u;
-    uint32_t tv[kQPre];
-    if (staged) {
+    const uint32_t lane = threadIdx.x & 63, l = lane & (kQLanes - 1), g = lane / kQLanes;
+    uint32_t *tile = sbuf + g * kQStride;
+    uint32_t mine = UNREACHED;
+    for (uint32_t r0 = 0; r0 < len; r0 += kQGroups) {
+        const uint32_t src = r0 + g;
+        const uint32_t a = __shfl(p.a, src), b = __shfl(p.b, src);
+        const uint32_t ls = __shfl(p.ls, src), lt = __shfl(p.lt, src);
+        const uint32_t *S = lab + shfl64(p.os, src), *T = lab + shfl64(p.ot, src);
+        const uint32_t ms = quad_max(p.ls, r0), mt = quad_max(p.lt, r0);
+        // (a group without a pair reads vertex 0's line and no labels)
+        const uint32_t wa = reinterpret_cast<const uint32_t *>(bpd + (uint64_t)a * kBpdStride)[l];
+        const uint32_t wb = reinterpret_cast<const uint32_t *>(bpd + (uint64_t)b * kBpdStride)[l];
+        u32x4 tv[kQPre];
 #pragma unroll
-        for (uint32_t u = 0; u < kQPre; ++u) {
-            const uint32_t j = u * 64 + lane;
-            tv[u] = j < lt ? T[j] : 0u;
-        }
-    }
-    // Bit-parallel slots.  A slot counts if the reference's gate passes; its
-    // result is td - {2, 1, 0}, so only slots with td <= m + 1 (m = the
-    // smallest counted td) can beat m.
-    int td = 0x7FFF;
-    bool gate = false;
-    if (lane < kBP) {
-        td = (int)(da + db);
-        if (W)
-            gate = da != kInf8 && db != kInf8;  // 255: the slot's BFS did not reach this vertex
-        else
-            gate = !(ref_compat && td < 2) && td - 2 <= 255;
-    }
-    const uint32_t m = wave_min_u32(gate ? (uint32_t)td : 0xFFFFu);
-    const bool use_sets = gate && (uint32_t)td <= m + 1u;
-    ulonglong2 sa = {0, 0}, sb = {0, 0};
-    if (use_sets) {
-        sa = bps[(uint64_t)a * kBP + lane];
-        sb = bps[(uint64_t)b * kBP + lane];
-    }
-    if (staged) {
+        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * kQStep + 4 * l, lt);
+        const u32x4 s0 = load4(S, 4 * l, ls);
+        // This lane's four slots (the last lanes have none).
+        uint32_t td[4];
+        {
+            const uint32_t lo = (wa & 0x00FF00FFu) + (wb & 0x00FF00FFu);
+            const uint32_t hi = ((wa >> 8) & 0x00FF00FFu) + ((wb >> 8) & 0x00FF00FFu);
+            td[0] = lo & 0xFFFFu;
+            td[1] = hi & 0xFFFFu;
+            td[2] = lo >> 16;
+            td[3] = hi >> 16;
 #pragma unroll
-        for (uint32_t u = 0; u < kQPre; ++u) {
-            const uint32_t j = u * 64 + lane;
-            if (j < lt) sbuf[j] = tv[u];
-        }
-        for (uint32_t j = kQPre * 64 + lane; j < lt; j += 64) sbuf[j] = T[j];
-        q_lds_sync();
-    }
-    uint32_t d = UNREACHED;
-    for (uint32_t j0 = 0; j0 < ls; j0 += 64) {
-        const uint32_t j = j0 + lane;
-        if (j < ls) {
-            const uint32_t s = j0 == 0 ? s0 : S[j];
-            const uint32_t key = s >> B;
-            const uint32_t *L = staged ? sbuf : T;
-            const uint32_t lo = lower_hub<W>(L, lt, key);
-            if (lo < lt && (L[lo] >> B) == key) {
-                const uint32_t t = (s & MASK) + (L[lo] & MASK);
-                if (t < d) d = t;
+            for (uint32_t j = 0; j < 4; ++j) {
+                bool ok = 4 * l + j < kBP;
+                if (W)  // 255: the slot's BFS did not reach this vertex
+                    ok = ok && ((wa >> (8 * j)) & 255u) != kInf8 && ((wb >> (8 * j)) & 255u) != kInf8;
+                else
+                    ok = ok && !(ref_compat && td[j] < 2u);
+                if (!ok) td[j] = kNoSlot;
             }
         }
+        // Which of this lane's slots have S^-1 sets on both sides (bits of
+        // `both`) and which S^-1 on one and S^0 on the other (`cross`).
+        uint32_t both, cross;
+        {
+            const uint32_t sh = 8 * ((kBpNzByte + l) & 3u), from = (lane & ~(kQLanes - 1)) + ((kBpNzByte + l) >> 2);
+            const uint32_t na = __shfl(wa, from) >> sh, nb = __shfl(wb, from) >> sh;
+            both = na & nb & 15u;
+            cross = ((na & (nb >> 4)) | ((na >> 4) & nb)) & 15u;
+        }
+        const ulonglong2 *ra = bps + (uint64_t)a * kBP + 4 * l, *rb = bps + (uint64_t)b * kBP + 4 * l;
+        if (min(min(td[0], td[1]), min(td[2], td[3])) < 2u) {
+            // A sum that its sets would take below zero does not count (no
+            // such slot in a built index: a root's own sets are empty).
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                if (td[j] >= 2u || !(((both | cross) >> j) & 1u)) continue;
+                const ulonglong2 xa = ra[j], xb = rb[j];
+                const uint64_t neg = (xa.x & xb.x) | (td[j] == 0u ? (xa.x & xb.y) | (xa.y & xb.x) : 0ull);
+                td[j] = neg ? kNoSlot : td[j];
+            }
+        }
+        const uint32_t m = group_min(min(min(td[0], td[1]), min(td[2], td[3])));
+        // The slots at m (cm) and m + 1 (cn) that their sets can lower: S^-1
+        // against S^-1 by two, S^-1 against S^0 by one (which does not help
+        // at m + 1).
+        uint32_t cm, cn;
+        {
+            uint32_t em = 0, en = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                em |= td[j] == m ? 1u << j : 0u;
+                en |= td[j] == m + 1u ? 1u << j : 0u;
+            }
+            if (m == kNoSlot || l > (kBP - 1) / 4) em = en = 0u;
+            cm = em & (both | cross);
+            cn = en & both;
+        }
+        // The lane's first set pair is requested before the search.
+        ulonglong2 sa = {0, 0}, sb = {0, 0};
+        uint32_t j0 = 0;
+        const bool first = (cm | cn) != 0u, first_m = cm != 0u;
+        if (first) {
+            j0 = (uint32_t)__builtin_ctz(first_m ? cm : cn);
+            sa = ra[j0];
+            sb = rb[j0];
+            if (first_m)
+                cm &= cm - 1u;
+            else
+                cn &= cn - 1u;
+        }
+        uint32_t d = m < UNREACHED && m != kNoSlot ? m : UNREACHED;
+        for (uint32_t t0 = 0; ms && t0 < mt; t0 += kQTile) {
+            const uint32_t left = min(mt - t0, kQTile), size = tile_size(left);
+            for (uint32_t u = 0; u * kQStep < size; ++u) {
+                const uint32_t j = t0 + u * kQStep + 4 * l;
+                const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
+                *reinterpret_cast<u32x4 *>(tile + u * kQStep + 4 * l) = mask4(v, j, lt);
+            }
+            q_lds_sync();
+            for (uint32_t i = 0; i < ms; i += kQStep) {
+                const u32x4 s = mask4(i == 0 ? s0 : load4(S, i + 4 * l, ls), i + 4 * l, ls);
+                // A packed label with the same hub is >= the hub with
+                // distance 0, so whole words compare as hubs do.
+                const u32x4 key = s & ~MASK;
+                uint32_t pos[4];
+                search4(tile, size, key, pos);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t x = tile[pos[q]];
+                    if ((x ^ s[q]) >> B == 0u && s[q] != ~0u) d = min(d, (x & MASK) + (s[q] & MASK));
+                }
+            }
+            // The next copy must not overtake these reads.
+            q_lds_sync();
+        }
+        d = group_min(d);
+        if (first) {
+            if (sa.x & sb.x)
+                d = min(d, first_m ? m - 2u : m - 1u);
+            else if (first_m && ((sa.x & sb.y) | (sa.y & sb.x)))
+                d = min(d, m - 1u);
+        }
+        // The others, where they can still lower the answer.
+        if (d + 1u <= m) cn = 0u, cm &= both;
+        if (d + 2u <= m) cm = 0u;
+        while (cm | cn) {
+            const bool at_m = cm != 0u;
+            const uint32_t j = (uint32_t)__builtin_ctz(at_m ? cm : cn);
+            const ulonglong2 xa = ra[j], xb = rb[j];
+            if (at_m)
+                cm &= cm - 1u;
+            else
+                cn &= cn - 1u;
+            if (xa.x & xb.x)
+                d = min(d, at_m ? m - 2u : m - 1u);
+            else if (at_m && ((xa.x & xb.y) | (xa.y & xb.x)))
+                d = min(d, m - 1u);
+        }
+        d = group_min(d);
+        if (!W && d >= 253u) d = 255u;
+        const uint32_t back = __shfl(d, (lane & (kQGroups - 1)) * kQLanes);
+        if (lane / kQGroups == r0 / kQGroups && p.in) mine = back;
     }
-    // The next pair's copy must not overtake this pair's reads.
-    if (staged) q_lds_sync();
-    if (use_sets) {
-        int t = td;
-        if (sa.x & sb.x)
-            t -= 2;
-        else if ((sa.x & sb.y) | (sa.y & sb.x))
-            t -= 1;
-        if ((uint32_t)t < d) d = (uint32_t)t;
-    }
-    d = wave_min_u32(d);
-    if (W) return d;
-    return d >= 253u ? 255u : d;
-}
-
-template <bool W>
-__device__ inline uint32_t pair_distance(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps, const uint64_t *loff,
-                                         const uint32_t *lab, uint32_t a, uint32_t b, bool ref_compat,
-                                         uint32_t *sbuf)
-{
-    if (a >= n || b >= n) return a == b ? 0u : (W ? 0xFFFFu : 255u);
-    const uint64_t oa = loff[a], ob = loff[b];
-    return pair_distance_at<W>(n, bpd, bps, lab, a, b, oa, (uint32_t)(loff[a + 1] - oa), ob,
-                               (uint32_t)(loff[b + 1] - ob), ref_compat, sbuf);
-}
-
-// A pair's ids and label offsets, loaded ahead of its turn.
-struct QPair {
-    uint32_t a, b;
-    uint64_t oa, ea, ob, eb;
-};
-
-__device__ inline void q_load_ids(QPair &p, const uint32_t *qa, const uint32_t *qb, uint64_t i, uint64_t k)
-{
-    p.a = 0;
-    p.b = 0;
-    if (i < k) {
-        p.a = qa[i];
-        p.b = qb[i];
-    }
-}
-
-__device__ inline void q_load_offsets(QPair &p, uint32_t n, const uint64_t *loff)
-{
-    p.oa = p.ea = p.ob = p.eb = 0;
-    if (p.a < n && p.b < n) {
-        p.oa = loff[p.a];
-        p.ea = loff[p.a + 1];
-        p.ob = loff[p.b];
-        p.eb = loff[p.b + 1];
-    }
-}
-
-// OT: the answer type (u8, or u16 for a wide index or widened answers).
-template <bool W, class OT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_query(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                               const uint64_t *loff, const uint32_t *lab, const uint32_t *qa,
-                                               const uint32_t *qb, uint64_t k, OT *out, int ref_compat)
-{
-    __shared__ uint32_t s_q[kQWaves][kQLds];
-    uint32_t *sbuf = s_q[threadIdx.x >> 6];
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (i >= k) return;
-    // Software pipeline over the wave's pairs i, i + nw, ...: while pair i is
-    // answered, pair i + nw's label offsets and pair i + 2nw's ids are in
-    // flight, so a pair's dependent chain starts at its bit-parallel bytes.
-    QPair cur, nxt, far;
-    q_load_ids(cur, qa, qb, i, k);
-    q_load_offsets(cur, n, loff);
-    q_load_ids(nxt, qa, qb, i + nw, k);
-    for (;;) {
-        q_load_offsets(nxt, n, loff);
-        q_load_ids(far, qa, qb, i + 2 * nw, k);
-        const uint32_t d = pair_distance_at<W>(n, bpd, bps, lab, cur.a, cur.b, cur.oa, (uint32_t)(cur.ea - cur.oa),
-                                               cur.ob, (uint32_t)(cur.eb - cur.ob), ref_compat != 0, sbuf);
-        if ((threadIdx.x & 63) == 0) out[i] = (OT)d;
-        i += nw;
-        if (i >= k) break;
-        cur = nxt;
-        nxt = far;
-    }
+    return mine;
 }
 
 // Weighted query_distance (WPARA:2125-2243): min over common hubs of
 // La(h) + Lb(h).  Exact u32 answers, 0xFFFFFFFF when no hub is shared; with
 // ref_compat the reference's int16 domain (>= 32765 -> 32767, ids out of
-// range -> a == b ? 0 : 32767).  One wave per pair, the shorter list's hubs
-// binary-searched in the longer one as for unweighted labels.
-template <uint32_t LDS = kQLds>
-__device__ inline uint32_t wpair_distance_at(uint32_t n, const uint32_t *hub, const uint32_t *dist, uint32_t a,
-                                             uint32_t b, uint64_t oa, uint32_t la, uint64_t ob, uint32_t lb,
-                                             bool ref_compat, uint32_t *sbuf)
+// range -> a == b ? 0 : 32767).  As answer_pairs, on the hub lists;
+// distances of the shorter list come in with its hubs, those of the longer
+// list are read where a hub matches.
+__device__ inline uint32_t answer_wpairs(const uint32_t *hub, const uint32_t *dist, const QPair &p, uint32_t len,
+                                         bool ref_compat, uint32_t *sbuf)
 {
+    const uint32_t lane = threadIdx.x & 63, l = lane & (kQLanes - 1), g = lane / kQLanes;
+    uint32_t *tile = sbuf + g * kQStride;
+    uint32_t mine = 0xFFFFFFFFu;
+    for (uint32_t r0 = 0; r0 < len; r0 += kQGroups) {
+        const uint32_t src = r0 + g;
+        const uint32_t ls = __shfl(p.ls, src), lt = __shfl(p.lt, src);
+        const uint64_t os = shfl64(p.os, src), ot = shfl64(p.ot, src);
+        const uint32_t ms = quad_max(p.ls, r0), mt = quad_max(p.lt, r0);
+        u32x4 tv[kQPre];
+#pragma unroll
+        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(hub + ot, u * kQStep + 4 * l, lt);
+        const u32x4 s0 = load4(hub + os, 4 * l, ls), d0 = load4(dist + os, 4 * l, ls);
+        uint32_t d = 0xFFFFFFFFu;
+        for (uint32_t t0 = 0; ms && t0 < mt; t0 += kQTile) {
+            const uint32_t left = min(mt - t0, kQTile), size = tile_size(left);
+            for (uint32_t u = 0; u * kQStep < size; ++u) {
+                const uint32_t j = t0 + u * kQStep + 4 * l;
+                const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(hub + ot, j, lt);
+                *reinterpret_cast<u32x4 *>(tile + u * kQStep + 4 * l) = mask4(v, j, lt);
+            }
+            q_lds_sync();
+            for (uint32_t i = 0; i < ms; i += kQStep) {
+                const u32x4 s = mask4(i == 0 ? s0 : load4(hub + os, i + 4 * l, ls), i + 4 * l, ls);
+                const u32x4 e = i == 0 ? d0 : load4(dist + os, i + 4 * l, ls);
+                uint32_t pos[4], x[4];
+                search4(tile, size, s, pos);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    x[q] = 0xFFFFFFFFu;
+                    if (tile[pos[q]] == s[q] && s[q] != ~0u) x[q] = dist[ot + t0 + pos[q]];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t td = x[q] + e[q];
+                    if (x[q] != 0xFFFFFFFFu && td >= e[q]) d = min(d, td);  // (a sum past 2^32 lowers nothing)
+                }
+            }
+            q_lds_sync();
+        }
+        d = group_min(d);
+        if (ref_compat && d >= 32765u) d = 32767u;
+        const uint32_t back = __shfl(d, (lane & (kQGroups - 1)) * kQLanes);
+        if (lane / kQGroups == r0 / kQGroups && p.in) mine = back;
+    }
+    return mine;
+}
+
+// The answer of a pair with an id past the index.
+__device__ inline uint32_t outside_answer(uint32_t a, uint32_t b, uint32_t far) { return a == b ? 0u : far; }
+
+}  // namespace
+
+// Batch queries: a wave takes `chunk` consecutive pairs at a time (see
+// query_chunk).  OT: the answer type (u8, or u16 for a wide index or widened
+// answers).
+template <bool W, class OT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
+                                               const uint64_t *loff, const uint32_t *lab, const uint32_t *qa,
+                                               const uint32_t *qb, uint64_t k, uint32_t chunk, OT *out,
+                                               int ref_compat)
+{
+    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
     const uint32_t lane = threadIdx.x & 63;
-    if (a >= n || b >= n) return a == b ? 0u : (ref_compat ? 32767u : 0xFFFFFFFFu);
-    const uint64_t os = la <= lb ? oa : ob, ot = la <= lb ? ob : oa;
-    const uint32_t ls = la <= lb ? la : lb, lt = la <= lb ? lb : la;
-    // The longer list's hubs go to the wave's LDS (distances are read only
-    // for matches); its first kWPre * 64 hubs and the shorter list's first 64
-    // are requested together.
-    const bool staged = lt <= LDS;
-    const uint32_t k0 = lane < ls ? hub[os + lane] : 0u;
-    if (staged) {
-        uint32_t tv[kWPre];
-#pragma unroll
-        for (uint32_t u = 0; u < kWPre; ++u) {
-            const uint32_t j = u * 64 + lane;
-            tv[u] = j < lt ? hub[ot + j] : 0u;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < kWPre; ++u) {
-            const uint32_t j = u * 64 + lane;
-            if (j < lt) sbuf[j] = tv[u];
-        }
-        for (uint32_t j = kWPre * 64 + lane; j < lt; j += 64) sbuf[j] = hub[ot + j];
-        q_lds_sync();
-    }
-    const uint32_t *H = staged ? sbuf : hub + ot;
-    uint32_t d = 0xFFFFFFFFu;
-    for (uint32_t j0 = 0; j0 < ls; j0 += 64) {
-        const uint32_t j = j0 + lane;
-        if (j < ls) {
-            const uint32_t key = j0 == 0 ? k0 : hub[os + j];
-            uint32_t lo = 0, hi = lt;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (H[mid] < key)
-                    lo = mid + 1;
-                else
-                    hi = mid;
-            }
-            if (lo < lt && H[lo] == key) {
-                const uint64_t td = (uint64_t)dist[os + j] + dist[ot + lo];
-                if (td < d) d = (uint32_t)td;
-            }
-        }
-    }
-    // The next pair's copy must not overtake this pair's reads.
-    if (staged) q_lds_sync();
-    d = wave_min_u32(d);
-    if (ref_compat && d >= 32765u) d = 32767u;
-    return d;
-}
-
-__device__ inline uint32_t wpair_distance(uint32_t n, const uint64_t *loff, const uint32_t *hub, const uint32_t *dist,
-                                          uint32_t a, uint32_t b, bool ref_compat, uint32_t *sbuf)
-{
-    if (a >= n || b >= n) return a == b ? 0u : (ref_compat ? 32767u : 0xFFFFFFFFu);
-    const uint64_t oa = loff[a], ob = loff[b];
-    return wpair_distance_at(n, hub, dist, a, b, oa, (uint32_t)(loff[a + 1] - oa), ob, (uint32_t)(loff[b + 1] - ob),
-                             ref_compat, sbuf);
-}
-
-__global__ __launch_bounds__(256) void k_wquery(uint32_t n, const uint64_t *loff, const uint32_t *hub,
-                                                const uint32_t *dist, const uint32_t *qa, const uint32_t *qb,
-                                                uint64_t k, uint32_t *out, int ref_compat)
-{
-    __shared__ uint32_t s_q[kQWaves][kQLds];
-    uint32_t *sbuf = s_q[threadIdx.x >> 6];
     const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    uint64_t i = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (i >= k) return;
-    // The same software pipeline as k_query.
-    QPair cur, nxt, far;
-    q_load_ids(cur, qa, qb, i, k);
-    q_load_offsets(cur, n, loff);
-    q_load_ids(nxt, qa, qb, i + nw, k);
-    for (;;) {
-        q_load_offsets(nxt, n, loff);
-        q_load_ids(far, qa, qb, i + 2 * nw, k);
-        const uint32_t d = wpair_distance_at(n, hub, dist, cur.a, cur.b, cur.oa, (uint32_t)(cur.ea - cur.oa), cur.ob,
-                                             (uint32_t)(cur.eb - cur.ob), ref_compat != 0, sbuf);
-        if ((threadIdx.x & 63) == 0) out[i] = d;
-        i += nw;
-        if (i >= k) break;
-        cur = nxt;
-        nxt = far;
+    const uint64_t w = uniform64(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    for (uint64_t c0 = w * chunk; c0 < k; c0 += nw * chunk) {
+        const uint32_t len = (uint32_t)min((uint64_t)chunk, k - c0);
+        const bool has = lane < len;
+        const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
+        const QPair p = load_pair(has, n, loff, a, b);
+        const uint32_t d = answer_pairs<W>(bpd, bps, lab, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        if (has) out[c0 + lane] = (OT)(p.in ? d : outside_answer(a, b, W ? 0xFFFFu : 255u));
+    }
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_wquery(uint32_t n, const uint64_t *loff, const uint32_t *hub,
+                                                const uint32_t *dist, const uint32_t *qa, const uint32_t *qb,
+                                                uint64_t k, uint32_t chunk, uint32_t *out, int ref_compat)
+{
+    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
+    const uint64_t w = uniform64(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    for (uint64_t c0 = w * chunk; c0 < k; c0 += nw * chunk) {
+        const uint32_t len = (uint32_t)min((uint64_t)chunk, k - c0);
+        const bool has = lane < len;
+        const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
+        const QPair p = load_pair(has, n, loff, a, b);
+        const uint32_t d = answer_wpairs(hub, dist, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        if (has) out[c0 + lane] = p.in ? d : outside_answer(a, b, ref_compat ? 32767u : 0xFFFFFFFFu);
     }
 }
 
@@ -342,45 +419,45 @@ __global__ __launch_bounds__(256) void k_wquery(uint32_t n, const uint64_t *loff
 // once the counter passes k.
 constexpr uint32_t kGrab = 16;
 
-__global__ __launch_bounds__(256) void k_query_ws(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query_ws(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
                                                   const uint64_t *loff, const uint32_t *lab, const uint32_t *qa,
                                                   const uint32_t *qb, uint64_t k, uint8_t *out, int ref_compat,
                                                   unsigned long long *work)
 {
-    __shared__ uint32_t s_q[kQWaves][kQLds];
-    uint32_t *sbuf = s_q[threadIdx.x >> 6];
+    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
     const uint32_t lane = threadIdx.x & 63;
     for (;;) {
         unsigned long long c0 = 0;
         if (lane == 0) c0 = atomicAdd(work, (unsigned long long)kGrab);
-        c0 = __shfl(c0, 0);
+        c0 = uniform64(c0);
         if (c0 >= k) break;
-        const uint64_t c1 = c0 + kGrab < k ? c0 + kGrab : k;
-        for (uint64_t i = c0; i < c1; ++i) {
-            const uint32_t d = pair_distance<false>(n, bpd, bps, loff, lab, qa[i], qb[i], ref_compat != 0, sbuf);
-            if (lane == 0) out[i] = (uint8_t)d;
-        }
+        const uint32_t len = (uint32_t)min((uint64_t)kGrab, k - c0);
+        const bool has = lane < len;
+        const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
+        const QPair p = load_pair(has, n, loff, a, b);
+        const uint32_t d = answer_pairs<false>(bpd, bps, lab, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        if (has) out[c0 + lane] = (uint8_t)(p.in ? d : outside_answer(a, b, 255u));
     }
 }
 
-__global__ __launch_bounds__(256) void k_wquery_ws(uint32_t n, const uint64_t *loff, const uint32_t *hub,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_wquery_ws(uint32_t n, const uint64_t *loff, const uint32_t *hub,
                                                    const uint32_t *dist, const uint32_t *qa, const uint32_t *qb,
                                                    uint64_t k, uint32_t *out, int ref_compat,
                                                    unsigned long long *work)
 {
-    __shared__ uint32_t s_q[kQWaves][kQLds];
-    uint32_t *sbuf = s_q[threadIdx.x >> 6];
+    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
     const uint32_t lane = threadIdx.x & 63;
     for (;;) {
         unsigned long long c0 = 0;
         if (lane == 0) c0 = atomicAdd(work, (unsigned long long)kGrab);
-        c0 = __shfl(c0, 0);
+        c0 = uniform64(c0);
         if (c0 >= k) break;
-        const uint64_t c1 = c0 + kGrab < k ? c0 + kGrab : k;
-        for (uint64_t i = c0; i < c1; ++i) {
-            const uint32_t d = wpair_distance(n, loff, hub, dist, qa[i], qb[i], ref_compat != 0, sbuf);
-            if (lane == 0) out[i] = d;
-        }
+        const uint32_t len = (uint32_t)min((uint64_t)kGrab, k - c0);
+        const bool has = lane < len;
+        const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
+        const QPair p = load_pair(has, n, loff, a, b);
+        const uint32_t d = answer_wpairs(hub, dist, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        if (has) out[c0 + lane] = p.in ? d : outside_answer(a, b, ref_compat ? 32767u : 0xFFFFFFFFu);
     }
 }
 
@@ -492,16 +569,11 @@ __device__ void serve_poll(const ServeKernelArgs &A)
 
 // K: 0 = u8 hop answers, 1 = wide index (u16 exact hops), 2 = weighted (u32).
 template <int K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_serve(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_serve(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
                                                const uint64_t *loff, const uint32_t *lab, const uint32_t *wdist,
                                                ServeKernelArgs A)
 {
-    // A smaller label buffer than the batch kernel's leaves room for the
-    // descriptor's pairs within 20 KB of LDS per workgroup (eight per CU).
-    __shared__ uint32_t s_q[kQWaves][kServeLds];
-    // The descriptor's pairs: ids and label offsets, lane j's pair at [j].
-    __shared__ uint32_t s_ab[kQWaves][2][kServeGroup], s_len[kQWaves][2][kServeGroup];
-    __shared__ uint64_t s_off[kQWaves][2][kServeGroup];
+    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (blockIdx.x == 0 && wv == 0) {
         serve_poll(A);
@@ -536,43 +608,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
         const uint64_t seq = uniform64(ld_sys(&dp->seq));
         const uint32_t rk = uniform32(ld_sys(&dp->k));
         const uint64_t phys = pos % A.cap;
-        {
-            uint32_t ia = 0, ib = 0;
-            if (lane < len) {
-                ia = ld_sys(A.ra + phys + lane);
-                ib = ld_sys(A.rb + phys + lane);
-            }
-            uint64_t oa = 0, ob = 0;
-            uint32_t la = 0, lb = 0;
-            if (lane < len && ia < n && ib < n) {
-                oa = loff[ia];
-                ob = loff[ib];
-                la = (uint32_t)(loff[ia + 1] - oa);
-                lb = (uint32_t)(loff[ib + 1] - ob);
-            }
-            s_ab[wv][0][lane] = ia;
-            s_ab[wv][1][lane] = ib;
-            s_off[wv][0][lane] = oa;
-            s_off[wv][1][lane] = ob;
-            s_len[wv][0][lane] = la;
-            s_len[wv][1][lane] = lb;
-            q_lds_sync();
+        uint32_t ia = 0, ib = 0;
+        if (lane < len) {
+            ia = ld_sys(A.ra + phys + lane);
+            ib = ld_sys(A.rb + phys + lane);
         }
-        uint32_t mine = 0;
-        for (uint32_t j = 0; j < len; ++j) {
-            const uint32_t a = s_ab[wv][0][j], b = s_ab[wv][1][j];
-            const uint64_t xa = s_off[wv][0][j], xb = s_off[wv][1][j];
-            const uint32_t ya = s_len[wv][0][j], yb = s_len[wv][1][j];
-            uint32_t d;
-            if (K == 2)
-                d = wpair_distance_at<kServeLds>(n, lab, wdist, a, b, xa, ya, xb, yb, A.ref_compat != 0, sbuf);
-            else
-                d = pair_distance_at<K == 1, kServeLds>(n, bpd, bps, lab, a, b, xa, ya, xb, yb, A.ref_compat != 0,
-                                                        sbuf);
-            if (lane == j) mine = d;
-        }
-        // The next descriptor's writes must not overtake these reads.
-        q_lds_sync();
+        const QPair p = load_pair(lane < len, n, loff, ia, ib);
+        uint32_t mine;
+        if constexpr (K == 2)
+            mine = answer_wpairs(lab, wdist, p, len, A.ref_compat != 0, sbuf);
+        else
+            mine = answer_pairs<K == 1>(bpd, bps, lab, p, len, A.ref_compat != 0, sbuf);
+        if (!p.in)
+            mine = outside_answer(ia, ib, K == 0 ? 255u : K == 1 ? 0xFFFFu : A.ref_compat ? 32767u : 0xFFFFFFFFu);
         if (lane < len) {
             if (K == 0) st_sys(static_cast<uint8_t *>(A.out) + phys + lane, (uint8_t)mine);
             if (K == 1) st_sys(static_cast<uint16_t *>(A.out) + phys + lane, (uint16_t)mine);
@@ -647,12 +695,14 @@ __global__ __launch_bounds__(64) void k_query_pair(uint32_t n, const uint8_t *bp
                                                    const uint64_t *loff, const uint32_t *lab, const uint32_t *wdist,
                                                    uint32_t a, uint32_t b, int ref_compat, uint32_t *out)
 {
-    __shared__ uint32_t sbuf[kQLds];
+    __shared__ alignas(16) uint32_t sbuf[kQBuf];
+    const QPair p = load_pair(threadIdx.x == 0, n, loff, a, b);
     uint32_t d;
-    if (K == 2)
-        d = wpair_distance(n, loff, lab, wdist, a, b, ref_compat != 0, sbuf);
+    if constexpr (K == 2)
+        d = answer_wpairs(lab, wdist, p, 1, ref_compat != 0, sbuf);
     else
-        d = pair_distance<K == 1>(n, bpd, bps, loff, lab, a, b, ref_compat != 0, sbuf);
+        d = answer_pairs<K == 1>(bpd, bps, lab, p, 1, ref_compat != 0, sbuf);
+    if (!p.in) d = outside_answer(a, b, K == 0 ? 255u : K == 1 ? 0xFFFFu : ref_compat ? 32767u : 0xFFFFFFFFu);
     if (threadIdx.x == 0) __hip_atomic_store(out, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -718,6 +768,23 @@ pado_gpu_status launch_query_any(const pado_gpu_index *idx, bool rank_space, con
     return PADO_GPU_OK;
 }
 
+namespace {
+
+// Consecutive pairs per wave: as many as leave each of the chip's 8,192
+// resident waves four chunks, in [4, 64].  A chunk's ids and offsets are two
+// dependent reads before its first pair, so long calls take 64; short ones
+// spread over the chip.
+uint32_t query_chunk(uint64_t k)
+{
+    uint32_t c = kQGroups;
+    while (c < 64 && (uint64_t)c * 2 * 4 * 8192 <= k) c *= 2;
+    return c;
+}
+
+uint32_t query_grid(uint64_t k, uint32_t chunk) { return grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20); }
+
+}  // namespace
+
 pado_gpu_status launch_wquery(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                               uint64_t k, uint32_t *out, bool ref_compat, hipStream_t st)
 {
@@ -725,8 +792,8 @@ pado_gpu_status launch_wquery(const pado_gpu_index *idx, bool rank_space, const 
     const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
     const uint32_t *hub = rank_space ? idx->whub.p : idx->qlab.p;
     const uint32_t *dist = rank_space ? idx->wdist.p : idx->qwdist.p;
-    uint32_t grid = grid_for(k * 64, 256, 65536);
-    hipLaunchKernelGGL(k_wquery, dim3(grid), dim3(256), 0, st, idx->n, loff, hub, dist, qa, qb, k, out,
+    const uint32_t chunk = query_chunk(k), grid = query_grid(k, chunk);
+    hipLaunchKernelGGL(k_wquery, dim3(grid), dim3(256), 0, st, idx->n, loff, hub, dist, qa, qb, k, chunk, out,
                        ref_compat ? 1 : 0);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
@@ -740,9 +807,9 @@ pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const u
     const ulonglong2 *bps = (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p);
     const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
     const uint32_t *lab = rank_space ? idx->lab.p : idx->qlab.p;
-    uint32_t grid = grid_for(k * 64, 256, 65536);
+    const uint32_t chunk = query_chunk(k), grid = query_grid(k, chunk);
     hipLaunchKernelGGL((k_query<false, uint8_t>), dim3(grid), dim3(256), 0, st, idx->n, bpd, bps, loff, lab, qa, qb,
-                       k, out, ref_compat ? 1 : 0);
+                       k, chunk, out, ref_compat ? 1 : 0);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
@@ -757,13 +824,13 @@ pado_gpu_status launch_query_wide(const pado_gpu_index *idx, bool rank_space, co
     const ulonglong2 *bps = (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p);
     const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
     const uint32_t *lab = rank_space ? idx->lab.p : idx->qlab.p;
-    uint32_t grid = grid_for(k * 64, 256, 65536);
+    const uint32_t chunk = query_chunk(k), grid = query_grid(k, chunk);
     if (idx->wide)
         hipLaunchKernelGGL((k_query<true, uint16_t>), dim3(grid), dim3(256), 0, st, idx->n, bpd, bps, loff, lab, qa,
-                           qb, k, out, 0);
+                           qb, k, chunk, out, 0);
     else
         hipLaunchKernelGGL((k_query<false, uint16_t>), dim3(grid), dim3(256), 0, st, idx->n, bpd, bps, loff, lab,
-                           qa, qb, k, out, ref_compat ? 1 : 0);
+                           qa, qb, k, chunk, out, ref_compat ? 1 : 0);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
