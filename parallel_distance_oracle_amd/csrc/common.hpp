@@ -91,6 +91,19 @@ inline std::recursive_mutex &capture_mutex()
     return m;
 }
 
+// The query copy's record of a vertex: everything about it that a query reads
+// but its sets and labels, in one 128-byte line (a weighted index has the
+// last four words only):
+//   bytes   0..63   the distance line (distances, nonempty-set bits)
+//   bytes  64..113  per slot the eight bytes of S^-1 OR-ed into one: two
+//                   vertices' sets can meet only where these bytes do
+//   word  29        component: vertices with different values are in different
+//                   components; 0 throughout an imported index
+//   words 30, 31    first label << 24 | label count
+constexpr uint32_t kQRecWords = 32, kQRecFold = 16, kQRecTail = 28;
+constexpr uint32_t kWRecWords = 4;
+constexpr uint32_t kListAlign = 32;  // label list alignment: one 128-byte line
+
 // Device buffer owned by a handle.  kBufSlack bytes past its end are its own
 // too: a 16-byte read that starts inside it may run over the end (query.hip).
 constexpr size_t kBufSlack = 16;
@@ -241,13 +254,14 @@ struct pado_gpu_index {
     // Weighted labels (hub u32, dist u32), rank space.
     pado::DevBuf<uint32_t> whub;
     pado::DevBuf<uint32_t> wdist;
-    // Query copy in original-id order (order_labels, PARA:2198-2281).
+    // Query copy in original-id order (order_labels, PARA:2198-2281): records
+    // (QRec below), sets, and label lists that start at multiples of
+    // kListAlign entries and are padded to them with all-ones.
     int ordered = 0;
-    pado::DevBuf<uint8_t> qbpd;
+    int built = 0;  // labeled by this library (not imported): components are known
+    pado::DevBuf<uint32_t> qrec;
     pado::DevBuf<uint64_t> qbps;
-    pado::DevBuf<uint64_t> qoff;
-    pado::DevBuf<uint32_t> qlab;
-    pado::DevBuf<uint32_t> qwhub;
+    pado::DevBuf<uint32_t> qlab;  // packed labels, or hubs of a weighted index
     pado::DevBuf<uint32_t> qwdist;
     // Staging for host-pointer queries.
     pado::DevBuf<uint32_t> qa, qb;

@@ -49,30 +49,74 @@ __global__ __launch_bounds__(256) void k_order_counts(uint32_t n, const uint32_t
     uint32_t stride = gridDim.x * blockDim.x;
     for (uint32_t x = blockIdx.x * blockDim.x + threadIdx.x; x < n; x += stride) {
         uint32_t v = rank[x];
-        cnt[x] = (uint32_t)(loff[v + 1] - loff[v]);
+        cnt[x] = ((uint32_t)(loff[v + 1] - loff[v]) + kListAlign - 1) / kListAlign * kListAlign;
     }
 }
 
+// Component of a vertex with label list lab[s, s + L): the lowest slot whose
+// BFS reached it (a BFS covers its root's component), or else the highest
+// vertex of its component, which is every member's first hub (nothing ranks
+// above it to prune it).
+__device__ inline uint32_t component(unsigned long long reached, const uint32_t *lab, uint64_t s, uint32_t L,
+                                     uint32_t hub_shift)
+{
+    if (reached) return (uint32_t)__ffsll(reached);
+    return kBP + 1u + (L ? lab[s] >> hub_shift : 0xFFFFFFu);
+}
+
+// One wave per vertex: its record, sets and padded label list.  slots: which
+// bit-parallel distances tell components (0 in a wide index whose BFS was cut
+// short); known: whether components are to be told at all.
+template <bool WEIGHTED>
 __global__ __launch_bounds__(256) void k_order_copy(uint32_t n, const uint32_t *rank, const uint8_t *bpd,
                                                     const ulonglong2 *bps, const uint64_t *loff, const uint32_t *lab,
-                                                    const uint32_t *wdist, uint8_t *qbpd, ulonglong2 *qbps,
-                                                    const uint64_t *qoff, uint32_t *qlab, uint32_t *qwdist)
+                                                    const uint32_t *wdist, const uint64_t *qoff, int known,
+                                                    unsigned long long slots, uint32_t hub_shift, uint32_t *qrec,
+                                                    ulonglong2 *qbps, uint32_t *qlab, uint32_t *qwdist)
 {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
     for (uint32_t x = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; x < n; x += nw) {
         const uint32_t v = rank[x];
-        if (bpd) {
-            qbpd[(uint64_t)x * kBpdStride + lane] = bpd[(uint64_t)v * kBpdStride + lane];
-            if (lane < kBP) qbps[(uint64_t)x * kBP + lane] = bps[(uint64_t)v * kBP + lane];
-        }
         const uint64_t s = loff[v], dsto = qoff[x];
         const uint32_t L = (uint32_t)(loff[v + 1] - s);
-        for (uint32_t j = lane; j < L; j += 64) {
-            qlab[dsto + j] = lab[s + j];
-            if (wdist) qwdist[dsto + j] = wdist[s + j];
+        uint32_t *rec = qrec + (uint64_t)x * (WEIGHTED ? kWRecWords : kQRecWords);
+        unsigned long long reached = 0;
+        if constexpr (!WEIGHTED) {
+            const uint32_t d = bpd[(uint64_t)v * kBpdStride + lane];
+            reinterpret_cast<uint8_t *>(rec)[lane] = (uint8_t)d;
+            reached = __ballot(lane < kBP && d != kInf8) & slots;
+            unsigned long long f = 0;
+            if (lane < kBP) {
+                const ulonglong2 set = bps[(uint64_t)v * kBP + lane];
+                qbps[(uint64_t)x * kBP + lane] = set;
+                f = set.x | (set.x >> 32);
+                f |= f >> 16;
+                f |= f >> 8;
+            }
+            // (bytes 50 and 51 of the folds are spare)
+            if (lane < kBP + 2) reinterpret_cast<uint8_t *>(rec + kQRecFold)[lane] = (uint8_t)f;
+        }
+        if (lane == 0) {
+            const uint64_t packed = (dsto << 24) | L;
+            uint32_t *tail = rec + (WEIGHTED ? 0 : kQRecTail);
+            if (WEIGHTED) tail[0] = 0u;
+            tail[1] = known ? component(reached, lab, s, L, hub_shift) : 0u;
+            tail[2] = (uint32_t)packed;
+            tail[3] = (uint32_t)(packed >> 32);
+        }
+        const uint32_t P = (L + kListAlign - 1) / kListAlign * kListAlign;
+        for (uint32_t j = lane; j < P; j += 64) {
+            qlab[dsto + j] = j < L ? lab[s + j] : ~0u;
+            if (WEIGHTED) qwdist[dsto + j] = j < L ? wdist[s + j] : ~0u;
         }
     }
+}
+
+__global__ void k_iota(uint32_t n, uint32_t *p)
+{
+    const uint32_t stride = gridDim.x * blockDim.x;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = i;
 }
 
 __global__ void k_pack_labels(uint64_t total, const uint32_t *hub, const uint8_t *dist, uint32_t *lab)
@@ -100,40 +144,53 @@ pado_gpu_status check_ctx(pado_gpu_ctx *ctx)
     return PADO_GPU_OK;
 }
 
-// Builds the original-id query copy from the rank-space index.
+// Builds the original-id query copy from the rank-space index (h_rank null:
+// the index is in original-id order already).
 pado_gpu_status order_index(pado_gpu_index *idx, const uint32_t *h_rank)
 {
     hipStream_t st = idx->ctx->stream;
     const uint32_t n = idx->n;
-    // rank must be a permutation of [0, n).
-    std::vector<uint8_t> seen(n, 0);
-    for (uint32_t x = 0; x < n; ++x) {
-        if (h_rank[x] >= n || seen[h_rank[x]]) {
-            set_error("rank is not a permutation of [0, n)");
-            return PADO_GPU_ERR_ARG;
+    if (h_rank) {
+        // rank must be a permutation of [0, n).
+        std::vector<uint8_t> seen(n, 0);
+        for (uint32_t x = 0; x < n; ++x) {
+            if (h_rank[x] >= n || seen[h_rank[x]]) {
+                set_error("rank is not a permutation of [0, n)");
+                return PADO_GPU_ERR_ARG;
+            }
+            seen[h_rank[x]] = 1;
         }
-        seen[h_rank[x]] = 1;
     }
     DevBuf<uint32_t> rank, cnt;
+    DevBuf<uint64_t> qoff;
     PADO_TRY(rank.alloc(n));
     PADO_TRY(cnt.alloc(n));
-    PADO_HIP(hipMemcpyAsync(rank.p, h_rank, sizeof(uint32_t) * n, hipMemcpyHostToDevice, st));
+    PADO_TRY(qoff.alloc((uint64_t)n + 1));
+    if (h_rank)
+        PADO_HIP(hipMemcpyAsync(rank.p, h_rank, sizeof(uint32_t) * n, hipMemcpyHostToDevice, st));
+    else
+        hipLaunchKernelGGL(k_iota, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, rank.p);
     hipLaunchKernelGGL(k_order_counts, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, rank.p, idx->loff.p, cnt.p);
-    PADO_TRY(idx->qoff.alloc((uint64_t)n + 1));
-    PADO_TRY(scan_u32_to_u64(cnt.p, idx->qoff.p, n, st));
-    const bool w = idx->weighted != 0;
-    if (!w) {
-        PADO_TRY(idx->qbpd.alloc((uint64_t)n * kBpdStride));
-        PADO_TRY(idx->qbps.alloc((uint64_t)n * kBP * 2));
+    PADO_TRY(scan_u32_to_u64(cnt.p, qoff.p, n, st));
+    uint64_t total = 0;
+    PADO_HIP(copy_sync(&total, qoff.p + n, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+    PADO_TRY(idx->qlab.alloc(total));
+    const dim3 grid(grid_for((uint64_t)n * 64, 256, 8192)), block(256);
+    if (idx->weighted) {
+        PADO_TRY(idx->qrec.alloc((uint64_t)n * kWRecWords));
+        PADO_TRY(idx->qwdist.alloc(total));
+        hipLaunchKernelGGL(k_order_copy<true>, grid, block, 0, st, n, rank.p, nullptr, nullptr, idx->loff.p,
+                           idx->whub.p, idx->wdist.p, qoff.p, idx->built, 0ull, 0u, idx->qrec.p, nullptr, idx->qlab.p,
+                           idx->qwdist.p);
     } else {
-        PADO_TRY(idx->qwdist.alloc(idx->num_labels));
+        PADO_TRY(idx->qrec.alloc((uint64_t)n * kQRecWords));
+        PADO_TRY(idx->qbps.alloc((uint64_t)n * kBP * 2));
+        hipLaunchKernelGGL(k_order_copy<false>, grid, block, 0, st, n, rank.p, idx->bpd.p,
+                           (const ulonglong2 *)idx->bps.p, idx->loff.p, idx->lab.p, nullptr, qoff.p, idx->built,
+                           idx->bp_pass_through ? 0ull : ~0ull, idx->wide ? Hop<true>::kBits : Hop<false>::kBits,
+                           idx->qrec.p, (ulonglong2 *)idx->qbps.p, idx->qlab.p, nullptr);
     }
-    PADO_TRY(idx->qlab.alloc(idx->num_labels));
-    hipLaunchKernelGGL(k_order_copy, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, rank.p,
-                       w ? nullptr : idx->bpd.p, w ? nullptr : (const ulonglong2 *)idx->bps.p, idx->loff.p,
-                       w ? idx->whub.p : idx->lab.p, w ? idx->wdist.p : nullptr, w ? nullptr : idx->qbpd.p,
-                       w ? nullptr : (ulonglong2 *)idx->qbps.p, idx->qoff.p, idx->qlab.p,
-                       w ? idx->qwdist.p : nullptr);
+    PADO_HIP(hipGetLastError());
     PADO_HIP(hipStreamSynchronize(st));
     idx->ordered = 1;
     return PADO_GPU_OK;
@@ -371,6 +428,7 @@ pado_gpu_status pado_gpu_build(pado_gpu_ctx *ctx, const pado_gpu_graph *graph, c
         delete idx;
         return s;
     }
+    idx->built = 1;
     *out = idx;
     return PADO_GPU_OK;
 }
@@ -951,18 +1009,19 @@ pado_gpu_status pado_gpu_index_load(pado_gpu_ctx *ctx, const char *filename, pad
         set_error("truncated index file");
         return PADO_GPU_ERR_IO;
     }
-    // The file is in original-id order: import it as-is and mark it ordered.
+    // The file is in original-id order: imported as it is, it gives the query
+    // copy, and there is no rank-space index.
     pado_gpu_index *idx = nullptr;
     PADO_TRY(pado_gpu_index_import(ctx, n, bd.data(), bs.data(), off.data(), hub.data(), dist.data(), &idx));
-    std::swap(idx->qbpd.p, idx->bpd.p);
-    std::swap(idx->qbpd.n, idx->bpd.n);
-    std::swap(idx->qbps.p, idx->bps.p);
-    std::swap(idx->qbps.n, idx->bps.n);
-    std::swap(idx->qoff.p, idx->loff.p);
-    std::swap(idx->qoff.n, idx->loff.n);
-    std::swap(idx->qlab.p, idx->lab.p);
-    std::swap(idx->qlab.n, idx->lab.n);
-    idx->ordered = 1;
+    const pado_gpu_status s = order_index(idx, nullptr);
+    if (s != PADO_GPU_OK) {
+        delete idx;
+        return s;
+    }
+    idx->bpd.release();
+    idx->bps.release();
+    idx->loff.release();
+    idx->lab.release();
     *out = idx;
     return PADO_GPU_OK;
 }
@@ -1068,22 +1127,30 @@ pado_gpu_status pado_gpu_windex_load(pado_gpu_ctx *ctx, const char *filename, pa
     idx->num_labels = hub.size();
     const uint64_t L = hub.size();
     hipStream_t st = ctx->stream;
-    pado_gpu_status s = idx->qoff.alloc((uint64_t)n + 1);
-    if (s == PADO_GPU_OK) s = idx->qlab.alloc(L);
-    if (s == PADO_GPU_OK) s = idx->qwdist.alloc(L);
+    pado_gpu_status s = idx->loff.alloc((uint64_t)n + 1);
+    if (s == PADO_GPU_OK) s = idx->whub.alloc(L);
+    if (s == PADO_GPU_OK) s = idx->wdist.alloc(L);
     if (s != PADO_GPU_OK) {
         delete idx;
         return s;
     }
-    if (hipMemcpyAsync(idx->qoff.p, off.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st) != hipSuccess ||
-        (L && hipMemcpyAsync(idx->qlab.p, hub.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
-        (L && hipMemcpyAsync(idx->qwdist.p, dist.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
+    if (hipMemcpyAsync(idx->loff.p, off.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st) != hipSuccess ||
+        (L && hipMemcpyAsync(idx->whub.p, hub.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
+        (L && hipMemcpyAsync(idx->wdist.p, dist.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
         hipStreamSynchronize(st) != hipSuccess) {
         delete idx;
         set_error("index upload failed");
         return PADO_GPU_ERR_HIP;
     }
-    idx->ordered = 1;
+    // As for the unweighted file: the query copy only.
+    s = order_index(idx, nullptr);
+    if (s != PADO_GPU_OK) {
+        delete idx;
+        return s;
+    }
+    idx->loff.release();
+    idx->whub.release();
+    idx->wdist.release();
     *out = idx;
     return PADO_GPU_OK;
 }

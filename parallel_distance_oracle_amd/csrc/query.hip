@@ -81,11 +81,12 @@ __device__ inline uint32_t group_min(uint32_t x)
     return min(x, row_ror<1>(x));
 }
 
-// The largest of the values that the four lanes r0 .. r0 + 3 hold, as a scalar.
-__device__ inline uint32_t quad_max(uint32_t x, uint32_t r0)
+// The largest of the four groups' values (the same in a group's lanes), as a
+// scalar.
+__device__ inline uint32_t groups_max(uint32_t x)
 {
-    const uint32_t a = __builtin_amdgcn_readlane(x, r0), b = __builtin_amdgcn_readlane(x, r0 + 1);
-    const uint32_t c = __builtin_amdgcn_readlane(x, r0 + 2), d = __builtin_amdgcn_readlane(x, r0 + 3);
+    const uint32_t a = __builtin_amdgcn_readlane(x, 0), b = __builtin_amdgcn_readlane(x, kQLanes);
+    const uint32_t c = __builtin_amdgcn_readlane(x, 2 * kQLanes), d = __builtin_amdgcn_readlane(x, 3 * kQLanes);
     return max(max(a, b), max(c, d));
 }
 
@@ -112,79 +113,149 @@ __device__ inline u32x4 mask4(u32x4 v, uint32_t j, uint32_t len)
 }
 
 // Lower bounds of four keys in a tile of `size` ascending words (a power of
-// two, at least 1): pos[q] = the tile position of the first word >= key[q],
-// or the last position.
+// two up to kQTile): pos[q] = the byte offset of the first word >= key[q], or
+// of the last word.  Three vector instructions and an LDS read a step.
+template <uint32_t H>
+__device__ inline void search_step(const char *tile, uint32_t size, const u32x4 &key, uint32_t (&pos)[4])
+{
+    if (size > H) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t x = *reinterpret_cast<const uint32_t *>(tile + pos[q] + (4 * H - 4));
+            pos[q] = x < key[q] ? pos[q] + 4 * H : pos[q];
+        }
+    }
+    if constexpr (H > 1) search_step<H / 2>(tile, size, key, pos);
+}
+
 __device__ inline void search4(const uint32_t *tile, uint32_t size, const u32x4 &key, uint32_t (&pos)[4])
 {
 #pragma unroll
     for (int q = 0; q < 4; ++q) pos[q] = 0;
-    for (uint32_t half = size >> 1; half; half >>= 1) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) pos[q] += tile[pos[q] + half - 1] < key[q] ? half : 0u;
-    }
+    search_step<kQTile / 2>(reinterpret_cast<const char *>(tile), size, key, pos);
 }
 
-// A lane's pair: ids and the two label lists, the shorter first.  `in` is
-// false for a lane without a pair or with an id past the index.
-struct QPair {
-    uint32_t a, b;
-    uint64_t os, ot;
-    uint32_t ls, lt;
-    bool in;
-};
-
-__device__ inline QPair load_pair(bool has, uint32_t n, const uint64_t *loff, uint32_t a, uint32_t b)
+__device__ inline uint32_t tile_at(const uint32_t *tile, uint32_t pos)
 {
-    QPair p{0, 0, 0, 0, 0, 0, has && a < n && b < n};
-    if (p.in) {
-        const uint64_t oa = loff[a], ob = loff[b];
-        const uint32_t la = (uint32_t)(loff[a + 1] - oa), lb = (uint32_t)(loff[b + 1] - ob);
-        const bool sw = la > lb;
-        p.a = a;
-        p.b = b;
-        p.os = sw ? ob : oa;
-        p.ot = sw ? oa : ob;
-        p.ls = sw ? lb : la;
-        p.lt = sw ? la : lb;
-    }
-    return p;
+    return *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(tile) + pos);
 }
 
-__device__ inline uint64_t shfl64(uint64_t x, uint32_t src)
-{
-    const uint32_t lo = __shfl((uint32_t)x, src), hi = __shfl((uint32_t)(x >> 32), src);
-    return ((uint64_t)hi << 32) | lo;
-}
+// A group's four list entries to its tile.
+__device__ inline void tile_put(uint32_t *tile, uint32_t j, const u32x4 &v) { *reinterpret_cast<u32x4 *>(tile + j) = v; }
 
 // The power of two at or above x (x in [1, kQTile]; 1 for 0).
 __device__ inline uint32_t tile_size(uint32_t x) { return x <= 1u ? 1u : 1u << (32 - __builtin_clz(x - 1u)); }
 
-// Answers the wave's pairs, lane j holding pair j < len: returns lane j's
-// answer.  Hop<false>: the reference's answers (255 for unreachable or >=
-// 253); Hop<true>: exact hops, 0xFFFF for unreachable, using only
-// bit-parallel slots reached on both sides.  sbuf: the wave's kQBuf words.
-template <bool W>
-__device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bps, const uint32_t *lab,
-                                        const QPair &p, uint32_t len, bool ref_compat, uint32_t *sbuf)
+}  // namespace
+
+// What the query kernels read of an index: the ordered copy's records, or the
+// rank-space arrays (rec null).
+struct QIndex {
+    uint32_t n;
+    const uint32_t *rec;
+    const uint8_t *bpd;
+    const ulonglong2 *bps;
+    const uint64_t *loff;
+    const uint32_t *lab;    // packed labels, or a weighted index's hubs
+    const uint32_t *wdist;  // a weighted index's distances
+};
+
+namespace {
+
+// A lane's pair, while it still has to be answered from sets and labels: ids
+// and the two label lists, the shorter first.
+struct alignas(16) QJob {
+    uint32_t a, b;
+    uint32_t ls, lt;  // ls: the lane in the top byte (lists have < 2^24 labels)
+    uint64_t os, ot;
+};
+
+// One wave's LDS.
+struct QBuf {
+    alignas(16) uint32_t tile[kQBuf];
+    QJob job[64];
+    uint32_t ans[64];
+};
+
+// Sorts out the wave's pairs (lane j: pair j if `has`): returns how many are
+// left to answer, in buf.job, and sets ans to the lane's answer if it needs
+// none of that: an id past the index (a == b ? 0 : far), two components (far).
+template <bool REC, uint32_t RECW>
+__device__ inline uint32_t make_jobs(const QIndex &X, bool has, uint32_t a, uint32_t b, uint32_t far, QBuf &buf,
+                                     uint32_t &ans, bool &job)
+{
+    const uint32_t lane = threadIdx.x & 63;
+    ans = a == b ? 0u : far;
+    job = has && a < X.n && b < X.n;
+    uint64_t oa = 0, ob = 0;
+    uint32_t la = 0, lb = 0;
+    if (job) {
+        if constexpr (REC) {
+            const uint4 ta = *reinterpret_cast<const uint4 *>(X.rec + (uint64_t)a * RECW + (RECW - 4));
+            const uint4 tb = *reinterpret_cast<const uint4 *>(X.rec + (uint64_t)b * RECW + (RECW - 4));
+            const uint64_t pa = ((uint64_t)ta.w << 32) | ta.z, pb = ((uint64_t)tb.w << 32) | tb.z;
+            oa = pa >> 24;
+            ob = pb >> 24;
+            la = ta.z & 0xFFFFFFu;
+            lb = tb.z & 0xFFFFFFu;
+            job = ta.y == tb.y;
+            if (!job) ans = far;
+        } else {
+            oa = X.loff[a];
+            ob = X.loff[b];
+            la = (uint32_t)(X.loff[a + 1] - oa);
+            lb = (uint32_t)(X.loff[b + 1] - ob);
+        }
+    }
+    const unsigned long long m = __ballot(job);
+    if (job) {
+        QJob j;
+        const bool sw = la > lb;
+        j.a = a;
+        j.b = b;
+        j.os = sw ? ob : oa;
+        j.ot = sw ? oa : ob;
+        j.ls = (sw ? lb : la) | (lane << 24);
+        j.lt = sw ? la : lb;
+        buf.job[__popcll(m & ((1ull << lane) - 1ull))] = j;
+    }
+    q_lds_sync();
+    return (uint32_t)__popcll(m);
+}
+
+// Answers the jobs four at a time, each job's answer to buf.ans[its lane].
+// Hop<false>: the reference's answers (255 for unreachable or >= 253);
+// Hop<true>: exact hops, 0xFFFF for unreachable, using only bit-parallel slots
+// reached on both sides.
+template <bool W, bool REC>
+__device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_compat, QBuf &buf)
 {
     constexpr uint32_t B = Hop<W>::kBits, MASK = Hop<W>::kInf;
     constexpr uint32_t UNREACHED = W ? 0xFFFFu : 255u;
     const uint32_t lane = threadIdx.x & 63, l = lane & (kQLanes - 1), g = lane / kQLanes;
-    uint32_t *tile = sbuf + g * kQStride;
-    uint32_t mine = UNREACHED;
-    for (uint32_t r0 = 0; r0 < len; r0 += kQGroups) {
-        const uint32_t src = r0 + g;
-        const uint32_t a = __shfl(p.a, src), b = __shfl(p.b, src);
-        const uint32_t ls = __shfl(p.ls, src), lt = __shfl(p.lt, src);
-        const uint32_t *S = lab + shfl64(p.os, src), *T = lab + shfl64(p.ot, src);
-        const uint32_t ms = quad_max(p.ls, r0), mt = quad_max(p.lt, r0);
-        // (a group without a pair reads vertex 0's line and no labels)
-        const uint32_t wa = reinterpret_cast<const uint32_t *>(bpd + (uint64_t)a * kBpdStride)[l];
-        const uint32_t wb = reinterpret_cast<const uint32_t *>(bpd + (uint64_t)b * kBpdStride)[l];
+    uint32_t *tile = buf.tile + g * kQStride;
+    for (uint32_t r0 = 0; r0 < njobs; r0 += kQGroups) {
+        // (a group without a job repeats the first one's)
+        const bool has = r0 + g < njobs;
+        const QJob job = buf.job[has ? r0 + g : r0];
+        const uint32_t ls = job.ls & 0xFFFFFFu, lt = job.lt;
+        const uint32_t *S = X.lab + job.os, *T = X.lab + job.ot;
+        uint32_t wa, wb, fa = 0, fb = 0;
+        if constexpr (REC) {
+            const uint32_t *pa = X.rec + (uint64_t)job.a * kQRecWords + l, *pb = X.rec + (uint64_t)job.b * kQRecWords + l;
+            wa = pa[0];
+            wb = pb[0];
+            fa = pa[kQRecFold];
+            fb = pb[kQRecFold];
+        } else {
+            wa = reinterpret_cast<const uint32_t *>(X.bpd + (uint64_t)job.a * kBpdStride)[l];
+            wb = reinterpret_cast<const uint32_t *>(X.bpd + (uint64_t)job.b * kBpdStride)[l];
+        }
         u32x4 tv[kQPre];
 #pragma unroll
         for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * kQStep + 4 * l, lt);
         const u32x4 s0 = load4(S, 4 * l, ls);
+        const uint32_t ms = groups_max(ls), mt = groups_max(lt);
         // This lane's four slots (the last lanes have none).
         uint32_t td[4];
         {
@@ -204,16 +275,23 @@ __device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bp
                 if (!ok) td[j] = kNoSlot;
             }
         }
-        // Which of this lane's slots have S^-1 sets on both sides (bits of
-        // `both`) and which S^-1 on one and S^0 on the other (`cross`).
+        // Which of this lane's slots can have S^-1 sets that meet (bits of
+        // `both`) and which S^-1 on one side and S^0 on the other (`cross`).
         uint32_t both, cross;
         {
             const uint32_t sh = 8 * ((kBpNzByte + l) & 3u), from = (lane & ~(kQLanes - 1)) + ((kBpNzByte + l) >> 2);
             const uint32_t na = __shfl(wa, from) >> sh, nb = __shfl(wb, from) >> sh;
-            both = na & nb & 15u;
+            if constexpr (REC) {
+                // the bytes of f that are not zero, as four bits
+                const uint32_t f = fa & fb;
+                const uint32_t h = (((f & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | f) & 0x80808080u;
+                both = (h * 0x00204081u) >> 28;
+            } else {
+                both = na & nb & 15u;
+            }
             cross = ((na & (nb >> 4)) | ((na >> 4) & nb)) & 15u;
         }
-        const ulonglong2 *ra = bps + (uint64_t)a * kBP + 4 * l, *rb = bps + (uint64_t)b * kBP + 4 * l;
+        const ulonglong2 *ra = X.bps + (uint64_t)job.a * kBP + 4 * l, *rb = X.bps + (uint64_t)job.b * kBP + 4 * l;
         if (min(min(td[0], td[1]), min(td[2], td[3])) < 2u) {
             // A sum that its sets would take below zero does not count (no
             // such slot in a built index: a root's own sets are empty).
@@ -242,8 +320,8 @@ __device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bp
             cn = en & both;
         }
         // The lane's first set pair is requested before the search.
-        ulonglong2 sa = {0, 0}, sb = {0, 0};
         uint32_t j0 = 0;
+        ulonglong2 sa = {0, 0}, sb = {0, 0};
         const bool first = (cm | cn) != 0u, first_m = cm != 0u;
         if (first) {
             j0 = (uint32_t)__builtin_ctz(first_m ? cm : cn);
@@ -256,15 +334,16 @@ __device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bp
         }
         uint32_t d = m < UNREACHED && m != kNoSlot ? m : UNREACHED;
         for (uint32_t t0 = 0; ms && t0 < mt; t0 += kQTile) {
-            const uint32_t left = min(mt - t0, kQTile), size = tile_size(left);
+            const uint32_t size = tile_size(min(mt - t0, kQTile));
             for (uint32_t u = 0; u * kQStep < size; ++u) {
                 const uint32_t j = t0 + u * kQStep + 4 * l;
                 const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
-                *reinterpret_cast<u32x4 *>(tile + u * kQStep + 4 * l) = mask4(v, j, lt);
+                tile_put(tile, u * kQStep + 4 * l, REC ? v : mask4(v, j, lt));
             }
             q_lds_sync();
             for (uint32_t i = 0; i < ms; i += kQStep) {
-                const u32x4 s = mask4(i == 0 ? s0 : load4(S, i + 4 * l, ls), i + 4 * l, ls);
+                const u32x4 v = i == 0 ? s0 : load4(S, i + 4 * l, ls);
+                const u32x4 s = REC ? v : mask4(v, i + 4 * l, ls);
                 // A packed label with the same hub is >= the hub with
                 // distance 0, so whole words compare as hubs do.
                 const u32x4 key = s & ~MASK;
@@ -272,13 +351,18 @@ __device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bp
                 search4(tile, size, key, pos);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const uint32_t x = tile[pos[q]];
-                    if ((x ^ s[q]) >> B == 0u && s[q] != ~0u) d = min(d, (x & MASK) + (s[q] & MASK));
+                    // x - key is the other distance if the hubs are equal,
+                    // else at least MASK + 1: a u8 answer it does not lower,
+                    // and neither do two entries past their lists (all-ones).
+                    const uint32_t u = tile_at(tile, pos[q]) - key[q];
+                    const uint32_t sum = __builtin_elementwise_add_sat(u, s[q] & MASK);
+                    d = min(d, W && u > MASK ? UNREACHED : sum);
                 }
             }
             // The next copy must not overtake these reads.
             q_lds_sync();
         }
+        if (W && d >= 2 * MASK) d = UNREACHED;
         d = group_min(d);
         if (first) {
             if (sa.x & sb.x)
@@ -304,10 +388,9 @@ __device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bp
         }
         d = group_min(d);
         if (!W && d >= 253u) d = 255u;
-        const uint32_t back = __shfl(d, (lane & (kQGroups - 1)) * kQLanes);
-        if (lane / kQGroups == r0 / kQGroups && p.in) mine = back;
+        if (has && l == 0) buf.ans[job.ls >> 24] = d;
     }
-    return mine;
+    q_lds_sync();
 }
 
 // Weighted query_distance (WPARA:2125-2243): min over common hubs of
@@ -316,99 +399,95 @@ __device__ inline uint32_t answer_pairs(const uint8_t *bpd, const ulonglong2 *bp
 // range -> a == b ? 0 : 32767).  As answer_pairs, on the hub lists;
 // distances of the shorter list come in with its hubs, those of the longer
 // list are read where a hub matches.
-__device__ inline uint32_t answer_wpairs(const uint32_t *hub, const uint32_t *dist, const QPair &p, uint32_t len,
-                                         bool ref_compat, uint32_t *sbuf)
+template <bool REC>
+__device__ inline void answer_wjobs(const QIndex &X, uint32_t njobs, bool ref_compat, QBuf &buf)
 {
     const uint32_t lane = threadIdx.x & 63, l = lane & (kQLanes - 1), g = lane / kQLanes;
-    uint32_t *tile = sbuf + g * kQStride;
-    uint32_t mine = 0xFFFFFFFFu;
-    for (uint32_t r0 = 0; r0 < len; r0 += kQGroups) {
-        const uint32_t src = r0 + g;
-        const uint32_t ls = __shfl(p.ls, src), lt = __shfl(p.lt, src);
-        const uint64_t os = shfl64(p.os, src), ot = shfl64(p.ot, src);
-        const uint32_t ms = quad_max(p.ls, r0), mt = quad_max(p.lt, r0);
+    uint32_t *tile = buf.tile + g * kQStride;
+    for (uint32_t r0 = 0; r0 < njobs; r0 += kQGroups) {
+        const bool has = r0 + g < njobs;
+        const QJob job = buf.job[has ? r0 + g : r0];
+        const uint32_t ls = job.ls & 0xFFFFFFu, lt = job.lt;
+        const uint32_t *S = X.lab + job.os, *T = X.lab + job.ot;
+        const uint32_t *DS = X.wdist + job.os, *DT = X.wdist + job.ot;
         u32x4 tv[kQPre];
 #pragma unroll
-        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(hub + ot, u * kQStep + 4 * l, lt);
-        const u32x4 s0 = load4(hub + os, 4 * l, ls), d0 = load4(dist + os, 4 * l, ls);
+        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * kQStep + 4 * l, lt);
+        const u32x4 s0 = load4(S, 4 * l, ls), d0 = load4(DS, 4 * l, ls);
+        const uint32_t ms = groups_max(ls), mt = groups_max(lt);
         uint32_t d = 0xFFFFFFFFu;
         for (uint32_t t0 = 0; ms && t0 < mt; t0 += kQTile) {
-            const uint32_t left = min(mt - t0, kQTile), size = tile_size(left);
+            const uint32_t size = tile_size(min(mt - t0, kQTile));
             for (uint32_t u = 0; u * kQStep < size; ++u) {
                 const uint32_t j = t0 + u * kQStep + 4 * l;
-                const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(hub + ot, j, lt);
-                *reinterpret_cast<u32x4 *>(tile + u * kQStep + 4 * l) = mask4(v, j, lt);
+                const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
+                tile_put(tile, u * kQStep + 4 * l, REC ? v : mask4(v, j, lt));
             }
             q_lds_sync();
             for (uint32_t i = 0; i < ms; i += kQStep) {
-                const u32x4 s = mask4(i == 0 ? s0 : load4(hub + os, i + 4 * l, ls), i + 4 * l, ls);
-                const u32x4 e = i == 0 ? d0 : load4(dist + os, i + 4 * l, ls);
+                const u32x4 v = i == 0 ? s0 : load4(S, i + 4 * l, ls);
+                const u32x4 s = REC ? v : mask4(v, i + 4 * l, ls);
+                const u32x4 e = i == 0 ? d0 : load4(DS, i + 4 * l, ls);
                 uint32_t pos[4], x[4];
                 search4(tile, size, s, pos);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     x[q] = 0xFFFFFFFFu;
-                    if (tile[pos[q]] == s[q] && s[q] != ~0u) x[q] = dist[ot + t0 + pos[q]];
+                    if (tile_at(tile, pos[q]) == s[q] && s[q] != ~0u) x[q] = DT[t0 + pos[q] / 4];
                 }
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t td = x[q] + e[q];
-                    if (x[q] != 0xFFFFFFFFu && td >= e[q]) d = min(d, td);  // (a sum past 2^32 lowers nothing)
-                }
+                for (int q = 0; q < 4; ++q)  // (no hub, or a sum past 2^32: all-ones, which lowers nothing)
+                    d = min(d, __builtin_elementwise_add_sat(x[q], e[q]));
             }
             q_lds_sync();
         }
         d = group_min(d);
         if (ref_compat && d >= 32765u) d = 32767u;
-        const uint32_t back = __shfl(d, (lane & (kQGroups - 1)) * kQLanes);
-        if (lane / kQGroups == r0 / kQGroups && p.in) mine = back;
+        if (has && l == 0) buf.ans[job.ls >> 24] = d;
     }
-    return mine;
+    q_lds_sync();
 }
 
-// The answer of a pair with an id past the index.
-__device__ inline uint32_t outside_answer(uint32_t a, uint32_t b, uint32_t far) { return a == b ? 0u : far; }
+// Kinds of index: u8 hops, the wide hop domain, weighted.
+enum { kHops = 0, kWideHops = 1, kWeights = 2 };
+
+// Answers the wave's pairs, lane j holding pair j if `has`; returns the lane's
+// answer.
+template <int K, bool REC>
+__device__ inline uint32_t answer_pairs(const QIndex &X, bool has, uint32_t a, uint32_t b, bool ref_compat, QBuf &buf)
+{
+    const uint32_t far = K == kHops ? 255u : K == kWideHops ? 0xFFFFu : ref_compat ? 32767u : 0xFFFFFFFFu;
+    uint32_t ans;
+    bool job;
+    const uint32_t njobs = make_jobs<REC, K == kWeights ? kWRecWords : kQRecWords>(X, has, a, b, far, buf, ans, job);
+    if constexpr (K == kWeights)
+        answer_wjobs<REC>(X, njobs, ref_compat, buf);
+    else
+        answer_jobs<K == kWideHops, REC>(X, njobs, ref_compat, buf);
+    return job ? buf.ans[threadIdx.x & 63] : ans;
+}
 
 }  // namespace
 
 // Batch queries: a wave takes `chunk` consecutive pairs at a time (see
-// query_chunk).  OT: the answer type (u8, or u16 for a wide index or widened
+// query_chunk).  OT: the answer type (u16 for a wide index or widened
 // answers).
-template <bool W, class OT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                               const uint64_t *loff, const uint32_t *lab, const uint32_t *qa,
+template <int K, bool REC, class OT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query(QIndex X, const uint32_t *qa,
                                                const uint32_t *qb, uint64_t k, uint32_t chunk, OT *out,
                                                int ref_compat)
 {
-    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
+    __shared__ QBuf s_q[kQWaves];
     const uint32_t lane = threadIdx.x & 63;
     const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
     const uint64_t w = uniform64(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     for (uint64_t c0 = w * chunk; c0 < k; c0 += nw * chunk) {
-        const uint32_t len = (uint32_t)min((uint64_t)chunk, k - c0);
-        const bool has = lane < len;
+        const bool has = lane < chunk && c0 + lane < k;
         const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const QPair p = load_pair(has, n, loff, a, b);
-        const uint32_t d = answer_pairs<W>(bpd, bps, lab, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
-        if (has) out[c0 + lane] = (OT)(p.in ? d : outside_answer(a, b, W ? 0xFFFFu : 255u));
-    }
-}
-
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_wquery(uint32_t n, const uint64_t *loff, const uint32_t *hub,
-                                                const uint32_t *dist, const uint32_t *qa, const uint32_t *qb,
-                                                uint64_t k, uint32_t chunk, uint32_t *out, int ref_compat)
-{
-    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    const uint64_t w = uniform64(((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    for (uint64_t c0 = w * chunk; c0 < k; c0 += nw * chunk) {
-        const uint32_t len = (uint32_t)min((uint64_t)chunk, k - c0);
-        const bool has = lane < len;
-        const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const QPair p = load_pair(has, n, loff, a, b);
-        const uint32_t d = answer_wpairs(hub, dist, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
-        if (has) out[c0 + lane] = p.in ? d : outside_answer(a, b, ref_compat ? 32767u : 0xFFFFFFFFu);
+        const uint32_t d = answer_pairs<K, REC>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        if (has) out[c0 + lane] = (OT)d;
+        // The next chunk's jobs and answers must not overtake these reads.
+        q_lds_sync();
     }
 }
 
@@ -419,45 +498,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
 // once the counter passes k.
 constexpr uint32_t kGrab = 16;
 
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query_ws(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                                  const uint64_t *loff, const uint32_t *lab, const uint32_t *qa,
-                                                  const uint32_t *qb, uint64_t k, uint8_t *out, int ref_compat,
+template <int K, class OT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query_ws(QIndex X, const uint32_t *qa,
+                                                  const uint32_t *qb, uint64_t k, OT *out, int ref_compat,
                                                   unsigned long long *work)
 {
-    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
+    __shared__ QBuf s_q[kQWaves];
     const uint32_t lane = threadIdx.x & 63;
     for (;;) {
         unsigned long long c0 = 0;
         if (lane == 0) c0 = atomicAdd(work, (unsigned long long)kGrab);
         c0 = uniform64(c0);
         if (c0 >= k) break;
-        const uint32_t len = (uint32_t)min((uint64_t)kGrab, k - c0);
-        const bool has = lane < len;
+        const bool has = lane < kGrab && c0 + lane < k;
         const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const QPair p = load_pair(has, n, loff, a, b);
-        const uint32_t d = answer_pairs<false>(bpd, bps, lab, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
-        if (has) out[c0 + lane] = (uint8_t)(p.in ? d : outside_answer(a, b, 255u));
-    }
-}
-
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_wquery_ws(uint32_t n, const uint64_t *loff, const uint32_t *hub,
-                                                   const uint32_t *dist, const uint32_t *qa, const uint32_t *qb,
-                                                   uint64_t k, uint32_t *out, int ref_compat,
-                                                   unsigned long long *work)
-{
-    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
-    const uint32_t lane = threadIdx.x & 63;
-    for (;;) {
-        unsigned long long c0 = 0;
-        if (lane == 0) c0 = atomicAdd(work, (unsigned long long)kGrab);
-        c0 = uniform64(c0);
-        if (c0 >= k) break;
-        const uint32_t len = (uint32_t)min((uint64_t)kGrab, k - c0);
-        const bool has = lane < len;
-        const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const QPair p = load_pair(has, n, loff, a, b);
-        const uint32_t d = answer_wpairs(hub, dist, p, len, ref_compat != 0, s_q[threadIdx.x >> 6]);
-        if (has) out[c0 + lane] = p.in ? d : outside_answer(a, b, ref_compat ? 32767u : 0xFFFFFFFFu);
+        const uint32_t d = answer_pairs<K, true>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        if (has) out[c0 + lane] = (OT)d;
+        q_lds_sync();
     }
 }
 
@@ -469,8 +526,8 @@ __global__ void k_zero_work(unsigned long long *work) { *work = 0ull; }
 uint32_t query_ws_blocks_per_cu(bool weighted)
 {
     int nb = 0;
-    const hipError_t e = weighted ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_wquery_ws, 256, 0)
-                                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws, 256, 0);
+    const hipError_t e = weighted ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws<kWeights, uint32_t>, 256, 0)
+                                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws<kHops, uint8_t>, 256, 0);
     return (e == hipSuccess && nb > 0) ? (uint32_t)nb : 4u;
 }
 
@@ -567,19 +624,15 @@ __device__ void serve_poll(const ServeKernelArgs &A)
     }
 }
 
-// K: 0 = u8 hop answers, 1 = wide index (u16 exact hops), 2 = weighted (u32).
 template <int K>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_serve(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                               const uint64_t *loff, const uint32_t *lab, const uint32_t *wdist,
-                                               ServeKernelArgs A)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_serve(QIndex X, ServeKernelArgs A)
 {
-    __shared__ alignas(16) uint32_t s_q[kQWaves][kQBuf];
+    __shared__ QBuf s_q[kQWaves];
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (blockIdx.x == 0 && wv == 0) {
         serve_poll(A);
         return;
     }
-    uint32_t *sbuf = s_q[wv];
     unsigned long long *S = A.state;
     const uint32_t q = blockIdx.x % kServeQueues;
     for (;;) {
@@ -613,18 +666,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
             ia = ld_sys(A.ra + phys + lane);
             ib = ld_sys(A.rb + phys + lane);
         }
-        const QPair p = load_pair(lane < len, n, loff, ia, ib);
-        uint32_t mine;
-        if constexpr (K == 2)
-            mine = answer_wpairs(lab, wdist, p, len, A.ref_compat != 0, sbuf);
-        else
-            mine = answer_pairs<K == 1>(bpd, bps, lab, p, len, A.ref_compat != 0, sbuf);
-        if (!p.in)
-            mine = outside_answer(ia, ib, K == 0 ? 255u : K == 1 ? 0xFFFFu : A.ref_compat ? 32767u : 0xFFFFFFFFu);
+        const uint32_t mine = answer_pairs<K, true>(X, lane < len, ia, ib, A.ref_compat != 0, s_q[wv]);
+        // The next descriptor's writes must not overtake these reads.
+        q_lds_sync();
         if (lane < len) {
-            if (K == 0) st_sys(static_cast<uint8_t *>(A.out) + phys + lane, (uint8_t)mine);
-            if (K == 1) st_sys(static_cast<uint16_t *>(A.out) + phys + lane, (uint16_t)mine);
-            if (K == 2) st_sys(static_cast<uint32_t *>(A.out) + phys + lane, mine);
+            if (K == kHops) st_sys(static_cast<uint8_t *>(A.out) + phys + lane, (uint8_t)mine);
+            if (K == kWideHops) st_sys(static_cast<uint16_t *>(A.out) + phys + lane, (uint16_t)mine);
+            if (K == kWeights) st_sys(static_cast<uint32_t *>(A.out) + phys + lane, mine);
         }
         // The answers have reached host memory before this wave's count
         // moves (the stores write through to the host; waiting for them is
@@ -662,108 +710,79 @@ uint32_t serve_resident_blocks_per_cu(const pado_gpu_index *idx)
     int nb = 0;
     hipError_t e;
     if (idx->weighted)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_serve<2>, 256, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_serve<kWeights>, 256, 0);
     else if (idx->wide)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_serve<1>, 256, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_serve<kWideHops>, 256, 0);
     else
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_serve<0>, 256, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_serve<kHops>, 256, 0);
     return (e == hipSuccess && nb > 0) ? (uint32_t)nb : 4u;
+}
+
+// The ordered copy of an index (or its rank-space arrays).
+static QIndex query_index(const pado_gpu_index *idx, bool rank_space)
+{
+    QIndex X{};
+    X.n = idx->n;
+    if (rank_space) {
+        X.bpd = idx->bpd.p;
+        X.bps = (const ulonglong2 *)idx->bps.p;
+        X.loff = idx->loff.p;
+        X.lab = idx->weighted ? idx->whub.p : idx->lab.p;
+        X.wdist = idx->wdist.p;
+    } else {
+        X.rec = idx->qrec.p;
+        X.bps = (const ulonglong2 *)idx->qbps.p;
+        X.lab = idx->qlab.p;
+        X.wdist = idx->qwdist.p;
+    }
+    return X;
 }
 
 pado_gpu_status launch_serve_resident(const pado_gpu_index *idx, const ServeKernelArgs &a, uint32_t blocks,
                                       hipStream_t st)
 {
+    const QIndex X = query_index(idx, false);
     hipLaunchKernelGGL(k_serve_reset, dim3(1), dim3(64), 0, st, a.state);
     if (idx->weighted)
-        hipLaunchKernelGGL(k_serve<2>, dim3(blocks), dim3(256), 0, st, idx->n, nullptr, nullptr, idx->qoff.p,
-                           idx->qlab.p, idx->qwdist.p, a);
+        hipLaunchKernelGGL(k_serve<kWeights>, dim3(blocks), dim3(256), 0, st, X, a);
     else if (idx->wide)
-        hipLaunchKernelGGL(k_serve<1>, dim3(blocks), dim3(256), 0, st, idx->n, idx->qbpd.p,
-                           (const ulonglong2 *)idx->qbps.p, idx->qoff.p, idx->qlab.p, nullptr, a);
+        hipLaunchKernelGGL(k_serve<kWideHops>, dim3(blocks), dim3(256), 0, st, X, a);
     else
-        hipLaunchKernelGGL(k_serve<0>, dim3(blocks), dim3(256), 0, st, idx->n, idx->qbpd.p,
-                           (const ulonglong2 *)idx->qbps.p, idx->qoff.p, idx->qlab.p, nullptr, a);
+        hipLaunchKernelGGL(k_serve<kHops>, dim3(blocks), dim3(256), 0, st, X, a);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
 
 // One pair, ids passed by value, the answer written into mapped host memory
 // with a system-scope store: a lone query costs one launch and one stream
-// synchronisation, no copies (K: 0 u8 hops, 1 wide, 2 weighted).
-template <int K>
-__global__ __launch_bounds__(64) void k_query_pair(uint32_t n, const uint8_t *bpd, const ulonglong2 *bps,
-                                                   const uint64_t *loff, const uint32_t *lab, const uint32_t *wdist,
-                                                   uint32_t a, uint32_t b, int ref_compat, uint32_t *out)
+// synchronisation, no copies.
+template <int K, bool REC>
+__global__ __launch_bounds__(64) void k_query_pair(QIndex X, uint32_t a, uint32_t b, int ref_compat, uint32_t *out)
 {
-    __shared__ alignas(16) uint32_t sbuf[kQBuf];
-    const QPair p = load_pair(threadIdx.x == 0, n, loff, a, b);
-    uint32_t d;
-    if constexpr (K == 2)
-        d = answer_wpairs(lab, wdist, p, 1, ref_compat != 0, sbuf);
-    else
-        d = answer_pairs<K == 1>(bpd, bps, lab, p, 1, ref_compat != 0, sbuf);
-    if (!p.in) d = outside_answer(a, b, K == 0 ? 255u : K == 1 ? 0xFFFFu : ref_compat ? 32767u : 0xFFFFFFFFu);
+    __shared__ QBuf buf;
+    const uint32_t d = answer_pairs<K, REC>(X, threadIdx.x == 0, a, b, ref_compat != 0, buf);
     if (threadIdx.x == 0) __hip_atomic_store(out, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+template <int K>
+static void launch_pair(const QIndex &X, uint32_t a, uint32_t b, bool ref, uint32_t *out_dev, hipStream_t st)
+{
+    if (X.rec)
+        hipLaunchKernelGGL((k_query_pair<K, true>), dim3(1), dim3(64), 0, st, X, a, b, ref ? 1 : 0, out_dev);
+    else
+        hipLaunchKernelGGL((k_query_pair<K, false>), dim3(1), dim3(64), 0, st, X, a, b, ref ? 1 : 0, out_dev);
 }
 
 pado_gpu_status launch_query_pair(const pado_gpu_index *idx, bool rank_space, uint32_t a, uint32_t b,
                                   bool ref_compat, uint32_t *out_dev, hipStream_t st)
 {
-    const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
+    const QIndex X = query_index(idx, rank_space);
     if (idx->weighted)
-        hipLaunchKernelGGL(k_query_pair<2>, dim3(1), dim3(64), 0, st, idx->n, nullptr, nullptr, loff,
-                           rank_space ? idx->whub.p : idx->qlab.p, rank_space ? idx->wdist.p : idx->qwdist.p, a, b,
-                           ref_compat ? 1 : 0, out_dev);
+        launch_pair<kWeights>(X, a, b, ref_compat, out_dev, st);
     else if (idx->wide)
-        hipLaunchKernelGGL(k_query_pair<1>, dim3(1), dim3(64), 0, st, idx->n, rank_space ? idx->bpd.p : idx->qbpd.p,
-                           (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p), loff,
-                           rank_space ? idx->lab.p : idx->qlab.p, nullptr, a, b, 0, out_dev);
+        launch_pair<kWideHops>(X, a, b, false, out_dev, st);
     else
-        hipLaunchKernelGGL(k_query_pair<0>, dim3(1), dim3(64), 0, st, idx->n, rank_space ? idx->bpd.p : idx->qbpd.p,
-                           (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p), loff,
-                           rank_space ? idx->lab.p : idx->qlab.p, nullptr, a, b, ref_compat ? 1 : 0, out_dev);
-    PADO_HIP(hipGetLastError());
-    return PADO_GPU_OK;
-}
-
-pado_gpu_status launch_wquery(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
-                              uint64_t k, uint32_t *out, bool ref_compat, hipStream_t st);
-pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
-                             uint64_t k, uint8_t *out, bool ref_compat, hipStream_t st);
-pado_gpu_status launch_query_wide(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
-                                  uint64_t k, uint16_t *out, bool ref_compat, hipStream_t st);
-
-// Query launch on device pairs for either index type: out holds u8
-// (unweighted) or u32 (weighted) answers.  work == nullptr selects the plain
-// grid-stride kernel; otherwise the persistent kernel with `blocks`
-// workgroups, its counter cleared on the same stream first.
-pado_gpu_status launch_query_any(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
-                                 uint64_t k, void *out, bool ref_compat, hipStream_t st,
-                                 unsigned long long *work, uint32_t blocks)
-{
-    if (k == 0) return PADO_GPU_OK;
-    const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
-    // A wide index always takes the grid-stride kernel (u16 answers).
-    if (idx->wide) return launch_query_wide(idx, rank_space, qa, qb, k, (uint16_t *)out, false, st);
-    if (!work) {
-        if (idx->weighted) return launch_wquery(idx, rank_space, qa, qb, k, (uint32_t *)out, ref_compat, st);
-        return launch_query(idx, rank_space, qa, qb, k, (uint8_t *)out, ref_compat, st);
-    }
-    const uint64_t need = (k + kGrab - 1) / kGrab;  // grabs; one wave per grab at most
-    uint32_t grid = blocks;
-    if ((uint64_t)grid * 4 > need) grid = (uint32_t)((need + 3) / 4);
-    if (grid == 0) grid = 1;
-    hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(1), 0, st, work);
-    if (idx->weighted) {
-        hipLaunchKernelGGL(k_wquery_ws, dim3(grid), dim3(256), 0, st, idx->n, loff,
-                           rank_space ? idx->whub.p : idx->qlab.p, rank_space ? idx->wdist.p : idx->qwdist.p, qa, qb,
-                           k, (uint32_t *)out, ref_compat ? 1 : 0, work);
-    } else {
-        hipLaunchKernelGGL(k_query_ws, dim3(grid), dim3(256), 0, st, idx->n, rank_space ? idx->bpd.p : idx->qbpd.p,
-                           (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p), loff,
-                           rank_space ? idx->lab.p : idx->qlab.p, qa, qb, k, (uint8_t *)out, ref_compat ? 1 : 0,
-                           work);
-    }
+        launch_pair<kHops>(X, a, b, ref_compat, out_dev, st);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
@@ -771,7 +790,7 @@ pado_gpu_status launch_query_any(const pado_gpu_index *idx, bool rank_space, con
 namespace {
 
 // Consecutive pairs per wave: as many as leave each of the chip's 8,192
-// resident waves four chunks, in [4, 64].  A chunk's ids and offsets are two
+// resident waves four chunks, in [4, 64].  A chunk's ids and records are two
 // dependent reads before its first pair, so long calls take 64; short ones
 // spread over the chip.
 uint32_t query_chunk(uint64_t k)
@@ -781,37 +800,33 @@ uint32_t query_chunk(uint64_t k)
     return c;
 }
 
-uint32_t query_grid(uint64_t k, uint32_t chunk) { return grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20); }
+template <int K, class OT>
+pado_gpu_status launch_batch(const QIndex &X, const uint32_t *qa, const uint32_t *qb, uint64_t k, OT *out, bool ref,
+                             hipStream_t st)
+{
+    if (k == 0) return PADO_GPU_OK;
+    const uint32_t chunk = query_chunk(k), grid = grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20);
+    if (X.rec)
+        hipLaunchKernelGGL((k_query<K, true, OT>), dim3(grid), dim3(256), 0, st, X, qa, qb, k, chunk, out, ref ? 1 : 0);
+    else
+        hipLaunchKernelGGL((k_query<K, false, OT>), dim3(grid), dim3(256), 0, st, X, qa, qb, k, chunk, out,
+                           ref ? 1 : 0);
+    PADO_HIP(hipGetLastError());
+    return PADO_GPU_OK;
+}
 
 }  // namespace
 
 pado_gpu_status launch_wquery(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                               uint64_t k, uint32_t *out, bool ref_compat, hipStream_t st)
 {
-    if (k == 0) return PADO_GPU_OK;
-    const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
-    const uint32_t *hub = rank_space ? idx->whub.p : idx->qlab.p;
-    const uint32_t *dist = rank_space ? idx->wdist.p : idx->qwdist.p;
-    const uint32_t chunk = query_chunk(k), grid = query_grid(k, chunk);
-    hipLaunchKernelGGL(k_wquery, dim3(grid), dim3(256), 0, st, idx->n, loff, hub, dist, qa, qb, k, chunk, out,
-                       ref_compat ? 1 : 0);
-    PADO_HIP(hipGetLastError());
-    return PADO_GPU_OK;
+    return launch_batch<kWeights>(query_index(idx, rank_space), qa, qb, k, out, ref_compat, st);
 }
 
 pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                              uint64_t k, uint8_t *out, bool ref_compat, hipStream_t st)
 {
-    if (k == 0) return PADO_GPU_OK;
-    const uint8_t *bpd = rank_space ? idx->bpd.p : idx->qbpd.p;
-    const ulonglong2 *bps = (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p);
-    const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
-    const uint32_t *lab = rank_space ? idx->lab.p : idx->qlab.p;
-    const uint32_t chunk = query_chunk(k), grid = query_grid(k, chunk);
-    hipLaunchKernelGGL((k_query<false, uint8_t>), dim3(grid), dim3(256), 0, st, idx->n, bpd, bps, loff, lab, qa, qb,
-                       k, chunk, out, ref_compat ? 1 : 0);
-    PADO_HIP(hipGetLastError());
-    return PADO_GPU_OK;
+    return launch_batch<kHops>(query_index(idx, rank_space), qa, qb, k, out, ref_compat, st);
 }
 
 // u16 answers on device pairs: exact hops for a wide index, the reference's
@@ -819,18 +834,37 @@ pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const u
 pado_gpu_status launch_query_wide(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                                   uint64_t k, uint16_t *out, bool ref_compat, hipStream_t st)
 {
+    const QIndex X = query_index(idx, rank_space);
+    if (idx->wide) return launch_batch<kWideHops>(X, qa, qb, k, out, false, st);
+    return launch_batch<kHops>(X, qa, qb, k, out, ref_compat, st);
+}
+
+// Query launch on device pairs for either index type, ordered ids: out holds
+// u8, u16 (wide) or u32 (weighted) answers.  work == nullptr selects the batch
+// kernel; otherwise the persistent kernel with `blocks` workgroups, its
+// counter cleared on the same stream first (a wide index always takes the
+// batch kernel).
+pado_gpu_status launch_query_any(const pado_gpu_index *idx, const uint32_t *qa, const uint32_t *qb, uint64_t k,
+                                 void *out, bool ref_compat, hipStream_t st, unsigned long long *work, uint32_t blocks)
+{
     if (k == 0) return PADO_GPU_OK;
-    const uint8_t *bpd = rank_space ? idx->bpd.p : idx->qbpd.p;
-    const ulonglong2 *bps = (const ulonglong2 *)(rank_space ? idx->bps.p : idx->qbps.p);
-    const uint64_t *loff = rank_space ? idx->loff.p : idx->qoff.p;
-    const uint32_t *lab = rank_space ? idx->lab.p : idx->qlab.p;
-    const uint32_t chunk = query_chunk(k), grid = query_grid(k, chunk);
-    if (idx->wide)
-        hipLaunchKernelGGL((k_query<true, uint16_t>), dim3(grid), dim3(256), 0, st, idx->n, bpd, bps, loff, lab, qa,
-                           qb, k, chunk, out, 0);
+    if (idx->wide) return launch_query_wide(idx, false, qa, qb, k, (uint16_t *)out, false, st);
+    if (!work) {
+        if (idx->weighted) return launch_wquery(idx, false, qa, qb, k, (uint32_t *)out, ref_compat, st);
+        return launch_query(idx, false, qa, qb, k, (uint8_t *)out, ref_compat, st);
+    }
+    const uint64_t need = (k + kGrab - 1) / kGrab;  // grabs; one wave per grab at most
+    uint32_t grid = blocks;
+    if ((uint64_t)grid * 4 > need) grid = (uint32_t)((need + 3) / 4);
+    if (grid == 0) grid = 1;
+    const QIndex X = query_index(idx, false);
+    hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(1), 0, st, work);
+    if (idx->weighted)
+        hipLaunchKernelGGL((k_query_ws<kWeights, uint32_t>), dim3(grid), dim3(256), 0, st, X, qa, qb, k,
+                           (uint32_t *)out, ref_compat ? 1 : 0, work);
     else
-        hipLaunchKernelGGL((k_query<false, uint16_t>), dim3(grid), dim3(256), 0, st, idx->n, bpd, bps, loff, lab,
-                           qa, qb, k, chunk, out, ref_compat ? 1 : 0);
+        hipLaunchKernelGGL((k_query_ws<kHops, uint8_t>), dim3(grid), dim3(256), 0, st, X, qa, qb, k, (uint8_t *)out,
+                           ref_compat ? 1 : 0, work);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }

@@ -26,9 +26,9 @@
 #include "internal.hpp"
 
 namespace pado {
-pado_gpu_status launch_query_any(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
-                                 uint64_t k, void *out, bool ref_compat, hipStream_t st,
-                                 unsigned long long *work, uint32_t blocks);
+pado_gpu_status launch_query_any(const pado_gpu_index *idx, const uint32_t *qa, const uint32_t *qb, uint64_t k,
+                                 void *out, bool ref_compat, hipStream_t st, unsigned long long *work,
+                                 uint32_t blocks);
 uint32_t query_ws_blocks_per_cu(bool weighted);
 }
 
@@ -246,7 +246,7 @@ void dispatcher_loop(pado_gpu_server *s)
             hipLaunchKernelGGL(k_stage_pairs, dim3(sgrid), dim3(256), 0, st, s->m_a + phys, s->m_b + phys,
                                s->d_a.p + phys, s->d_b.p + phys, k);
             const bool grid_stride = (s->cfg.flags & PADO_GPU_SERVE_PERSISTENT) == 0;
-            pado_gpu_status qs = launch_query_any(s->idx, false, s->d_a.p + phys, s->d_b.p + phys, k,
+            pado_gpu_status qs = launch_query_any(s->idx, s->d_a.p + phys, s->d_b.p + phys, k,
                                                   s->d_out.p + phys * s->es,
                                                   (s->cfg.flags & PADO_GPU_QUERY_REF_COMPAT) != 0, st,
                                                   grid_stride ? nullptr : s->work.p + si, s->ws_blocks);
