@@ -13,27 +13,36 @@
 // reproduces the reference's answers bit for bit.  Either way the slot order
 // does not matter: the result is a minimum over slots.
 //
-// Mapping: four pairs per wave, sixteen lanes (one DPP row) each; a wave
-// holds up to 64 consecutive pairs (lane j: pair j's ids and label offsets,
-// loaded together) and answers them four at a time.
+// Mapping: a wave takes up to 64 consecutive pairs.  Lane j reads pair j's ids
+// and the tails of their records (label list, component): pairs in different
+// components are answered from those alone, the others become jobs in LDS and
+// are answered four at a time, sixteen lanes (one DPP row) each, so that the
+// first kind leaves no lanes idle.
 //   Bit-parallel slots: a lane takes four slots as bytes of one word of the
-// distance line.  With m the smallest slot sum, only slots at m or m + 1 can
-// lower it, and only where the sets that decide are nonempty; the line's
-// spare bytes say which are (bp_nz_byte), so most set pairs are never read.
+// record.  With m the smallest slot sum, only slots at m or m + 1 can lower
+// it, and only where the deciding sets can meet: the record has two bits per
+// slot for nonempty sets and S^-1 folded to a byte, so most set pairs are
+// never read (46 slots a pair within one of m, 1.8 left, R-MAT 20).
 //   Labels: the longer list goes through the group's LDS tile (kQTile labels,
 // padded with all-ones to a power of two), and each lane searches four labels
 // of the shorter list in it at once, branch-free.  The reads that need only
-// the offsets go out together: distance words, the longer list's first 128
+// the record's tail go out together: slot words, the longer list's first 128
 // labels, the shorter list's first 64; the set pairs are requested next and
-// the search runs while they are in flight.
+// the search runs while they are in flight.  Lists start on 128-byte lines
+// and are padded to them with all-ones, so nothing is masked.
+// Rank-space queries (many-graph jobs, checks) read the build's own arrays
+// through the same code (REC = false).
 //
-// What bounds it: instruction issue.  One wave per pair spent 234 vector
-// instructions a pair (73% of the SIMDs' issue slots on R-MAT 20) and read
-// all set pairs within one of the smallest sum (46 slots a pair; the
-// nonempty-set bits leave 2.3).  One million pairs, half of them Zipf, on the
-// R-MAT 14 index: 264 -> 122 us; 2 million on the weighted R-MAT 18 index:
-// 744 -> 555 us; 6 million in host arrays, R-MAT 18: 3.66 -> 2.76 ms; 10
-// million uniform pairs on R-MAT 20: 4.99 -> 4.47 ms.
+// What bounds it: on a large index the lines read at random (81 M of 128 B for
+// 10 M uniform pairs on R-MAT 20: 4.5 TB/s, a copy's rate), on a small one
+// instruction issue.  Against one wave per pair with the set pairs of every
+// slot within one of m read, in us:
+//                                            start   four pairs   records
+//   10 M uniform pairs, R-MAT 20 (HBM)        4,980       4,465     2,325
+//   1 M pairs, half Zipf, R-MAT 14 (L2)         264         122        87
+//   2 M pairs, weighted R-MAT 18                742         555       344
+//   6 M pairs in host arrays, R-MAT 18        3,600       2,760     2,190
+// (62% of uniform R-MAT 20 pairs have an isolated end.)
 #include "internal.hpp"
 
 namespace pado {
@@ -50,8 +59,8 @@ constexpr uint32_t kQPre = 2;                 // such loads of the longer list i
 constexpr uint32_t kQStride = kQTile + 8;
 constexpr uint32_t kQBuf = kQGroups * kQStride;  // LDS words per wave
 // Waves per SIMD the query kernels are compiled for: five is what their
-// registers take without spilling (at eight, 22 spilled registers made the
-// small-index batch below 171 us).
+// registers take without spilling (R-MAT 20 batch: 2,325 us at four or five,
+// 2,657 at six).
 constexpr int kQOcc = 5;
 constexpr uint32_t kNoSlot = 0x7FFFu;         // sum of a slot that does not count
 
@@ -789,14 +798,14 @@ pado_gpu_status launch_query_pair(const pado_gpu_index *idx, bool rank_space, ui
 
 namespace {
 
-// Consecutive pairs per wave: as many as leave each of the chip's 8,192
-// resident waves four chunks, in [4, 64].  A chunk's ids and records are two
-// dependent reads before its first pair, so long calls take 64; short ones
-// spread over the chip.
+// Consecutive pairs per wave: as many as leave 8,192 waves work, in [4, 64].
+// A chunk's ids and records are two dependent reads before its first pair, so
+// long calls take 64 (1 M pairs: 87 us against 97 with 16 and 161 with 4);
+// short ones spread over the chip.
 uint32_t query_chunk(uint64_t k)
 {
     uint32_t c = kQGroups;
-    while (c < 64 && (uint64_t)c * 2 * 4 * 8192 <= k) c *= 2;
+    while (c < 64 && (uint64_t)c * 2 * 8192 <= k) c *= 2;
     return c;
 }
 

@@ -8,7 +8,9 @@ import struct
 import numpy as np
 import pytest
 
+import oracle
 import parallel_distance_oracle_amd as pado
+from helpers import rank_space
 
 pytestmark = pytest.mark.gpu
 
@@ -126,3 +128,49 @@ def test_weighted_list_lengths(gpu_ctx, tmp_path):
     assert np.array_equal(idx.query(a, b, ref_compat=True), np.where(exp >= 32765, 32767, exp))
     assert np.array_equal(np.array([idx.query_pair(int(x), int(y)) for x, y in zip(a[:300], b[:300])], np.uint32),
                           exp[:300])
+
+
+@pytest.mark.parametrize("kind", ("hops", "wide", "cut", "weighted"))
+def test_components(gpu_ctx, kind):
+    """More components than bit-parallel slots, isolated vertices among them;
+    "cut" has a path deeper than the slots' BFS goes."""
+    rng = np.random.default_rng(3)
+    parts, n = [], 0
+
+    def add(edges, size):
+        nonlocal n
+        parts.append(np.asarray(edges, np.uint32).reshape(-1, 2) + np.uint32(n))
+        n += size
+
+    add(pado.rmat_edges(8, 6, seed=4), 256)
+    add(pado.grid_edges(9, 0.1, 2), 81)
+    if kind == "cut":
+        add([(i, i + 1) for i in range(399)], 400)
+    for k in range(120):
+        size = 2 + k % 5
+        add([(i, i + 1) for i in range(size - 1)], size)
+        n += k % 2  # an isolated vertex
+    edges = np.concatenate(parts + [np.array([[n, n + 1]], np.uint32)])
+    n += 2
+    w = pado.edge_weights(edges.shape[0], 1, 100, 5)
+    G, rank, _ = rank_space(edges)
+    dg, _, _ = pado.DeviceGraph.from_edges(gpu_ctx, edges, w if kind == "weighted" else None, rank)
+    idx = pado.Index.build(gpu_ctx, dg, wide=kind in ("wide", "cut"))
+    idx.order(rank)
+    a, b = rng.integers(0, n, 20000).astype(np.uint32), rng.integers(0, n, 20000).astype(np.uint32)
+    a[:n] = b[:n] = np.arange(n)
+    if kind == "weighted":
+        import scipy.sparse as sp
+        from scipy.sparse.csgraph import dijkstra
+
+        e = edges.astype(np.int64)
+        A = sp.coo_matrix((w.astype(float), (e[:, 0], e[:, 1])), shape=(n, n)).tocsr()
+        d = dijkstra(A, directed=False)[a, b]
+        exp = np.where(np.isinf(d), float(pado.WINF), d).astype(np.uint32)
+    else:
+        hops = oracle.bfs_pairs(G.num_v, G.off, G.adj, rank[a], rank[b])
+        exp = oracle.bfs_to_u8(hops) if kind == "hops" else np.minimum(hops, pado.WIDE_INF).astype(np.uint16)
+    print(f"[gpu] {kind}: {n} vertices", flush=True)
+    assert np.array_equal(idx.query(a, b), exp)
+    assert np.array_equal(idx.query(rank[a], rank[b], rank_space=True), exp)
+
