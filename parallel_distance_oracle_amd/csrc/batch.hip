@@ -62,10 +62,48 @@ __device__ inline uint32_t wave_sum_u32(uint32_t x)
     return x;
 }
 
-__device__ inline unsigned long long wave_sum_u64(unsigned long long x)
+template <int CTRL, int ROWS>
+__device__ inline uint32_t dpp0(uint32_t x)  // x moved by DPP, 0 where nothing moves in
 {
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false);
+}
+
+// Inclusive prefix sum over the 64 lanes of a wave (all of them active): four
+// shifts inside the rows of sixteen lanes, then the row totals passed on.  Six
+// dependent adds in registers where shuffles were six LDS round trips.
+__device__ inline uint32_t wave_incl_scan(uint32_t x)
+{
+    x += dpp0<0x111, 0xF>(x);
+    x += dpp0<0x112, 0xF>(x);
+    x += dpp0<0x114, 0xF>(x);
+    x += dpp0<0x118, 0xF>(x);
+    x += dpp0<0x142, 0xA>(x);
+    x += dpp0<0x143, 0xC>(x);
     return x;
+}
+
+__device__ inline uint32_t wave_total(uint32_t x) { return __builtin_amdgcn_readlane(wave_incl_scan(x), 63); }
+
+// Adds the wave's sums of the lanes' counts x to statistics FIRST .. FIRST + N
+// - 1 of its row.  A row has few writers and nobody reads it during the build:
+// with all waves adding to one set of totals, the queue on their line was 4.7
+// us of the average batch kernel (R-MAT 20 build: 317 ms, 292 without the
+// totals).  With the rows, the scans by DPP and the working counters on lines
+// of their own: 250 ms; a 161 x 161 wide grid 80 -> 64.6 ms.
+template <int FIRST, int N>
+__device__ inline void add_stats(BuildCounters *C, uint32_t wave, const uint32_t (&x)[N])
+{
+    static_assert(FIRST + N <= (int)kStats, "a statistic per entry");
+    const uint32_t lane = lane_id();
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        // (each half's total fits 32 bits)
+        const unsigned long long s = wave_total(x[i] & 0xFFFFu) + ((unsigned long long)wave_total(x[i] >> 16) << 16);
+        if (lane == (uint32_t)i) mine = s;
+    }
+    unsigned long long *row = reinterpret_cast<unsigned long long *>(C + 1) + (uint64_t)(wave % kStatRows) * kStatCols;
+    if (mine) atomicAdd(&row[FIRST + lane], mine);
 }
 
 // Push descriptor written into reserved chunk slots that carry no work: its
@@ -242,17 +280,6 @@ __device__ inline bool bp_mask_scan(uint32_t iter, const unsigned long long *rm,
     }
 }
 
-// Inclusive prefix sum over the 64 lanes of a wave.
-__device__ inline uint32_t wave_incl_scan(uint32_t x)
-{
-    const uint32_t lane = threadIdx.x & 63;
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o);
-        if (lane >= (uint32_t)o) x += y;
-    }
-    return x;
-}
-
 // Orders LDS writes of some lanes of a wave before reads by other lanes of
 // the same wave.
 __device__ inline void wave_lds_sync()
@@ -359,7 +386,7 @@ __device__ inline bool bp_set_phase(unsigned long long rem, unsigned long long o
     }
     const uint32_t cnt = (uint32_t)__popcll(rem);
     const uint32_t incl = wave_incl_scan(cnt);
-    const uint32_t total = __shfl(incl, 63);
+    const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
     if (total == 0) return pr;
     sc.rem[lane] = rem;
     sc.one[lane] = one;
@@ -654,7 +681,7 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
         // One update per block of each shared counter (every root would
         // otherwise queue on the same two addresses).
         s_base = tot ? atomicAdd(&C->n_chunk[1], tot) : 0u;
-        if (tot_e) atomicAdd(&C->n_pedge[1], tot_e);
+        if (tot_e && C->pull) atomicAdd(&C->n_pedge[1], tot_e);
     }
     __syncthreads();
     if (nch) {
@@ -799,7 +826,7 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
         const uint32_t cnt = (uint32_t)__popcll(nb);
         n_pass += cnt;
         const uint32_t incl = wave_incl_scan(cnt);
-        const uint32_t total = __shfl(incl, 63);
+        const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
         unsigned long long keep = 0ull;
         if (total) {
             s_nb[lane] = nb;
@@ -941,7 +968,6 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                 C->domain = 1;
             } else {
                 C->iterations += 1;
-                C->actives += n_act0;
                 if (pull) C->pulls += 1;
             }
         }
@@ -1022,7 +1048,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                 n_pass += cnt;
             }
             const uint32_t incl = wave_incl_scan(cnt);
-            const uint32_t total = __shfl(incl, 63);
+            const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
             if (total == 0) continue;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
@@ -1124,17 +1150,8 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
         // s_t is rewritten by the next step.
         wave_lds_sync();
     }
-    const unsigned long long t_push = wave_sum_u64(n_push), t_pass = wave_sum_u64(n_pass);
-    const unsigned long long t_bp = wave_sum_u64(n_bp), t_cand = wave_sum_u64(n_cand);
-    const unsigned long long t_edge = wave_sum_u64(n_edge), t_tail = wave_sum_u64(n_tail);
-    if (lane == 0) {
-        if (t_edge) atomicAdd(&C->edges, t_edge);
-        if (t_tail) atomicAdd(&C->tails, t_tail);
-        if (t_push) atomicAdd(&C->pushes, t_push);
-        if (t_pass) atomicAdd(&C->ind_pass, t_pass);
-        if (t_bp) atomicAdd(&C->bp_pruned, t_bp);
-        if (t_cand) atomicAdd(&C->cands, t_cand);
-    }
+    if (__ballot(n_edge != 0u) != 0ull)
+        add_stats<0>(C, wave, {n_edge, n_tail, n_push, n_pass, n_bp, n_cand});
 }
 
 template <bool W, uint32_t CH, uint32_t PW>
@@ -1169,6 +1186,7 @@ __device__ inline void batch_begin_write(BuildCounters *C, uint32_t b, uint32_t 
     C->n_cand[0] = C->n_cand[1] = 0;
     C->n_touched = rsz;
     C->labels += cnt;
+    C->actives += cnt;
 }
 
 // Start of a batch (construct's loop over batches, PARA:1791-1812): roots
@@ -1512,12 +1530,8 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         const uint32_t surv = cb & ~prune;
         n_dq += __popc(cb & prune);
         const uint32_t cnt = __popc(surv);
-        uint32_t incl = cnt;
-        for (int o = 1; o < 64; o <<= 1) {
-            uint32_t y = __shfl_up(incl, o);
-            if (lane >= (uint32_t)o) incl += y;
-        }
-        const uint32_t total = __shfl(incl, 63);
+        const uint32_t incl = wave_incl_scan(cnt);
+        const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
         if (total == 0) continue;
         n_lab += total;
         const unsigned long long nb = store_reserve_at(S, C, v, len, base, cap, total);
@@ -1554,7 +1568,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         ++my_act;
         my_pedge += __builtin_amdgcn_readfirstlane(pdeg);
         if (my_pedge >= 0x80000000u) {
-            if (lane == 0) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
+            if (lane == 0 && C->pull) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
             my_pedge = 0;
         }
         reinterpret_cast<uint16_t *>(ag + (uint64_t)v * kWords)[lane] = (uint16_t)surv;
@@ -1584,14 +1598,11 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         c_left -= nch;
     }
     for (uint32_t q = lane; q < c_left; q += 64) chunks[c_next + q] = kChunkPad;
-    if (lane == 0 && my_act) atomicAdd(&C->n_act[p ^ 1u], my_act);
-    if (lane == 0 && my_pedge) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
-    const unsigned long long t_dq = wave_sum_u64(n_dq), t_read = wave_sum_u64(n_read);
-    if (lane == 0) {
-        if (t_read) atomicAdd(&C->dq_labels, t_read);
-        if (t_dq) atomicAdd(&C->dq_pruned, t_dq);
-        if (n_lab) atomicAdd(&C->labels, (unsigned long long)n_lab);
-        if (n_rows) atomicAdd(&C->dq_rows, n_rows);
+    if (lane == 0 && my_act) C->n_act[p ^ 1u] = 1u;  // (every writer writes the same)
+    if (lane == 0 && my_pedge && C->pull) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
+    if (wave < ncand) {
+        const bool one = lane == 0;
+        add_stats<6>(C, wave, {n_read, n_dq, one ? n_lab : 0u, one ? n_rows : 0u, one ? my_act : 0u});
     }
 }
 
@@ -1607,10 +1618,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
 }
 
 // The graph's shape in the counters (once, at allocation).
-__global__ void k_ctr_shape(BuildCounters *C, uint32_t n, uint32_t nw)
+__global__ void k_ctr_shape(BuildCounters *C, uint32_t n, uint32_t nw, uint32_t pull)
 {
     C->n_vert = n;
     C->abits_words = nw;
+    C->pull = pull;
+}
+
+// The statistics rows' sums into the totals (one block, sixteen threads per
+// row step; once, at the end).
+__global__ __launch_bounds__(1024) void k_fold_stats(BuildCounters *C)
+{
+    __shared__ unsigned long long s[kStatCols];
+    const uint32_t col = threadIdx.x % kStatCols;
+    if (threadIdx.x < kStatCols) s[threadIdx.x] = 0ull;
+    __syncthreads();
+    const unsigned long long *rows = reinterpret_cast<const unsigned long long *>(C + 1);
+    unsigned long long sum = 0;
+    for (uint32_t i = threadIdx.x; i < kStatRows * kStatCols; i += 1024) sum += rows[i];
+    atomicAdd(&s[col], sum);
+    __syncthreads();
+    if (threadIdx.x < kStats) (&C->edges)[threadIdx.x] += s[threadIdx.x];
 }
 
 __global__ void k_unhold(BuildCounters *C) { C->hold = 0u; }
@@ -1847,7 +1875,7 @@ struct BatchBuffers {
 // rows (255).
 template <bool W>
 static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index *idx, uint64_t add_waves,
-                                   uint32_t chunk, unsigned long long pool_size, uint32_t dc_rows,
+                                   uint32_t chunk, unsigned long long pool_size, uint32_t dc_rows, bool pull,
                                    BatchBuffers<W> &B)
 {
     using DT = typename Hop<W>::Dist;
@@ -1870,7 +1898,7 @@ static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index
     PADO_TRY(B.rset.alloc((uint64_t)kBP * kBatch));
     PADO_TRY(B.lmask.alloc((uint64_t)n * kLmWords));
     PADO_TRY(B.rmask.alloc((kLmNz0 + 1ull) * kBatch));
-    PADO_TRY(B.ctr.alloc(1));
+    PADO_TRY(B.ctr.alloc(1 + kStatRows * kStatCols * 8 / sizeof(BuildCounters)));
     PADO_TRY(B.pool.alloc(pool_size));
     PADO_TRY(B.dc.alloc((uint64_t)dc_rows * kBatch));
     B.pool_size = pool_size;
@@ -1886,9 +1914,9 @@ static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index
     hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, reinterpret_cast<unsigned long long *>(B.lrec.p),
                        2ull * n);
     hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.abits.p, 2ull * nw);
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, reinterpret_cast<uint32_t *>(B.ctr.p),
-                       (uint64_t)(sizeof(BuildCounters) / 4), 0u);
-    hipLaunchKernelGGL(k_ctr_shape, dim3(1), dim3(1), 0, st, B.ctr.p, n, nw);
+    hipLaunchKernelGGL(k_fill_u32, dim3(64), dim3(256), 0, st, reinterpret_cast<uint32_t *>(B.ctr.p),
+                       (uint64_t)(B.ctr.n * sizeof(BuildCounters) / 4), 0u);
+    hipLaunchKernelGGL(k_ctr_shape, dim3(1), dim3(1), 0, st, B.ctr.p, n, nw, pull ? 1u : 0u);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
@@ -1903,6 +1931,7 @@ static pado_gpu_status batch_finish(pado_gpu_graph *g, pado_gpu_index *idx, cons
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
     hipLaunchKernelGGL(k_batch_end, dim3(1024), dim3(256), 0, st, B.ind.p, B.tlist.p, B.abits.p, B.ctr.p);
+    hipLaunchKernelGGL(k_fold_stats, dim3(1), dim3(1024), 0, st, B.ctr.p);
     BuildCounters c{};
     PADO_HIP(copy_sync(&c, B.ctr.p, sizeof(BuildCounters), hipMemcpyDeviceToHost, st));
     idx->counters = c;
@@ -1982,6 +2011,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         W ? "batch iteration reached 4095: distances outside the wide (12-bit) hop domain"
           : "batch iteration reached 255: distances outside the uint8 domain of the reference";
 
+    const uint32_t pull_ratio = cfg.pull_ratio ? cfg.pull_ratio : kPullRatio;
     // Per-wave reservations in k_add leave holes in the active list and the
     // descriptor array (see batch_alloc).
     const uint64_t add_waves = 4ull * (cfg.add_blocks ? cfg.add_blocks : default_add_grid(n));
@@ -1993,7 +2023,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     BatchBuffers<W> B;
     PADO_TRY(batch_alloc<W>(g, idx, add_waves, chunk,
                             std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, 64ull * n), pool_min),
-                            std::min<uint32_t>(n, 1u << 16), B));
+                            std::min<uint32_t>(n, 1u << 16), pull_ratio != ~0u, B));
     auto &ind = B.ind, &cand = B.cand, &ag = B.ag, &chunks = B.chunks, &abits = B.abits;
     unsigned long long *vmark = B.lmask.p + kLmMark;  // word kLmMark of each mask row (stride kLmWords)
     auto &lmask = B.lmask, &rmask = B.rmask;
@@ -2023,7 +2053,6 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     const uint32_t push_grid = cfg.push_blocks ? cfg.push_blocks : default_push_grid(n);
     const uint32_t add_grid = cfg.add_blocks ? cfg.add_blocks : default_add_grid(n);
     const uint32_t root_blocks = (batch * 64 + 255) / 256;
-    const uint32_t pull_ratio = cfg.pull_ratio ? cfg.pull_ratio : kPullRatio;
 
     // Stream mode brackets every push and add launch with HIP events (read
     // after the host check that follows each block of U iterations).
@@ -2360,7 +2389,7 @@ static pado_gpu_status batch_loop_t(std::vector<LoopJob> &jobs, hipStream_t st)
         // growable per-vertex arrays take up to four times their length.
         const unsigned long long pool =
             std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, 384ull * n), J.pool_min);
-        PADO_TRY(batch_alloc<W>(J.g, J.idx, kLoopWaves, kChunk, pool, n, bufs[j]));
+        PADO_TRY(batch_alloc<W>(J.g, J.idx, kLoopWaves, kChunk, pool, n, false, bufs[j]));
         plans[j] = batch_plan<W>(J.g, J.idx, J.used, J.batch, bufs[j]);
     }
     DevBuf<BatchPlan<W>> dplans;

@@ -168,43 +168,51 @@ __device__ inline uint32_t wave_append(uint32_t *counter, bool pred)
     return base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
 }
 
-// Device-side counters shared by the labeling kernels (one struct per build).
+// Device-side counters shared by the labeling kernels (one struct per build,
+// kStatRows statistics rows behind it).  Counters that a kernel's waves update
+// lie on lines of their own: updates of one line queue behind each other.
 struct BuildCounters {
-    // Frontier and candidate counts of batch iteration i live in slot i & 1:
-    // each kernel reads its own slot and empties the other one for the next
-    // kernel to fill, so no control launch runs between iterations.
-    uint32_t n_act[2];     // active vertices of the iteration
+    // Device-side schedule: the batch step reads its parameters from here, so
+    // one launch sequence (or one captured hipGraph) serves every batch.
     uint32_t n_vert;       // vertices of the graph
     uint32_t abits_words;  // 64-bit words of one frontier bitmap slot
-    uint32_t n_chunk[2];   // push work descriptors of the iteration
-    uint32_t n_cand[2];    // candidate vertices of the iteration
-    uint32_t n_touched;    // vertices whose indicator row was touched this batch
+    uint32_t pull;         // the frontier's push edges are wanted (n_pedge)
     // Batch gate: a batch enqueued before the host has seen the previous one
     // finish runs as no-ops if the previous batch still has a frontier.
     uint32_t hold;         // set: every batch kernel returns at once
     uint32_t iter_last;    // last iteration k_push ran (not held)
-    uint32_t overflow;     // label pool exhausted
-    uint32_t dq_rows;      // root-distance rows scanned (statistic)
-    unsigned long long pool_top;  // next free label slot in the pool
-    unsigned long long n_pedge[2];  // push edges of the iteration's frontier (sum of push degrees)
-    unsigned long long pulls;     // iterations run in pull form (statistic)
-    unsigned long long pushes;    // (tail, root) pairs offered by push
-    unsigned long long ind_pass;  // pairs that set a fresh indicator bit
-    unsigned long long bp_pruned; // pairs pruned by the bit-parallel check
-    unsigned long long cands;     // (vertex, root) candidates after the BP check
-    unsigned long long dq_pruned; // candidates pruned by the distance query
-    unsigned long long labels;    // labels appended
-    unsigned long long edges;     // push edges scanned (tails >= roots_start)
-    unsigned long long tails;     // distinct tails with a fresh indicator bit, summed over iterations
-    unsigned long long dq_labels; // labels with dist < iter read by distance queries
-    unsigned long long actives;   // active vertices, summed over iterations
-    // Device-side schedule: the batch step reads its parameters from here, so
-    // one launch sequence (or one captured hipGraph) serves every batch.
     uint32_t next_batch;          // batch index the next k_batch_begin starts
     uint32_t rs, rsz, gen_batch;  // current batch: roots [rs, rs + rsz)
     uint32_t domain;              // an iteration reached 255 (u8 domain)
     unsigned long long iterations;  // live iterations, summed over batches
+    unsigned long long pulls;     // iterations run in pull form (statistic)
+    // Frontier and candidate counts of batch iteration i live in slot i & 1:
+    // each kernel reads its own slot and empties the other one for the next
+    // kernel to fill, so no control launch runs between iterations.
+    alignas(128) uint32_t n_act[2];    // nonzero: the iteration has active vertices
+    alignas(128) uint32_t n_chunk[2];  // push work descriptors of the iteration
+    alignas(128) uint32_t n_cand[2];   // candidate vertices of the iteration
+    alignas(128) uint32_t n_touched;   // vertices whose indicator row was touched this batch
+    alignas(128) unsigned long long pool_top;  // next free label slot in the pool
+    uint32_t overflow;     // label pool exhausted
+    alignas(128) unsigned long long n_pedge[2];  // push edges of the iteration's frontier (sum of push degrees)
+    // Statistics: the sums of the rows' entries (fold_stats).
+    alignas(128) unsigned long long edges;  // push edges scanned (tails >= roots_start)
+    unsigned long long tails;     // distinct tails with a fresh indicator bit, summed over iterations
+    unsigned long long pushes;    // (tail, root) pairs offered by push
+    unsigned long long ind_pass;  // pairs that set a fresh indicator bit
+    unsigned long long bp_pruned; // pairs pruned by the bit-parallel check
+    unsigned long long cands;     // (vertex, root) candidates after the BP check
+    unsigned long long dq_labels; // labels with dist < iter read by distance queries
+    unsigned long long dq_pruned; // candidates pruned by the distance query
+    unsigned long long labels;    // labels appended
+    unsigned long long dq_rows;   // root-distance rows scanned
+    unsigned long long actives;   // active vertices, summed over iterations
 };
+// A statistics row: one 128-byte line, entries in the order of the struct's
+// last fields.  A wave adds its counts to row (wave mod kStatRows).
+constexpr uint32_t kStatRows = 1024, kStatCols = 16, kStats = 11;
+static_assert(kStatRows * kStatCols * 8 % sizeof(BuildCounters) == 0, "rows are allocated in units of the struct");
 
 // Host-side timing of the labeling kernels (HIP events on the build stream).
 struct KernelTimes {
