@@ -556,15 +556,16 @@ __global__ __launch_bounds__(256) void k_bp_masks(uint32_t n, const uint8_t *bpd
 // dist(root r, hub h) at column r - rs for the hubs of the batch roots'
 // labels, 255 elsewhere; hinfo[h] summarises the row (HubInfo).  Root
 // offset ro's labels pool[base, base + len) are entered (fill) or their
-// entries reset, by one wave; each lane handles four labels per step so the
-// dependent loads of a step overlap.
+// entries reset, by `parts` waves of which this is number `part`; each lane
+// handles four labels per step so the dependent loads of a step overlap.
 template <bool W>
-__device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned long long base, uint32_t len, LabelStore S,
-                                         HubInfo *hinfo, typename Hop<W>::Dist *dc)
+__device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned long long base, uint32_t len,
+                                         uint32_t part, uint32_t parts, LabelStore S, HubInfo *hinfo,
+                                         typename Hop<W>::Dist *dc)
 {
     constexpr uint32_t B = Hop<W>::kBits, INF = Hop<W>::kInf;
     const uint32_t lane = lane_id();
-    for (uint32_t j0 = 0; j0 < len; j0 += 256) {
+    for (uint32_t j0 = part * 256; j0 < len; j0 += parts * 256) {
         uint32_t lab[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -606,11 +607,15 @@ __device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned lo
 
 // initialize (PARA:848-1080): non-BP roots become active with their own bit as
 // last group, get the self label (r, 0), and set their own indicator bit;
-// then their labels go into the root-distance table (PARA:986-1013).  One
-// wave per root, four roots per block.  Root offset ro owns touched-list
+// their labels go into the root-distance table (PARA:986-1013).  Four waves per
+// root, kInitRoots roots per block of the launch schedule: the first wave of a
+// root sets it up while the other three enter its labels -- with one wave for
+// both, the root with the longest list (1,435 labels on R-MAT 20, six
+// dependent steps) set the kernel's time.  Root offset ro owns touched-list
 // slot ro (k_batch_begin sets the count and the frontier size), so the shared
 // counters left are the push-descriptor count, updated once per block, and
 // the frontier's push-edge count.
+constexpr uint32_t kRootWaves = 4, kInitRoots = 4;
 template <bool W, uint32_t CH>
 __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, const uint8_t *used, const uint64_t *off, const uint32_t *adj,
                                                      LabelStore S, HubInfo *hinfo, typename Hop<W>::Dist *dc,
@@ -621,13 +626,26 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
                                                      const unsigned long long *lmask, unsigned long long *rmask,
                                                      BuildCounters *C)
 {
-    __shared__ uint32_t s_nch[16], s_pdeg[16];
+    __shared__ uint32_t s_nch[kInitRoots], s_pdeg[kInitRoots];
     __shared__ uint32_t s_base;
     if (C->hold) return;
-    const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
-    const uint32_t ro = (bid * blockDim.x + threadIdx.x) >> 6;
+    const uint32_t lane = lane_id(), part = (threadIdx.x >> 6) % kRootWaves, rb = threadIdx.x / (64 * kRootWaves);
+    const uint32_t roots = blockDim.x / (64 * kRootWaves);  // of this block
+    const uint32_t ro = bid * roots + rb;
     const uint32_t rs = C->rs, rsz = C->rsz, gen_batch = C->gen_batch;
     const uint32_t r = rs + ro;
+    // Every wave of a root reads its label record before the first one
+    // appends to the list (which may move it: the old array stays as it is).
+    const bool live = ro < rsz && !used[r];
+    LRec rec0{};
+    if (live) rec0 = S.rec[r];
+    __syncthreads();
+    if (part != 0) {
+        if (live) hub_rows<W>(1u, ro, rec0.base, rec0.len, part - 1u, kRootWaves - 1u, S, hinfo, dc);
+        __syncthreads();
+        __syncthreads();
+        return;
+    }
     // Every root of the batch (bit-parallel roots included) is on the
     // touched list; a row that stays empty is cleared at no harm.
     if (ro < rsz && lane == 0) {
@@ -639,19 +657,14 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     if (ro < rsz && lane < kBP) rset[lane * kBatch + ro] = bps[(uint64_t)r * kBP + lane];
     if (ro < rsz && lane < kLmNz0 + 1) rmask[lane * kBatch + ro] = lmask[(uint64_t)r * kLmWords + lane];
     uint32_t pdeg = 0;
-    // the root's labels before its self label (their array, even if it moves)
-    uint32_t len0 = 0;
-    unsigned long long base0 = 0;
-    bool table = false;
-    if (ro < rsz && !used[r]) {
-        const LRec rec0 = S.rec[r];
-        len0 = rec0.len;
-        base0 = rec0.base;
-        const uint32_t len = len0;
+    if (live) {
+        const uint32_t len = rec0.len;
         const unsigned long long base = store_reserve_at(S, C, r, len, rec0.base, rec0.cap, 1);
         if (base != ~0ull) {
-            table = true;
             if (lane == 0) {
+                // the root-distance entry of the self label
+                dc[(uint64_t)r * kBatch + ro] = 0;
+                atomicMin(&hinfo[r].info, ~Hop<W>::kInf);
                 S.pool[base + len] = r << Hop<W>::kBits;  // (hub r, dist 0), PARA:932-949
                 S.rec[r].len = len + 1;
                 ind[(uint64_t)r * kWords + (ro >> 6)] |= 1ull << (ro & 63);
@@ -666,14 +679,14 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     }
     const uint32_t nch = (pdeg + CH - 1) / CH;
     if (lane == 0) {
-        s_nch[wv] = nch;
-        s_pdeg[wv] = pdeg;
+        s_nch[rb] = nch;
+        s_pdeg[rb] = pdeg;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t tot = 0;
         unsigned long long tot_e = 0;
-        for (uint32_t w = 0; w < blockDim.x / 64; ++w) {
+        for (uint32_t w = 0; w < roots; ++w) {
             tot += s_nch[w];
             tot_e += s_pdeg[w];
         }
@@ -686,21 +699,13 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     __syncthreads();
     if (nch) {
         uint32_t c0 = s_base;
-        for (uint32_t w = 0; w < wv; ++w) c0 += s_nch[w];
+        for (uint32_t w = 0; w < rb; ++w) c0 += s_nch[w];
         for (uint32_t q = lane; q < nch; q += 64) chunks[c0 + q] = ((unsigned long long)(q * CH) << 32) | r;
-    }
-    if (table) {
-        // root-distance entries: the earlier labels, then the self label
-        hub_rows<W>(1u, ro, base0, len0, S, hinfo, dc);
-        if (lane == 0) {
-            dc[(uint64_t)r * kBatch + ro] = 0;
-            atomicMin(&hinfo[r].info, ~Hop<W>::kInf);
-        }
     }
 }
 
 template <bool W, uint32_t CH>
-__global__ __launch_bounds__(256) void k_batch_init(const uint8_t *used, const uint64_t *off, const uint32_t *adj,
+__global__ __launch_bounds__(kInitRoots * kRootWaves * 64) void k_batch_init(const uint8_t *used, const uint64_t *off, const uint32_t *adj,
                                                      LabelStore S, HubInfo *hinfo, typename Hop<W>::Dist *dc,
                                                      unsigned long long *ind, unsigned long long *vmark,
                                                      uint32_t *tlist, unsigned long long *abits, unsigned long long *ag,
@@ -713,22 +718,21 @@ __global__ __launch_bounds__(256) void k_batch_init(const uint8_t *used, const u
                            chunks, bps, rset, lmask, rmask, C);
 }
 
-// One root's entries of the root-distance table from the batch roots'
-// offsets (one wave per root): with `fill` its labels are entered, without,
-// the entries of the previous batch's roots (the labels they held at its end,
-// which include every entry written during it) are reset.
+// The root-distance entries of the previous batch's roots (the labels they
+// held at its end, which include every entry written during it) are reset,
+// kRootWaves waves per root.
 template <bool W>
-__device__ __forceinline__ void hub_table_body(uint32_t bid, uint32_t nblk, uint32_t fill, const uint8_t *used, LabelStore S, HubInfo *hinfo,
-                                                   typename Hop<W>::Dist *dc, const BuildCounters *C)
+__device__ __forceinline__ void hub_reset_body(uint32_t bid, const uint8_t *used, LabelStore S, HubInfo *hinfo,
+                                               typename Hop<W>::Dist *dc, const BuildCounters *C)
 {
     if (C->hold) return;
-    const uint32_t ro = (bid * blockDim.x + threadIdx.x) >> 6;
+    const uint32_t w = (bid * blockDim.x + threadIdx.x) >> 6, ro = w / kRootWaves;
     const uint32_t rs = C->rs, rsz = C->rsz;
     if (ro >= rsz) return;
     const uint32_t r = rs + ro;
     if (used[r]) return;
     const LRec rec = S.rec[r];
-    hub_rows<W>(fill, ro, rec.base, rec.len, S, hinfo, dc);
+    hub_rows<W>(0u, ro, rec.base, rec.len, w % kRootWaves, kRootWaves, S, hinfo, dc);
 }
 
 
@@ -1645,7 +1649,7 @@ __global__ void k_unhold(BuildCounters *C) { C->hold = 0u; }
 
 // reset_at_end (PARA:1328-1410) and the next batch's indicator reset
 // (PARA:877-901): clear the indicator rows of the touched vertices (the
-// root-distance table is reset by hub_table_body), and frontier bitmap slot 1,
+// root-distance table is reset by hub_reset_body), and frontier bitmap slot 1,
 // which the next batch's first frontier goes into.
 __device__ __forceinline__ void batch_end_body(uint32_t bid, uint32_t nblk, unsigned long long *ind, const uint32_t *tlist,
                                                    unsigned long long *abits, const BuildCounters *C)
@@ -1669,8 +1673,8 @@ __global__ __launch_bounds__(256) void k_batch_end(unsigned long long *ind, cons
 // still has a frontier (its next iteration's count in slot (iter_last + 1) &
 // 1), this batch was enqueued too early and everything up to the host's
 // k_unhold is a no-op (a no-op before the first batch: all counts zero) --
-// then the previous batch's reset -- its roots' root-distance entries (one wave per
-// root in the first blocks) and batch_end_body -- which are independent of
+// then the previous batch's reset -- its roots' root-distance entries (four waves
+// per root) and batch_end_body -- which are independent of
 // each other.  Every block takes the gate's decision itself from counters
 // that nothing in this kernel changes.
 template <bool W>
@@ -1682,7 +1686,7 @@ __global__ __launch_bounds__(256) void k_batch_close(const uint8_t *used, LabelS
         if (blockIdx.x == 0 && threadIdx.x == 0) C->hold = 1u;
         return;
     }
-    hub_table_body<W>(blockIdx.x, gridDim.x, 0u, used, S, hinfo, dc, C);
+    hub_reset_body<W>(blockIdx.x, used, S, hinfo, dc, C);
     batch_end_body(blockIdx.x, gridDim.x, ind, tlist, abits, C);
 }
 
@@ -1734,8 +1738,8 @@ __global__ __launch_bounds__(kLoopWaves * 64) void k_batch_loop(const BatchPlan<
     for (uint32_t b = 0; b < nb; ++b) {
         // The previous batch's root-distance entries and indicator rows.
         const uint32_t prsz = C->rsz;
-        for (uint32_t vb = 0; vb * kLoopWaves < prsz; ++vb)
-            hub_table_body<W>(vb, 1, 0u, P.used, P.S, P.hinfo, P.dc, C);
+        for (uint32_t vb = 0; vb * (kLoopWaves / kRootWaves) < prsz; ++vb)
+            hub_reset_body<W>(vb, P.used, P.S, P.hinfo, P.dc, C);
         batch_end_body(0, 1, P.ind, P.tlist, P.abits, C);
         // Batch b: its non-bit-parallel roots are the first frontier.
         const uint32_t rs = b * P.batch, rsz = min(P.batch, P.n - rs);
@@ -1748,7 +1752,7 @@ __global__ __launch_bounds__(kLoopWaves * 64) void k_batch_loop(const BatchPlan<
         __syncthreads();
         if (threadIdx.x == 0) batch_begin_write(C, b, rs, rsz, s_cnt);
         __syncthreads();
-        for (uint32_t vb = 0; vb * kLoopWaves < rsz; ++vb)
+        for (uint32_t vb = 0; vb * (kLoopWaves / kRootWaves) < rsz; ++vb)
             batch_init_body<W, kChunk>(vb, 1, P.used, P.off, P.adj, P.S, P.hinfo, P.dc, P.ind, P.vmark, P.tlist,
                                        P.abits, P.ag, P.amask, P.aend, P.chunks, P.bps, P.rset, P.lmask, P.rmask, C);
         __syncthreads();
@@ -2052,7 +2056,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     const uint32_t U = cfg.iters_per_sync ? std::min<uint32_t>(cfg.iters_per_sync, 64u) : 8u;
     const uint32_t push_grid = cfg.push_blocks ? cfg.push_blocks : default_push_grid(n);
     const uint32_t add_grid = cfg.add_blocks ? cfg.add_blocks : default_add_grid(n);
-    const uint32_t root_blocks = (batch * 64 + 255) / 256;
+    const uint32_t root_blocks = (batch * kRootWaves * 64 + 255) / 256;
 
     // Stream mode brackets every push and add launch with HIP events (read
     // after the host check that follows each block of U iterations).
@@ -2077,7 +2081,8 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         hipLaunchKernelGGL(k_batch_close<W>, dim3(std::max<uint32_t>(1024u, root_blocks)), dim3(256), 0, st, d_used.p,
                            S, hinfo.p, dc.p, ind.p, tlist.p, abits.p, ctr.p);
         hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(batch), 0, st, d_used.p, ctr.p, batch, n);
-        hipLaunchKernelGGL(K.init, dim3((batch + 3) / 4), dim3(256), 0, st, d_used.p, g->off.p, g->adj.p, S,
+        hipLaunchKernelGGL(K.init, dim3((batch + kInitRoots - 1) / kInitRoots), dim3(kInitRoots * kRootWaves * 64), 0, st,
+                           d_used.p, g->off.p, g->adj.p, S,
                            hinfo.p, dc.p, ind.p, vmark, tlist.p, abits.p, ag.p, amask.p, aend.p, chunks.p,
                            (const ulonglong2 *)idx->bps.p, rset.p, lmask.p, rmask.p, ctr.p);
     };
