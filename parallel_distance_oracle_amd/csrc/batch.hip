@@ -62,48 +62,9 @@ __device__ inline uint32_t wave_sum_u32(uint32_t x)
     return x;
 }
 
-template <int CTRL, int ROWS>
-__device__ inline uint32_t dpp0(uint32_t x)  // x moved by DPP, 0 where nothing moves in
+__device__ inline unsigned long long *stat_rows(BuildCounters *C)
 {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false);
-}
-
-// Inclusive prefix sum over the 64 lanes of a wave (all of them active): four
-// shifts inside the rows of sixteen lanes, then the row totals passed on.  Six
-// dependent adds in registers where shuffles were six LDS round trips.
-__device__ inline uint32_t wave_incl_scan(uint32_t x)
-{
-    x += dpp0<0x111, 0xF>(x);
-    x += dpp0<0x112, 0xF>(x);
-    x += dpp0<0x114, 0xF>(x);
-    x += dpp0<0x118, 0xF>(x);
-    x += dpp0<0x142, 0xA>(x);
-    x += dpp0<0x143, 0xC>(x);
-    return x;
-}
-
-__device__ inline uint32_t wave_total(uint32_t x) { return __builtin_amdgcn_readlane(wave_incl_scan(x), 63); }
-
-// Adds the wave's sums of the lanes' counts x to statistics FIRST .. FIRST + N
-// - 1 of its row.  A row has few writers and nobody reads it during the build:
-// with all waves adding to one set of totals, the queue on their line was 4.7
-// us of the average batch kernel (R-MAT 20 build: 317 ms, 292 without the
-// totals).  With the rows, the scans by DPP and the working counters on lines
-// of their own: 250 ms; a 161 x 161 wide grid 80 -> 64.6 ms.
-template <int FIRST, int N>
-__device__ inline void add_stats(BuildCounters *C, uint32_t wave, const uint32_t (&x)[N])
-{
-    static_assert(FIRST + N <= (int)kStats, "a statistic per entry");
-    const uint32_t lane = lane_id();
-    unsigned long long mine = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        // (each half's total fits 32 bits)
-        const unsigned long long s = wave_total(x[i] & 0xFFFFu) + ((unsigned long long)wave_total(x[i] >> 16) << 16);
-        if (lane == (uint32_t)i) mine = s;
-    }
-    unsigned long long *row = reinterpret_cast<unsigned long long *>(C + 1) + (uint64_t)(wave % kStatRows) * kStatCols;
-    if (mine) atomicAdd(&row[FIRST + lane], mine);
+    return reinterpret_cast<unsigned long long *>(C + 1);
 }
 
 // Push descriptor written into reserved chunk slots that carry no work: its
@@ -1004,9 +965,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
             }
         }
         s_t[wv][lane] = t;
-        uint32_t wall = words;
-        for (int o = 32; o > 0; o >>= 1) wall |= __shfl_xor(wall, o);
-        wall = uniform32(wall);  // the same in every lane: the step's word choice lives in scalar registers
+        uint32_t wall = wave_or(words);  // a scalar: the step's word choice lives in scalar registers
         bool touched = false, got = false;
         while (wall) {
             // Up to four root words per step (wave-uniform): their indicator
@@ -1155,7 +1114,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
         wave_lds_sync();
     }
     if (__ballot(n_edge != 0u) != 0ull)
-        add_stats<0>(C, wave, {n_edge, n_tail, n_push, n_pass, n_bp, n_cand});
+        add_stats<0>(stat_rows(C), wave, {n_edge, n_tail, n_push, n_pass, n_bp, n_cand});
 }
 
 template <bool W, uint32_t CH, uint32_t PW>
@@ -1606,7 +1565,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
     if (lane == 0 && my_pedge && C->pull) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
     if (wave < ncand) {
         const bool one = lane == 0;
-        add_stats<6>(C, wave, {n_read, n_dq, one ? n_lab : 0u, one ? n_rows : 0u, one ? my_act : 0u});
+        add_stats<6>(stat_rows(C), wave, {n_read, n_dq, one ? n_lab : 0u, one ? n_rows : 0u, one ? my_act : 0u});
     }
 }
 
@@ -1637,7 +1596,7 @@ __global__ __launch_bounds__(1024) void k_fold_stats(BuildCounters *C)
     const uint32_t col = threadIdx.x % kStatCols;
     if (threadIdx.x < kStatCols) s[threadIdx.x] = 0ull;
     __syncthreads();
-    const unsigned long long *rows = reinterpret_cast<const unsigned long long *>(C + 1);
+    const unsigned long long *rows = stat_rows(C);
     unsigned long long sum = 0;
     for (uint32_t i = threadIdx.x; i < kStatRows * kStatCols; i += 1024) sum += rows[i];
     atomicAdd(&s[col], sum);

@@ -152,6 +152,64 @@ __device__ inline uint64_t uniform64(uint64_t x)
 
 __device__ inline uint32_t uniform32(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
+template <int CTRL, int ROWS>
+__device__ inline uint32_t dpp0(uint32_t x)  // x moved by DPP, 0 where nothing moves in
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false);
+}
+
+// Inclusive prefix sum over the 64 lanes of a wave (all of them active): four
+// shifts inside the rows of sixteen lanes, then the row totals passed on.  Six
+// dependent adds in registers where shuffles were six LDS round trips.
+__device__ inline uint32_t wave_incl_scan(uint32_t x)
+{
+    x += dpp0<0x111, 0xF>(x);
+    x += dpp0<0x112, 0xF>(x);
+    x += dpp0<0x114, 0xF>(x);
+    x += dpp0<0x118, 0xF>(x);
+    x += dpp0<0x142, 0xA>(x);
+    x += dpp0<0x143, 0xC>(x);
+    return x;
+}
+
+__device__ inline uint32_t wave_total(uint32_t x) { return __builtin_amdgcn_readlane(wave_incl_scan(x), 63); }
+
+// The wave's OR of x.
+__device__ inline uint32_t wave_or(uint32_t x)
+{
+    x |= dpp0<0x111, 0xF>(x);
+    x |= dpp0<0x112, 0xF>(x);
+    x |= dpp0<0x114, 0xF>(x);
+    x |= dpp0<0x118, 0xF>(x);
+    x |= dpp0<0x142, 0xA>(x);
+    x |= dpp0<0x143, 0xC>(x);
+    return __builtin_amdgcn_readlane(x, 63);
+}
+
+// Adds the wave's sums of the lanes' counts x to entries FIRST .. FIRST + N -
+// 1 of the wave's row of statistics: kStatRows rows of one 128-byte line each,
+// summed once at the end of a build.  A row has few writers and nobody reads
+// it during the build: with all waves adding to one set of totals, the queue
+// on their line was 4.7 us of the average batch kernel (R-MAT 20 build: 317
+// ms, 292 without the totals).  With the rows, the scans by DPP and the
+// working counters on lines of their own: 250 ms; a 161 x 161 wide grid 80 ->
+// 64.6 ms.
+constexpr uint32_t kStatRows = 1024, kStatCols = 16;
+template <int FIRST, int N>
+__device__ inline void add_stats(unsigned long long *rows, uint32_t wave, const uint32_t (&x)[N])
+{
+    static_assert(FIRST + N <= (int)kStatCols, "an entry per count");
+    const uint32_t lane = threadIdx.x & 63;
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        // (each half's total fits 32 bits)
+        const unsigned long long s = wave_total(x[i] & 0xFFFFu) + ((unsigned long long)wave_total(x[i] >> 16) << 16);
+        if (lane == (uint32_t)i) mine = s;
+    }
+    if (mine) atomicAdd(&rows[(uint64_t)(wave % kStatRows) * kStatCols + FIRST + lane], mine);
+}
+
 // Append one item per lane with `pred` to a list counted by *counter: the
 // active lanes of the wave take consecutive slots with a single atomic, so a
 // shared counter sees one update per wave instead of one per item.  Returns
@@ -169,7 +227,7 @@ __device__ inline uint32_t wave_append(uint32_t *counter, bool pred)
 }
 
 // Device-side counters shared by the labeling kernels (one struct per build,
-// kStatRows statistics rows behind it).  Counters that a kernel's waves update
+// the statistics rows of add_stats behind it).  Counters that a kernel's waves update
 // lie on lines of their own: updates of one line queue behind each other.
 struct BuildCounters {
     // Device-side schedule: the batch step reads its parameters from here, so
@@ -196,7 +254,7 @@ struct BuildCounters {
     alignas(128) unsigned long long pool_top;  // next free label slot in the pool
     uint32_t overflow;     // label pool exhausted
     alignas(128) unsigned long long n_pedge[2];  // push edges of the iteration's frontier (sum of push degrees)
-    // Statistics: the sums of the rows' entries (fold_stats).
+    // Statistics: the sums of the rows' entries (k_fold_stats).
     alignas(128) unsigned long long edges;  // push edges scanned (tails >= roots_start)
     unsigned long long tails;     // distinct tails with a fresh indicator bit, summed over iterations
     unsigned long long pushes;    // (tail, root) pairs offered by push
@@ -209,9 +267,7 @@ struct BuildCounters {
     unsigned long long dq_rows;   // root-distance rows scanned
     unsigned long long actives;   // active vertices, summed over iterations
 };
-// A statistics row: one 128-byte line, entries in the order of the struct's
-// last fields.  A wave adds its counts to row (wave mod kStatRows).
-constexpr uint32_t kStatRows = 1024, kStatCols = 16, kStats = 11;
+constexpr uint32_t kStats = 11;  // the last fields, in the order of a row's entries
 static_assert(kStatRows * kStatCols * 8 % sizeof(BuildCounters) == 0, "rows are allocated in units of the struct");
 
 // Host-side timing of the labeling kernels (HIP events on the build stream).

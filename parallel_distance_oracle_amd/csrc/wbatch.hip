@@ -46,14 +46,27 @@ using u64 = unsigned long long;
 
 // Frontier / improved-tail counts of round i live in slot i & 1: each round's
 // kernels read their slot and empty the other one for the next kernel.
+// Counters that a kernel's waves update lie on lines of their own; add_stats'
+// rows follow the struct (with the scans by DPP, weighted R-MAT 20: 719 -> 627
+// ms; the filter of a late batch, 2,048 blocks of which most are idle, 11.5 ->
+// 6.6 us).
 struct WCounters {
-    uint32_t n_act[2], n_chunk[2], n_imp[2], n_touched, overflow;
-    uint32_t a_top[2];  // active-list slots handed out (>= n_act: per-wave reservations)
-    u64 pool_top, relax, improved, pruned, labels, filtered, rounds, need;
+    uint32_t n_act[2];              // nonzero: the round has active vertices
+    u64 rounds;
+    alignas(128) uint32_t a_top[2];    // active-list slots handed out (per-wave reservations)
+    alignas(128) uint32_t n_chunk[2];
+    alignas(128) uint32_t n_imp[2];
+    alignas(128) uint32_t n_touched;
+    alignas(128) u64 pool_top;
+    uint32_t overflow;
     // Pool words the batch's commit can reserve at most: per touched vertex
     // the reservation its list would take if every batch root were kept.
-    u64 need_bound;
+    alignas(128) u64 need_bound;
+    alignas(128) u64 need, labels;
+    // Statistics: the sums of the rows' entries (k_w_fold_stats).
+    alignas(128) u64 relax, improved, pruned, filtered;
 };
+constexpr uint32_t kWStats = 4;
 
 struct WStore {
     u64 *pool;
@@ -64,10 +77,17 @@ struct WStore {
 
 __device__ inline uint32_t lane_id() { return threadIdx.x & 63; }
 
-__device__ inline u64 wave_sum(u64 x)
+__device__ inline u64 *stat_rows(WCounters *C) { return reinterpret_cast<u64 *>(C + 1); }
+
+__device__ inline uint32_t wave_max(uint32_t x)
 {
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
+    x = max(x, dpp0<0x111, 0xF>(x));
+    x = max(x, dpp0<0x112, 0xF>(x));
+    x = max(x, dpp0<0x114, 0xF>(x));
+    x = max(x, dpp0<0x118, 0xF>(x));
+    x = max(x, dpp0<0x142, 0xA>(x));
+    x = max(x, dpp0<0x143, 0xC>(x));
+    return __builtin_amdgcn_readlane(x, 63);
 }
 
 // Tails > lo form a prefix of a descending adjacency list (WPARA:457 breaks
@@ -130,13 +150,28 @@ __device__ inline u64 reserve_words(uint32_t len, uint32_t cap, uint32_t add)
     return ncap;
 }
 
+// The statistics rows' sums into the totals (once, at the end).
+__global__ __launch_bounds__(1024) void k_w_fold_stats(WCounters *C)
+{
+    __shared__ u64 s[kStatCols];
+    if (threadIdx.x < kStatCols) s[threadIdx.x] = 0ull;
+    __syncthreads();
+    const u64 *rows = stat_rows(C);
+    u64 sum = 0;
+    for (uint32_t i = threadIdx.x; i < kStatRows * kStatCols; i += 1024) sum += rows[i];
+    atomicAdd(&s[threadIdx.x % kStatCols], sum);
+    __syncthreads();
+    if (threadIdx.x < kWStats) (&C->relax)[threadIdx.x] += s[threadIdx.x];
+}
+
 // Round 1's frontier is the batch's roots in order: root offset ro holds
 // active-list slot ro and touched-list entry ro (k_w_init).
 __global__ void k_w_reset_counters(WCounters *C, uint32_t rsz)
 {
     C->n_act[0] = C->n_chunk[0] = C->n_chunk[1] = C->n_imp[0] = C->n_imp[1] = 0;
     C->a_top[0] = 0;
-    C->n_act[1] = C->a_top[1] = rsz;
+    C->n_act[1] = 1;
+    C->a_top[1] = rsz;
     C->n_touched = rsz;
     C->need = C->need_bound = 0;
 }
@@ -145,35 +180,58 @@ __global__ void k_w_reset_counters(WCounters *C, uint32_t rsz)
 // (roots_labels_buffer, WPARA:322-348, transposed): dcw[h][ro] = d(root
 // rs + ro, hub h), indexed by hub id, and hmin[h] = the least of them.  Both
 // are INF outside the batch roots' hubs (k_w_commit resets what was written).
-__device__ inline void w_hub_fill(uint32_t ro, uint32_t r, WStore S, uint32_t *hmin, uint32_t *dcw)
+// Lists are hub-sorted and every root holds the top-ranked hubs: walking them
+// from the end staggers the roots' arrival at those hubs, so the plain read of
+// hmin skips most atomics.  The root's list of `len` labels is walked by
+// `parts` waves of which this is number `part`, two labels per lane and step.
+__device__ inline void w_hub_fill(uint32_t ro, u64 base, uint32_t len, uint32_t part, uint32_t parts, WStore S,
+                                  uint32_t *hmin, uint32_t *dcw)
 {
     const uint32_t lane = lane_id();
-    const uint32_t len = S.len[r];
-    const u64 base = S.base[r];
-    // Lists are hub-sorted and every root holds the top-ranked hubs: walking
-    // them from the end staggers the roots' arrival at those hubs, so the
-    // plain read of hmin skips most atomics.
-    for (uint32_t j0 = (len + 63) & ~63u; j0 > 0; j0 -= 64) {
-        const uint32_t j = j0 - 64 + lane;
-        if (j >= len) continue;
-        const u64 lab = S.pool[base + j];
-        const uint32_t h = (uint32_t)(lab >> 32), d = (uint32_t)lab;
-        dcw[(uint64_t)h * kWB + ro] = d;
-        if (d < hmin[h]) atomicMin(&hmin[h], d);
+    for (uint32_t k0 = part * 128; k0 < len; k0 += parts * 128) {
+        u64 lab[2];
+        uint32_t hm[2];
+        bool ok[2];
+#pragma unroll
+        for (uint32_t u = 0; u < 2; ++u) {
+            const uint32_t k = k0 + 64 * u + lane;  // from the end
+            ok[u] = k < len;
+            lab[u] = ok[u] ? S.pool[base + (len - 1 - k)] : 0ull;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 2; ++u) {
+            const uint32_t h = (uint32_t)(lab[u] >> 32);
+            if (ok[u]) {
+                hm[u] = hmin[h];
+                dcw[(uint64_t)h * kWB + ro] = (uint32_t)lab[u];
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 2; ++u)
+            if (ok[u] && (uint32_t)lab[u] < hm[u]) atomicMin(&hmin[lab[u] >> 32], (uint32_t)lab[u]);
     }
 }
 
 // initialize_tables (WPARA:305-383): every root at distance 0 from itself,
 // active with its own bit, and its earlier labels in the root-distance table.
-// One wave per root, one chunk reservation per block.
-__global__ __launch_bounds__(256) void k_w_init(uint32_t rs, uint32_t rsz, uint32_t gen_batch, const uint64_t *off,
+// Four roots per block: the first four waves set the roots up, the other
+// twelve (three per root) enter their labels, which nothing here changes.  One
+// chunk reservation per block.
+constexpr uint32_t kWInitFill = 3;
+__global__ __launch_bounds__(256 * (1 + kWInitFill)) void k_w_init(uint32_t rs, uint32_t rsz, uint32_t gen_batch, const uint64_t *off,
                                                 const uint32_t *adj, uint32_t *T, uint32_t *tmark, uint32_t *tlist,
                                                 uint32_t *alist, u64 *ag, uint32_t *amask, uint32_t *aend, u64 *chunks,
                                                 uint32_t *hmin, uint32_t *dcw, WStore S, WCounters *C)
 {
     __shared__ uint32_t s_nch[4], s_c0;
-    const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
+    const uint32_t lane = lane_id(), wv = (threadIdx.x >> 6) & 3u, part = threadIdx.x >> 8;
     const uint32_t ro = blockIdx.x * 4 + wv;
+    if (part) {
+        if (ro < rsz) w_hub_fill(ro, S.base[rs + ro], S.len[rs + ro], part - 1u, kWInitFill, S, hmin, dcw);
+        __syncthreads();
+        __syncthreads();
+        return;
+    }
     uint32_t nch = 0;
     if (ro < rsz) {
         const uint32_t r = rs + ro;
@@ -201,7 +259,6 @@ __global__ __launch_bounds__(256) void k_w_init(uint32_t rs, uint32_t rsz, uint3
     uint32_t c0 = s_c0;
     for (uint32_t w = 0; w < wv; ++w) c0 += s_nch[w];
     for (uint32_t q = lane; q < nch; q += 64) chunks[c0 + q] = ((u64)(q * kChunk) << 32) | ro;
-    if (ro < rsz) w_hub_fill(ro, rs + ro, S, hmin, dcw);
 }
 
 
@@ -279,8 +336,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         C->a_top[p ^ 1u] = 0;
         C->n_chunk[p ^ 1u] = 0;
     }
-    uint32_t n_relax = 0, n_imp = 0;
-    u64 n_bound = 0;
+    uint32_t n_relax = 0, n_imp = 0, n_bound = 0;  // (a list's reservation fits 32 bits, and a lane's few do)
     for (uint32_t c0 = wave * 4; c0 < nc; c0 += nwaves * 4) {
         const uint32_t c = c0 + (lane >> 4);
         uint32_t k = 0, u = 0, t = 0, w = 0, lim = 0, words = 0;
@@ -300,8 +356,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         s_u[wv][lane] = u;
         s_t[wv][lane] = t;
         s_w[wv][lane] = w;
-        uint32_t wall = words;
-        for (int o = 32; o > 0; o >>= 1) wall |= __shfl_xor(wall, o);
+        uint32_t wall = wave_or(words);
         bool got = false;
         while (wall) {
             const uint32_t wd = __ffs(wall) - 1;
@@ -312,12 +367,8 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
                 if (lim < (wd + 1) * 64) g &= (1ull << (lim - wd * 64)) - 1ull;
             }
             const uint32_t cnt = (uint32_t)__popcll(g);
-            uint32_t incl = cnt;
-            for (int o = 1; o < 64; o <<= 1) {
-                const uint32_t y = __shfl_up(incl, o);
-                if (lane >= (uint32_t)o) incl += y;
-            }
-            const uint32_t total = __shfl(incl, 63);
+            const uint32_t incl = wave_incl_scan(cnt);
+            const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
             if (total == 0) continue;
             s_g[wv][lane] = g;
             s_ex[wv][lane] = incl - cnt;
@@ -358,7 +409,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         const uint32_t ti = wave_append(&C->n_touched, new_t);
         if (new_t) {
             tlist[ti] = t;
-            n_bound += reserve_words(S.len[t], S.cap[t], rsz);
+            n_bound += (uint32_t)reserve_words(S.len[t], S.cap[t], rsz);
         }
         const uint32_t ii = wave_append(&C->n_imp[p], new_i);
         if (new_i) {
@@ -368,11 +419,10 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         // s_u / s_t / s_w are rewritten by the next step.
         w_lds_sync();
     }
-    const u64 t_relax = wave_sum(n_relax), t_imp = wave_sum(n_imp), t_bound = wave_sum(n_bound);
-    if (lane == 0) {
-        if (t_relax) atomicAdd(&C->relax, t_relax);
-        if (t_imp) atomicAdd(&C->improved, t_imp);
-        if (t_bound) atomicAdd(&C->need_bound, t_bound);
+    if (wave * 4 < nc) {
+        const u64 t_bound = wave_total(n_bound & 0xFFFFu) + ((u64)wave_total(n_bound >> 16) << 16);
+        if (lane == 0 && t_bound) atomicAdd(&C->need_bound, t_bound);
+        add_stats<0>(stat_rows(C), wave, {n_relax, n_imp});
     }
 }
 
@@ -391,7 +441,7 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
     const uint32_t p = round & 1u;
     const uint32_t nimp = C->n_imp[p];
     if (blockIdx.x == 0 && threadIdx.x == 0) C->n_imp[p ^ 1u] = 0;
-    u64 n_pruned = 0;
+    uint32_t n_pruned = 0;
     uint32_t a_next = 0, a_left = 0, c_next = 0, c_left = 0, my_act = 0;
     for (uint32_t i = wave; i < nimp; i += nwaves) {
         const uint32_t t = ilist[i];
@@ -407,11 +457,7 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
             dv[q] = (imp >> q) & 1u ? T[(uint64_t)t * kWB + lane * 8 + q] : 0u;
             if (((imp >> q) & 1u) && dv[q] > maxd) maxd = dv[q];
         }
-        uint32_t wmax = maxd;
-        for (int o = 32; o > 0; o >>= 1) {
-            uint32_t y = __shfl_xor(wmax, o);
-            wmax = y > wmax ? y : wmax;
-        }
+        const uint32_t wmax = wave_max(maxd);
         uint32_t prune = 0;
         const uint32_t len = uniform32(S.len[t]);
         const u64 base = uniform64(S.base[t]);
@@ -421,7 +467,7 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
         // at most kWGather unpruned, the labels not yet read go to the gather
         // phase.
         uint32_t j_gather = 0;
-        if (wave_sum((u64)__popc(imp)) > kWGather) {
+        if (wave_total(__popc(imp)) > kWGather) {
             j_gather = len;
             for (uint32_t j0 = 0; j0 < len; j0 += 64) {
                 const uint32_t j = j0 + lane;
@@ -468,7 +514,7 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
                         for (int q = 0; q < 8; ++q)
                             if (((imp >> q) & 1u) && x[q] != kWInf && (uint64_t)dd[u] + x[q] <= dv[q]) prune |= 1u << q;
                     }
-                    if (wave_sum((u64)__popc(imp & ~prune)) <= kWGather) {
+                    if (wave_total(__popc(imp & ~prune)) <= kWGather) {
                         few = true;
                         break;
                     }
@@ -599,9 +645,8 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
         c_left -= nch;
     }
     for (uint32_t q = lane; q < c_left; q += 64) chunks[c_next + q] = kWChunkPad;
-    if (lane == 0 && my_act) atomicAdd(&C->n_act[p ^ 1u], my_act);
-    n_pruned = wave_sum(n_pruned);
-    if (lane == 0 && n_pruned) atomicAdd(&C->pruned, n_pruned);
+    if (lane == 0 && my_act) C->n_act[p ^ 1u] = 1u;  // (every writer writes the same)
+    if (wave < nimp) add_stats<2>(stat_rows(C), wave, {n_pruned});
 }
 
 // The batch roots' mutual entries, transposed for the filter: RT[h][r] =
@@ -651,7 +696,11 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t nt = C->n_touched;
-    u64 n_lab = 0, n_filt = 0, n_need = 0;
+    __shared__ u64 s_lab, s_need;
+    if (threadIdx.x == 0) s_lab = s_need = 0ull;
+    __syncthreads();
+    uint32_t n_filt = 0;
+    u64 n_lab = 0, n_need = 0;
     for (uint32_t i = wave; i < nt; i += nwaves) {
         const uint32_t v = tlist[i];
         const uint8_t pb = reinterpret_cast<const uint8_t *>(P + (uint64_t)v * kWW)[lane];
@@ -710,16 +759,20 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
         // The improved bitmap is all zero once the rounds end; it carries the
         // kept pairs to the commit kernel.
         reinterpret_cast<uint8_t *>(I + (uint64_t)v * kWW)[lane] = (uint8_t)keep;
-        const uint32_t total = (uint32_t)wave_sum((u64)__popc(keep));
+        const uint32_t total = wave_total(__popc(keep));
         if (!total) continue;
         n_lab += total;
         if (lane == 0) n_need += reserve_words(S.len[v], S.cap[v], total);
     }
-    n_filt = wave_sum(n_filt);
+    if (wave < nt) add_stats<3>(stat_rows(C), wave, {n_filt});
     if (lane == 0) {
-        if (n_lab) atomicAdd(&C->labels, n_lab);
-        if (n_filt) atomicAdd(&C->filtered, n_filt);
-        if (n_need) atomicAdd(&C->need, n_need);
+        if (n_lab) atomicAdd(&s_lab, n_lab);
+        if (n_need) atomicAdd(&s_need, n_need);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_lab) atomicAdd(&C->labels, s_lab);
+        if (s_need) atomicAdd(&C->need, s_need);
     }
 }
 
@@ -752,12 +805,8 @@ __global__ __launch_bounds__(256) void k_w_commit(uint32_t rs, uint32_t rsz, con
         uint8_t *Kb = reinterpret_cast<uint8_t *>(I + (uint64_t)v * kWW);
         const uint32_t keep = Kb[lane];
         const uint32_t cnt = __popc(keep);
-        uint32_t incl = cnt;
-        for (int o = 1; o < 64; o <<= 1) {
-            uint32_t y = __shfl_up(incl, o);
-            if (lane >= (uint32_t)o) incl += y;
-        }
-        const uint32_t total = __shfl(incl, 63);
+        const uint32_t incl = wave_incl_scan(cnt);
+        const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
         if (total) {
             if (keep) Kb[lane] = 0;
             const uint32_t len = S.len[v];
@@ -847,7 +896,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     PADO_TRY(len.alloc(n));
     PADO_TRY(cap.alloc(n));
     PADO_TRY(base.alloc(n));
-    PADO_TRY(ctr.alloc(1));
+    PADO_TRY(ctr.alloc(1 + (kStatRows * kStatCols * 8 + sizeof(WCounters) - 1) / sizeof(WCounters)));
     u64 pool_size = std::max<u64>(1ull << 22, 32ull * n);
     PADO_TRY(pool.alloc(pool_size));
     uint32_t dc_slots = std::min<uint32_t>(n, 1u << 14);
@@ -863,7 +912,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, len.p, (uint64_t)n, 0u);
     hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, cap.p, (uint64_t)n, 0u);
     hipLaunchKernelGGL(k_w_zero64, dim3(fg), dim3(256), 0, st, base.p, (uint64_t)n);
-    PADO_HIP(hipMemsetAsync(ctr.p, 0, sizeof(WCounters), st));
+    PADO_HIP(hipMemsetAsync(ctr.p, 0, ctr.n * sizeof(WCounters), st));
     WCounters *h = nullptr;
     PADO_HIP(hipHostMalloc((void **)&h, sizeof(WCounters), hipHostMallocDefault));
     std::memset(h, 0, sizeof(WCounters));
@@ -896,7 +945,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
             PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB));
             hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, dcw.p, (uint64_t)dc_slots * kWB, kWInf);
         }
-        hipLaunchKernelGGL(k_w_init, dim3(rb), dim3(256), 0, st, rs, rsz, gen_batch, g->off.p, g->adj.p, T.p, tmark.p,
+        hipLaunchKernelGGL(k_w_init, dim3(rb), dim3(256 * (1 + kWInitFill)), 0, st, rs, rsz, gen_batch, g->off.p, g->adj.p, T.p, tmark.p,
                            tlist.p, alist.p, ag.p, amask.p, aend.p, chunks.p, hmin.p, dcw.p, S, ctr.p);
         // Rounds per host check: the previous batch's round count + 1 first
         // (enough when this batch takes no more), then blocks of 2^j that
@@ -986,6 +1035,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
         hipLaunchKernelGGL(k_w_commit, dim3(2048), dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, I.p, hmin.p, dcw.p,
                            S, ctr.p);
     }
+    hipLaunchKernelGGL(k_w_fold_stats, dim3(1), dim3(1024), 0, st, ctr.p);
     PADO_HIP(hipMemcpyAsync(h, ctr.p, sizeof(WCounters), hipMemcpyDeviceToHost, st));
     PADO_HIP(hipStreamSynchronize(st));
     if (h->overflow) {
