@@ -17,13 +17,14 @@
 // and the tails of their records (label list, component): pairs in different
 // components are answered from those alone, the others become jobs in LDS and
 // are answered four at a time, sixteen lanes (one DPP row) each, so that the
-// first kind leaves no lanes idle.
+// first kind leaves no lanes idle.  Pairs with long lists are left to the end
+// and take the whole wave, one at a time; so do all pairs of a short call.
 //   Bit-parallel slots: a lane takes four slots as bytes of one word of the
 // record.  With m the smallest slot sum, only slots at m or m + 1 can lower
 // it, and only where the deciding sets can meet: the record has two bits per
 // slot for nonempty sets and S^-1 folded to a byte, so most set pairs are
 // never read (46 slots a pair within one of m, 1.8 left, R-MAT 20).
-//   Labels: the longer list goes through the group's LDS tile (kQTile labels,
+//   Labels: the longer list goes through the group's LDS tile (256 labels,
 // padded with all-ones to a power of two), and each lane searches four labels
 // of the shorter list in it at once, branch-free.  The reads that need only
 // the record's tail go out together: slot words, the longer list's first 128
@@ -37,11 +38,11 @@
 // 10 M uniform pairs on R-MAT 20: 4.5 TB/s, a copy's rate), on a small one
 // instruction issue.  Against one wave per pair with the set pairs of every
 // slot within one of m read, in us:
-//                                            start   four pairs   records
-//   10 M uniform pairs, R-MAT 20 (HBM)        4,980       4,465     2,325
-//   1 M pairs, half Zipf, R-MAT 14 (L2)         264         122        87
-//   2 M pairs, weighted R-MAT 18                742         555       344
-//   6 M pairs in host arrays, R-MAT 18        3,600       2,760     2,190
+//                                      first   four pairs   records   long alone
+//   10 M uniform pairs, R-MAT 20 (HBM) 4,980       4,465     2,325        1,970
+//   1 M pairs, half Zipf, R-MAT 14       264         122        87           87
+//   2 M pairs, weighted R-MAT 18         742         555       344          341
+//   6 M host pairs, R-MAT 18           3,600       2,760     2,190        2,180
 // (62% of uniform R-MAT 20 pairs have an isolated end.)
 #include "internal.hpp"
 
@@ -50,19 +51,31 @@ namespace {
 
 constexpr uint32_t kQWaves = 4;               // waves per query block
 constexpr uint32_t kQLanes = 16;              // lanes per pair: one DPP row
-constexpr uint32_t kQGroups = 64 / kQLanes;   // pairs a wave answers at once
-constexpr uint32_t kQTile = 256;              // labels of the longer list held in LDS
-constexpr uint32_t kQStep = 4 * kQLanes;      // labels a group moves per load: four per lane
-constexpr uint32_t kQPre = 2;                 // such loads of the longer list issued with the first reads
-// Groups' tiles start at different LDS banks: the first search steps of all
-// groups read the same tile position.
-constexpr uint32_t kQStride = kQTile + 8;
-constexpr uint32_t kQBuf = kQGroups * kQStride;  // LDS words per wave
+constexpr uint32_t kQPre = 2;                 // loads of the longer list issued with the first reads
+constexpr uint32_t kQBuf = 64 / kQLanes * (16 * kQLanes + 8);  // LDS words per wave
 // Waves per SIMD the query kernels are compiled for: five is what their
 // registers take without spilling (R-MAT 20 batch: 2,325 us at four or five,
 // 2,657 at six).
 constexpr int kQOcc = 5;
+// Searches a group would do one after the other, from which on the whole wave
+// takes the pair instead: it needs one or two, and the wave's other groups
+// would have waited for the longest (10 M pairs on R-MAT 20: 1,970 us at 3,
+// 2,060 at 2, 2,035 at 4, 2,610 without; weighted R-MAT 18: 364 us at 4, 378
+// at 3, 341 without: see kWMixedPairs).
+constexpr uint32_t kLongSteps = 3, kWLongSteps = 4;
 constexpr uint32_t kNoSlot = 0x7FFFu;         // sum of a slot that does not count
+
+// L lanes work on a pair: a group of a wave, or all of it.
+template <uint32_t L>
+struct Lanes {
+    static constexpr uint32_t kGroups = 64 / L;  // pairs a wave answers at once
+    static constexpr uint32_t kTile = 16 * L;    // labels of the longer list held in LDS
+    static constexpr uint32_t kStep = 4 * L;     // labels a group moves per load: four per lane
+    // Groups' tiles start at different LDS banks: the first search steps of
+    // all groups read the same tile position.
+    static constexpr uint32_t kStride = kTile + 8;
+    static_assert(kGroups * kTile + (kGroups - 1) * 8 <= kQBuf);
+};
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_at4 __attribute__((aligned(4)));  // four words at any word address
@@ -81,19 +94,28 @@ __device__ inline uint32_t row_ror(uint32_t x)
     return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x120 + N, 0xF, 0xF, false);
 }
 
-// The least value of the sixteen lanes of a group, in all of them.
+// The least value of a group's lanes, in all of them.
+template <uint32_t L>
 __device__ inline uint32_t group_min(uint32_t x)
 {
     x = min(x, row_ror<8>(x));
     x = min(x, row_ror<4>(x));
     x = min(x, row_ror<2>(x));
-    return min(x, row_ror<1>(x));
+    x = min(x, row_ror<1>(x));
+    if constexpr (L == 64) {
+        const uint32_t a = __builtin_amdgcn_readlane(x, 0), b = __builtin_amdgcn_readlane(x, 16);
+        const uint32_t c = __builtin_amdgcn_readlane(x, 32), d = __builtin_amdgcn_readlane(x, 48);
+        x = min(min(a, b), min(c, d));
+    }
+    return x;
 }
 
-// The largest of the four groups' values (the same in a group's lanes), as a
+// The largest of the groups' values (the same in a group's lanes), as a
 // scalar.
+template <uint32_t L>
 __device__ inline uint32_t groups_max(uint32_t x)
 {
+    if constexpr (L == 64) return uniform32(x);
     const uint32_t a = __builtin_amdgcn_readlane(x, 0), b = __builtin_amdgcn_readlane(x, kQLanes);
     const uint32_t c = __builtin_amdgcn_readlane(x, 2 * kQLanes), d = __builtin_amdgcn_readlane(x, 3 * kQLanes);
     return max(max(a, b), max(c, d));
@@ -122,7 +144,7 @@ __device__ inline u32x4 mask4(u32x4 v, uint32_t j, uint32_t len)
 }
 
 // Lower bounds of four keys in a tile of `size` ascending words (a power of
-// two up to kQTile): pos[q] = the byte offset of the first word >= key[q], or
+// two up to TILE): pos[q] = the byte offset of the first word >= key[q], or
 // of the last word.  Three vector instructions and an LDS read a step.
 template <uint32_t H>
 __device__ inline void search_step(const char *tile, uint32_t size, const u32x4 &key, uint32_t (&pos)[4])
@@ -137,11 +159,12 @@ __device__ inline void search_step(const char *tile, uint32_t size, const u32x4 
     if constexpr (H > 1) search_step<H / 2>(tile, size, key, pos);
 }
 
+template <uint32_t TILE>
 __device__ inline void search4(const uint32_t *tile, uint32_t size, const u32x4 &key, uint32_t (&pos)[4])
 {
 #pragma unroll
     for (int q = 0; q < 4; ++q) pos[q] = 0;
-    search_step<kQTile / 2>(reinterpret_cast<const char *>(tile), size, key, pos);
+    search_step<TILE / 2>(reinterpret_cast<const char *>(tile), size, key, pos);
 }
 
 __device__ inline uint32_t tile_at(const uint32_t *tile, uint32_t pos)
@@ -152,7 +175,7 @@ __device__ inline uint32_t tile_at(const uint32_t *tile, uint32_t pos)
 // A group's four list entries to its tile.
 __device__ inline void tile_put(uint32_t *tile, uint32_t j, const u32x4 &v) { *reinterpret_cast<u32x4 *>(tile + j) = v; }
 
-// The power of two at or above x (x in [1, kQTile]; 1 for 0).
+// The power of two at or above x (1 for 0).
 __device__ inline uint32_t tile_size(uint32_t x) { return x <= 1u ? 1u : 1u << (32 - __builtin_clz(x - 1u)); }
 
 }  // namespace
@@ -186,12 +209,27 @@ struct QBuf {
     uint32_t ans[64];
 };
 
-// Sorts out the wave's pairs (lane j: pair j if `has`): returns how many are
-// left to answer, in buf.job, and sets ans to the lane's answer if it needs
-// none of that: an id past the index (a == b ? 0 : far), two components (far).
-template <bool REC, uint32_t RECW>
-__device__ inline uint32_t make_jobs(const QIndex &X, bool has, uint32_t a, uint32_t b, uint32_t far, QBuf &buf,
-                                     uint32_t &ans, bool &job)
+// How a wave's pairs are shared out: all to groups, the ones with long lists
+// to the whole wave, or all of them.
+enum { kGrouped = 0, kMixed = 1, kAlone = 2 };
+
+// Whether a whole wave takes a pair by itself: where a group would need
+// kLongSteps searches or more.
+template <bool W>
+__device__ inline bool long_lists(uint32_t ls, uint32_t lt)
+{
+    constexpr uint32_t s = Lanes<kQLanes>::kStep, t = Lanes<kQLanes>::kTile;
+    return ((ls + s - 1) / s) * ((lt + t - 1) / t) >= (W ? kWLongSteps : kLongSteps);
+}
+
+// Sorts out the wave's pairs (lane j: pair j if `has`): the ones left to
+// answer go to buf.job, njobs of them, the first ngroup for groups, the others
+// for the whole wave; sets ans to the lane's answer if
+// it needs none of that: an id past the index (a == b ? 0 : far), two
+// components (far).
+template <bool REC, uint32_t RECW, int M>
+__device__ inline void make_jobs(const QIndex &X, bool has, uint32_t a, uint32_t b, uint32_t far, QBuf &buf,
+                                 uint32_t &ans, bool &job, uint32_t &ngroup, uint32_t &njobs)
 {
     const uint32_t lane = threadIdx.x & 63;
     ans = a == b ? 0u : far;
@@ -216,34 +254,39 @@ __device__ inline uint32_t make_jobs(const QIndex &X, bool has, uint32_t a, uint
             lb = (uint32_t)(X.loff[b + 1] - ob);
         }
     }
-    const unsigned long long m = __ballot(job);
-    if (job) {
-        QJob j;
-        const bool sw = la > lb;
-        j.a = a;
-        j.b = b;
-        j.os = sw ? ob : oa;
-        j.ot = sw ? oa : ob;
-        j.ls = (sw ? lb : la) | (lane << 24);
-        j.lt = sw ? la : lb;
-        buf.job[__popcll(m & ((1ull << lane) - 1ull))] = j;
-    }
+    const bool sw = la > lb;
+    QJob j;
+    j.a = a;
+    j.b = b;
+    j.os = sw ? ob : oa;
+    j.ot = sw ? oa : ob;
+    j.ls = (sw ? lb : la) | (lane << 24);
+    j.lt = sw ? la : lb;
+    const bool alone = M == kAlone || M == kMixed && long_lists<RECW == kWRecWords>(sw ? lb : la, j.lt);
+    const unsigned long long mg = __ballot(job && !alone), ma = __ballot(job && alone);
+    ngroup = (uint32_t)__popcll(mg);
+    njobs = ngroup + (uint32_t)__popcll(ma);
+    if (job) buf.job[(alone ? ngroup : 0u) + (uint32_t)__popcll((alone ? ma : mg) & ((1ull << lane) - 1ull))] = j;
     q_lds_sync();
-    return (uint32_t)__popcll(m);
 }
 
-// Answers the jobs four at a time, each job's answer to buf.ans[its lane].
+// Answers jobs r0 to njobs, 64 / L at a time, each job's answer to
+// buf.ans[its lane].
 // Hop<false>: the reference's answers (255 for unreachable or >= 253);
 // Hop<true>: exact hops, 0xFFFF for unreachable, using only bit-parallel slots
 // reached on both sides.
-template <bool W, bool REC>
-__device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_compat, QBuf &buf)
+template <bool W, bool REC, uint32_t L>
+__device__ inline void answer_jobs(const QIndex &X, uint32_t r0, uint32_t njobs, bool ref_compat, QBuf &buf)
 {
     constexpr uint32_t B = Hop<W>::kBits, MASK = Hop<W>::kInf;
     constexpr uint32_t UNREACHED = W ? 0xFFFFu : 255u;
-    const uint32_t lane = threadIdx.x & 63, l = lane & (kQLanes - 1), g = lane / kQLanes;
-    uint32_t *tile = buf.tile + g * kQStride;
-    for (uint32_t r0 = 0; r0 < njobs; r0 += kQGroups) {
+    using G = Lanes<L>;
+    // (the slots take one row of lanes: the rows of a wave that works on one
+    // pair all do the same)
+    const uint32_t sl = threadIdx.x & (kQLanes - 1);
+    const uint32_t lane = threadIdx.x & 63, l = lane & (L - 1), g = lane / L;
+    uint32_t *tile = buf.tile + g * G::kStride;
+    for (; r0 < njobs; r0 += G::kGroups) {
         // (a group without a job repeats the first one's)
         const bool has = r0 + g < njobs;
         const QJob job = buf.job[has ? r0 + g : r0];
@@ -251,20 +294,20 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
         const uint32_t *S = X.lab + job.os, *T = X.lab + job.ot;
         uint32_t wa, wb, fa = 0, fb = 0;
         if constexpr (REC) {
-            const uint32_t *pa = X.rec + (uint64_t)job.a * kQRecWords + l, *pb = X.rec + (uint64_t)job.b * kQRecWords + l;
+            const uint32_t *pa = X.rec + (uint64_t)job.a * kQRecWords + sl, *pb = X.rec + (uint64_t)job.b * kQRecWords + sl;
             wa = pa[0];
             wb = pb[0];
             fa = pa[kQRecFold];
             fb = pb[kQRecFold];
         } else {
-            wa = reinterpret_cast<const uint32_t *>(X.bpd + (uint64_t)job.a * kBpdStride)[l];
-            wb = reinterpret_cast<const uint32_t *>(X.bpd + (uint64_t)job.b * kBpdStride)[l];
+            wa = reinterpret_cast<const uint32_t *>(X.bpd + (uint64_t)job.a * kBpdStride)[sl];
+            wb = reinterpret_cast<const uint32_t *>(X.bpd + (uint64_t)job.b * kBpdStride)[sl];
         }
         u32x4 tv[kQPre];
 #pragma unroll
-        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * kQStep + 4 * l, lt);
+        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * G::kStep + 4 * l, lt);
         const u32x4 s0 = load4(S, 4 * l, ls);
-        const uint32_t ms = groups_max(ls), mt = groups_max(lt);
+        const uint32_t ms = groups_max<L>(ls), mt = groups_max<L>(lt);
         // This lane's four slots (the last lanes have none).
         uint32_t td[4];
         {
@@ -276,7 +319,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
             td[3] = hi >> 16;
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) {
-                bool ok = 4 * l + j < kBP;
+                bool ok = 4 * sl + j < kBP;
                 if (W)  // 255: the slot's BFS did not reach this vertex
                     ok = ok && ((wa >> (8 * j)) & 255u) != kInf8 && ((wb >> (8 * j)) & 255u) != kInf8;
                 else
@@ -288,7 +331,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
         // `both`) and which S^-1 on one side and S^0 on the other (`cross`).
         uint32_t both, cross;
         {
-            const uint32_t sh = 8 * ((kBpNzByte + l) & 3u), from = (lane & ~(kQLanes - 1)) + ((kBpNzByte + l) >> 2);
+            const uint32_t sh = 8 * ((kBpNzByte + sl) & 3u), from = (lane & ~(kQLanes - 1)) + ((kBpNzByte + sl) >> 2);
             const uint32_t na = __shfl(wa, from) >> sh, nb = __shfl(wb, from) >> sh;
             if constexpr (REC) {
                 // the bytes of f that are not zero, as four bits
@@ -300,7 +343,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
             }
             cross = ((na & (nb >> 4)) | ((na >> 4) & nb)) & 15u;
         }
-        const ulonglong2 *ra = X.bps + (uint64_t)job.a * kBP + 4 * l, *rb = X.bps + (uint64_t)job.b * kBP + 4 * l;
+        const ulonglong2 *ra = X.bps + (uint64_t)job.a * kBP + 4 * sl, *rb = X.bps + (uint64_t)job.b * kBP + 4 * sl;
         if (min(min(td[0], td[1]), min(td[2], td[3])) < 2u) {
             // A sum that its sets would take below zero does not count (no
             // such slot in a built index: a root's own sets are empty).
@@ -312,7 +355,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
                 td[j] = neg ? kNoSlot : td[j];
             }
         }
-        const uint32_t m = group_min(min(min(td[0], td[1]), min(td[2], td[3])));
+        const uint32_t m = group_min<L>(min(min(td[0], td[1]), min(td[2], td[3])));
         // The slots at m (cm) and m + 1 (cn) that their sets can lower: S^-1
         // against S^-1 by two, S^-1 against S^0 by one (which does not help
         // at m + 1).
@@ -324,7 +367,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
                 em |= td[j] == m ? 1u << j : 0u;
                 en |= td[j] == m + 1u ? 1u << j : 0u;
             }
-            if (m == kNoSlot || l > (kBP - 1) / 4) em = en = 0u;
+            if (m == kNoSlot || sl > (kBP - 1) / 4) em = en = 0u;
             cm = em & (both | cross);
             cn = en & both;
         }
@@ -342,22 +385,22 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
                 cn &= cn - 1u;
         }
         uint32_t d = m < UNREACHED && m != kNoSlot ? m : UNREACHED;
-        for (uint32_t t0 = 0; ms && t0 < mt; t0 += kQTile) {
-            const uint32_t size = tile_size(min(mt - t0, kQTile));
-            for (uint32_t u = 0; u * kQStep < size; ++u) {
-                const uint32_t j = t0 + u * kQStep + 4 * l;
+        for (uint32_t t0 = 0; ms && t0 < mt; t0 += G::kTile) {
+            const uint32_t size = tile_size(min(mt - t0, G::kTile));
+            for (uint32_t u = 0; u * G::kStep < size; ++u) {
+                const uint32_t j = t0 + u * G::kStep + 4 * l;
                 const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
-                tile_put(tile, u * kQStep + 4 * l, REC ? v : mask4(v, j, lt));
+                tile_put(tile, u * G::kStep + 4 * l, REC ? v : mask4(v, j, lt));
             }
             q_lds_sync();
-            for (uint32_t i = 0; i < ms; i += kQStep) {
+            for (uint32_t i = 0; i < ms; i += G::kStep) {
                 const u32x4 v = i == 0 ? s0 : load4(S, i + 4 * l, ls);
                 const u32x4 s = REC ? v : mask4(v, i + 4 * l, ls);
                 // A packed label with the same hub is >= the hub with
                 // distance 0, so whole words compare as hubs do.
                 const u32x4 key = s & ~MASK;
                 uint32_t pos[4];
-                search4(tile, size, key, pos);
+                search4<G::kTile>(tile, size, key, pos);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     // x - key is the other distance if the hubs are equal,
@@ -372,7 +415,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
             q_lds_sync();
         }
         if (W && d >= 2 * MASK) d = UNREACHED;
-        d = group_min(d);
+        d = group_min<L>(d);
         if (first) {
             if (sa.x & sb.x)
                 d = min(d, first_m ? m - 2u : m - 1u);
@@ -395,7 +438,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
             else if (at_m && ((xa.x & xb.y) | (xa.y & xb.x)))
                 d = min(d, m - 1u);
         }
-        d = group_min(d);
+        d = group_min<L>(d);
         if (!W && d >= 253u) d = 255u;
         if (has && l == 0) buf.ans[job.ls >> 24] = d;
     }
@@ -408,12 +451,13 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t njobs, bool ref_com
 // range -> a == b ? 0 : 32767).  As answer_pairs, on the hub lists;
 // distances of the shorter list come in with its hubs, those of the longer
 // list are read where a hub matches.
-template <bool REC>
-__device__ inline void answer_wjobs(const QIndex &X, uint32_t njobs, bool ref_compat, QBuf &buf)
+template <bool REC, uint32_t L>
+__device__ inline void answer_wjobs(const QIndex &X, uint32_t r0, uint32_t njobs, bool ref_compat, QBuf &buf)
 {
-    const uint32_t lane = threadIdx.x & 63, l = lane & (kQLanes - 1), g = lane / kQLanes;
-    uint32_t *tile = buf.tile + g * kQStride;
-    for (uint32_t r0 = 0; r0 < njobs; r0 += kQGroups) {
+    using G = Lanes<L>;
+    const uint32_t lane = threadIdx.x & 63, l = lane & (L - 1), g = lane / L;
+    uint32_t *tile = buf.tile + g * G::kStride;
+    for (; r0 < njobs; r0 += G::kGroups) {
         const bool has = r0 + g < njobs;
         const QJob job = buf.job[has ? r0 + g : r0];
         const uint32_t ls = job.ls & 0xFFFFFFu, lt = job.lt;
@@ -421,24 +465,24 @@ __device__ inline void answer_wjobs(const QIndex &X, uint32_t njobs, bool ref_co
         const uint32_t *DS = X.wdist + job.os, *DT = X.wdist + job.ot;
         u32x4 tv[kQPre];
 #pragma unroll
-        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * kQStep + 4 * l, lt);
+        for (uint32_t u = 0; u < kQPre; ++u) tv[u] = load4(T, u * G::kStep + 4 * l, lt);
         const u32x4 s0 = load4(S, 4 * l, ls), d0 = load4(DS, 4 * l, ls);
-        const uint32_t ms = groups_max(ls), mt = groups_max(lt);
+        const uint32_t ms = groups_max<L>(ls), mt = groups_max<L>(lt);
         uint32_t d = 0xFFFFFFFFu;
-        for (uint32_t t0 = 0; ms && t0 < mt; t0 += kQTile) {
-            const uint32_t size = tile_size(min(mt - t0, kQTile));
-            for (uint32_t u = 0; u * kQStep < size; ++u) {
-                const uint32_t j = t0 + u * kQStep + 4 * l;
+        for (uint32_t t0 = 0; ms && t0 < mt; t0 += G::kTile) {
+            const uint32_t size = tile_size(min(mt - t0, G::kTile));
+            for (uint32_t u = 0; u * G::kStep < size; ++u) {
+                const uint32_t j = t0 + u * G::kStep + 4 * l;
                 const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
-                tile_put(tile, u * kQStep + 4 * l, REC ? v : mask4(v, j, lt));
+                tile_put(tile, u * G::kStep + 4 * l, REC ? v : mask4(v, j, lt));
             }
             q_lds_sync();
-            for (uint32_t i = 0; i < ms; i += kQStep) {
+            for (uint32_t i = 0; i < ms; i += G::kStep) {
                 const u32x4 v = i == 0 ? s0 : load4(S, i + 4 * l, ls);
                 const u32x4 s = REC ? v : mask4(v, i + 4 * l, ls);
                 const u32x4 e = i == 0 ? d0 : load4(DS, i + 4 * l, ls);
                 uint32_t pos[4], x[4];
-                search4(tile, size, s, pos);
+                search4<G::kTile>(tile, size, s, pos);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     x[q] = 0xFFFFFFFFu;
@@ -450,7 +494,7 @@ __device__ inline void answer_wjobs(const QIndex &X, uint32_t njobs, bool ref_co
             }
             q_lds_sync();
         }
-        d = group_min(d);
+        d = group_min<L>(d);
         if (ref_compat && d >= 32765u) d = 32767u;
         if (has && l == 0) buf.ans[job.ls >> 24] = d;
     }
@@ -462,17 +506,21 @@ enum { kHops = 0, kWideHops = 1, kWeights = 2 };
 
 // Answers the wave's pairs, lane j holding pair j if `has`; returns the lane's
 // answer.
-template <int K, bool REC>
+template <int K, bool REC, int M>
 __device__ inline uint32_t answer_pairs(const QIndex &X, bool has, uint32_t a, uint32_t b, bool ref_compat, QBuf &buf)
 {
     const uint32_t far = K == kHops ? 255u : K == kWideHops ? 0xFFFFu : ref_compat ? 32767u : 0xFFFFFFFFu;
     uint32_t ans;
     bool job;
-    const uint32_t njobs = make_jobs<REC, K == kWeights ? kWRecWords : kQRecWords>(X, has, a, b, far, buf, ans, job);
-    if constexpr (K == kWeights)
-        answer_wjobs<REC>(X, njobs, ref_compat, buf);
-    else
-        answer_jobs<K == kWideHops, REC>(X, njobs, ref_compat, buf);
+    uint32_t ngroup, njobs;
+    make_jobs<REC, K == kWeights ? kWRecWords : kQRecWords, M>(X, has, a, b, far, buf, ans, job, ngroup, njobs);
+    if constexpr (K == kWeights) {
+        if constexpr (M != kAlone) answer_wjobs<REC, kQLanes>(X, 0, ngroup, ref_compat, buf);
+        if constexpr (M != kGrouped) answer_wjobs<REC, 64>(X, ngroup, njobs, ref_compat, buf);
+    } else {
+        if constexpr (M != kAlone) answer_jobs<K == kWideHops, REC, kQLanes>(X, 0, ngroup, ref_compat, buf);
+        if constexpr (M != kGrouped) answer_jobs<K == kWideHops, REC, 64>(X, ngroup, njobs, ref_compat, buf);
+    }
     return job ? buf.ans[threadIdx.x & 63] : ans;
 }
 
@@ -481,7 +529,7 @@ __device__ inline uint32_t answer_pairs(const QIndex &X, bool has, uint32_t a, u
 // Batch queries: a wave takes `chunk` consecutive pairs at a time (see
 // query_chunk).  OT: the answer type (u16 for a wide index or widened
 // answers).
-template <int K, bool REC, class OT>
+template <int K, bool REC, int M, class OT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query(QIndex X, const uint32_t *qa,
                                                const uint32_t *qb, uint64_t k, uint32_t chunk, OT *out,
                                                int ref_compat)
@@ -493,7 +541,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
     for (uint64_t c0 = w * chunk; c0 < k; c0 += nw * chunk) {
         const bool has = lane < chunk && c0 + lane < k;
         const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const uint32_t d = answer_pairs<K, REC>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        const uint32_t d = answer_pairs<K, REC, M>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
         if (has) out[c0 + lane] = (OT)d;
         // The next chunk's jobs and answers must not overtake these reads.
         q_lds_sync();
@@ -521,7 +569,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
         if (c0 >= k) break;
         const bool has = lane < kGrab && c0 + lane < k;
         const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const uint32_t d = answer_pairs<K, true>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        const uint32_t d = answer_pairs<K, true, K == kWeights ? kGrouped : kMixed>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
         if (has) out[c0 + lane] = (OT)d;
         q_lds_sync();
     }
@@ -675,7 +723,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
             ia = ld_sys(A.ra + phys + lane);
             ib = ld_sys(A.rb + phys + lane);
         }
-        const uint32_t mine = answer_pairs<K, true>(X, lane < len, ia, ib, A.ref_compat != 0, s_q[wv]);
+        const uint32_t mine = answer_pairs<K, true, kMixed>(X, lane < len, ia, ib, A.ref_compat != 0, s_q[wv]);
         // The next descriptor's writes must not overtake these reads.
         q_lds_sync();
         if (lane < len) {
@@ -769,7 +817,7 @@ template <int K, bool REC>
 __global__ __launch_bounds__(64) void k_query_pair(QIndex X, uint32_t a, uint32_t b, int ref_compat, uint32_t *out)
 {
     __shared__ QBuf buf;
-    const uint32_t d = answer_pairs<K, REC>(X, threadIdx.x == 0, a, b, ref_compat != 0, buf);
+    const uint32_t d = answer_pairs<K, REC, kAlone>(X, threadIdx.x == 0, a, b, ref_compat != 0, buf);
     if (threadIdx.x == 0) __hip_atomic_store(out, d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -798,13 +846,29 @@ pado_gpu_status launch_query_pair(const pado_gpu_index *idx, bool rank_space, ui
 
 namespace {
 
-// Consecutive pairs per wave: as many as leave 8,192 waves work, in [4, 64].
-// A chunk's ids and records are two dependent reads before its first pair, so
-// long calls take 64 (1 M pairs: 87 us against 97 with 16 and 161 with 4);
-// short ones spread over the chip.
+// Up to here a whole wave takes each pair: the waves are on the chip together,
+// and a call takes as long as its longest lists, which the wave goes through
+// in fewer steps.  4,000 pairs, 900 K vertex R-MAT: 6.2 us, 22.2 in groups;
+// 200 K vertices weighted: 4.7 and 9.9; short lists 4.6 to 5.3 either way.
+// 8,000 pairs with short lists: 6.4 us, 4.5 in groups.
+constexpr uint64_t kAlonePairs = 4096;
+
+// Weighted pairs go to groups only from here on: the whole wave's part costs
+// registers and scheduling (2 M pairs: 341 us, 362 mixed) and only a call's
+// last waves gain by it (16,000 pairs: 10.4 us, 9.3 mixed).
+constexpr uint64_t kWMixedPairs = 32768;
+
+// Consecutive pairs per wave otherwise: as many as leave 8,192 waves work, in
+// [4, 64].  A chunk's ids and records are two dependent reads before its first
+// pair, so long calls take 64 (1 M pairs: 87 us against 97 with 16 and 161
+// with 4); short ones spread over the chip.  Weighted pairs, whose distances
+// are one more dependent read, start at 2 (6,000 pairs, 200 K vertices: 7.3
+// us, 7.9 with 4; 12,000: 10.2 and 8.7).
+template <int K>
 uint32_t query_chunk(uint64_t k)
 {
-    uint32_t c = kQGroups;
+    if (K == kWeights && k <= 2 * kAlonePairs) return 2;
+    uint32_t c = 64 / kQLanes;
     while (c < 64 && (uint64_t)c * 2 * 8192 <= k) c *= 2;
     return c;
 }
@@ -814,12 +878,13 @@ pado_gpu_status launch_batch(const QIndex &X, const uint32_t *qa, const uint32_t
                              hipStream_t st)
 {
     if (k == 0) return PADO_GPU_OK;
-    const uint32_t chunk = query_chunk(k), grid = grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20);
-    if (X.rec)
-        hipLaunchKernelGGL((k_query<K, true, OT>), dim3(grid), dim3(256), 0, st, X, qa, qb, k, chunk, out, ref ? 1 : 0);
-    else
-        hipLaunchKernelGGL((k_query<K, false, OT>), dim3(grid), dim3(256), 0, st, X, qa, qb, k, chunk, out,
-                           ref ? 1 : 0);
+    const bool alone = k <= kAlonePairs;
+    const uint32_t chunk = alone ? 1u : query_chunk<K>(k), grid = grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20);
+    auto kern = X.rec ? (alone ? k_query<K, true, kAlone, OT> : k_query<K, true, kMixed, OT>)
+                      : (alone ? k_query<K, false, kAlone, OT> : k_query<K, false, kMixed, OT>);
+    if (K == kWeights && k > kWMixedPairs)
+        kern = X.rec ? k_query<K, true, kGrouped, OT> : k_query<K, false, kGrouped, OT>;
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, st, X, qa, qb, k, chunk, out, ref ? 1 : 0);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
