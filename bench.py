@@ -168,7 +168,7 @@ def serving_leg(ctx, scale=14, ef=8, duration_s=4.0, seed=5, stream=False):
     uniform, half Zipf(1.1) over degree rank.  Latency = completion - arrival
     (admission waits included).  Compared with the plain path: the same pairs
     in one query launch.  stream=True builds the index with per-kernel
-    launches instead of hipGraphs (for profiler runs)."""
+    launches and batches one by one (for profiler runs)."""
     edges, G, rank, rank2id = make_graph(scale, ef)
     cfg = pado.BuildCfg()
     cfg.batch_size = pado.BATCH_SIZE
@@ -441,7 +441,7 @@ def main():
     ap.add_argument("--copy-calibrate", type=int, default=0, metavar="MIB",
                     help="only run a plain device copy of MIB MiB (PMC byte-counter calibration) and exit")
     ap.add_argument("--stream", action="store_true",
-                    help="run the batch step as per-kernel launches with HIP-event timing instead of the default hipGraphs")
+                    help="run batches one by one with HIP-event timing of each launch instead of four at a time")
     ap.add_argument("--weighted-scale", type=int, default=22,
                     help="also build and serve a weighted R-MAT of this scale (0 = skip)")
     ap.add_argument("--multi-graphs", type=int, default=1024, metavar="N",
@@ -526,8 +526,8 @@ def main():
 
     # Roofline of the dominant labeling kernel (push or add), per launch.  The
     # stream-mode build brackets each push / add launch with HIP events on the
-    # build stream; a hipGraph build records none, so then one extra
-    # stream-mode build of the same graph (same kernels and grids) times them.
+    # build stream; a default build records none, so then one extra
+    # stream-mode build of the same graph (a batch at a time) times them.
     timing_src = "timed builds (HIP events on the build stream)"
     if not args.stream:
         tcfg = pado.BuildCfg()
@@ -539,7 +539,7 @@ def main():
         tb.close()
         for k in ("ms_push", "ms_add", "n_push", "n_add"):
             st[k] = st_t[k]
-        timing_src = "one stream-mode build after the timed hipGraph builds (HIP events on the build stream)"
+        timing_src = "one stream-mode build after the timed builds (HIP events on the build stream)"
     push_bytes = 8 * st["actives"] + 4 * st["edges"] + BP_RECORD_BYTES * st["tails"]
     add_bytes = 5 * st["dq_labels"] + 5 * st["labels_appended"]
     kern = {
@@ -658,7 +658,7 @@ def main():
         "config": {"workload": f"R-MAT scale {args.scale} ef {args.edge_factor} (0.57,0.19,0.19,0.05) seed 1, "
                                f"BATCH_SIZE=1024, BITPARALLEL_SIZE=50; full index build",
                    "num_v": G.num_v, "num_edges": int(edges.shape[0]),
-                   "batch_step": "stream (launch-ahead blocks)" if args.stream else "hipGraph"},
+                   "batch_step": "stream (launch-ahead blocks)" if args.stream else "four batches at a time"},
         "parity": parity, "query": query, "serving": serving, "weighted": weighted, "multi": multi,
         "roofline": roofline, "cpu_baseline": cpu,
         "build_breakdown_ms": {"bp": round(st["ms_bp"], 1), "batches_and_sort": round(st["ms_batch"], 1)},

@@ -191,11 +191,13 @@ typedef struct {
 /* Bit-parallel labeling one BFS per slot (as the reference runs it) instead of
  * the default single multi-source sweep over all 50 slots; same output. */
 #define PADO_GPU_BUILD_BP_PER_SLOT 1u
-/* The batch step runs by default as captured hipGraphs (batch prologue plus a
- * block of iterations, then iteration blocks until the frontier is empty).
- * With this flag it runs as per-kernel launches instead, each push / add
- * launch bracketed by HIP events (pado_gpu_index_info's ms_push / ms_add).
- * Same output either way. */
+/* The batch step runs by default four batches of 1,024 roots at a time, one such
+ * group ahead of the host's check (in captured hipGraphs where several builds
+ * run at once).  With this flag batches run one by one and each push / add
+ * launch is bracketed by HIP events (pado_gpu_index_info's ms_push / ms_add).
+ * Same labels either way, and the same iterations, pushes, ind_pass,
+ * bp_pruned, cands and dq_pruned; edges, tails, actives, dq_labels and dq_rows
+ * count what the chosen schedule scanned. */
 #define PADO_GPU_BUILD_STREAM 2u
 /* Wide hop domain (no reference counterpart: the reference's u8 level and
  * iteration counters wrap at 255, GLB:29-40, PARA:711/1470).  Labels carry

@@ -31,7 +31,7 @@ QUERY_DEVICE_PTRS = 1
 QUERY_REF_COMPAT = 2
 QUERY_RANK_SPACE = 4
 BUILD_BP_PER_SLOT = 1
-BUILD_STREAM = 2  # per-kernel launches with HIP-event timing (default: hipGraph batch step)
+BUILD_STREAM = 2  # batches one by one, launches timed with HIP events
 BUILD_WIDE = 4  # wide hop domain: 12-bit label distances, u16 answers (graphs deeper than 254)
 BUILD_DEVICE_LOOP = 8  # whole batch phase in one workgroup (deep graphs: many small iterations)
 WIDE_INF = 0xFFFF  # wide-domain query: unreachable

@@ -62,6 +62,34 @@ __device__ inline uint32_t wave_sum_u32(uint32_t x)
     return x;
 }
 
+// Bitmap rows of RW 64-bit words hold one bit per root of a batch.  RW = 16 is
+// the reference's batch of 1,024 roots; RW = 64 runs four of them as one (the
+// default schedule, see build_batches), lane l then owning word l of a row.
+template <uint32_t RW>
+struct Rows {
+    static constexpr uint32_t kRoots = RW * 64;
+    static constexpr uint32_t kPer = RW;  // roots per lane
+    using Bits = typename std::conditional<RW <= 32, uint32_t, uint64_t>::type;  // one lane's roots
+    using Mask = typename std::conditional<RW <= 32, uint32_t, uint64_t>::type;  // set of words of a row
+    static_assert(RW == 16 || RW == 64, "rows of 16 or 64 words");
+};
+constexpr uint32_t kRow = 16;       // words per row of the reference's batch
+constexpr uint32_t kWideRow = 64;   // four of them
+constexpr uint32_t kWideRowVertices = 1u << 22;
+
+__device__ inline uint32_t ctz_any(uint32_t x) { return (uint32_t)__builtin_ctz(x); }
+__device__ inline uint32_t ctz_any(uint64_t x) { return (uint32_t)__builtin_ctzll(x); }
+__device__ inline uint32_t popc_any(uint32_t x) { return (uint32_t)__popc(x); }
+__device__ inline uint32_t popc_any(uint64_t x) { return (uint32_t)__popcll(x); }
+__device__ inline uint32_t readlane_any(uint32_t x, uint32_t l) { return __builtin_amdgcn_readlane(x, l); }
+__device__ inline uint64_t readlane_any(uint64_t x, uint32_t l)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, l), hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), l);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+__device__ inline bool any_active(const uint32_t (&n_act)[4]) { return (n_act[0] | n_act[1] | n_act[2] | n_act[3]) != 0u; }
+
 __device__ inline unsigned long long *stat_rows(BuildCounters *C)
 {
     return reinterpret_cast<unsigned long long *>(C + 1);
@@ -193,7 +221,7 @@ __device__ inline unsigned long long bp_nz_filter(unsigned long long cs, unsigne
     return (two & nz1r & nz1t) | (o1 & ((nz1r & (nz1t | nz0t)) | (nz0r & nz1t)));
 }
 
-template <int IT>
+template <uint32_t R, int IT>
 __device__ inline bool bp_mask_scan_it(const unsigned long long *rm, uint32_t ro, const unsigned long long *lt,
                                        unsigned long long &cand, unsigned long long &one)
 {
@@ -202,7 +230,7 @@ __device__ inline bool bp_mask_scan_it(const unsigned long long *rm, uint32_t ro
     unsigned long long lr[L], tl[L];
 #pragma unroll
     for (int a = 0; a < L; ++a) {
-        lr[a] = rm[a * kBatch + ro];
+        lr[a] = rm[a * R + ro];
         tl[a] = lt[a];
     }
     unsigned long long hit = 0, e1 = 0, e2 = 0;
@@ -226,18 +254,19 @@ __device__ inline bool bp_mask_scan_it(const unsigned long long *rm, uint32_t ro
 
 // Same contract as bp_dist_scan for 1 <= iter <= kMaskIters (wave-uniform):
 // root offset ro's masks come from the batch's word-major root table rm
-// (rm[k * kBatch + ro]: lanes holding consecutive roots read consecutive
+// (rm[k * R + ro], R roots per batch: lanes holding consecutive roots read consecutive
 // words), the tail's from its mask row lt.
+template <uint32_t R>
 __device__ inline bool bp_mask_scan(uint32_t iter, const unsigned long long *rm, uint32_t ro,
                                     const unsigned long long *lt, unsigned long long &cand,
                                     unsigned long long &one)
 {
     switch (iter) {
-    case 1: return bp_mask_scan_it<1>(rm, ro, lt, cand, one);
-    case 2: return bp_mask_scan_it<2>(rm, ro, lt, cand, one);
-    case 3: return bp_mask_scan_it<3>(rm, ro, lt, cand, one);
-    case 4: return bp_mask_scan_it<4>(rm, ro, lt, cand, one);
-    default: return bp_mask_scan_it<5>(rm, ro, lt, cand, one);
+    case 1: return bp_mask_scan_it<R, 1>(rm, ro, lt, cand, one);
+    case 2: return bp_mask_scan_it<R, 2>(rm, ro, lt, cand, one);
+    case 3: return bp_mask_scan_it<R, 3>(rm, ro, lt, cand, one);
+    case 4: return bp_mask_scan_it<R, 4>(rm, ro, lt, cand, one);
+    default: return bp_mask_scan_it<R, 5>(rm, ro, lt, cand, one);
     }
 }
 
@@ -323,6 +352,7 @@ struct SetScratch {
 // L2 cache), tail set pairs from the vertex-major table (in the spread steps
 // lanes hold slots of the same few tails, whose records they share).
 // Returns whether the lane's pair is pruned.
+template <uint32_t R>
 __device__ inline bool bp_set_phase(unsigned long long rem, unsigned long long one, const ulonglong2 *rset,
                                     uint32_t ro, const ulonglong2 *bps, uint32_t t, const SetScratch &sc)
 {
@@ -334,10 +364,10 @@ __device__ inline bool bp_set_phase(unsigned long long rem, unsigned long long o
         const bool two = rem != 0ull;
         const uint32_t i1 = two ? (uint32_t)__ffsll(rem) - 1 : i0;
         if (two) rem &= rem - 1;
-        const ulonglong2 r0 = rset[i0 * kBatch + ro], t0 = bps[(uint64_t)t * kBP + i0];
+        const ulonglong2 r0 = rset[i0 * R + ro], t0 = bps[(uint64_t)t * kBP + i0];
         ulonglong2 r1 = make_ulonglong2(0ull, 0ull), t1 = r1;
         if (two) {
-            r1 = rset[i1 * kBatch + ro];
+            r1 = rset[i1 * R + ro];
             t1 = bps[(uint64_t)t * kBP + i1];
         }
         if (bp_set_hit(r0, t0, (one >> i0) & 1ull) || (two && bp_set_hit(r1, t1, (one >> i1) & 1ull))) {
@@ -362,7 +392,7 @@ __device__ inline bool bp_set_phase(unsigned long long rem, unsigned long long o
         const uint32_t o = item_owner(sc.ex, x);
         const unsigned long long ro_rem = sc.rem[o];
         const uint32_t i = nth_set_bit(ro_rem, x - sc.ex[o]);
-        const ulonglong2 rr = rset[i * kBatch + sc.r[o]], tt = bps[(uint64_t)sc.t[o] * kBP + i];
+        const ulonglong2 rr = rset[i * R + sc.r[o]], tt = bps[(uint64_t)sc.t[o] * kBP + i];
         if (bp_set_hit(rr, tt, (sc.one[o] >> i) & 1ull)) atomicOr(&sc.hit[o], 1u);
     }
     wave_lds_sync();
@@ -408,8 +438,8 @@ struct HubList1 {
 };
 
 // Summary of one row of the root-distance table (hub h): near[k] has bit l
-// set iff some batch root in [16l, 16l+16) -- the roots lane l of k_add owns --
-// is at distance k + 1 from h; info is 0xFFFFFF00 | the minimum distance of
+// set iff one of the batch roots that lane l of k_add owns (Rows::kPer) is at
+// distance k + 1 from h; info is 0xFFFFFF00 | the minimum distance of
 // any batch root (0xFFFFFFFF when h is no hub of any of them).  A hub can
 // prune a candidate root r of v only if d_r(h) <= iter - d_v(h), so for
 // thresholds up to kNear the masks name the lanes whose row slices can
@@ -519,7 +549,7 @@ __global__ __launch_bounds__(256) void k_bp_masks(uint32_t n, const uint8_t *bpd
 // offset ro's labels pool[base, base + len) are entered (fill) or their
 // entries reset, by `parts` waves of which this is number `part`; each lane
 // handles four labels per step so the dependent loads of a step overlap.
-template <bool W>
+template <bool W, uint32_t RW>
 __device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned long long base, uint32_t len,
                                          uint32_t part, uint32_t parts, LabelStore S, HubInfo *hinfo,
                                          typename Hop<W>::Dist *dc)
@@ -538,7 +568,7 @@ __device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned lo
             for (int u = 0; u < 4; ++u) {
                 if (lab[u] == kEmpty) continue;
                 const uint32_t h = lab[u] >> B;
-                dc[(uint64_t)h * kBatch + ro] = (typename Hop<W>::Dist)~0u;
+                dc[(uint64_t)h * Rows<RW>::kRoots + ro] = (typename Hop<W>::Dist)~0u;
                 hub_info_clear(hinfo[h]);
             }
             continue;
@@ -547,12 +577,12 @@ __device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned lo
 #pragma unroll
         for (int u = 0; u < 4; ++u)
             if (lab[u] != kEmpty) hi[u] = hinfo[lab[u] >> B];
-        const unsigned long long bit = 1ull << (ro >> 4);
+        const unsigned long long bit = 1ull << (ro / Rows<RW>::kPer);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             if (lab[u] == kEmpty) continue;
             const uint32_t h = lab[u] >> B, d = lab[u] & INF;
-            dc[(uint64_t)h * kBatch + ro] = (typename Hop<W>::Dist)d;
+            dc[(uint64_t)h * Rows<RW>::kRoots + ro] = (typename Hop<W>::Dist)d;
             // The minimum only falls and mask bits are only set during the
             // kernel, so a value read as already there (even a stale one)
             // makes the atomic a no-op.
@@ -577,12 +607,12 @@ __device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned lo
 // counters left are the push-descriptor count, updated once per block, and
 // the frontier's push-edge count.
 constexpr uint32_t kRootWaves = 4, kInitRoots = 4;
-template <bool W, uint32_t CH>
+template <bool W, uint32_t CH, uint32_t RW>
 __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, const uint8_t *used, const uint64_t *off, const uint32_t *adj,
                                                      LabelStore S, HubInfo *hinfo, typename Hop<W>::Dist *dc,
                                                      unsigned long long *ind, unsigned long long *vmark,
                                                      uint32_t *tlist, unsigned long long *abits, unsigned long long *ag,
-                                                     uint32_t *amask, uint32_t *aend, unsigned long long *chunks,
+                                                     uint64_t *amask, uint32_t *aend, unsigned long long *chunks,
                                                      const ulonglong2 *bps, ulonglong2 *rset,
                                                      const unsigned long long *lmask, unsigned long long *rmask,
                                                      BuildCounters *C)
@@ -602,7 +632,7 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     if (live) rec0 = S.rec[r];
     __syncthreads();
     if (part != 0) {
-        if (live) hub_rows<W>(1u, ro, rec0.base, rec0.len, part - 1u, kRootWaves - 1u, S, hinfo, dc);
+        if (live) hub_rows<W, RW>(1u, ro, rec0.base, rec0.len, part - 1u, kRootWaves - 1u, S, hinfo, dc);
         __syncthreads();
         __syncthreads();
         return;
@@ -615,8 +645,8 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     }
     // Slot-major copy of the batch roots' bit-parallel sets and word-major
     // copy of their mask rows (push's bit-parallel check).
-    if (ro < rsz && lane < kBP) rset[lane * kBatch + ro] = bps[(uint64_t)r * kBP + lane];
-    if (ro < rsz && lane < kLmNz0 + 1) rmask[lane * kBatch + ro] = lmask[(uint64_t)r * kLmWords + lane];
+    if (ro < rsz && lane < kBP) rset[lane * Rows<RW>::kRoots + ro] = bps[(uint64_t)r * kBP + lane];
+    if (ro < rsz && lane < kLmNz0 + 1) rmask[lane * Rows<RW>::kRoots + ro] = lmask[(uint64_t)r * kLmWords + lane];
     uint32_t pdeg = 0;
     if (live) {
         const uint32_t len = rec0.len;
@@ -624,16 +654,16 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
         if (base != ~0ull) {
             if (lane == 0) {
                 // the root-distance entry of the self label
-                dc[(uint64_t)r * kBatch + ro] = 0;
+                dc[(uint64_t)r * Rows<RW>::kRoots + ro] = 0;
                 atomicMin(&hinfo[r].info, ~Hop<W>::kInf);
                 S.pool[base + len] = r << Hop<W>::kBits;  // (hub r, dist 0), PARA:932-949
                 S.rec[r].len = len + 1;
-                ind[(uint64_t)r * kWords + (ro >> 6)] |= 1ull << (ro & 63);
-                amask[r] = 1u << (ro >> 6);
+                ind[(uint64_t)r * RW + (ro >> 6)] |= 1ull << (ro & 63);
+                amask[r] = 1ull << (ro >> 6);
                 // frontier of iteration 1: slot 1 of the bitmap
                 atomicOr(&abits[C->abits_words + (r >> 6)], 1ull << (r & 63));
             }
-            if (lane < kWords) ag[(uint64_t)r * kWords + lane] = (lane == (ro >> 6)) ? (1ull << (ro & 63)) : 0ull;
+            if (lane < RW) ag[(uint64_t)r * RW + lane] = (lane == (ro >> 6)) ? (1ull << (ro & 63)) : 0ull;
             pdeg = push_degree(off, adj, r, rs);
             if (lane == 0) aend[r] = pdeg;
         }
@@ -665,24 +695,24 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     }
 }
 
-template <bool W, uint32_t CH>
+template <bool W, uint32_t CH, uint32_t RW>
 __global__ __launch_bounds__(kInitRoots * kRootWaves * 64) void k_batch_init(const uint8_t *used, const uint64_t *off, const uint32_t *adj,
                                                      LabelStore S, HubInfo *hinfo, typename Hop<W>::Dist *dc,
                                                      unsigned long long *ind, unsigned long long *vmark,
                                                      uint32_t *tlist, unsigned long long *abits, unsigned long long *ag,
-                                                     uint32_t *amask, uint32_t *aend, unsigned long long *chunks,
+                                                     uint64_t *amask, uint32_t *aend, unsigned long long *chunks,
                                                      const ulonglong2 *bps, ulonglong2 *rset,
                                                      const unsigned long long *lmask, unsigned long long *rmask,
                                                      BuildCounters *C)
 {
-    batch_init_body<W, CH>(blockIdx.x, gridDim.x, used, off, adj, S, hinfo, dc, ind, vmark, tlist, abits, ag, amask, aend,
+    batch_init_body<W, CH, RW>(blockIdx.x, gridDim.x, used, off, adj, S, hinfo, dc, ind, vmark, tlist, abits, ag, amask, aend,
                            chunks, bps, rset, lmask, rmask, C);
 }
 
 // The root-distance entries of the previous batch's roots (the labels they
 // held at its end, which include every entry written during it) are reset,
 // kRootWaves waves per root.
-template <bool W>
+template <bool W, uint32_t RW>
 __device__ __forceinline__ void hub_reset_body(uint32_t bid, const uint8_t *used, LabelStore S, HubInfo *hinfo,
                                                typename Hop<W>::Dist *dc, const BuildCounters *C)
 {
@@ -693,7 +723,7 @@ __device__ __forceinline__ void hub_reset_body(uint32_t bid, const uint8_t *used
     const uint32_t r = rs + ro;
     if (used[r]) return;
     const LRec rec = S.rec[r];
-    hub_rows<W>(0u, ro, rec.base, rec.len, w % kRootWaves, kRootWaves, S, hinfo, dc);
+    hub_rows<W, RW>(0u, ro, rec.base, rec.len, w % kRootWaves, kRootWaves, S, hinfo, dc);
 }
 
 
@@ -765,7 +795,7 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
                     const uint32_t kk = __shfl(k, (int)(16 * g + sl));
                     x[u] = 0ull;
                     if (gm) {
-                        x[u] = ag[(uint64_t)kk * kWords + w] & wm;
+                        x[u] = ag[(uint64_t)kk * kRow + w] & wm;
                         gm &= gm - 1u;
                     }
                 }
@@ -784,9 +814,9 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
         // this iteration)
         unsigned long long nb = 0ull;
         if (acc) {
-            const unsigned long long seen = ind[(uint64_t)t * kWords + w];
+            const unsigned long long seen = ind[(uint64_t)t * kRow + w];
             nb = acc & ~seen;
-            if (nb) ind[(uint64_t)t * kWords + w] = seen | acc;
+            if (nb) ind[(uint64_t)t * kRow + w] = seen | acc;
         }
         const uint32_t cnt = (uint32_t)__popcll(nb);
         n_pass += cnt;
@@ -812,7 +842,7 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
                     to = s_t[o];
                     const unsigned long long *lt = lmask + (uint64_t)to * kLmWords;
                     if (use_masks) {
-                        dist_pr = bp_mask_scan(iter, rmask, ro, lt, cs, one);
+                        dist_pr = bp_mask_scan<kBatch>(iter, rmask, ro, lt, cs, one);
                     } else {
                         uint32_t dr[13], dt[13];
                         load_dline(bpd, rs + ro, dr);
@@ -827,7 +857,7 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
                         cs = bp_nz_filter(cs, one, rmask[kLmNz1 * kBatch + ro], rmask[kLmNz0 * kBatch + ro], lt[kLmNz1],
                                           lt[kLmNz0]);
                 }
-                const bool set_pr = bp_set_phase(dist_pr ? 0ull : cs, one, rset, ro, bps, to, sc);
+                const bool set_pr = bp_set_phase<kBatch>(dist_pr ? 0ull : cs, one, rset, ro, bps, to, sc);
                 if (xa) {
                     if (dist_pr || set_pr)
                         ++n_bp;
@@ -841,7 +871,7 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
             wave_lds_sync();
         }
         if (keep) {
-            cand[(uint64_t)t * kWords + w] = keep;  // the row was empty (k_add clears what it takes)
+            cand[(uint64_t)t * kRow + w] = keep;  // the row was empty (k_add clears what it takes)
             n_cand += (uint32_t)__popcll(keep);
         }
         const bool touched = ((__ballot(nb != 0ull) >> (16 * g)) & 0xFFFFull) != 0ull;
@@ -876,11 +906,11 @@ __device__ __forceinline__ void pull_step(uint32_t wave, uint32_t nwaves, uint32
 // An iteration whose frontier has more push edges than pull_ratio / 1000 of
 // the adjacency entries at or above roots_start runs in pull form instead
 // (pull_step; ~0u: never; PL = false compiles the pull form out).
-template <bool W, uint32_t CH, uint32_t PW, bool PL = true>
+template <bool W, uint32_t CH, uint32_t PW, uint32_t RW, bool PL = RW == kRow>
 __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t iter, const uint64_t *off,
                                               const uint32_t *adj, unsigned long long *abits,
                                               const unsigned long long *ag,
-                                              const uint32_t *amask, const uint32_t *aend,
+                                              const uint64_t *amask, const uint32_t *aend,
                                               const unsigned long long *chunks, unsigned long long *ind,
                                               unsigned long long *cand, unsigned long long *vmark, uint32_t *tlist,
                                               uint32_t *clist,
@@ -890,12 +920,16 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                                               uint32_t pull_ratio)
 {
     static_assert(CH >= 4 && CH <= 64 && (CH & (CH - 1)) == 0, "chunk: a power of two in [4, 64]");
+    static_assert(!PL || RW == kRow, "the pull form is written for rows of 16 words");
     constexpr uint32_t DPS = 64 / CH;  // descriptors per wave step
+    constexpr uint32_t R = Rows<RW>::kRoots;
+    using Mask = typename Rows<RW>::Mask;
     __shared__ unsigned long long s_nb[PW][4][64]; // fresh roots of each lane's edge, per word of the step
     __shared__ unsigned long long s_keep[PW][4][64];  // of those, the ones the BP check keeps
     __shared__ uint32_t s_ex[PW][64];              // exclusive prefix of the lanes' fresh counts
     __shared__ uint32_t s_cu[PW][64];              // a lane's running counts over its four words
     __shared__ uint32_t s_t[PW][64];               // each lane's tail
+    __shared__ uint32_t s_w[PW][64];               // a lane's words of the step, one per byte
     // set-phase scratch (bp_set_phase)
     __shared__ unsigned long long s_srem[PW][64], s_sone[PW][64];
     __shared__ uint32_t s_sro[PW][64], s_st[PW][64], s_sex[PW][64], s_shit[PW][64];
@@ -913,8 +947,8 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
     // other slot, which k_add fills with the next frontier.
     if (C->hold) return;
     const uint32_t p = iter & 1u;
-    const uint32_t n_act0 = C->n_act[p];
-    const bool live = n_act0 != 0 && iter < Hop<W>::kInf;
+    const bool act0 = any_active(C->n_act[p]);
+    const bool live = act0 && iter < Hop<W>::kInf;
     const uint32_t nc = live ? C->n_chunk[p] : 0u;
     const uint32_t rs = C->rs, gen_batch = C->gen_batch;
     const unsigned long long gen_iter = ((unsigned long long)gen_batch << 16) | iter;
@@ -925,14 +959,17 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                       C->n_pedge[p] * 1000ull > (unsigned long long)(off[n] - off[rs]) * pull_ratio;
     if (bid == 0 && threadIdx.x == 0) {
         C->iter_last = iter;
-        C->n_act[p ^ 1u] = 0;
+        for (uint32_t q = 0; q < 4; ++q) C->n_act[p ^ 1u][q] = 0;
         C->n_chunk[p ^ 1u] = 0;
         C->n_pedge[p ^ 1u] = 0;
-        if (n_act0 != 0) {
+        if (act0) {
             if (iter >= Hop<W>::kInf) {
                 C->domain = 1;
             } else {
-                C->iterations += 1;
+                uint32_t subs = 0;
+                for (uint32_t q = 0; q < 4; ++q) subs += C->n_act[p][q] != 0u ? 1u : 0u;
+                C->iterations += subs;
+                C->steps += 1;
                 if (pull) C->pulls += 1;
             }
         }
@@ -952,7 +989,8 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
     for (uint32_t c0 = wave * DPS; !pull && c0 < nc; c0 += nwaves * DPS) {
         const uint32_t c = c0 + lane / CH;
         const unsigned long long desc = c < nc ? chunks[c] : kChunkPad;
-        uint32_t k = 0, t = 0, lim = 0, words = 0;
+        uint32_t k = 0, t = 0, lim = 0;
+        Mask words = 0;
         if (desc != kChunkPad) {
             k = (uint32_t)desc;
             const uint32_t e = (uint32_t)(desc >> 32) + (lane & (CH - 1));
@@ -961,22 +999,23 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                 t = adj[off[k] + e];
                 lim = t - rs;  // roots with offset < lim satisfy root < tail (PARA:1134)
                 // words w with w * 64 < lim
-                words = amask[k] & (lim >= kBatch ? 0xFFFFu : ((1u << ((lim + 63) / 64)) - 1u));
+                const uint32_t nw64 = lim >= R ? RW : (lim + 63) / 64;
+                words = (Mask)(amask[k] & (nw64 == 64 ? ~0ull : (1ull << nw64) - 1ull));
             }
         }
         s_t[wv][lane] = t;
-        uint32_t wall = wave_or(words);  // a scalar: the step's word choice lives in scalar registers
         bool touched = false, got = false;
-        while (wall) {
-            // Up to four root words per step (wave-uniform): their indicator
-            // test-and-sets are issued together, and their fresh pairs share
-            // the bit-parallel passes.
-            uint32_t wsel[4] = {0u, 0u, 0u, 0u}, gsel = 0;
+        while (__ballot(words != 0) != 0ull) {
+            // Up to four of each lane's root words per step: their indicator
+            // test-and-sets are issued together, and the fresh pairs of all
+            // lanes share the bit-parallel passes.
+            uint32_t wsel[4], gsel = 0;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                if (wall) {
-                    wsel[u] = __ffs(wall) - 1;
-                    wall &= wall - 1;
+                wsel[u] = 0;
+                if (words) {
+                    wsel[u] = ctz_any(words);
+                    words &= words - 1;
                     gsel |= 1u << u;
                 }
             }
@@ -986,10 +1025,10 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                 g[u] = 0ull;
                 seen[u] = 0ull;
                 const uint32_t w = wsel[u];
-                if (((gsel >> u) & 1u) && ((words >> w) & 1u)) {
-                    g[u] = ag[(uint64_t)k * kWords + w];
+                if ((gsel >> u) & 1u) {
+                    g[u] = ag[(uint64_t)k * RW + w];
                     if (lim < (w + 1) * 64) g[u] &= (1ull << (lim - w * 64)) - 1ull;
-                    seen[u] = ind[(uint64_t)t * kWords + w];
+                    seen[u] = ind[(uint64_t)t * RW + w];
                 }
             }
             // Bits are only set during the kernel, so bits read as set are
@@ -999,7 +1038,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                 nb[u] = 0ull;
                 if (g[u]) {
                     n_push += __popcll(g[u]);
-                    if (g[u] & ~seen[u]) nb[u] = g[u] & ~atomicOr(&ind[(uint64_t)t * kWords + wsel[u]], g[u]);
+                    if (g[u] & ~seen[u]) nb[u] = g[u] & ~atomicOr(&ind[(uint64_t)t * RW + wsel[u]], g[u]);
                 }
             }
             const uint32_t cu1 = (uint32_t)__popcll(nb[0]);
@@ -1020,6 +1059,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
             }
             s_ex[wv][lane] = incl - cnt;
             s_cu[wv][lane] = cu1 | (cu2 << 10) | (cu3 << 20);
+            s_w[wv][lane] = wsel[0] | (wsel[1] << 8) | (wsel[2] << 16) | (wsel[3] << 24);
             wave_lds_sync();
             // Fresh pair x of the wave: owner lane o (the last lane whose
             // prefix is <= x; it has a fresh root), then its word u and root
@@ -1040,10 +1080,10 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                     u = (rank >= c1 ? 1u : 0u) + (rank >= c2 ? 1u : 0u) + (rank >= c3 ? 1u : 0u);
                     const uint32_t base = u == 0 ? 0u : (u == 1 ? c1 : (u == 2 ? c2 : c3));
                     b = nth_set_bit(s_nb[wv][u][o], rank - base);
-                    w = u == 0 ? wsel[0] : (u == 1 ? wsel[1] : (u == 2 ? wsel[2] : wsel[3]));
+                    w = (s_w[wv][o] >> (8 * u)) & 255u;
                     to = s_t[wv][o];
                     if (use_masks) {
-                        dist_pr = bp_mask_scan(iter, rmask, w * 64 + b, lmask + (uint64_t)to * kLmWords, cs, one);
+                        dist_pr = bp_mask_scan<R>(iter, rmask, w * 64 + b, lmask + (uint64_t)to * kLmWords, cs, one);
                     } else {
                         const uint4 *rl = reinterpret_cast<const uint4 *>(bpd + (uint64_t)(rs + w * 64 + b) * kBpdStride);
                         const uint4 *tl = reinterpret_cast<const uint4 *>(bpd + (uint64_t)to * kBpdStride);
@@ -1065,11 +1105,11 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                     if (!dist_pr && cs) {
                         const uint32_t ro = w * 64 + b;
                         const unsigned long long *lt = lmask + (uint64_t)to * kLmWords;
-                        cs = bp_nz_filter(cs, one, rmask[kLmNz1 * kBatch + ro], rmask[kLmNz0 * kBatch + ro], lt[kLmNz1],
+                        cs = bp_nz_filter(cs, one, rmask[kLmNz1 * R + ro], rmask[kLmNz0 * R + ro], lt[kLmNz1],
                                           lt[kLmNz0]);
                     }
                 }
-                const bool set_pr = bp_set_phase(dist_pr ? 0ull : cs, one, rset, w * 64 + b, bps, to, sc);
+                const bool set_pr = bp_set_phase<R>(dist_pr ? 0ull : cs, one, rset, w * 64 + b, bps, to, sc);
                 if (act) {
                     if (dist_pr || set_pr)
                         ++n_bp;
@@ -1082,7 +1122,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
             for (int u = 0; u < 4; ++u) {
                 const unsigned long long pass = s_keep[wv][u][lane];
                 if (pass) {
-                    atomicOr(&cand[(uint64_t)t * kWords + wsel[u]], pass);
+                    atomicOr(&cand[(uint64_t)t * RW + wsel[u]], pass);
                     n_cand += __popcll(pass);
                     got = true;
                 }
@@ -1117,11 +1157,11 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
         add_stats<0>(stat_rows(C), wave, {n_edge, n_tail, n_push, n_pass, n_bp, n_cand});
 }
 
-template <bool W, uint32_t CH, uint32_t PW>
+template <bool W, uint32_t CH, uint32_t PW, uint32_t RW>
 __global__ __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_push(uint32_t iter, const uint64_t *off,
                                               const uint32_t *adj, unsigned long long *abits,
                                               const unsigned long long *ag,
-                                              const uint32_t *amask, const uint32_t *aend,
+                                              const uint64_t *amask, const uint32_t *aend,
                                               const unsigned long long *chunks, unsigned long long *ind,
                                               unsigned long long *cand, unsigned long long *vmark, uint32_t *tlist,
                                               uint32_t *clist,
@@ -1130,55 +1170,56 @@ __global__ __launch_bounds__(PW * 64) __attribute__((amdgpu_waves_per_eu(4))) vo
                                               const ulonglong2 *rset, BuildCounters *C, uint32_t bp_prune,
                                               uint32_t pull_ratio)
 {
-    push_body<W, CH, PW>(blockIdx.x, gridDim.x, iter, off, adj, abits, ag, amask, aend, chunks, ind, cand, vmark, tlist,
+    push_body<W, CH, PW, RW>(blockIdx.x, gridDim.x, iter, off, adj, abits, ag, amask, aend, chunks, ind, cand, vmark, tlist,
                          clist, bpd, lmask, rmask, bps, rset, C, bp_prune, pull_ratio);
 }
 
-// Batch b's schedule into the counters: roots [rs, rs + rsz), cnt of them
-// not bit-parallel (the first frontier, one self label each).
-__device__ inline void batch_begin_write(BuildCounters *C, uint32_t b, uint32_t rs, uint32_t rsz, uint32_t cnt)
+// Batch b's schedule into the counters: roots [rs, rs + rsz), cnt[q] of the
+// q-th 1,024 not bit-parallel (the first frontier, one self label each).
+__device__ inline void batch_begin_write(BuildCounters *C, uint32_t b, uint32_t rs, uint32_t rsz,
+                                         const uint32_t (&cnt)[4])
 {
     C->next_batch = b + 1;
     C->rs = rs;
     C->rsz = rsz;
     C->gen_batch = b + 1;
-    C->n_act[0] = 0;
-    C->n_act[1] = cnt;
+    uint32_t all = 0;
+    for (uint32_t q = 0; q < 4; ++q) {
+        C->n_act[0][q] = 0;
+        C->n_act[1][q] = cnt[q];
+        all += cnt[q];
+    }
     C->n_pedge[0] = C->n_pedge[1] = 0;
     C->n_chunk[0] = C->n_chunk[1] = 0;
     C->n_cand[0] = C->n_cand[1] = 0;
     C->n_touched = rsz;
-    C->labels += cnt;
-    C->actives += cnt;
+    C->labels += all;
+    C->actives += all;
 }
 
 // Start of a batch (construct's loop over batches, PARA:1791-1812): roots
 // [b * batch, ...) with b taken from the device-side batch counter.  One
-// thread per root offset: the block also counts the batch's
-// non-bit-parallel roots, which are the first frontier (active slots and
-// touched-list slots [0, rsz) belong to the root offsets, filled by
-// k_batch_init) and get one self label each.
-__device__ __forceinline__ void batch_begin_body(uint32_t bid, uint32_t nblk, const uint8_t *used, BuildCounters *C, uint32_t batch,
+// block of 1,024 threads: it also counts the batch's non-bit-parallel roots,
+// which are the first frontier (active slots and touched-list slots [0, rsz)
+// belong to the root offsets, filled by k_batch_init) and get one self label
+// each.
+__global__ __launch_bounds__(1024) void k_batch_begin(const uint8_t *used, BuildCounters *C, uint32_t batch,
                                                       uint32_t n)
 {
     if (C->hold) return;
     const uint32_t b = C->next_batch;
     const uint32_t rs = b * batch;
     const uint32_t rsz = rs < n ? min(batch, n - rs) : 0u;
-    const uint32_t o = threadIdx.x;
-    const uint32_t cnt = (uint32_t)__syncthreads_count(o < rsz && !used[rs + o]);
-    if (o != 0) return;
-    batch_begin_write(C, b, rs, rsz, cnt);
+    uint32_t cnt[4];
+    for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t o = q * kBatch + threadIdx.x;
+        cnt[q] = (uint32_t)__syncthreads_count(o < rsz && !used[rs + o]);
+    }
+    if (threadIdx.x == 0) batch_begin_write(C, b, rs, rsz, cnt);
 }
 
-__global__ __launch_bounds__(1024) void k_batch_begin(const uint8_t *used, BuildCounters *C, uint32_t batch,
-                                                      uint32_t n)
-{
-    batch_begin_body(blockIdx.x, gridDim.x, used, C, batch, n);
-}
-
-// add (PARA:1568-1665): one wave per candidate vertex v.  Lane l owns roots
-// [16l, 16l+16).  distance_query (PARA:1218-1270) runs over v's labels with
+// add (PARA:1568-1665): one wave per candidate vertex v.  Lane l owns
+// Rows::kPer consecutive roots.  distance_query (PARA:1218-1270) runs over v's labels with
 // dist < iter: a hub h can prune only if d_v(h) + min_r d_r(h) <= iter, so a
 // per-hub minimum filters most hubs before the 1 KB root-distance row of the
 // survivors is read (16 B per lane).  Only hubs below the candidate root
@@ -1186,20 +1227,53 @@ __global__ __launch_bounds__(1024) void k_batch_begin(const uint8_t *used, Build
 // pushes to v) never prunes: iteration 1, whose only labels with dist < 1 are
 // such self labels, scans nothing, and iteration 2 scans v's distance-1 list
 // instead of the whole label array.
-constexpr uint32_t kAddHubs = 2;  // root-distance rows k_add loads per step
+// Root-distance rows k_add loads per step (two: a wide row's slice in the wide
+// hop domain, 128 bytes, fills 32 registers).
+template <bool W, uint32_t RW>
+constexpr uint32_t kAddHubs = W && RW == kWideRow ? 1 : 2;
 constexpr uint32_t kGather = 8;   // candidate roots up to which k_add reads single entries
+
+// Which of the N entries of a root-distance slice are at most thr, as bits: u8
+// entries four to a word (u16: two), compared as packed values.
+template <bool W, uint32_t N>
+__device__ inline typename std::conditional<N <= 32, uint32_t, uint64_t>::type slice_le(const uint32_t *x, uint32_t thr)
+{
+    using Bits = typename std::conditional<N <= 32, uint32_t, uint64_t>::type;
+    Bits bits = 0;
+    if constexpr (W) {
+        const uint32_t k = (0x7FFFu - thr) * 0x00010001u;  // thr < 4095
+#pragma unroll
+        for (uint32_t q = 0; q < N / 2; ++q) {
+            const uint32_t le = ~(((x[q] & 0x7FFF7FFFu) + k) | x[q]);
+            bits |= (Bits)(((le >> 15) & 1u) | ((le >> 30) & 2u)) << (2 * q);
+        }
+    } else {
+        // s: the low seven bits are above thr's; then by the top bits.
+        const uint32_t k = (0x7Fu - (thr & 0x7Fu)) * 0x01010101u;
+        const bool low = thr < 128u;
+#pragma unroll
+        for (uint32_t q = 0; q < N / 4; ++q) {
+            const uint32_t s = (x[q] & 0x7F7F7F7Fu) + k;
+            const uint32_t le = ~(low ? s | x[q] : s & x[q]) & 0x80808080u;
+            bits |= (Bits)((le * 0x00204081u) >> 28) << (4 * q);
+        }
+    }
+    return bits;
+}
 
 // DEEP compiles in the hub-parallel distance query (see below), which only
 // iterations past kNear + 1 use; the launch schedule runs the other
 // instantiation for the iterations before, whose code it leaves as lean as
 // it was.
-template <bool W, uint32_t CH, bool DEEP = true>
+template <bool W, uint32_t CH, uint32_t RW, bool DEEP = true>
 __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t iter, const uint8_t *used, const uint64_t *off, const uint32_t *adj, const uint32_t *clist,
                                              unsigned long long *cand, LabelStore S, HubList1 H1, HubInfo *hinfo,
                                              typename Hop<W>::Dist *dc,
-                                             unsigned long long *abits, unsigned long long *ag, uint32_t *amask,
+                                             unsigned long long *abits, unsigned long long *ag, uint64_t *amask,
                                              uint32_t *aend, unsigned long long *chunks, BuildCounters *C)
 {
+    constexpr uint32_t R = Rows<RW>::kRoots, PER = Rows<RW>::kPer, HUBS = kAddHubs<W, RW>;
+    using Bits = typename Rows<RW>::Bits;
     const uint32_t lane = lane_id();
     const uint32_t wave = (bid * blockDim.x + threadIdx.x) >> 6;
     const uint32_t nwaves = (nblk * blockDim.x) >> 6;
@@ -1218,7 +1292,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
     // per wave, so the shared counter sees one atomic per reservation, not per
     // vertex; unused descriptor slots are padded.  The active count and the
     // frontier's push edges are added once per wave at the end.
-    uint32_t c_next = 0, c_left = 0, my_act = 0;
+    uint32_t c_next = 0, c_left = 0, my_act = 0, my_subs = 0;
     uint32_t my_pedge = 0;  // push edges of this wave's new frontier entries (flushed below 2^31)
     unsigned long long *nbits = abits + (uint64_t)(p ^ 1u) * C->abits_words;
     // The loop over this wave's candidates (grid-stride: i, i + nwaves, ...)
@@ -1230,7 +1304,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
     // read three ahead.  The vertices differ, so none of these loads can see
     // a store of an earlier candidate.
     struct StageA {
-        unsigned long long word;  // candidate bits of this lane's four words' quarter
+        unsigned long long word;  // the row word with this lane's candidate bits
         LRec rec;
         uint64_t e0, e1;
         uint32_t v, used, n1;
@@ -1242,7 +1316,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         StageA a{};
         a.v = v;
         if (ok) {
-            a.word = cand[(uint64_t)v * kWords + (lane >> 2)];
+            a.word = cand[(uint64_t)v * RW + lane * PER / 64];
             a.rec = S.rec[v];
             a.used = used[v];
             a.e0 = off[v];
@@ -1311,56 +1385,59 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
                               : e1 - e0 <= 64u
                                   ? (uint32_t)__popcll(__ballot(lane < e1 - e0 && cbl.probe >= rs))
                                   : push_degree_range(adj, e0, e1, rs);
-        const uint32_t cb = (uint32_t)(word >> (16 * (lane & 3))) & 0xFFFFu;
+        Bits cb;
+        if constexpr (RW == kRow)
+            cb = (uint32_t)(word >> (16 * (lane & 3))) & 0xFFFFu;
+        else
+            cb = word;
         // The clear below is control-dependent on every lane's loaded word
         // (through the ballot), so no lane can clear a word before all lanes
         // have read it.
-        if (__ballot(cb != 0) != 0ull && lane < kWords) cand[(uint64_t)v * kWords + lane] = 0ull;
-        uint32_t prune = 0;
-        const uint32_t my_lo = rs + 16 * lane;  // real id of this lane's first root
+        if (__ballot(cb != 0) != 0ull && lane < RW) cand[(uint64_t)v * RW + lane] = 0ull;
+        Bits prune = 0;
+        const uint32_t my_lo = rs + PER * lane;  // real id of this lane's first root
         // The passing hubs of one set of 64 labels (h, d, lm per lane): up to
-        // kAddHubs per step, their row loads issued together; only lanes of
-        // the hub's mask that still hold an unpruned candidate load their
-        // slice of a row (16 entries: 16 bytes, 32 wide).
+        // HUBS per step, their row loads issued together; only lanes of the
+        // hub's mask that still hold an unpruned candidate load their slice of
+        // a row (PER entries).
         auto hub_pass = [&](uint32_t h, uint32_t d, unsigned long long lm) {
             // A hub is worth a row only if some lane that still holds an
             // unpruned candidate has a root close enough to it.
-            const unsigned long long live = __ballot((cb & ~prune) != 0u);
+            const unsigned long long live = __ballot((cb & ~prune) != 0);
             unsigned long long m = __ballot((lm & live) != 0ull);
             while (m) {
-                int src[kAddHubs];
-                bool ok[kAddHubs];
+                int src[HUBS];
+                bool ok[HUBS];
 #pragma unroll
-                for (int u = 0; u < (int)kAddHubs; ++u) {
+                for (int u = 0; u < (int)HUBS; ++u) {
                     ok[u] = m != 0ull;
                     src[u] = ok[u] ? __ffsll(m) - 1 : 0;
                     if (ok[u]) m &= m - 1;
                 }
-                const bool need = (cb & ~prune) != 0u;
-                constexpr uint32_t RV = W ? 2 : 1;  // 16-byte vectors of a lane's slice
-                uint32_t hh[kAddHubs], thr[kAddHubs];
-                uint4 row[kAddHubs][RV];
+                const bool need = (cb & ~prune) != 0;
+                constexpr uint32_t RV = PER * sizeof(typename Hop<W>::Dist) / 16;  // 16-byte vectors of a lane's slice
+                uint32_t hh[HUBS], thr[HUBS];
+                uint4 row[HUBS][RV];
 #pragma unroll
-                for (int u = 0; u < (int)kAddHubs; ++u) {
-                    hh[u] = __shfl(h, src[u]);
+                for (int u = 0; u < (int)HUBS; ++u) {
+                    hh[u] = __builtin_amdgcn_readlane(h, src[u]);
                     // prune root r if d_r(h) <= iter - d_v(h); an unused slot u
-                    // (fewer than kAddHubs hubs left) gets threshold 0, which the
+                    // (fewer than HUBS hubs left) gets threshold 0, which the
                     // all-INF row never meets
-                    const uint32_t du = __shfl(d, src[u]);
+                    const uint32_t du = __builtin_amdgcn_readlane(d, src[u]);
                     thr[u] = ok[u] ? iter - du : 0u;
-                    const uint32_t mlo = __shfl((uint32_t)lm, src[u]), mhi = __shfl((uint32_t)(lm >> 32), src[u]);
-                    const bool mine = ((lane < 32 ? mlo : mhi) >> (lane & 31)) & 1u;
+                    const bool mine = (readlane_any((uint64_t)lm, (uint32_t)src[u]) >> lane) & 1ull;
 #pragma unroll
                     for (uint32_t q = 0; q < RV; ++q) row[u][q] = make_uint4(~0u, ~0u, ~0u, ~0u);
                     if (ok[u] && need && mine) {
-                        const uint4 *rp = reinterpret_cast<const uint4 *>(dc + (uint64_t)hh[u] * kBatch) + RV * lane;
+                        const uint4 *rp = reinterpret_cast<const uint4 *>(dc + (uint64_t)hh[u] * R) + RV * lane;
 #pragma unroll
                         for (uint32_t q = 0; q < RV; ++q) row[u][q] = rp[q];
                     }
                     n_rows += ok[u] ? 1 : 0;
                 }
 #pragma unroll
-                for (int u = 0; u < (int)kAddHubs; ++u) {
+                for (int u = 0; u < (int)HUBS; ++u) {
                     uint32_t wds[4 * RV];
 #pragma unroll
                     for (uint32_t q = 0; q < RV; ++q) {
@@ -1369,12 +1446,10 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
                         wds[4 * q + 2] = row[u][q].z;
                         wds[4 * q + 3] = row[u][q].w;
                     }
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) {
-                        const uint32_t x = W ? (wds[q >> 1] >> ((q & 1) * 16)) & 0xFFFFu
-                                             : (wds[q >> 2] >> ((q & 3) * 8)) & 255u;
-                        if (x <= thr[u] && hh[u] < my_lo + q) prune |= 1u << q;
-                    }
+                    // only roots above the hub (PARA:1250-1254)
+                    const int o = (int)hh[u] - (int)my_lo;
+                    const Bits above = o < 0 ? ~(Bits)0 : (o >= (int)PER - 1 ? (Bits)0 : ~(Bits)1 << o);
+                    prune |= slice_le<W, PER>(wds, thr[u]) & above;
                 }
             }
         };
@@ -1407,20 +1482,19 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         uint32_t ncand_v = kGather + 1, cpr = 0;
         if (DEEP && iter > kNear + 1 && slen != 0) {
             ncand_v = 0;
-            uint32_t rest = cb;
+            Bits rest = cb;
 #pragma unroll
             for (uint32_t k = 0; k < kGather; ++k) {
-                const unsigned long long m = __ballot(rest != 0u);
+                const unsigned long long m = __ballot(rest != 0);
                 croot[k] = ~0u;
                 if (m) {
                     const uint32_t l0 = (uint32_t)__ffsll(m) - 1;
-                    const uint32_t bits = uniform32(__shfl(rest, (int)l0));
-                    croot[k] = 16 * l0 + (uint32_t)__ffs(bits) - 1;
+                    croot[k] = PER * l0 + ctz_any(readlane_any(rest, l0));
                     if (lane == l0) rest &= rest - 1;
                     ++ncand_v;
                 }
             }
-            if (__ballot(rest != 0u) != 0ull) ncand_v = kGather + 1;  // too many: row slices
+            if (__ballot(rest != 0) != 0ull) ncand_v = kGather + 1;  // too many: row slices
         }
         const bool gather = ncand_v <= kGather;
         // One label per lane against the listed candidates: prune candidate k
@@ -1432,8 +1506,8 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
             for (uint32_t k = 0; k < kGather; ++k) {
                 const uint32_t ro = croot[k];
                 x[k] = ~0u;
-                if (k < ncand_v && !((cpr >> k) & 1u) && ((lm >> (ro >> 4)) & 1ull) && h < rs + ro)
-                    x[k] = dc[(uint64_t)h * kBatch + ro];
+                if (k < ncand_v && !((cpr >> k) & 1u) && ((lm >> (ro / PER)) & 1ull) && h < rs + ro)
+                    x[k] = dc[(uint64_t)h * R + ro];
             }
             bool any = false;
 #pragma unroll
@@ -1483,16 +1557,16 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
             });
 #pragma unroll
             for (uint32_t k = 0; k < kGather; ++k)
-                if (((cpr >> k) & 1u) && lane == (croot[k] >> 4)) prune |= 1u << (croot[k] & 15u);
+                if (((cpr >> k) & 1u) && lane == croot[k] / PER) prune |= (Bits)1 << (croot[k] % PER);
         } else {
             scan_labels([&](uint32_t h, uint32_t d, unsigned long long lm) {
                 hub_pass(h, d, lm);
-                return __ballot((cb & ~prune) != 0u) == 0ull;
+                return __ballot((cb & ~prune) != 0) == 0ull;
             });
         }
-        const uint32_t surv = cb & ~prune;
-        n_dq += __popc(cb & prune);
-        const uint32_t cnt = __popc(surv);
+        const Bits surv = cb & ~prune;
+        n_dq += popc_any((Bits)(cb & prune));
+        const uint32_t cnt = popc_any(surv);
         const uint32_t incl = wave_incl_scan(cnt);
         const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
         if (total == 0) continue;
@@ -1500,25 +1574,25 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         const unsigned long long nb = store_reserve_at(S, C, v, len, base, cap, total);
         if (nb == ~0ull) continue;
         uint32_t pos = len + incl - cnt;
-        for (uint32_t sb = surv; sb; sb &= sb - 1) {
-            const uint32_t q = __ffs(sb) - 1;
+        for (Bits sb = surv; sb; sb &= sb - 1) {
+            const uint32_t q = ctz_any(sb);
             S.pool[nb + pos++] = ((my_lo + q) << B) | iter;  // insert_label_only, PARA:1285
         }
         if (lane == 0) S.rec[v].len = len + total;
         if (iter == 1u) {
             // The new labels are at distance 1: v's list gets them too.
             uint32_t p1 = n1 + incl - cnt;
-            for (uint32_t sb = surv; sb; sb &= sb - 1) H1.lab[e0 + p1++] = ((my_lo + __ffs(sb) - 1) << B) | 1u;
+            for (Bits sb = surv; sb; sb &= sb - 1) H1.lab[e0 + p1++] = ((my_lo + ctz_any(sb)) << B) | 1u;
             if (lane == 0) H1.len[v] = n1 + total;
         }
         // Roots of this batch also record the new label in the root table
         // (dist_matrix[v_root][cand_real] = iter, PARA:1287-1290).
         if (v >= rs && v < rs + rsz) {
-            for (uint32_t sb = surv; sb; sb &= sb - 1) {
-                const uint32_t h = my_lo + __ffs(sb) - 1;
-                dc[(uint64_t)h * kBatch + (v - rs)] = (typename Hop<W>::Dist)iter;
+            for (Bits sb = surv; sb; sb &= sb - 1) {
+                const uint32_t h = my_lo + ctz_any(sb);
+                dc[(uint64_t)h * R + (v - rs)] = (typename Hop<W>::Dist)iter;
                 if (iter < (hinfo[h].info & INF)) atomicMin(&hinfo[h].info, ~INF | iter);
-                if (iter <= kNear) atomicOr(&hinfo[h].near[iter - 1], 1ull << ((v - rs) >> 4));
+                if (iter <= kNear) atomicOr(&hinfo[h].near[iter - 1], 1ull << ((v - rs) / PER));
             }
         }
         // v becomes active with the new distance group as its last group
@@ -1534,12 +1608,21 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
             if (lane == 0 && C->pull) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
             my_pedge = 0;
         }
-        reinterpret_cast<uint16_t *>(ag + (uint64_t)v * kWords)[lane] = (uint16_t)surv;
         const unsigned long long nzm = __ballot(surv != 0);
-        uint32_t wmask = 0;
+        uint64_t wmask = 0;
+        if constexpr (RW == kRow) {
+            reinterpret_cast<uint16_t *>(ag + (uint64_t)v * RW)[lane] = (uint16_t)surv;
 #pragma unroll
-        for (int w = 0; w < (int)kWords; ++w)
-            if ((nzm >> (4 * w)) & 0xFull) wmask |= 1u << w;
+            for (int w = 0; w < (int)RW; ++w)
+                if ((nzm >> (4 * w)) & 0xFull) wmask |= 1ull << w;
+            my_subs = 1u;
+        } else {
+            ag[(uint64_t)v * RW + lane] = surv;
+            wmask = nzm;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if ((nzm >> (16 * q)) & 0xFFFFull) my_subs |= 1u << q;
+        }
         if (lane == 0) {
             amask[v] = wmask;
             aend[v] = pdeg;
@@ -1561,7 +1644,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         c_left -= nch;
     }
     for (uint32_t q = lane; q < c_left; q += 64) chunks[c_next + q] = kChunkPad;
-    if (lane == 0 && my_act) C->n_act[p ^ 1u] = 1u;  // (every writer writes the same)
+    if (lane < 4 && ((my_subs >> lane) & 1u)) C->n_act[p ^ 1u][lane] = 1u;  // (every writer writes the same)
     if (lane == 0 && my_pedge && C->pull) atomicAdd(&C->n_pedge[p ^ 1u], (unsigned long long)my_pedge);
     if (wave < ncand) {
         const bool one = lane == 0;
@@ -1569,14 +1652,14 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
     }
 }
 
-template <bool W, uint32_t CH, bool DEEP>
+template <bool W, uint32_t CH, uint32_t RW, bool DEEP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_add(uint32_t iter, const uint8_t *used, const uint64_t *off, const uint32_t *adj, const uint32_t *clist,
                                              unsigned long long *cand, LabelStore S, HubList1 H1, HubInfo *hinfo,
                                              typename Hop<W>::Dist *dc,
-                                             unsigned long long *abits, unsigned long long *ag, uint32_t *amask,
+                                             unsigned long long *abits, unsigned long long *ag, uint64_t *amask,
                                              uint32_t *aend, unsigned long long *chunks, BuildCounters *C)
 {
-    add_body<W, CH, DEEP>(blockIdx.x, gridDim.x, iter, used, off, adj, clist, cand, S, H1, hinfo, dc, abits, ag, amask,
+    add_body<W, CH, RW, DEEP>(blockIdx.x, gridDim.x, iter, used, off, adj, clist, cand, S, H1, hinfo, dc, abits, ag, amask,
                           aend, chunks, C);
 }
 
@@ -1610,22 +1693,24 @@ __global__ void k_unhold(BuildCounters *C) { C->hold = 0u; }
 // (PARA:877-901): clear the indicator rows of the touched vertices (the
 // root-distance table is reset by hub_reset_body), and frontier bitmap slot 1,
 // which the next batch's first frontier goes into.
+template <uint32_t RW>
 __device__ __forceinline__ void batch_end_body(uint32_t bid, uint32_t nblk, unsigned long long *ind, const uint32_t *tlist,
                                                    unsigned long long *abits, const BuildCounters *C)
 {
     if (C->hold) return;
     const uint32_t nt = C->n_touched, nw = C->abits_words;
     const uint64_t stride = (uint64_t)nblk * blockDim.x;
-    const uint64_t tot = (uint64_t)nt * kWords;
+    const uint64_t tot = (uint64_t)nt * RW;
     for (uint64_t i = (uint64_t)bid * blockDim.x + threadIdx.x; i < tot; i += stride)
-        ind[(uint64_t)tlist[i / kWords] * kWords + (i % kWords)] = 0ull;
+        ind[(uint64_t)tlist[i / RW] * RW + (i % RW)] = 0ull;
     for (uint64_t i = (uint64_t)bid * blockDim.x + threadIdx.x; i < nw; i += stride) abits[nw + i] = 0ull;
 }
 
+template <uint32_t RW>
 __global__ __launch_bounds__(256) void k_batch_end(unsigned long long *ind, const uint32_t *tlist,
                                                    unsigned long long *abits, const BuildCounters *C)
 {
-    batch_end_body(blockIdx.x, gridDim.x, ind, tlist, abits, C);
+    batch_end_body<RW>(blockIdx.x, gridDim.x, ind, tlist, abits, C);
 }
 
 // First kernel of a batch's prologue: the gate -- if the previous batch
@@ -1636,17 +1721,17 @@ __global__ __launch_bounds__(256) void k_batch_end(unsigned long long *ind, cons
 // per root) and batch_end_body -- which are independent of
 // each other.  Every block takes the gate's decision itself from counters
 // that nothing in this kernel changes.
-template <bool W>
+template <bool W, uint32_t RW>
 __global__ __launch_bounds__(256) void k_batch_close(const uint8_t *used, LabelStore S, HubInfo *hinfo,
                                                      typename Hop<W>::Dist *dc, unsigned long long *ind,
                                                      const uint32_t *tlist, unsigned long long *abits, BuildCounters *C)
 {
-    if (C->hold || C->n_act[(C->iter_last + 1u) & 1u] != 0u) {
+    if (C->hold || any_active(C->n_act[(C->iter_last + 1u) & 1u])) {
         if (blockIdx.x == 0 && threadIdx.x == 0) C->hold = 1u;
         return;
     }
-    hub_reset_body<W>(blockIdx.x, used, S, hinfo, dc, C);
-    batch_end_body(blockIdx.x, gridDim.x, ind, tlist, abits, C);
+    hub_reset_body<W, RW>(blockIdx.x, used, S, hinfo, dc, C);
+    batch_end_body<RW>(blockIdx.x, gridDim.x, ind, tlist, abits, C);
 }
 
 // One graph's whole batch phase in one workgroup (no reference
@@ -1668,7 +1753,8 @@ struct BatchPlan {
     unsigned long long *ind, *cand, *vmark;
     uint32_t *tlist, *clist;
     unsigned long long *abits, *ag;
-    uint32_t *amask, *aend;
+    uint64_t *amask;
+    uint32_t *aend;
     unsigned long long *chunks;
     const uint8_t *bpd;
     const unsigned long long *lmask;
@@ -1698,8 +1784,8 @@ __global__ __launch_bounds__(kLoopWaves * 64) void k_batch_loop(const BatchPlan<
         // The previous batch's root-distance entries and indicator rows.
         const uint32_t prsz = C->rsz;
         for (uint32_t vb = 0; vb * (kLoopWaves / kRootWaves) < prsz; ++vb)
-            hub_reset_body<W>(vb, P.used, P.S, P.hinfo, P.dc, C);
-        batch_end_body(0, 1, P.ind, P.tlist, P.abits, C);
+            hub_reset_body<W, kRow>(vb, P.used, P.S, P.hinfo, P.dc, C);
+        batch_end_body<kRow>(0, 1, P.ind, P.tlist, P.abits, C);
         // Batch b: its non-bit-parallel roots are the first frontier.
         const uint32_t rs = b * P.batch, rsz = min(P.batch, P.n - rs);
         uint32_t c = 0;
@@ -1709,22 +1795,22 @@ __global__ __launch_bounds__(kLoopWaves * 64) void k_batch_loop(const BatchPlan<
         __syncthreads();
         if ((threadIdx.x & 63) == 0) atomicAdd(&s_cnt, c);
         __syncthreads();
-        if (threadIdx.x == 0) batch_begin_write(C, b, rs, rsz, s_cnt);
+        if (threadIdx.x == 0) batch_begin_write(C, b, rs, rsz, {s_cnt, 0u, 0u, 0u});
         __syncthreads();
         for (uint32_t vb = 0; vb * (kLoopWaves / kRootWaves) < rsz; ++vb)
-            batch_init_body<W, kChunk>(vb, 1, P.used, P.off, P.adj, P.S, P.hinfo, P.dc, P.ind, P.vmark, P.tlist,
+            batch_init_body<W, kChunk, kRow>(vb, 1, P.used, P.off, P.adj, P.S, P.hinfo, P.dc, P.ind, P.vmark, P.tlist,
                                        P.abits, P.ag, P.amask, P.aend, P.chunks, P.bps, P.rset, P.lmask, P.rmask, C);
         __syncthreads();
         for (uint32_t iter = 1;; ++iter) {
-            push_body<W, kChunk, kLoopWaves, false>(0, 1, iter, P.off, P.adj, P.abits, P.ag, P.amask, P.aend, P.chunks,
+            push_body<W, kChunk, kLoopWaves, kRow, false>(0, 1, iter, P.off, P.adj, P.abits, P.ag, P.amask, P.aend, P.chunks,
                                              P.ind, P.cand, P.vmark, P.tlist, P.clist, P.bpd, P.lmask, P.rmask,
                                              P.bps, P.rset, C, P.bp_prune, P.pull_ratio);
             __syncthreads();
-            add_body<W, kChunk>(0, 1, iter, P.used, P.off, P.adj, P.clist, P.cand, P.S, P.H1, P.hinfo, P.dc, P.abits,
+            add_body<W, kChunk, kRow>(0, 1, iter, P.used, P.off, P.adj, P.clist, P.cand, P.S, P.H1, P.hinfo, P.dc, P.abits,
                                 P.ag, P.amask, P.aend, P.chunks, C);
             __syncthreads();
             const bool stop = C->overflow != 0u || C->domain != 0u;
-            const bool done = C->n_act[(iter + 1) & 1u] == 0u;
+            const bool done = !any_active(C->n_act[(iter + 1) & 1u]);
             __syncthreads();  // every thread has read the counters before any writes them
             if (stop) return;
             if (done) break;
@@ -1779,9 +1865,10 @@ __global__ __launch_bounds__(256) void k_gather_labels(uint32_t n, const uint32_
 
 }  // namespace
 
-// Grows (or just compacts) the label pool between batches.
+// Compacts the label pool between batches, into one that the lists take up at
+// most a quarter of and that has room for `room` words twice over.
 static pado_gpu_status pool_repack(hipStream_t st, uint32_t n, DevBuf<uint32_t> &pool, DevBuf<LRec> &rec,
-                                   unsigned long long new_size, unsigned long long *new_top)
+                                   unsigned long long room, unsigned long long *new_top)
 {
     DevBuf<uint32_t> ncap;
     DevBuf<uint64_t> nbase;
@@ -1791,7 +1878,8 @@ static pado_gpu_status pool_repack(hipStream_t st, uint32_t n, DevBuf<uint32_t> 
     PADO_TRY(scan_u32_to_u64(ncap.p, nbase.p, n, st));
     uint64_t need = 0;
     PADO_HIP(copy_sync(&need, nbase.p + n, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-    if (new_size < need * 2) new_size = need * 2;
+    const unsigned long long new_size =
+        std::max<unsigned long long>(pool.n, std::max<unsigned long long>(4 * need, 2 * (need + room)));
     DevBuf<uint32_t> npool;
     PADO_TRY(npool.alloc(new_size));
     hipLaunchKernelGGL(k_pool_move, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, pool.p, rec.p,
@@ -1810,7 +1898,8 @@ struct BatchBuffers {
     DevBuf<unsigned long long> abits;  // frontier bitmaps, two slots of ceil(n / 64) words
     DevBuf<unsigned long long> lmask;  // bit-parallel mask rows, kLmWords words per vertex
     DevBuf<unsigned long long> rmask;  // batch roots' mask words 0..kLmNz0, word-major [10][kBatch]
-    DevBuf<uint32_t> tlist, clist, amask, aend, pool;
+    DevBuf<uint64_t> amask;
+    DevBuf<uint32_t> tlist, clist, aend, pool;
     DevBuf<HubInfo> hinfo;
     DevBuf<uint32_t> d1, d1len;  // distance-1 lists (HubList1): m slots, n counts
     DevBuf<LRec> lrec;
@@ -1822,7 +1911,8 @@ struct BatchBuffers {
     void release()
     {
         for (auto *b : {&ind, &cand, &ag, &chunks, &abits, &lmask, &rmask}) b->release();
-        for (auto *b : {&tlist, &clist, &amask, &aend, &pool, &d1, &d1len}) b->release();
+        for (auto *b : {&tlist, &clist, &aend, &pool, &d1, &d1len}) b->release();
+        amask.release();
         hinfo.release();
         lrec.release();
         dc.release();
@@ -1834,9 +1924,9 @@ struct BatchBuffers {
 // Allocates and initialises them on the graph's stream.  add_waves bounds
 // the padding of k_add's per-wave descriptor reservations: padded
 // descriptors are fewer than the real ones plus kChunkGrab per wave.  The
-// pool holds pool_size label words, the root-distance table dc_rows 1 KB
-// rows (255).
-template <bool W>
+// pool holds pool_size label words, the root-distance table dc_rows rows of
+// one entry per root (255).
+template <bool W, uint32_t RW>
 static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index *idx, uint64_t add_waves,
                                    uint32_t chunk, unsigned long long pool_size, uint32_t dc_rows, bool pull,
                                    BatchBuffers<W> &B)
@@ -1845,9 +1935,9 @@ static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
     const uint32_t nw = (n + 63) / 64;  // words of one frontier bitmap slot
-    PADO_TRY(B.ind.alloc((uint64_t)n * kWords));
-    PADO_TRY(B.cand.alloc((uint64_t)n * kWords));
-    PADO_TRY(B.ag.alloc((uint64_t)n * kWords));
+    PADO_TRY(B.ind.alloc((uint64_t)n * RW));
+    PADO_TRY(B.cand.alloc((uint64_t)n * RW));
+    PADO_TRY(B.ag.alloc((uint64_t)n * RW));
     PADO_TRY(B.abits.alloc(2ull * nw));
     PADO_TRY(B.chunks.alloc(2 * (g->m / chunk + (uint64_t)n) + kChunkGrab * add_waves + 64));
     PADO_TRY(B.tlist.alloc(n));
@@ -1858,19 +1948,19 @@ static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index
     PADO_TRY(B.d1.alloc(g->m ? g->m : 1));
     PADO_TRY(B.d1len.alloc(n));
     PADO_TRY(B.lrec.alloc(n));
-    PADO_TRY(B.rset.alloc((uint64_t)kBP * kBatch));
+    PADO_TRY(B.rset.alloc((uint64_t)kBP * Rows<RW>::kRoots));
     PADO_TRY(B.lmask.alloc((uint64_t)n * kLmWords));
-    PADO_TRY(B.rmask.alloc((kLmNz0 + 1ull) * kBatch));
+    PADO_TRY(B.rmask.alloc((kLmNz0 + 1ull) * Rows<RW>::kRoots));
     PADO_TRY(B.ctr.alloc(1 + kStatRows * kStatCols * 8 / sizeof(BuildCounters)));
     PADO_TRY(B.pool.alloc(pool_size));
-    PADO_TRY(B.dc.alloc((uint64_t)dc_rows * kBatch));
+    PADO_TRY(B.dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots));
     B.pool_size = pool_size;
     B.dc_rows = dc_rows;
     const uint32_t fg = 4096;
     hipLaunchKernelGGL(k_fill_u32, dim3(fg), dim3(256), 0, st, reinterpret_cast<uint32_t *>(B.dc.p),
-                       (uint64_t)dc_rows * kBatch * sizeof(DT) / 4, ~0u);
-    hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.ind.p, (uint64_t)n * kWords);
-    hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.cand.p, (uint64_t)n * kWords);
+                       (uint64_t)dc_rows * Rows<RW>::kRoots * sizeof(DT) / 4, ~0u);
+    hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.ind.p, (uint64_t)n * RW);
+    hipLaunchKernelGGL(k_zero_u64, dim3(fg), dim3(256), 0, st, B.cand.p, (uint64_t)n * RW);
     hipLaunchKernelGGL(k_bp_masks, dim3(fg), dim3(256), 0, st, n, idx->bpd.p, B.lmask.p);
     hipLaunchKernelGGL(k_hub_info_init, dim3(fg), dim3(256), 0, st, B.hinfo.p, (uint64_t)n);
     hipLaunchKernelGGL(k_fill_u32, dim3(fg), dim3(256), 0, st, B.d1len.p, (uint64_t)n, 0u);
@@ -1887,13 +1977,13 @@ static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index
 // End of the batch phase: clear the indicator rows still marked, keep the
 // counters, and build the canonical rank-space CSR -- each vertex's labels
 // gathered and sorted by hub (order_labels' per-vertex std::sort, PARA:2240).
-template <bool W>
+template <bool W, uint32_t RW>
 static pado_gpu_status batch_finish(pado_gpu_graph *g, pado_gpu_index *idx, const pado_gpu_build_cfg &cfg,
                                     BatchBuffers<W> &B, const KernelTimes &kt)
 {
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
-    hipLaunchKernelGGL(k_batch_end, dim3(1024), dim3(256), 0, st, B.ind.p, B.tlist.p, B.abits.p, B.ctr.p);
+    hipLaunchKernelGGL(k_batch_end<RW>, dim3(1024), dim3(256), 0, st, B.ind.p, B.tlist.p, B.abits.p, B.ctr.p);
     hipLaunchKernelGGL(k_fold_stats, dim3(1), dim3(1024), 0, st, B.ctr.p);
     BuildCounters c{};
     PADO_HIP(copy_sync(&c, B.ctr.p, sizeof(BuildCounters), hipMemcpyDeviceToHost, st));
@@ -1916,36 +2006,40 @@ static pado_gpu_status batch_finish(pado_gpu_graph *g, pado_gpu_index *idx, cons
 }
 
 // The batch kernels of one (chunk, push waves) choice.
-template <bool W>
+template <bool W, uint32_t RW>
 struct BatchKernels {
-    decltype(&k_batch_init<W, kChunk>) init;
-    decltype(&k_push<W, kChunk, kPushWaves>) push;
-    decltype(&k_add<W, kChunk, false>) add;       // iterations up to kNear + 1
-    decltype(&k_add<W, kChunk, true>) add_deep;   // the later ones
+    decltype(&k_batch_init<W, kChunk, RW>) init;
+    decltype(&k_push<W, kChunk, kPushWaves, RW>) push;
+    decltype(&k_add<W, kChunk, RW, false>) add;       // iterations up to kNear + 1
+    decltype(&k_add<W, kChunk, RW, true>) add_deep;   // the later ones
     uint32_t chunk, waves;
 };
 
-template <bool W, uint32_t CH>
-static BatchKernels<W> batch_kernels_ch(uint32_t waves)
+template <bool W, uint32_t RW, uint32_t CH>
+static BatchKernels<W, RW> batch_kernels_ch(uint32_t waves)
 {
-    BatchKernels<W> K{k_batch_init<W, CH>, k_push<W, CH, kPushWaves>, k_add<W, CH, false>, k_add<W, CH, true>, CH,
-                      kPushWaves};
-    if (waves == 2) K.push = k_push<W, CH, 2>;
-    if (waves == 8) K.push = k_push<W, CH, 8>;
-    if (waves == 2 || waves == 8) K.waves = waves;
+    BatchKernels<W, RW> K{k_batch_init<W, CH, RW>,       k_push<W, CH, kPushWaves, RW>, k_add<W, CH, RW, false>,
+                          k_add<W, CH, RW, true>, CH, kPushWaves};
+    if constexpr (RW == kRow) {
+        if (waves == 2) K.push = k_push<W, CH, 2, RW>;
+        if (waves == 8) K.push = k_push<W, CH, 8, RW>;
+        if (waves == 2 || waves == 8) K.waves = waves;
+    }
     return K;
 }
 
-template <bool W>
-static BatchKernels<W> batch_kernels(uint32_t chunk, uint32_t waves)
+template <bool W, uint32_t RW>
+static BatchKernels<W, RW> batch_kernels(uint32_t chunk, uint32_t waves)
 {
-    if (chunk == 4) return batch_kernels_ch<W, 4>(waves);
-    if (chunk == 8) return batch_kernels_ch<W, 8>(waves);
-    if (chunk == 32) return batch_kernels_ch<W, 32>(waves);
-    return batch_kernels_ch<W, kChunk>(waves);
+    if constexpr (RW == kRow) {
+        if (chunk == 4) return batch_kernels_ch<W, RW, 4>(waves);
+        if (chunk == 32) return batch_kernels_ch<W, RW, 32>(waves);
+        if (chunk == kChunk) return batch_kernels_ch<W, RW, kChunk>(waves);
+    }
+    return batch_kernels_ch<W, RW, kPushChunk>(waves);
 }
 
-template <bool W>
+template <bool W, uint32_t RW>
 static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, const DevBuf<uint8_t> &d_used,
                                        const pado_gpu_build_cfg &cfg, unsigned long long pool_min,
                                        unsigned long long *pool_exhausted)
@@ -1954,8 +2048,8 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     constexpr uint32_t kIterEnd = Hop<W>::kInf;  // the first iteration that is never run
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
-    const uint32_t batch = cfg.batch_size ? cfg.batch_size : kBatch;
-    if (batch == 0 || batch > kBatch) {
+    const uint32_t batch = RW == kRow ? (cfg.batch_size ? cfg.batch_size : kBatch) : Rows<RW>::kRoots;
+    if (batch == 0 || batch > Rows<RW>::kRoots) {
         set_error("batch_size must be in [1, 1024]");
         return PADO_GPU_ERR_ARG;
     }
@@ -1969,7 +2063,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         set_error("push_chunk must be 4, 8, 16 or 32 and push_waves 2, 4 or 8");
         return PADO_GPU_ERR_ARG;
     }
-    const BatchKernels<W> K = batch_kernels<W>(chunk, waves);
+    const BatchKernels<W, RW> K = batch_kernels<W, RW>(chunk, waves);
     const std::string domain_msg =
         W ? "batch iteration reached 4095: distances outside the wide (12-bit) hop domain"
           : "batch iteration reached 255: distances outside the uint8 domain of the reference";
@@ -1978,19 +2072,25 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     // Per-wave reservations in k_add leave holes in the active list and the
     // descriptor array (see batch_alloc).
     const uint64_t add_waves = 4ull * (cfg.add_blocks ? cfg.add_blocks : default_add_grid(n));
-    // The label pool starts at 64 words per vertex and doubles whenever a
-    // host check finds it over 40% full; the checks come every
-    // iters_per_sync iterations, so the headroom covers several iterations.
-    // The root-distance table covers the hubs of the first 2^16 ids and
-    // grows on the host before a batch that could exceed it.
+    // The label pool starts at 64 words per vertex (320 for batches of four
+    // times the roots, whose first iterations append as much more) and is
+    // compacted, and grown where that is not enough, whenever a host check
+    // finds it over 40% full or without room for what may come before the
+    // next check.  The root-distance table covers the hubs of the first 2^16
+    // ids and grows fourfold on the host before a batch that could exceed it.
+    // Both are kept from growing further than they must: device memory that
+    // was in use before is cleared again before it is handed out (builds of
+    // R-MAT 20 that took 25 GB each slowed from 155 ms to 390 and more once
+    // the card's memory had gone round).
     BatchBuffers<W> B;
-    PADO_TRY(batch_alloc<W>(g, idx, add_waves, chunk,
-                            std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, 64ull * n), pool_min),
-                            std::min<uint32_t>(n, 1u << 16), pull_ratio != ~0u, B));
+    PADO_TRY((batch_alloc<W, RW>(g, idx, add_waves, chunk,
+                            std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, (RW == kRow ? 64ull : 320ull) * n), pool_min),
+                            std::min<uint32_t>(n, 1u << 16), pull_ratio != ~0u, B)));
     auto &ind = B.ind, &cand = B.cand, &ag = B.ag, &chunks = B.chunks, &abits = B.abits;
     unsigned long long *vmark = B.lmask.p + kLmMark;  // word kLmMark of each mask row (stride kLmWords)
     auto &lmask = B.lmask, &rmask = B.rmask;
-    auto &tlist = B.tlist, &clist = B.clist, &amask = B.amask, &aend = B.aend, &pool = B.pool;
+    auto &tlist = B.tlist, &clist = B.clist, &aend = B.aend, &pool = B.pool;
+    auto &amask = B.amask;
     auto &hinfo = B.hinfo;
     auto &lrec = B.lrec;
     auto &dc = B.dc;
@@ -2011,7 +2111,13 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         }
     } pin{h_ctr};
 
-    const bool use_graph = (cfg.flags & PADO_GPU_BUILD_STREAM) == 0;
+    // Launches go straight to the stream unless several builds run at once:
+    // then their threads queue in the runtime, and captured graphs (one launch
+    // for a whole block) are ahead.  R-MAT 20 build 154 ms direct, 156 with
+    // graphs; 161 x 161 wide grid 39.6 / 43.7; R-MAT 14 from edges 6.2 / 6.8;
+    // 24 graphs on four threads 57 / 52.
+    const bool events = (cfg.flags & PADO_GPU_BUILD_STREAM) != 0;
+    const bool use_graph = !events && g->ctx->concurrent;
     const uint32_t U = cfg.iters_per_sync ? std::min<uint32_t>(cfg.iters_per_sync, 64u) : 8u;
     const uint32_t push_grid = cfg.push_blocks ? cfg.push_blocks : default_push_grid(n);
     const uint32_t add_grid = cfg.add_blocks ? cfg.add_blocks : default_add_grid(n);
@@ -2027,8 +2133,8 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
             for (auto x : *e) (void)hipEventDestroy(x);
         }
     } evf{&ev};
-    if (!use_graph) {
-        ev.resize(4 * U);
+    if (events) {
+        ev.resize(4 * 64);
         for (auto &e : ev) PADO_HIP(hipEventCreate(&e));
     }
     KernelTimes kt{};
@@ -2037,9 +2143,9 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     const HubList1 H1{B.d1.p, B.d1len.p};
     auto enqueue_prologue = [&]() {
         // Previous batch's reset_at_end first (a no-op before the first batch).
-        hipLaunchKernelGGL(k_batch_close<W>, dim3(std::max<uint32_t>(1024u, root_blocks)), dim3(256), 0, st, d_used.p,
+        hipLaunchKernelGGL((k_batch_close<W, RW>), dim3(std::max<uint32_t>(1024u, root_blocks)), dim3(256), 0, st, d_used.p,
                            S, hinfo.p, dc.p, ind.p, tlist.p, abits.p, ctr.p);
-        hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(batch), 0, st, d_used.p, ctr.p, batch, n);
+        hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(1024), 0, st, d_used.p, ctr.p, batch, n);
         hipLaunchKernelGGL(K.init, dim3((batch + kInitRoots - 1) / kInitRoots), dim3(kInitRoots * kRootWaves * 64), 0, st,
                            d_used.p, g->off.p, g->adj.p, S,
                            hinfo.p, dc.p, ind.p, vmark, tlist.p, abits.p, ag.p, amask.p, aend.p, chunks.p,
@@ -2103,7 +2209,14 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         }
         return PADO_GPU_OK;
     };
-    auto first_block = [&](uint32_t prev) { return std::max<uint32_t>(1u, std::min<uint32_t>(prev, U)); };
+    // A batch's first block: the iterations that recent batches needed.  Above
+    // eight they are rounded up to a multiple of eight, so that few graphs are
+    // captured, and go up to 64 unless the caller set a limit.
+    const uint32_t first_max = cfg.iters_per_sync ? U : 64u;
+    auto first_block = [&](uint32_t prev) {
+        const uint32_t want = prev <= 8 ? prev : (prev + 7) / 8 * 8;
+        return std::max<uint32_t>(1u, std::min<uint32_t>(want, first_max));
+    };
 
     // Counter snapshots: each enqueued block of iterations is followed by a
     // copy of the counters into its own pinned slot and an event, so the host
@@ -2134,18 +2247,19 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
             PADO_HIP(hipGraphLaunch(gx, st));
         } else {
             if (first == 0) enqueue_prologue();
-            PADO_TRY(enqueue_iterations(first, count, timed));
+            PADO_TRY(enqueue_iterations(first, count, timed && events));
         }
         return PADO_GPU_OK;
     };
 
-    // Graph mode runs one batch ahead when the label pool has ample room: the
+    // One batch runs ahead when the label pool has ample room (not when launches
+    // are timed): the
     // next batch's first block is enqueued before the host has checked the
     // current one, and its gate makes it a no-op if the current batch turns
     // out to need more iterations (the host then clears the gate, runs them,
     // and enqueues the next batch again).
     const uint32_t nb = (n + batch - 1) / batch;
-    uint64_t iterations_seen = 0;
+    uint64_t steps_seen = 0;
     uint32_t prev_batch_iters = 1;
     constexpr uint32_t kIterHistory = 8;
     uint32_t iters_hist[kIterHistory] = {1, 1, 1, 1, 1, 1, 1, 1}, hist_pos = 0;
@@ -2165,13 +2279,13 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
             // table already covers it.  hipFree/hipMalloc synchronise.  The new
             // table starts all 255, so the previous batch's reset is a no-op on it.
             PADO_HIP(hipStreamSynchronize(st));
-            dc_rows = std::min<uint32_t>(n, std::max<uint32_t>(batch_end, dc_rows * 2));
-            PADO_TRY(dc.alloc((uint64_t)dc_rows * kBatch));
+            dc_rows = (uint32_t)std::min<uint64_t>(n, std::max<uint64_t>(batch_end, dc_rows * 4ull));
+            PADO_TRY(dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots));
             hipLaunchKernelGGL(k_fill_u32, dim3(fg), dim3(256), 0, st, reinterpret_cast<uint32_t *>(dc.p),
-                               (uint64_t)dc_rows * kBatch * sizeof(DT) / 4, ~0u);
+                               (uint64_t)dc_rows * Rows<RW>::kRoots * sizeof(DT) / 4, ~0u);
             drop_graphs();
         }
-        const uint64_t batch_first_iter = iterations_seen;
+        const uint64_t batch_first_step = steps_seen;
         uint32_t next_count = std::min<uint32_t>(2u, U);  // a continuation block's size
         bool repacked = false;
         unsigned long long last_top = 0;
@@ -2188,7 +2302,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
             PADO_TRY(snapshot(&cur_slot));
         }
         const uint32_t next_end = std::min<uint64_t>((uint64_t)(b + 2) * batch, n);
-        bool spec = use_graph && b + 1 < nb && next_end <= dc_rows && growth != ~0ull &&
+        bool spec = !events && b + 1 < nb && next_end <= dc_rows && growth != ~0ull &&
                     (top_prev + 4 * growth) * 5 < pool_size * 2;
         if (spec) {
             ahead_count = std::min<uint32_t>(first_block(prev_batch_iters), kIterEnd);
@@ -2200,8 +2314,8 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
             PADO_HIP(hipGetLastError());
             const BuildCounters snap = h_ctr[cur_slot];
             last_top = snap.pool_top;
-            if (!use_graph) {
-                const uint64_t live = snap.iterations - iterations_seen;
+            if (events) {
+                const uint64_t live = snap.steps - steps_seen;
                 for (uint64_t u = 0; u < live && u < cur_count; ++u) {
                     float t_push = 0.f, t_add = 0.f;
                     PADO_HIP(hipEventElapsedTime(&t_push, ev[4 * u], ev[4 * u + 1]));
@@ -2212,7 +2326,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
                     kt.n_add += 1;
                 }
             }
-            iterations_seen = snap.iterations;
+            steps_seen = snap.steps;
             // Work enqueued after this block (a block ahead) still uses the
             // buffers: it drains before an error return frees them.
             if (snap.overflow) {
@@ -2231,17 +2345,16 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
                 rate = std::max(r, rate * 0.75);
             }
             snap_top_prev = snap.pool_top;
-            // Keep at least 60% of the pool free, and room for four times the
-            // recent growth over the next blocks (this batch's next block and
-            // a block run ahead: U iterations each at most); a block ahead
-            // runs to completion first.
-            const double need = rate * 4.0 * (spec ? 2.0 * U : (double)U);
+            // Keep at least 60% of the pool free, and room for four blocks of
+            // the recent growth (two can run before the next check: this
+            // batch's next and the one ahead); a block ahead runs to
+            // completion first.
+            const double ahead_iters = std::max<uint32_t>(U, first_block(prev_batch_iters));
+            const double need = rate * 4.0 * ahead_iters;
             if (snap.pool_top * 5 > pool_size * 2 || (double)snap.pool_top + need > 0.8 * (double)pool_size) {
                 PADO_HIP(hipStreamSynchronize(st));
                 unsigned long long top = 0;
-                const unsigned long long want =
-                    std::max<unsigned long long>(pool_size * 2, (unsigned long long)(2.0 * (snap.pool_top + need)));
-                PADO_TRY(pool_repack(st, n, pool, lrec, want, &top));
+                PADO_TRY(pool_repack(st, n, pool, lrec, (unsigned long long)need, &top));
                 snap_top_prev = top;
                 pool_size = pool.n;
                 S.pool = pool.p;
@@ -2254,7 +2367,8 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
                 if (spec) PADO_TRY(snapshot(&ahead_slot));
             }
             // The frontier of the next iteration is in slot (launched + 1) & 1.
-            if (snap.n_act[(launched + 1) & 1u] == 0) break;
+            const uint32_t(&left)[4] = snap.n_act[(launched + 1) & 1u];
+            if ((left[0] | left[1] | left[2] | left[3]) == 0) break;
             if (launched >= kIterEnd) {
                 (void)hipStreamSynchronize(st);
                 set_error(domain_msg);
@@ -2278,7 +2392,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         // end costs two empty launches.  On R-MAT 20 this policy takes 9 such
         // round trips and 282 empty iterations where the previous batch's count
         // alone takes 81 and 86.
-        iters_hist[hist_pos++ % kIterHistory] = (uint32_t)(iterations_seen - batch_first_iter);
+        iters_hist[hist_pos++ % kIterHistory] = (uint32_t)(steps_seen - batch_first_step);
         prev_batch_iters = *std::max_element(iters_hist, iters_hist + kIterHistory);
         // Pool growth of this batch (unknown across a repack, which blocks
         // running ahead until a batch has been measured again).
@@ -2292,7 +2406,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         }
         ahead = spec;
     }
-    return batch_finish<W>(g, idx, cfg, B, kt);
+    return batch_finish<W, RW>(g, idx, cfg, B, kt);
 }
 
 template <bool W>
@@ -2353,7 +2467,7 @@ static pado_gpu_status batch_loop_t(std::vector<LoopJob> &jobs, hipStream_t st)
         // growable per-vertex arrays take up to four times their length.
         const unsigned long long pool =
             std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, 384ull * n), J.pool_min);
-        PADO_TRY(batch_alloc<W>(J.g, J.idx, kLoopWaves, kChunk, pool, n, false, bufs[j]));
+        PADO_TRY((batch_alloc<W, kRow>(J.g, J.idx, kLoopWaves, kChunk, pool, n, false, bufs[j])));
         plans[j] = batch_plan<W>(J.g, J.idx, J.used, J.batch, bufs[j]);
     }
     DevBuf<BatchPlan<W>> dplans;
@@ -2377,7 +2491,7 @@ static pado_gpu_status batch_loop_t(std::vector<LoopJob> &jobs, hipStream_t st)
         }
         pado_gpu_build_cfg cfg{};
         cfg.batch_size = J.batch;
-        J.status = batch_finish<W>(J.g, J.idx, cfg, bufs[j], KernelTimes{});
+        J.status = batch_finish<W, kRow>(J.g, J.idx, cfg, bufs[j], KernelTimes{});
         bufs[j].release();  // this graph's buffers go before the next finish allocates
     }
     return PADO_GPU_OK;
@@ -2408,10 +2522,19 @@ pado_gpu_status build_batches(pado_gpu_graph *g, pado_gpu_index *idx, const DevB
         if (job[0].status != PADO_GPU_ERR_NOMEM) return job[0].status;
         pool_min = job[0].pool_exhausted * 2;
     }
+    // Batches of 1,024 roots run four at a time wherever nothing asks for them
+    // one by one (any batch size gives the same labels, and `iterations` counts
+    // the same either way): a batch costs its prologue and two launches per
+    // iteration however little is in it.  Above kWideRowVertices the wider rows
+    // would take too much memory (5.6 KB more per vertex).
+    const bool four = g->n > kBatch && g->n <= kWideRowVertices && (cfg.batch_size == 0 || cfg.batch_size == kBatch) &&
+                      (cfg.flags & PADO_GPU_BUILD_STREAM) == 0 && (cfg.push_chunk == 0 || cfg.push_chunk == kPushChunk) &&
+                      (cfg.push_waves == 0 || cfg.push_waves == kPushWaves) && cfg.pull_ratio == 0;
     for (int attempt = 0;; ++attempt) {
         exhausted = 0;
-        const pado_gpu_status s = idx->wide ? build_batches_t<true>(g, idx, d_used, cfg, pool_min, &exhausted)
-                                            : build_batches_t<false>(g, idx, d_used, cfg, pool_min, &exhausted);
+        const auto build = idx->wide ? (four ? build_batches_t<true, kWideRow> : build_batches_t<true, kRow>)
+                                     : (four ? build_batches_t<false, kWideRow> : build_batches_t<false, kRow>);
+        const pado_gpu_status s = build(g, idx, d_used, cfg, pool_min, &exhausted);
         if (s != PADO_GPU_ERR_NOMEM || !exhausted || attempt == 2) return s;
         pool_min = exhausted * 4;
         (void)hipStreamSynchronize(g->ctx->stream);

@@ -21,7 +21,6 @@ constexpr uint32_t kBpdStride = 64;   // bytes per vertex in the bp_dist array (
 // The queries read the line anyway and skip the sets that it rules out.
 constexpr uint32_t kBpNzByte = 51;
 constexpr uint32_t kBatch = 1024;     // BATCH_SIZE (PARA:42)
-constexpr uint32_t kWords = kBatch / 64;  // 64-bit words per 1024-root bitmap row
 constexpr uint8_t kInf8 = 255;        // SMALLI_MAX (GLB:40)
 constexpr uint32_t kHubBits = 24;     // packed label = (hub << 8) | dist
 constexpr uint32_t kMaxVertices = 1u << kHubBits;
@@ -242,12 +241,15 @@ struct BuildCounters {
     uint32_t next_batch;          // batch index the next k_batch_begin starts
     uint32_t rs, rsz, gen_batch;  // current batch: roots [rs, rs + rsz)
     uint32_t domain;              // an iteration reached 255 (u8 domain)
-    unsigned long long iterations;  // live iterations, summed over batches
+    // Live iterations summed over batches of 1,024 roots (a batch of 4,096
+    // counts for each quarter that has active vertices), and over batches as
+    // they are run.
+    unsigned long long iterations, steps;
     unsigned long long pulls;     // iterations run in pull form (statistic)
     // Frontier and candidate counts of batch iteration i live in slot i & 1:
     // each kernel reads its own slot and empties the other one for the next
     // kernel to fill, so no control launch runs between iterations.
-    alignas(128) uint32_t n_act[2];    // nonzero: the iteration has active vertices
+    alignas(128) uint32_t n_act[2][4];  // nonzero: the iteration has active vertices (of that quarter)
     alignas(128) uint32_t n_chunk[2];  // push work descriptors of the iteration
     alignas(128) uint32_t n_cand[2];   // candidate vertices of the iteration
     alignas(128) uint32_t n_touched;   // vertices whose indicator row was touched this batch
@@ -285,6 +287,7 @@ struct pado_gpu_ctx {
     hipStream_t side = nullptr;       // second stream of chunked host-array queries
     hipEvent_t side_ev = nullptr;     // orders the side stream after work queued before a query
     int num_cu = 0;
+    bool concurrent = false;          // one of several contexts whose builds run at once (a many-graph job)
 };
 
 struct pado_gpu_graph {

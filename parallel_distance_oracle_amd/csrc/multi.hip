@@ -388,9 +388,11 @@ pado_gpu_status pado_gpu_build_multi(pado_gpu_ctx *ctx, uint32_t num_graphs, con
     std::mutex err_mu;
     pado_gpu_status first_status = PADO_GPU_OK;
     std::string first_error;
+    const uint32_t nthreads = std::max<uint32_t>(1, std::min<uint32_t>(workers, (uint32_t)tasks.size()));
     auto worker = [&]() {
         pado_gpu_ctx *wctx = nullptr;
         pado_gpu_status s = pado_gpu_ctx_create(ctx->device, &wctx);
+        if (wctx) wctx->concurrent = nthreads > 1;
         for (size_t t; s == PADO_GPU_OK && !failed.load() && (t = next_task.fetch_add(1)) < tasks.size();) {
             const Task &T = tasks[t];
             if (T.union_id >= 0) {
@@ -419,7 +421,6 @@ pado_gpu_status pado_gpu_build_multi(pado_gpu_ctx *ctx, uint32_t num_graphs, con
         }
     };
     std::vector<std::thread> pool;
-    const uint32_t nthreads = std::max<uint32_t>(1, std::min<uint32_t>(workers, (uint32_t)tasks.size()));
     for (uint32_t w = 0; w < nthreads; ++w) pool.emplace_back(worker);
     for (auto &t : pool) t.join();
     (void)hipSetDevice(ctx->device);
