@@ -1867,26 +1867,25 @@ __global__ __launch_bounds__(256) void k_gather_labels(uint32_t n, const uint32_
 
 // Compacts the label pool between batches, into one that the lists take up at
 // most a quarter of and that has room for `room` words twice over.
-static pado_gpu_status pool_repack(hipStream_t st, uint32_t n, DevBuf<uint32_t> &pool, DevBuf<LRec> &rec,
-                                   unsigned long long room, unsigned long long *new_top)
+static pado_gpu_status pool_repack(hipStream_t st, WorkPool *wp, uint32_t n, DevBuf<uint32_t> &pool,
+                                   DevBuf<LRec> &rec, unsigned long long room, unsigned long long *new_top)
 {
     DevBuf<uint32_t> ncap;
     DevBuf<uint64_t> nbase;
-    PADO_TRY(ncap.alloc(n));
-    PADO_TRY(nbase.alloc((uint64_t)n + 1));
+    PADO_TRY(ncap.alloc(n, wp));
+    PADO_TRY(nbase.alloc((uint64_t)n + 1, wp));
     hipLaunchKernelGGL(k_cap_for_len, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, rec.p, ncap.p, 0u);
-    PADO_TRY(scan_u32_to_u64(ncap.p, nbase.p, n, st));
+    PADO_TRY(scan_u32_to_u64(ncap.p, nbase.p, n, st, wp));
     uint64_t need = 0;
     PADO_HIP(copy_sync(&need, nbase.p + n, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
     const unsigned long long new_size =
         std::max<unsigned long long>(pool.n, std::max<unsigned long long>(4 * need, 2 * (need + room)));
     DevBuf<uint32_t> npool;
-    PADO_TRY(npool.alloc(new_size));
+    PADO_TRY(npool.alloc(new_size, wp));
     hipLaunchKernelGGL(k_pool_move, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, pool.p, rec.p,
                        nbase.p, npool.p, ncap.p);
     PADO_HIP(hipStreamSynchronize(st));
-    std::swap(pool.p, npool.p);
-    std::swap(pool.n, npool.n);
+    pool.swap(npool);
     *new_top = need;
     return PADO_GPU_OK;
 }
@@ -1929,31 +1928,31 @@ struct BatchBuffers {
 template <bool W, uint32_t RW>
 static pado_gpu_status batch_alloc(const pado_gpu_graph *g, const pado_gpu_index *idx, uint64_t add_waves,
                                    uint32_t chunk, unsigned long long pool_size, uint32_t dc_rows, bool pull,
-                                   BatchBuffers<W> &B)
+                                   WorkPool *wp, BatchBuffers<W> &B)
 {
     using DT = typename Hop<W>::Dist;
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
     const uint32_t nw = (n + 63) / 64;  // words of one frontier bitmap slot
-    PADO_TRY(B.ind.alloc((uint64_t)n * RW));
-    PADO_TRY(B.cand.alloc((uint64_t)n * RW));
-    PADO_TRY(B.ag.alloc((uint64_t)n * RW));
-    PADO_TRY(B.abits.alloc(2ull * nw));
-    PADO_TRY(B.chunks.alloc(2 * (g->m / chunk + (uint64_t)n) + kChunkGrab * add_waves + 64));
-    PADO_TRY(B.tlist.alloc(n));
-    PADO_TRY(B.clist.alloc(n));
-    PADO_TRY(B.amask.alloc(n));
-    PADO_TRY(B.aend.alloc(n));
-    PADO_TRY(B.hinfo.alloc(n));
-    PADO_TRY(B.d1.alloc(g->m ? g->m : 1));
-    PADO_TRY(B.d1len.alloc(n));
-    PADO_TRY(B.lrec.alloc(n));
-    PADO_TRY(B.rset.alloc((uint64_t)kBP * Rows<RW>::kRoots));
-    PADO_TRY(B.lmask.alloc((uint64_t)n * kLmWords));
-    PADO_TRY(B.rmask.alloc((kLmNz0 + 1ull) * Rows<RW>::kRoots));
-    PADO_TRY(B.ctr.alloc(1 + kStatRows * kStatCols * 8 / sizeof(BuildCounters)));
-    PADO_TRY(B.pool.alloc(pool_size));
-    PADO_TRY(B.dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots));
+    PADO_TRY(B.ind.alloc((uint64_t)n * RW, wp));
+    PADO_TRY(B.cand.alloc((uint64_t)n * RW, wp));
+    PADO_TRY(B.ag.alloc((uint64_t)n * RW, wp));
+    PADO_TRY(B.abits.alloc(2ull * nw, wp));
+    PADO_TRY(B.chunks.alloc(2 * (g->m / chunk + (uint64_t)n) + kChunkGrab * add_waves + 64, wp));
+    PADO_TRY(B.tlist.alloc(n, wp));
+    PADO_TRY(B.clist.alloc(n, wp));
+    PADO_TRY(B.amask.alloc(n, wp));
+    PADO_TRY(B.aend.alloc(n, wp));
+    PADO_TRY(B.hinfo.alloc(n, wp));
+    PADO_TRY(B.d1.alloc(g->m ? g->m : 1, wp));
+    PADO_TRY(B.d1len.alloc(n, wp));
+    PADO_TRY(B.lrec.alloc(n, wp));
+    PADO_TRY(B.rset.alloc((uint64_t)kBP * Rows<RW>::kRoots, wp));
+    PADO_TRY(B.lmask.alloc((uint64_t)n * kLmWords, wp));
+    PADO_TRY(B.rmask.alloc((kLmNz0 + 1ull) * Rows<RW>::kRoots, wp));
+    PADO_TRY(B.ctr.alloc(1 + kStatRows * kStatCols * 8 / sizeof(BuildCounters), wp));
+    PADO_TRY(B.pool.alloc(pool_size, wp));
+    PADO_TRY(B.dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots, wp));
     B.pool_size = pool_size;
     B.dc_rows = dc_rows;
     const uint32_t fg = 4096;
@@ -1992,16 +1991,17 @@ static pado_gpu_status batch_finish(pado_gpu_graph *g, pado_gpu_index *idx, cons
     idx->ktimes = kt;
     PADO_TRY(idx->loff.alloc((uint64_t)n + 1));
     DevBuf<uint32_t> lens;  // label counts (lives until the end: the scan is asynchronous)
-    PADO_TRY(lens.alloc(n));
+    WorkPool *wp = g->work.get();
+    PADO_TRY(lens.alloc(n, wp));
     hipLaunchKernelGGL(k_cap_for_len, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, B.lrec.p, lens.p, 1u);
-    PADO_TRY(scan_u32_to_u64(lens.p, idx->loff.p, n, st));
+    PADO_TRY(scan_u32_to_u64(lens.p, idx->loff.p, n, st, wp));
     uint64_t total = 0;
     PADO_HIP(copy_sync(&total, idx->loff.p + n, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
     idx->num_labels = total;
     PADO_TRY(idx->lab.alloc(total));
     hipLaunchKernelGGL(k_gather_labels, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, B.pool.p,
                        B.lrec.p, idx->loff.p, idx->lab.p);
-    PADO_TRY(segmented_sort_u32(idx->lab.p, total, idx->loff.p, n, st, cfg.sort_max_items));
+    PADO_TRY(segmented_sort_u32(idx->lab.p, total, idx->loff.p, n, st, cfg.sort_max_items, wp));
     return PADO_GPU_OK;
 }
 
@@ -2082,10 +2082,11 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     // was in use before is cleared again before it is handed out (builds of
     // R-MAT 20 that took 25 GB each slowed from 155 ms to 390 and more once
     // the card's memory had gone round).
+    WorkPool *wp = g->work.get();
     BatchBuffers<W> B;
     PADO_TRY((batch_alloc<W, RW>(g, idx, add_waves, chunk,
                             std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, (RW == kRow ? 64ull : 320ull) * n), pool_min),
-                            std::min<uint32_t>(n, 1u << 16), pull_ratio != ~0u, B)));
+                            std::min<uint32_t>(n, 1u << 16), pull_ratio != ~0u, wp, B)));
     auto &ind = B.ind, &cand = B.cand, &ag = B.ag, &chunks = B.chunks, &abits = B.abits;
     unsigned long long *vmark = B.lmask.p + kLmMark;  // word kLmMark of each mask row (stride kLmWords)
     auto &lmask = B.lmask, &rmask = B.rmask;
@@ -2100,16 +2101,9 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     uint32_t dc_rows = B.dc_rows;
     const uint32_t fg = 4096;
 
-    BuildCounters *h_ctr = nullptr;
-    PADO_HIP(hipHostMalloc((void **)&h_ctr, 4 * sizeof(BuildCounters), hipHostMallocDefault));
-    struct PinnedFree {
-        BuildCounters *p;
-        ~PinnedFree()
-        {
-            std::lock_guard<std::recursive_mutex> g(capture_mutex());
-            (void)hipHostFree(p);
-        }
-    } pin{h_ctr};
+    PinnedBuf<BuildCounters[4]> pin;
+    PADO_TRY(pin.alloc(wp, st));
+    BuildCounters *h_ctr = *pin.p;
 
     // Launches go straight to the stream unless several builds run at once:
     // then their threads queue in the runtime, and captured graphs (one launch
@@ -2276,11 +2270,11 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         const uint32_t batch_end = std::min<uint64_t>((uint64_t)(b + 1) * batch, n);
         if (batch_end > dc_rows) {
             // Never with a block ahead: a batch is only enqueued early when the
-            // table already covers it.  hipFree/hipMalloc synchronise.  The new
+            // table already covers it.  The new
             // table starts all 255, so the previous batch's reset is a no-op on it.
             PADO_HIP(hipStreamSynchronize(st));
             dc_rows = (uint32_t)std::min<uint64_t>(n, std::max<uint64_t>(batch_end, dc_rows * 4ull));
-            PADO_TRY(dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots));
+            PADO_TRY(dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots, wp));
             hipLaunchKernelGGL(k_fill_u32, dim3(fg), dim3(256), 0, st, reinterpret_cast<uint32_t *>(dc.p),
                                (uint64_t)dc_rows * Rows<RW>::kRoots * sizeof(DT) / 4, ~0u);
             drop_graphs();
@@ -2354,7 +2348,7 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
             if (snap.pool_top * 5 > pool_size * 2 || (double)snap.pool_top + need > 0.8 * (double)pool_size) {
                 PADO_HIP(hipStreamSynchronize(st));
                 unsigned long long top = 0;
-                PADO_TRY(pool_repack(st, n, pool, lrec, (unsigned long long)need, &top));
+                PADO_TRY(pool_repack(st, wp, n, pool, lrec, (unsigned long long)need, &top));
                 snap_top_prev = top;
                 pool_size = pool.n;
                 S.pool = pool.p;
@@ -2467,7 +2461,7 @@ static pado_gpu_status batch_loop_t(std::vector<LoopJob> &jobs, hipStream_t st)
         // growable per-vertex arrays take up to four times their length.
         const unsigned long long pool =
             std::max<unsigned long long>(std::max<unsigned long long>(1ull << 22, 384ull * n), J.pool_min);
-        PADO_TRY((batch_alloc<W, kRow>(J.g, J.idx, kLoopWaves, kChunk, pool, n, false, bufs[j])));
+        PADO_TRY((batch_alloc<W, kRow>(J.g, J.idx, kLoopWaves, kChunk, pool, n, false, nullptr, bufs[j])));
         plans[j] = batch_plan<W>(J.g, J.idx, J.used, J.batch, bufs[j]);
     }
     DevBuf<BatchPlan<W>> dplans;

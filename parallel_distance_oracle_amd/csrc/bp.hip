@@ -160,9 +160,10 @@ pado_gpu_status build_bp(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<uint8_t>
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
     const uint64_t m = g->m;
+    WorkPool *wp = g->work.get();
     PADO_TRY(idx->bpd.alloc((uint64_t)n * kBpdStride));
     PADO_TRY(idx->bps.alloc((uint64_t)n * kBP * 2));
-    PADO_TRY(d_used.alloc(n));
+    PADO_TRY(d_used.alloc(n, wp));
     // Unused slots keep bp_dist = 255 and empty sets (PARA:674-679).
     hipLaunchKernelGGL(k_fill_u8, dim3(grid_for((uint64_t)n * kBpdStride, 256, 8192)), dim3(256), 0, st,
                        idx->bpd.p, (uint64_t)n * kBpdStride, kInf8);
@@ -197,15 +198,15 @@ pado_gpu_status build_bp(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<uint8_t>
     DevBuf<uint8_t> lvl;
     DevBuf<unsigned long long> s1, s0, ca, cb;
     DevBuf<uint32_t> vis, sel, cnt;
-    PADO_TRY(lvl.alloc(n));
-    PADO_TRY(s1.alloc(n));
-    PADO_TRY(s0.alloc(n));
-    PADO_TRY(vis.alloc((n + 31) / 32 + 1));
+    PADO_TRY(lvl.alloc(n, wp));
+    PADO_TRY(s1.alloc(n, wp));
+    PADO_TRY(s0.alloc(n, wp));
+    PADO_TRY(vis.alloc((n + 31) / 32 + 1, wp));
     const uint64_t max_chunks = m / kChunk + n + 64;
-    PADO_TRY(ca.alloc(max_chunks));
-    PADO_TRY(cb.alloc(max_chunks));
-    PADO_TRY(sel.alloc(kBP * 64));
-    PADO_TRY(cnt.alloc(2));
+    PADO_TRY(ca.alloc(max_chunks, wp));
+    PADO_TRY(cb.alloc(max_chunks, wp));
+    PADO_TRY(sel.alloc(kBP * 64, wp));
+    PADO_TRY(cnt.alloc(2, wp));
     PADO_HIP(hipMemcpyAsync(sel.p, sel_all.data(), sizeof(uint32_t) * kBP * 64, hipMemcpyHostToDevice, st));
 
     uint32_t *h_cnt = nullptr;

@@ -393,9 +393,10 @@ pado_gpu_status build_bp_seeded(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<u
     hipStream_t st = g->ctx->stream;
     const uint32_t n = g->n;
     const uint64_t m = g->m;
+    WorkPool *wp = g->work.get();
     PADO_TRY(idx->bpd.alloc((uint64_t)n * kBpdStride));
     PADO_TRY(idx->bps.alloc((uint64_t)n * kBP * 2));
-    PADO_TRY(d_used.alloc(n));
+    PADO_TRY(d_used.alloc(n, wp));
     const std::vector<uint32_t> &sv = seeds.v, &ss = seeds.slot, &sj = seeds.j;
     PADO_HIP(hipMemcpyAsync(d_used.p, h_used.data(), n, hipMemcpyHostToDevice, st));
 
@@ -403,14 +404,14 @@ pado_gpu_status build_bp_seeded(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<u
     DevBuf<u64> masks, pieces[2];
     DevBuf<uint32_t> lists, dseeds;
     DevBuf<MsCounts> cnt;
-    PADO_TRY(masks.alloc(5ull * n));
+    PADO_TRY(masks.alloc(5ull * n, wp));
     const uint64_t max_pieces = m / kMsPiece + n;
-    PADO_TRY(pieces[0].alloc(max_pieces));
-    PADO_TRY(pieces[1].alloc(max_pieces));
-    PADO_TRY(lists.alloc(3ull * n));
-    PADO_TRY(cnt.alloc(1));
+    PADO_TRY(pieces[0].alloc(max_pieces, wp));
+    PADO_TRY(pieces[1].alloc(max_pieces, wp));
+    PADO_TRY(lists.alloc(3ull * n, wp));
+    PADO_TRY(cnt.alloc(1, wp));
     const uint32_t ns = (uint32_t)sv.size();
-    PADO_TRY(dseeds.alloc(3ull * (ns ? ns : 1)));
+    PADO_TRY(dseeds.alloc(3ull * (ns ? ns : 1), wp));
     std::vector<uint32_t> packed(sv);
     packed.insert(packed.end(), ss.begin(), ss.end());
     packed.insert(packed.end(), sj.begin(), sj.end());
@@ -423,19 +424,9 @@ pado_gpu_status build_bp_seeded(pado_gpu_graph *g, pado_gpu_index *idx, DevBuf<u
     hipLaunchKernelGGL(k_ms_fill, dim3(32), dim3(256), 0, st, (uint8_t *)nullptr, 0ull, (u64 *)cnt.p,
                        (uint64_t)sizeof(MsCounts) / 8);
 
-    MsCounts *h_cnt = nullptr;
-    {
-        std::lock_guard<std::recursive_mutex> cap_lock(capture_mutex());
-        PADO_HIP(hipHostMalloc((void **)&h_cnt, sizeof(MsCounts), hipHostMallocDefault));
-    }
-    struct PinnedFree {
-        MsCounts *p;
-        ~PinnedFree()
-        {
-            std::lock_guard<std::recursive_mutex> g(capture_mutex());
-            (void)hipHostFree(p);
-        }
-    } pin{h_cnt};
+    PinnedBuf<MsCounts> pin;
+    PADO_TRY(pin.alloc(wp, st));
+    MsCounts *h_cnt = pin.p;
     struct Events {
         hipEvent_t e[2] = {nullptr, nullptr};
         ~Events()

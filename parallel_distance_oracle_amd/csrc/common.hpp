@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -103,22 +104,70 @@ constexpr uint32_t kQRecWords = 32, kQRecFold = 16, kQRecTail = 28;
 constexpr uint32_t kWRecWords = 4;
 constexpr uint32_t kListAlign = 32;  // label list alignment: one 128-byte line
 
-// Device buffer owned by a handle.  kBufSlack bytes past its end are its own
-// too: a 16-byte read that starts inside it may run over the end (query.hip).
+// Temporary device memory of one context's calls, kept from one call for the
+// next: a build of R-MAT 20 spent 15 ms of 152 in hipMalloc and hipFree, and
+// memory that goes back to the driver is cleared before it is handed out again
+// (a build now and then took 300 ms longer once the card's memory had gone
+// round).  Everything that takes blocks from it uses them on the context's
+// stream only, so a block given back while that stream still works on it is
+// safe with the next taker.  What lies idle in it is bounded: a sixteenth of
+// the card while a graph of the context lives (it may be built again), else
+// kIdleWork; all of it goes back when the context is destroyed and whenever an
+// allocation fails.  Safe with several threads.
+class WorkPool {
+public:
+    explicit WorkPool(size_t card_bytes);
+    ~WorkPool();
+    // A block of at least `bytes` bytes (its size in *got), or null.
+    void *take(size_t bytes, size_t *got);
+    void give(void *p, size_t bytes);
+    // Page-locked host memory of kPinned bytes, or null.
+    void *take_pinned();
+    void give_pinned(void *p);
+    void hold(int graphs);  // graphs of the context that live, more or fewer
+    void collect(size_t keep, std::vector<void *> *out);  // takes out idle blocks, oldest first
+    void close();                                         // the context is gone
+    static constexpr size_t kPinned = 131072;
+
+private:
+    struct Block {
+        void *p;
+        size_t bytes;
+    };
+    std::mutex mu_;
+    std::vector<Block> idle_;  // in the order they were given back
+    std::vector<void *> pinned_;
+    size_t idle_bytes_ = 0, card_bytes_ = 0;
+    int graphs_ = 0;
+    bool closed_ = false;
+    size_t limit() const;
+};
+
+// hipMalloc under capture_mutex; where it fails, what the process's pools hold
+// idle goes back and it is tried once more.
+hipError_t device_alloc(void **p, size_t bytes);
+
+// Device buffer owned by a handle or, with a pool, by a call.  kBufSlack bytes
+// past its end are its own too: a 16-byte read that starts inside it may run
+// over the end (query.hip).
 constexpr size_t kBufSlack = 16;
 template <class T>
 struct DevBuf {
     T *p = nullptr;
     size_t n = 0;
-    pado_gpu_status alloc(size_t count)
+    pado_gpu_status alloc(size_t count, WorkPool *pool = nullptr)
     {
         release();
         if (count == 0) count = 1;
-        std::lock_guard<std::recursive_mutex> g(capture_mutex());
-        hipError_t e = hipMalloc((void **)&p, count * sizeof(T) + kBufSlack);
-        if (e != hipSuccess) {
+        const size_t bytes = count * sizeof(T) + kBufSlack;
+        if (pool) {
+            p = static_cast<T *>(pool->take(bytes, &held_));
+            pool_ = p ? pool : nullptr;
+        } else if (device_alloc((void **)&p, bytes) != hipSuccess) {
             p = nullptr;
-            set_error("hipMalloc(" + std::to_string(count * sizeof(T)) + " B): " + hipGetErrorString(e));
+        }
+        if (!p) {
+            set_error("hipMalloc(" + std::to_string(count * sizeof(T)) + " B): out of memory");
             return PADO_GPU_ERR_NOMEM;
         }
         n = count;
@@ -126,17 +175,63 @@ struct DevBuf {
     }
     void release()
     {
-        if (p) {
+        if (p && pool_) {
+            pool_->give(p, held_);
+        } else if (p) {
             std::lock_guard<std::recursive_mutex> g(capture_mutex());
             (void)hipFree(p);
         }
         p = nullptr;
         n = 0;
+        pool_ = nullptr;
+    }
+    void swap(DevBuf &o)
+    {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+        std::swap(pool_, o.pool_);
+        std::swap(held_, o.held_);
     }
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { release(); }
+
+private:
+    WorkPool *pool_ = nullptr;
+    size_t held_ = 0;  // the pool block's bytes
+};
+
+// A call's page-locked T, written by copies on stream st: they are done before
+// it goes back.
+template <class T>
+struct PinnedBuf {
+    static_assert(sizeof(T) <= WorkPool::kPinned);
+    T *p = nullptr;
+    pado_gpu_status alloc(WorkPool *pool, hipStream_t st)
+    {
+        p = static_cast<T *>(pool->take_pinned());
+        if (!p) {
+            set_error("hipHostMalloc failed");
+            return PADO_GPU_ERR_NOMEM;
+        }
+        pool_ = pool;
+        st_ = st;
+        return PADO_GPU_OK;
+    }
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf &) = delete;
+    PinnedBuf &operator=(const PinnedBuf &) = delete;
+    ~PinnedBuf()
+    {
+        if (!p) return;
+        (void)hipStreamSynchronize(st_);
+        pool_->give_pinned(p);
+    }
+
+private:
+    WorkPool *pool_ = nullptr;
+    hipStream_t st_ = nullptr;
 };
 
 // The first active lane's value, in scalar registers: for values that are the
@@ -288,10 +383,16 @@ struct pado_gpu_ctx {
     hipEvent_t side_ev = nullptr;     // orders the side stream after work queued before a query
     int num_cu = 0;
     bool concurrent = false;          // one of several contexts whose builds run at once (a many-graph job)
+    std::shared_ptr<pado::WorkPool> work;  // temporaries of calls on `stream`
 };
 
 struct pado_gpu_graph {
+    explicit pado_gpu_graph(pado_gpu_ctx *c) : ctx(c), work(c->work) { work->hold(1); }
+    ~pado_gpu_graph() { work->hold(-1); }
+    pado_gpu_graph(const pado_gpu_graph &) = delete;
+    pado_gpu_graph &operator=(const pado_gpu_graph &) = delete;
     pado_gpu_ctx *ctx = nullptr;
+    std::shared_ptr<pado::WorkPool> work;  // (a graph may outlive its context)
     uint32_t n = 0;
     uint64_t m = 0;  // directed edge count (2x undirected)
     pado::DevBuf<uint64_t> off;

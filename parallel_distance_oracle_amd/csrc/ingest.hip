@@ -95,14 +95,15 @@ extern "C" pado_gpu_status pado_gpu_graph_from_edges(pado_gpu_ctx *ctx, const ui
         }
     }
     hipStream_t st = ctx->stream;
+    WorkPool *wp = ctx->work.get();
     DevBuf<uint32_t> d_e, deg, rank, deg_new, cursor;
     DevBuf<uint8_t> d_w;
     DevBuf<unsigned long long> keys, sorted;
-    PADO_TRY(d_e.alloc(md));
-    PADO_TRY(deg.alloc(n));
+    PADO_TRY(d_e.alloc(md, wp));
+    PADO_TRY(deg.alloc(n, wp));
     PADO_HIP(hipMemcpyAsync(d_e.p, edges, 4 * md, hipMemcpyHostToDevice, st));
     if (weights) {
-        PADO_TRY(d_w.alloc(m));
+        PADO_TRY(d_w.alloc(m, wp));
         PADO_HIP(hipMemcpyAsync(d_w.p, w8.data(), m, hipMemcpyHostToDevice, st));
     }
     PADO_HIP(hipMemsetAsync(deg.p, 0, 4ull * n, st));
@@ -131,26 +132,25 @@ extern "C" pado_gpu_status pado_gpu_graph_from_edges(pado_gpu_ctx *ctx, const ui
         }
     }
     // id_transfer (GR:176-206): renumber, then each list sorted descending.
-    auto *g = new pado_gpu_graph();
+    auto *g = new pado_gpu_graph(ctx);
     struct Guard {
         pado_gpu_graph *&g;
         ~Guard() { delete g; }
     } guard{g};
-    g->ctx = ctx;
     g->n = n;
     g->m = md;
     g->weighted = weights != nullptr;
-    PADO_TRY(rank.alloc(n));
-    PADO_TRY(deg_new.alloc(n));
-    PADO_TRY(cursor.alloc(n));
+    PADO_TRY(rank.alloc(n, wp));
+    PADO_TRY(deg_new.alloc(n, wp));
+    PADO_TRY(cursor.alloc(n, wp));
     PADO_TRY(g->off.alloc((uint64_t)n + 1));
     PADO_TRY(g->adj.alloc(md));
     if (weights) PADO_TRY(g->w.alloc(md));
-    PADO_TRY(keys.alloc(md));
-    PADO_TRY(sorted.alloc(md));
+    PADO_TRY(keys.alloc(md, wp));
+    PADO_TRY(sorted.alloc(md, wp));
     PADO_HIP(hipMemcpyAsync(rank.p, h_rank.data(), 4ull * n, hipMemcpyHostToDevice, st));
     hipLaunchKernelGGL(k_permute, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, rank.p, deg.p, deg_new.p);
-    PADO_TRY(scan_u32_to_u64(deg_new.p, g->off.p, n, st));
+    PADO_TRY(scan_u32_to_u64(deg_new.p, g->off.p, n, st, wp));
     PADO_HIP(hipMemsetAsync(cursor.p, 0, 4ull * n, st));
     hipLaunchKernelGGL(k_scatter, dim3(grid_for(m, 256, 8192)), dim3(256), 0, st, d_e.p,
                        weights ? d_w.p : (const uint8_t *)nullptr, m, rank.p, g->off.p, cursor.p, keys.p);
@@ -158,7 +158,7 @@ extern "C" pado_gpu_status pado_gpu_graph_from_edges(pado_gpu_ctx *ctx, const ui
     PADO_HIP(hipcub::DeviceSegmentedSort::SortKeysDescending(nullptr, bytes, keys.p, sorted.p, (int)md, (int)n,
                                                              g->off.p, g->off.p + 1, st));
     DevBuf<uint8_t> ws;
-    PADO_TRY(ws.alloc(bytes));
+    PADO_TRY(ws.alloc(bytes, wp));
     PADO_HIP(hipcub::DeviceSegmentedSort::SortKeysDescending(ws.p, bytes, keys.p, sorted.p, (int)md, (int)n,
                                                              g->off.p, g->off.p + 1, st));
     hipLaunchKernelGGL(k_split_keys, dim3(grid_for(md, 256, 8192)), dim3(256), 0, st, md, sorted.p, g->adj.p,

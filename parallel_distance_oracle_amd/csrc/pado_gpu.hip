@@ -30,6 +30,186 @@ static thread_local std::string g_last_error;
 void set_error(const std::string &msg) { g_last_error = msg; }
 void clear_error() { g_last_error.clear(); }
 
+namespace {
+
+// Every context's pool, for an allocation that fails (never destroyed: a
+// context may be let go at the process's end).
+struct Pools {
+    std::mutex mu;
+    std::vector<WorkPool *> v;
+};
+Pools &pools()
+{
+    static Pools *p = new Pools;
+    return *p;
+}
+
+constexpr size_t kIdleWork = 256ull << 20;
+
+// Block sizes in steps of an eighth, so that calls of about one size share
+// their blocks.
+size_t block_size(size_t bytes)
+{
+    size_t step = 4096;
+    while (step * 16 <= bytes) step *= 2;
+    return (bytes + step - 1) / step * step;
+}
+
+void free_blocks(const std::vector<void *> &v)
+{
+    if (v.empty()) return;
+    std::lock_guard<std::recursive_mutex> g(capture_mutex());
+    for (void *p : v) (void)hipFree(p);
+}
+
+}  // namespace
+
+hipError_t device_alloc(void **p, size_t bytes)
+{
+    {
+        std::lock_guard<std::recursive_mutex> g(capture_mutex());
+        const hipError_t e = hipMalloc(p, bytes);
+        if (e == hipSuccess) return e;
+        (void)hipGetLastError();
+    }
+    std::vector<void *> out;
+    {
+        std::lock_guard<std::mutex> g(pools().mu);
+        for (WorkPool *w : pools().v) w->collect(0, &out);
+    }
+    free_blocks(out);
+    std::lock_guard<std::recursive_mutex> g(capture_mutex());
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
+WorkPool::WorkPool(size_t card_bytes) : card_bytes_(card_bytes)
+{
+    std::lock_guard<std::mutex> g(pools().mu);
+    pools().v.push_back(this);
+}
+
+WorkPool::~WorkPool()
+{
+    {
+        std::lock_guard<std::mutex> g(pools().mu);
+        auto &v = pools().v;
+        v.erase(std::find(v.begin(), v.end(), this));
+    }
+    close();
+}
+
+size_t WorkPool::limit() const
+{
+    return closed_ ? 0 : graphs_ > 0 ? std::max(card_bytes_ / 16, kIdleWork) : kIdleWork;
+}
+
+void WorkPool::close()
+{
+    std::vector<void *> out, pinned;
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        closed_ = true;
+        pinned.swap(pinned_);
+    }
+    collect(0, &out);
+    free_blocks(out);
+    std::lock_guard<std::recursive_mutex> g(capture_mutex());
+    for (void *p : pinned) (void)hipHostFree(p);
+}
+
+void *WorkPool::take(size_t bytes, size_t *got)
+{
+    bytes = block_size(bytes);
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        size_t best = idle_.size();
+        for (size_t i = 0; i < idle_.size(); ++i)
+            if (idle_[i].bytes >= bytes && idle_[i].bytes <= bytes + bytes / 4 &&
+                (best == idle_.size() || idle_[i].bytes < idle_[best].bytes))
+                best = i;
+        if (best < idle_.size()) {
+            const Block b = idle_[best];
+            idle_.erase(idle_.begin() + (ptrdiff_t)best);
+            idle_bytes_ -= b.bytes;
+            *got = b.bytes;
+            return b.p;
+        }
+    }
+    void *p = nullptr;
+    if (device_alloc(&p, bytes) != hipSuccess) return nullptr;
+    *got = bytes;
+    return p;
+}
+
+void WorkPool::give(void *p, size_t bytes)
+{
+    std::vector<void *> out;
+    size_t keep;
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        idle_.push_back({p, bytes});
+        idle_bytes_ += bytes;
+        keep = limit();
+    }
+    collect(keep, &out);
+    free_blocks(out);
+}
+
+void WorkPool::collect(size_t keep, std::vector<void *> *out)
+{
+    std::lock_guard<std::mutex> g(mu_);
+    size_t k = 0;
+    while (k < idle_.size() && idle_bytes_ > keep) {
+        out->push_back(idle_[k].p);
+        idle_bytes_ -= idle_[k].bytes;
+        ++k;
+    }
+    idle_.erase(idle_.begin(), idle_.begin() + (ptrdiff_t)k);
+}
+
+void WorkPool::hold(int graphs)
+{
+    std::vector<void *> out;
+    size_t keep;
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        graphs_ += graphs;
+        keep = limit();
+    }
+    collect(keep, &out);
+    free_blocks(out);
+}
+
+void *WorkPool::take_pinned()
+{
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        if (!pinned_.empty()) {
+            void *p = pinned_.back();
+            pinned_.pop_back();
+            return p;
+        }
+    }
+    void *p = nullptr;
+    std::lock_guard<std::recursive_mutex> g(capture_mutex());
+    return hipHostMalloc(&p, kPinned, hipHostMallocDefault) == hipSuccess ? p : nullptr;
+}
+
+void WorkPool::give_pinned(void *p)
+{
+    {
+        std::lock_guard<std::mutex> g(mu_);
+        if (!closed_ && pinned_.size() < 4) {
+            pinned_.push_back(p);
+            return;
+        }
+    }
+    std::lock_guard<std::recursive_mutex> g(capture_mutex());
+    (void)hipHostFree(p);
+}
+
 pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                              uint64_t k, uint8_t *out, bool ref_compat, hipStream_t st);
 pado_gpu_status launch_wquery(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
@@ -163,15 +343,16 @@ pado_gpu_status order_index(pado_gpu_index *idx, const uint32_t *h_rank)
     }
     DevBuf<uint32_t> rank, cnt;
     DevBuf<uint64_t> qoff;
-    PADO_TRY(rank.alloc(n));
-    PADO_TRY(cnt.alloc(n));
-    PADO_TRY(qoff.alloc((uint64_t)n + 1));
+    WorkPool *wp = idx->ctx->work.get();
+    PADO_TRY(rank.alloc(n, wp));
+    PADO_TRY(cnt.alloc(n, wp));
+    PADO_TRY(qoff.alloc((uint64_t)n + 1, wp));
     if (h_rank)
         PADO_HIP(hipMemcpyAsync(rank.p, h_rank, sizeof(uint32_t) * n, hipMemcpyHostToDevice, st));
     else
         hipLaunchKernelGGL(k_iota, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, rank.p);
     hipLaunchKernelGGL(k_order_counts, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, n, rank.p, idx->loff.p, cnt.p);
-    PADO_TRY(scan_u32_to_u64(cnt.p, qoff.p, n, st));
+    PADO_TRY(scan_u32_to_u64(cnt.p, qoff.p, n, st, wp));
     uint64_t total = 0;
     PADO_HIP(copy_sync(&total, qoff.p + n, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
     PADO_TRY(idx->qlab.alloc(total));
@@ -270,7 +451,12 @@ pado_gpu_status pado_gpu_ctx_create(int device, pado_gpu_ctx **out)
     auto *c = new pado_gpu_ctx();
     c->device = device;
     hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, device) == hipSuccess) c->num_cu = prop.multiProcessorCount;
+    size_t card = 0;
+    if (hipGetDeviceProperties(&prop, device) == hipSuccess) {
+        c->num_cu = prop.multiProcessorCount;
+        card = prop.totalGlobalMem;
+    }
+    c->work = std::make_shared<WorkPool>(card);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&c->side_ev, hipEventDisableTiming) != hipSuccess) {
@@ -291,6 +477,7 @@ void pado_gpu_ctx_destroy(pado_gpu_ctx *ctx)
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->side_ev) (void)hipEventDestroy(ctx->side_ev);
+    ctx->work->close();
     delete ctx;
 }
 
@@ -344,8 +531,7 @@ pado_gpu_status pado_gpu_graph_upload(pado_gpu_ctx *ctx, uint32_t n, uint64_t m_
                 set_error("adjacency lists must be sorted descending (rank space, after id_transfer)");
                 return PADO_GPU_ERR_ARG;
             }
-    auto *g = new pado_gpu_graph();
-    g->ctx = ctx;
+    auto *g = new pado_gpu_graph(ctx);
     g->n = n;
     g->m = m_dir;
     g->h_off.assign(off, off + n + 1);
@@ -423,6 +609,11 @@ pado_gpu_status pado_gpu_build(pado_gpu_ctx *ctx, const pado_gpu_graph *graph, c
             s = build_batches(g, idx, used, c);
             idx->ms_batch = t1.ms();
         }
+    }
+    // Other streams may read the index as soon as this returns.
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess && s == PADO_GPU_OK) {
+        set_error("labeling failed on the device");
+        s = PADO_GPU_ERR_HIP;
     }
     if (s != PADO_GPU_OK) {
         delete idx;

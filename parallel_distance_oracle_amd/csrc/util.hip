@@ -46,15 +46,15 @@ extern "C" pado_gpu_status pado_gpu_copy_bytes(pado_gpu_ctx *ctx, void *dst, con
     return PADO_GPU_OK;
 }
 
-pado_gpu_status scan_u32_to_u64(const uint32_t *in, uint64_t *out, uint32_t n, hipStream_t s)
+pado_gpu_status scan_u32_to_u64(const uint32_t *in, uint64_t *out, uint32_t n, hipStream_t s, WorkPool *wp)
 {
     DevBuf<uint64_t> tmp;
-    PADO_TRY(tmp.alloc((uint64_t)n + 1));
+    PADO_TRY(tmp.alloc((uint64_t)n + 1, wp));
     hipLaunchKernelGGL(k_widen, dim3(grid_for((uint64_t)n + 1, 256, 8192)), dim3(256), 0, s, in, tmp.p, n);
     size_t bytes = 0;
     PADO_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, tmp.p, out, (int)(n + 1), s));
     DevBuf<uint8_t> ws;
-    PADO_TRY(ws.alloc(bytes));
+    PADO_TRY(ws.alloc(bytes, wp));
     PADO_HIP(hipcub::DeviceScan::ExclusiveSum(ws.p, bytes, tmp.p, out, (int)(n + 1), s));
     PADO_HIP(hipStreamSynchronize(s));
     return PADO_GPU_OK;
@@ -69,7 +69,7 @@ __global__ void k_rel_offsets(const uint64_t *off, uint32_t v0, uint32_t cnt, ui
 }
 
 pado_gpu_status segmented_sort_u32(uint32_t *keys, uint64_t total, const uint64_t *off, uint32_t n,
-                                   hipStream_t s, uint64_t max_items)
+                                   hipStream_t s, uint64_t max_items, WorkPool *wp)
 {
     if (total == 0 || n == 0) return PADO_GPU_OK;
     // hipCUB takes the item and segment counts as int: an index with more than
@@ -102,9 +102,9 @@ pado_gpu_status segmented_sort_u32(uint32_t *keys, uint64_t total, const uint64_
     uint64_t biggest = 0;
     for (size_t r = 0; r + 1 < cuts.size(); ++r) biggest = std::max<uint64_t>(biggest, h_base[r + 1] - h_base[r]);
     DevBuf<uint32_t> out;
-    PADO_TRY(out.alloc(biggest));
+    PADO_TRY(out.alloc(biggest, wp));
     DevBuf<uint64_t> rel;
-    if (cuts.size() > 2) PADO_TRY(rel.alloc((uint64_t)n + 1));
+    if (cuts.size() > 2) PADO_TRY(rel.alloc((uint64_t)n + 1, wp));
     DevBuf<uint8_t> ws;
     for (size_t r = 0; r + 1 < cuts.size(); ++r) {
         const uint32_t v0 = cuts[r], v1 = cuts[r + 1];
@@ -120,7 +120,7 @@ pado_gpu_status segmented_sort_u32(uint32_t *keys, uint64_t total, const uint64_
         size_t bytes = 0;
         PADO_HIP(hipcub::DeviceSegmentedSort::SortKeys(nullptr, bytes, kr, out.p, (int)items, (int)(v1 - v0), o,
                                                        o + 1, s));
-        if (bytes > ws.n) PADO_TRY(ws.alloc(bytes));
+        if (bytes > ws.n) PADO_TRY(ws.alloc(bytes, wp));
         PADO_HIP(hipcub::DeviceSegmentedSort::SortKeys(ws.p, bytes, kr, out.p, (int)items, (int)(v1 - v0), o, o + 1,
                                                        s));
         PADO_HIP(hipMemcpyAsync(kr, out.p, items * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));

@@ -873,34 +873,35 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     DevBuf<uint32_t> RT;  // batch roots' entries, transposed for the filter
     DevBuf<u64> PT;
     DevBuf<WCounters> ctr;
-    PADO_TRY(T.alloc((uint64_t)n * kWB));
-    PADO_TRY(RT.alloc((uint64_t)kWB * kWB));
-    PADO_TRY(PT.alloc((uint64_t)kWB * kWW));
-    PADO_TRY(P.alloc((uint64_t)n * kWW));
-    PADO_TRY(I.alloc((uint64_t)n * kWW));
+    WorkPool *wp = g->work.get();
+    PADO_TRY(T.alloc((uint64_t)n * kWB, wp));
+    PADO_TRY(RT.alloc((uint64_t)kWB * kWB, wp));
+    PADO_TRY(PT.alloc((uint64_t)kWB * kWW, wp));
+    PADO_TRY(P.alloc((uint64_t)n * kWW, wp));
+    PADO_TRY(I.alloc((uint64_t)n * kWW, wp));
     // Per-wave reservations in k_w_check leave holes: up to kWAlistGrab
     // active-list slots per wave beyond the real ones, and padded
     // descriptors fewer than the real ones plus kWChunkGrab per wave.
     const uint64_t check_waves = 4ull * kAddGrid;
     const uint64_t alist_cap = (uint64_t)n + kWAlistGrab * check_waves;
-    PADO_TRY(ag.alloc(alist_cap * kWW));
-    PADO_TRY(chunks.alloc(2 * (g->m / kChunk + (uint64_t)n) + kWChunkGrab * check_waves + 64));
-    PADO_TRY(tmark.alloc(n));
-    PADO_TRY(tlist.alloc(n));
-    PADO_TRY(imark.alloc(n));
-    PADO_TRY(ilist.alloc(n));
-    PADO_TRY(alist.alloc(alist_cap));
-    PADO_TRY(amask.alloc(alist_cap));
-    PADO_TRY(aend.alloc(alist_cap));
-    PADO_TRY(hmin.alloc(n));
-    PADO_TRY(len.alloc(n));
-    PADO_TRY(cap.alloc(n));
-    PADO_TRY(base.alloc(n));
-    PADO_TRY(ctr.alloc(1 + (kStatRows * kStatCols * 8 + sizeof(WCounters) - 1) / sizeof(WCounters)));
+    PADO_TRY(ag.alloc(alist_cap * kWW, wp));
+    PADO_TRY(chunks.alloc(2 * (g->m / kChunk + (uint64_t)n) + kWChunkGrab * check_waves + 64, wp));
+    PADO_TRY(tmark.alloc(n, wp));
+    PADO_TRY(tlist.alloc(n, wp));
+    PADO_TRY(imark.alloc(n, wp));
+    PADO_TRY(ilist.alloc(n, wp));
+    PADO_TRY(alist.alloc(alist_cap, wp));
+    PADO_TRY(amask.alloc(alist_cap, wp));
+    PADO_TRY(aend.alloc(alist_cap, wp));
+    PADO_TRY(hmin.alloc(n, wp));
+    PADO_TRY(len.alloc(n, wp));
+    PADO_TRY(cap.alloc(n, wp));
+    PADO_TRY(base.alloc(n, wp));
+    PADO_TRY(ctr.alloc(1 + (kStatRows * kStatCols * 8 + sizeof(WCounters) - 1) / sizeof(WCounters), wp));
     u64 pool_size = std::max<u64>(1ull << 22, 32ull * n);
-    PADO_TRY(pool.alloc(pool_size));
+    PADO_TRY(pool.alloc(pool_size, wp));
     uint32_t dc_slots = std::min<uint32_t>(n, 1u << 14);
-    PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB));
+    PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB, wp));
     const uint32_t fg = 4096;
     hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, dcw.p, (uint64_t)dc_slots * kWB, kWInf);
     hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, T.p, (uint64_t)n * kWB, kWInf);
@@ -913,17 +914,10 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, cap.p, (uint64_t)n, 0u);
     hipLaunchKernelGGL(k_w_zero64, dim3(fg), dim3(256), 0, st, base.p, (uint64_t)n);
     PADO_HIP(hipMemsetAsync(ctr.p, 0, ctr.n * sizeof(WCounters), st));
-    WCounters *h = nullptr;
-    PADO_HIP(hipHostMalloc((void **)&h, sizeof(WCounters), hipHostMallocDefault));
+    PinnedBuf<WCounters> pin;
+    PADO_TRY(pin.alloc(wp, st));
+    WCounters *h = pin.p;
     std::memset(h, 0, sizeof(WCounters));
-    struct PinnedFree {
-        WCounters *p;
-        ~PinnedFree()
-        {
-            std::lock_guard<std::recursive_mutex> g(capture_mutex());
-            (void)hipHostFree(p);
-        }
-    } pin{h};
 
     WStore S{pool.p, base.p, len.p, cap.p, pool_size};
     // The first batch takes a quarter of the roots: nothing prunes its
@@ -942,7 +936,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
         // that many table rows always suffice (no device round trip).
         if (rs + rsz > dc_slots) {
             dc_slots = std::min<uint32_t>(n, std::max<uint32_t>(rs + rsz, dc_slots * 2));
-            PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB));
+            PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB, wp));
             hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, dcw.p, (uint64_t)dc_slots * kWB, kWInf);
         }
         hipLaunchKernelGGL(k_w_init, dim3(rb), dim3(256 * (1 + kWInitFill)), 0, st, rs, rsz, gen_batch, g->off.p, g->adj.p, T.p, tmark.p,
@@ -1015,8 +1009,8 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
             const u64 nsize = std::max<u64>(pool_size * 2, 4 * no[n] + 2 * added + 8ull * h->n_touched + 1024);
             DevBuf<u64> np;
             DevBuf<uint64_t> dno;
-            PADO_TRY(np.alloc(nsize));
-            PADO_TRY(dno.alloc((uint64_t)n + 1));
+            PADO_TRY(np.alloc(nsize, wp));
+            PADO_TRY(dno.alloc((uint64_t)n + 1, wp));
             PADO_HIP(copy_sync(dno.p, no.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st));
             hipLaunchKernelGGL(k_w_move, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, pool.p,
                                base.p, len.p, dno.p, np.p);
@@ -1024,8 +1018,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
             std::vector<u64> nb64(no.begin(), no.end() - 1);
             PADO_HIP(copy_sync(base.p, nb64.data(), 8ull * n, hipMemcpyHostToDevice, st));
             PADO_HIP(copy_sync(cap.p, nc.data(), 4ull * n, hipMemcpyHostToDevice, st));
-            std::swap(pool.p, np.p);
-            std::swap(pool.n, np.n);
+            pool.swap(np);
             pool_size = nsize;
             S.pool = pool.p;
             S.pool_size = pool_size;
@@ -1053,12 +1046,12 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     // root order and k_w_commit writes a batch's roots in ascending order, as
     // the reference's update_index appends them (WPARA:961-990).
     PADO_TRY(idx->loff.alloc((uint64_t)n + 1));
-    PADO_TRY(scan_u32_to_u64(len.p, idx->loff.p, n, st));
+    PADO_TRY(scan_u32_to_u64(len.p, idx->loff.p, n, st, wp));
     uint64_t total = 0;
     PADO_HIP(copy_sync(&total, idx->loff.p + n, 8, hipMemcpyDeviceToHost, st));
     idx->num_labels = total;
     DevBuf<u64> packed;
-    PADO_TRY(packed.alloc(total));
+    PADO_TRY(packed.alloc(total, wp));
     PADO_TRY(idx->whub.alloc(total));
     PADO_TRY(idx->wdist.alloc(total));
     hipLaunchKernelGGL(k_w_move, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, pool.p, base.p,
