@@ -2270,8 +2270,8 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         const uint32_t batch_end = std::min<uint64_t>((uint64_t)(b + 1) * batch, n);
         if (batch_end > dc_rows) {
             // Never with a block ahead: a batch is only enqueued early when the
-            // table already covers it.  The new
-            // table starts all 255, so the previous batch's reset is a no-op on it.
+            // table already covers it.  The new table starts all 255, so the
+            // previous batch's reset is a no-op on it.
             PADO_HIP(hipStreamSynchronize(st));
             dc_rows = (uint32_t)std::min<uint64_t>(n, std::max<uint64_t>(batch_end, dc_rows * 4ull));
             PADO_TRY(dc.alloc((uint64_t)dc_rows * Rows<RW>::kRoots, wp));

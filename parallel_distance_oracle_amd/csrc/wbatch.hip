@@ -294,6 +294,10 @@ __device__ inline void w_lds_sync()
 }
 
 constexpr uint32_t kWPushWaves = 4;  // waves per k_w_push block
+// Roots in a frontier word from which on k_w_push takes the word lane by lane,
+// kWPushEdges edges at a time (weighted R-MAT 20: 612 ms without, 597 at 16,
+// 598 at 24, 604 at 8; eight edges at a time 598).
+constexpr uint32_t kWDense = 16, kWPushEdges = 4;
 
 // Touched vertices up to which k_w_filter reads the roots' entries in place.
 constexpr uint32_t kWDirectFilter = 4096;
@@ -310,9 +314,13 @@ constexpr u64 kWChunkPad = 0xFFFFFFF0ull << 32;
 
 // send_messages (WPARA:435-522): relax the frontier's edges toward tails
 // ranked below each root.  A wave takes four 16-edge chunks (one edge per
-// lane) and walks the root words of its edges' groups in step; per word the
-// (edge, root) relaxations of all 64 lanes are spread over the wave, 64 per
-// step, so an edge with many roots does not hold up the others.
+// lane) and walks the root words of its edges' groups in step.  Chunks with
+// many roots in a word go edge by edge, lane = root: the source's distances
+// are read once for the chunk's edges, the tails' in whole lines.  For the
+// others the (edge, root) relaxations of all 64 lanes are spread over the
+// wave, 64 per step, so an edge with many roots does not hold up the others.
+// The first batches' rounds, most of the time, are bound by the random lines
+// of T that they read and update (about 2 TB/s).
 __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uint32_t rsz, uint32_t gen_batch,
                                                 const uint64_t *off, const uint32_t *adj, const uint8_t *wgt,
                                                 const uint32_t *alist, const u64 *ag, const uint32_t *amask,
@@ -361,42 +369,80 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         while (wall) {
             const uint32_t wd = __ffs(wall) - 1;
             wall &= wall - 1;
-            u64 g = 0;
+            u64 g = 0, all = 0;
             if ((words >> wd) & 1u) {
-                g = ag[(uint64_t)k * kWW + wd];
+                g = all = ag[(uint64_t)k * kWW + wd];
                 if (lim < (wd + 1) * 64) g &= (1ull << (lim - wd * 64)) - 1ull;
             }
+            // Chunks with many roots in this word: lane = root.
+            u64 imp = 0;
+            const u64 dense = __ballot(__popcll(all) >= (int)kWDense);
+            for (u64 todo = dense; todo;) {
+                const uint32_t l0 = (uint32_t)__ffsll(todo) - 1;
+                u64 edges = todo & (0xFFFFull << (l0 & ~(kChunk - 1)));  // this chunk's
+                todo &= ~edges;
+                const u64 roots = ((u64)__builtin_amdgcn_readlane((uint32_t)(all >> 32), l0) << 32) |
+                                  __builtin_amdgcn_readlane((uint32_t)all, l0);
+                const uint32_t *from = T + (uint64_t)__builtin_amdgcn_readlane(u, l0) * kWB + wd * 64;
+                const uint32_t du = (roots >> lane) & 1ull ? from[lane] : kWInf;
+                while (edges) {
+                    uint32_t e[kWPushEdges], cur[kWPushEdges], cand[kWPushEdges], *to[kWPushEdges];
+#pragma unroll
+                    for (uint32_t j = 0; j < kWPushEdges; ++j) {
+                        // (past the chunk's last edge: that edge again, relaxed by no lane)
+                        const bool more = edges != 0ull;
+                        e[j] = more ? (uint32_t)__ffsll(edges) - 1 : l0;
+                        edges &= edges - 1;
+                        const uint32_t le = more ? __builtin_amdgcn_readlane(lim, e[j]) : 0u;
+                        to[j] = T + (uint64_t)__builtin_amdgcn_readlane(t, e[j]) * kWB + wd * 64;
+                        const bool on = du != kWInf && wd * 64 + lane < le;
+                        cand[j] = on ? du + __builtin_amdgcn_readlane(w, e[j]) : kWInf;
+                        cur[j] = 0;
+                        if (on) cur[j] = to[j][lane];
+                        n_relax += on ? 1u : 0u;
+                    }
+#pragma unroll
+                    for (uint32_t j = 0; j < kWPushEdges; ++j) {
+                        bool better = false;
+                        if (cand[j] < cur[j]) better = cand[j] < atomicMin(to[j] + lane, cand[j]);
+                        const u64 who = __ballot(better);
+                        if (lane == e[j]) imp |= who;
+                    }
+                }
+            }
+            if ((dense >> lane) & 1ull) g = 0;
             const uint32_t cnt = (uint32_t)__popcll(g);
             const uint32_t incl = wave_incl_scan(cnt);
             const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-            if (total == 0) continue;
-            s_g[wv][lane] = g;
-            s_ex[wv][lane] = incl - cnt;
-            s_imp[wv][lane] = 0ull;
-            w_lds_sync();
-            for (uint32_t x0 = 0; x0 < total; x0 += 64) {
-                const uint32_t x = x0 + lane;
-                if (x >= total) continue;
-                uint32_t o = 0;
+            if (total) {
+                s_g[wv][lane] = g;
+                s_ex[wv][lane] = incl - cnt;
+                s_imp[wv][lane] = 0ull;
+                w_lds_sync();
+                for (uint32_t x0 = 0; x0 < total; x0 += 64) {
+                    const uint32_t x = x0 + lane;
+                    if (x >= total) continue;
+                    uint32_t o = 0;
 #pragma unroll
-                for (uint32_t sft = 32; sft; sft >>= 1)
-                    if (s_ex[wv][o + sft] <= x) o += sft;
-                const uint32_t b = w_nth_set_bit(s_g[wv][o], x - s_ex[wv][o]);
-                const uint32_t ro = wd * 64 + b;
-                const uint32_t du = T[(uint64_t)s_u[wv][o] * kWB + ro];
-                if (du == kWInf) continue;
-                const uint32_t cand = du + s_w[wv][o];
-                ++n_relax;
-                // A plain read first: values only fall during the kernel, so
-                // one read as <= cand (even a stale one) makes the atomic a no-op.
-                uint32_t *tt = &T[(uint64_t)s_t[wv][o] * kWB + ro];
-                if (cand < *tt) {
-                    const uint32_t old = atomicMin(tt, cand);
-                    if (cand < old) atomicOr(&s_imp[wv][o], 1ull << b);
+                    for (uint32_t sft = 32; sft; sft >>= 1)
+                        if (s_ex[wv][o + sft] <= x) o += sft;
+                    const uint32_t b = w_nth_set_bit(s_g[wv][o], x - s_ex[wv][o]);
+                    const uint32_t ro = wd * 64 + b;
+                    const uint32_t du = T[(uint64_t)s_u[wv][o] * kWB + ro];
+                    if (du == kWInf) continue;
+                    const uint32_t cand = du + s_w[wv][o];
+                    ++n_relax;
+                    // A plain read first: values only fall during the kernel, so
+                    // one read as <= cand (even a stale one) makes the atomic a no-op.
+                    uint32_t *tt = &T[(uint64_t)s_t[wv][o] * kWB + ro];
+                    if (cand < *tt) {
+                        const uint32_t old = atomicMin(tt, cand);
+                        if (cand < old) atomicOr(&s_imp[wv][o], 1ull << b);
+                    }
                 }
+                w_lds_sync();
+                imp |= s_imp[wv][lane];
             }
-            w_lds_sync();
-            const u64 imp = s_imp[wv][lane];
             if (imp) {
                 atomicOr(&I[(uint64_t)t * kWW + wd], imp);
                 got = true;
