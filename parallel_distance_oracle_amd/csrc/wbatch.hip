@@ -53,6 +53,7 @@ using u64 = unsigned long long;
 struct WCounters {
     uint32_t n_act[2];              // nonzero: the round has active vertices
     u64 rounds;
+    uint32_t hold;                  // a batch is not done: nothing after it runs (k_w_filter)
     alignas(128) uint32_t a_top[2];    // active-list slots handed out (per-wave reservations)
     alignas(128) uint32_t n_chunk[2];
     alignas(128) uint32_t n_imp[2];
@@ -67,6 +68,17 @@ struct WCounters {
     alignas(128) u64 relax, improved, pruned, filtered;
 };
 constexpr uint32_t kWStats = 4;
+
+// What the host learns of a batch (in page-locked memory).
+struct WClosed {
+    u64 rounds;
+    uint32_t held, n_touched;
+};
+constexpr uint32_t kWRing = 4;
+struct WHost {
+    WCounters c;
+    WClosed ring[kWRing];
+};
 
 struct WStore {
     u64 *pool;
@@ -164,10 +176,19 @@ __global__ __launch_bounds__(1024) void k_w_fold_stats(WCounters *C)
     if (threadIdx.x < kWStats) (&C->relax)[threadIdx.x] += s[threadIdx.x];
 }
 
-// Round 1's frontier is the batch's roots in order: root offset ro holds
-// active-list slot ro and touched-list entry ro (k_w_init).
-__global__ void k_w_reset_counters(WCounters *C, uint32_t rsz)
+// After a batch: its record for the host (`out`, unless null) and, if it is
+// done, the counters for a next batch of rsz roots (none if 0).  Round 1's
+// frontier is the batch's roots in order: root offset ro holds active-list
+// slot ro and touched-list entry ro (k_w_init).
+__global__ void k_w_close(WCounters *C, uint32_t rsz, WClosed *out)
 {
+    const uint32_t hold = C->hold;
+    if (out) {
+        out->rounds = C->rounds;
+        out->held = hold;
+        out->n_touched = C->n_touched;
+    }
+    if (hold || rsz == 0) return;
     C->n_act[0] = C->n_chunk[0] = C->n_chunk[1] = C->n_imp[0] = C->n_imp[1] = 0;
     C->a_top[0] = 0;
     C->n_act[1] = 1;
@@ -175,6 +196,8 @@ __global__ void k_w_reset_counters(WCounters *C, uint32_t rsz)
     C->n_touched = rsz;
     C->need = C->need_bound = 0;
 }
+
+__global__ void k_w_unhold(WCounters *C) { C->hold = 0; }
 
 // Earlier-batch labels of the batch roots -> root-distance table
 // (roots_labels_buffer, WPARA:322-348, transposed): dcw[h][ro] = d(root
@@ -226,6 +249,7 @@ __global__ __launch_bounds__(256 * (1 + kWInitFill)) void k_w_init(uint32_t rs, 
     __shared__ uint32_t s_nch[4], s_c0;
     const uint32_t lane = lane_id(), wv = (threadIdx.x >> 6) & 3u, part = threadIdx.x >> 8;
     const uint32_t ro = blockIdx.x * 4 + wv;
+    if (C->hold) return;
     if (part) {
         if (ro < rsz) w_hub_fill(ro, S.base[rs + ro], S.len[rs + ro], part - 1u, kWInitFill, S, hmin, dcw);
         __syncthreads();
@@ -302,6 +326,11 @@ constexpr uint32_t kWDense = 16, kWPushEdges = 4;
 // Touched vertices up to which k_w_filter reads the roots' entries in place.
 constexpr uint32_t kWDirectFilter = 4096;
 
+// Batches in flight, from the kWAheadFrom-th on (weighted R-MAT 20: 2: 575
+// ms, 1: 585, 3: 584, 4: 585, 7: 599 -- a batch that is held costs the empty
+// launches of those behind it).
+constexpr uint32_t kWAhead = 2, kWAheadFrom = 8;
+
 // Improved pairs of a tail up to which k_w_check reads single table entries.
 constexpr uint32_t kWGather = 8;
 
@@ -336,6 +365,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
     // Round `round` of the batch (slot round & 1; empty past the batch's
     // end).  Block 0 empties the other slot, which k_w_check fills.
     const uint32_t p = round & 1u;
+    if (C->hold) return;
     const uint32_t nc = C->n_chunk[p];
     const u64 gen_round = ((u64)gen_batch << 24) | round;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
@@ -485,6 +515,7 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t p = round & 1u;
+    if (C->hold) return;
     const uint32_t nimp = C->n_imp[p];
     if (blockIdx.x == 0 && threadIdx.x == 0) C->n_imp[p ^ 1u] = 0;
     uint32_t n_pruned = 0;
@@ -731,11 +762,23 @@ __global__ __launch_bounds__(256) void k_w_roots_t(uint32_t rs, uint32_t rsz, co
 // may reserve are summed into C->need.  kDirect: the roots' entries come from
 // T/P rows directly (8 scattered reads per witness and lane, no transpose
 // kernel; for batches that touch few vertices), else from RT/PT.
+// A batch enqueued in one go (gate) is held here if its rounds have not ended
+// (`slot`: where the next frontier would be) or if its commit might not fit
+// the pool: then this kernel and all later ones do nothing until the host has
+// seen to it.
 template <bool kDirect>
 __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, const uint32_t *tlist,
                                                   const uint32_t *T, const u64 *P, const uint32_t *RT, const u64 *PT,
-                                                  u64 *I, WStore S, WCounters *C)
+                                                  u64 *I, WStore S, WCounters *C, uint32_t gate, uint32_t slot)
 {
+    // (every block decides alike: nothing here changes what it reads)
+    if (gate) {
+        if (C->hold) return;
+        if (C->n_act[slot] != 0 || C->pool_top + C->need_bound > S.pool_size) {
+            if (blockIdx.x == 0 && threadIdx.x == 0) C->hold = 1;
+            return;
+        }
+    }
     __shared__ uint8_t sv[4][64];
     const uint32_t lane = lane_id();
     const uint32_t wib = threadIdx.x >> 6;
@@ -832,6 +875,7 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
 __global__ __launch_bounds__(256) void k_w_commit(uint32_t rs, uint32_t rsz, const uint32_t *tlist, uint32_t *T, u64 *P,
                                                   u64 *I, uint32_t *hmin, uint32_t *dcw, WStore S, WCounters *C)
 {
+    if (C->hold) return;
     const uint32_t lane = lane_id();
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
@@ -960,119 +1004,168 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, cap.p, (uint64_t)n, 0u);
     hipLaunchKernelGGL(k_w_zero64, dim3(fg), dim3(256), 0, st, base.p, (uint64_t)n);
     PADO_HIP(hipMemsetAsync(ctr.p, 0, ctr.n * sizeof(WCounters), st));
-    PinnedBuf<WCounters> pin;
+    PinnedBuf<WHost> pin;
     PADO_TRY(pin.alloc(wp, st));
-    WCounters *h = pin.p;
-    std::memset(h, 0, sizeof(WCounters));
+    std::memset(pin.p, 0, sizeof(WHost));
+    WCounters *h = &pin.p->c;
+    volatile WClosed *ring = pin.p->ring;
+    void *ring_dev = nullptr;
+    PADO_HIP(hipHostGetDevicePointer(&ring_dev, pin.p->ring, 0));
+    hipEvent_t ev[kWRing] = {};
+    struct EventFree {
+        hipEvent_t *e;
+        ~EventFree()
+        {
+            for (uint32_t i = 0; i < kWRing; ++i)
+                if (e[i]) (void)hipEventDestroy(e[i]);
+        }
+    } evf{ev};
+    for (hipEvent_t &e : ev) PADO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 
     WStore S{pool.p, base.p, len.p, cap.p, pool_size};
     // The first batch takes a quarter of the roots: nothing prunes its
     // searches, and its labels prune the next batch's (measured on weighted
     // R-MAT 20 / 22: 1.04 -> 0.95 s / 6.5 -> 6.3 s).  Any split of the rank
     // order into batches yields the same label set.
-    const uint32_t first = std::max<uint32_t>(1u, batch / 4);
-    uint32_t prev_rounds = 1;
-    uint32_t rs_next = 0;
-    for (uint32_t b = 0; rs_next < n; ++b) {
-        const uint32_t rs = rs_next, rsz = std::min(b ? batch : first, n - rs), gen_batch = b + 1;
-        rs_next = rs + rsz;
-        const uint32_t rb = (rsz * 64 + 255) / 256;
-        hipLaunchKernelGGL(k_w_reset_counters, dim3(1), dim3(1), 0, st, ctr.p, rsz);
-        // The hubs of the batch roots' labels are ids below the batch end, so
-        // that many table rows always suffice (no device round trip).
-        if (rs + rsz > dc_slots) {
-            dc_slots = std::min<uint32_t>(n, std::max<uint32_t>(rs + rsz, dc_slots * 2));
-            PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB, wp));
-            hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, dcw.p, (uint64_t)dc_slots * kWB, kWInf);
+    const uint32_t first = std::min(n, std::max<uint32_t>(1u, batch / 4));
+    const uint32_t nb = 1 + (n - first + batch - 1) / batch;
+    auto roots_start = [&](uint32_t b) { return b ? first + (b - 1) * batch : 0u; };
+    auto roots_size = [&](uint32_t b) { return b >= nb ? 0u : std::min(b ? batch : first, n - roots_start(b)); };
+    auto rounds = [&](uint32_t b, uint32_t done, uint32_t more) {
+        const uint32_t rs = roots_start(b), rsz = roots_size(b), gen_batch = b + 1;
+        for (uint32_t round = done + 1; round <= done + more; ++round) {
+            hipLaunchKernelGGL(k_w_push, dim3(kPushGrid), dim3(256), 0, st, round, rs, rsz, gen_batch, g->off.p,
+                               g->adj.p, g->w.p, alist.p, ag.p, amask.p, aend.p, chunks.p, T.p, I.p, tmark.p,
+                               tlist.p, imark.p, ilist.p, S, ctr.p);
+            hipLaunchKernelGGL(k_w_check, dim3(kAddGrid), dim3(256), 0, st, round, rs, ilist.p, g->off.p, g->adj.p,
+                               T.p, I.p, P.p, S, hmin.p, dcw.p, alist.p, ag.p, amask.p, aend.p,
+                               chunks.p, ctr.p);
         }
-        hipLaunchKernelGGL(k_w_init, dim3(rb), dim3(256 * (1 + kWInitFill)), 0, st, rs, rsz, gen_batch, g->off.p, g->adj.p, T.p, tmark.p,
-                           tlist.p, alist.p, ag.p, amask.p, aend.p, chunks.p, hmin.p, dcw.p, S, ctr.p);
-        // Rounds per host check: the previous batch's round count + 1 first
-        // (enough when this batch takes no more), then blocks of 2^j that
-        // double while a batch runs long.
-        // Round 1's frontier is the batch's roots (never empty); the counters
-        // seen last (after the previous batch's filter) hold every round so far.
-        uint32_t live = rsz;
-        const uint64_t rounds_before = h->rounds;
-        uint32_t launched = 0;
-        int j = 0;
-        while ((1u << j) < prev_rounds + 1 && j < 6) ++j;
-        while (live) {
-            const uint32_t blk = launched ? 1u << j : std::min<uint32_t>(prev_rounds + 1, 64u);
-            if (launched + blk >= (1u << 24)) {
-                set_error("a weighted batch needs more than 2^24 Bellman-Ford rounds");
-                return PADO_GPU_ERR_DOMAIN;
-            }
-            for (uint32_t u = 0; u < blk; ++u) {
-                const uint32_t round = launched + 1 + u;
-                hipLaunchKernelGGL(k_w_push, dim3(kPushGrid), dim3(256), 0, st, round, rs, rsz, gen_batch, g->off.p,
-                                   g->adj.p, g->w.p, alist.p, ag.p, amask.p, aend.p, chunks.p, T.p, I.p, tmark.p,
-                                   tlist.p, imark.p, ilist.p, S, ctr.p);
-                hipLaunchKernelGGL(k_w_check, dim3(kAddGrid), dim3(256), 0, st, round, rs, ilist.p, g->off.p, g->adj.p,
-                                   T.p, I.p, P.p, S, hmin.p, dcw.p, alist.p, ag.p, amask.p, aend.p,
-                                   chunks.p, ctr.p);
-            }
-            launched += blk;
-            PADO_HIP(hipMemcpyAsync(h, ctr.p, sizeof(WCounters), hipMemcpyDeviceToHost, st));
-            PADO_HIP(hipStreamSynchronize(st));
-            live = h->n_act[(launched + 1) & 1u];  // frontier of the next round
-            if (j < 6) ++j;
-        }
-        prev_rounds = (uint32_t)(h->rounds - rounds_before);
-        const u64 labels_before = h->labels;
-        // Few touched vertices: the filter reads the roots' entries in place
-        // instead of transposing them first.
-        if (h->n_touched <= kWDirectFilter) {
-            hipLaunchKernelGGL(k_w_filter<true>, dim3(2048), dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, RT.p, PT.p,
-                               I.p, S, ctr.p);
+    };
+    // Blocks for the touched vertices, by how many the last batch had.
+    auto touched_grid = [](uint32_t touched) { return std::min<uint32_t>(2048u, std::max<uint32_t>(256u, touched / 2)); };
+    // Few touched vertices: the filter reads the roots' entries in place
+    // instead of transposing them first.
+    auto filter = [&](uint32_t b, uint32_t touched, uint32_t gate, uint32_t slot) {
+        const uint32_t rs = roots_start(b), rsz = roots_size(b);
+        const dim3 grid(touched_grid(touched));
+        if (touched <= kWDirectFilter) {
+            hipLaunchKernelGGL(k_w_filter<true>, grid, dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, RT.p, PT.p, I.p,
+                               S, ctr.p, gate, slot);
         } else {
             hipLaunchKernelGGL(k_w_roots_t, dim3((kWB / 64) * (kWB / 64)), dim3(256), 0, st, rs, rsz, T.p, P.p, RT.p,
                                PT.p);
-            hipLaunchKernelGGL(k_w_filter<false>, dim3(2048), dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, RT.p,
-                               PT.p, I.p, S, ctr.p);
+            hipLaunchKernelGGL(k_w_filter<false>, grid, dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, RT.p, PT.p, I.p,
+                               S, ctr.p, gate, slot);
         }
-        // The touched vertices are known once the rounds end: when even the
-        // reservation bound fits the pool, the commit needs no host check.
-        bool grow = h->pool_top + h->need_bound > pool_size;
-        if (grow) {
-            PADO_HIP(hipMemcpyAsync(h, ctr.p, sizeof(WCounters), hipMemcpyDeviceToHost, st));
-            PADO_HIP(hipStreamSynchronize(st));
-            grow = h->pool_top + h->need > pool_size;
-        }
-        if (grow) {
-            // Compact every list into a larger pool.  After compaction a list of
-            // length L has capacity L + L/4 + 4, so the commit can reserve at
-            // most 2.5 * live + new + 8 * touched words.
-            const u64 added = h->labels - labels_before;
-            std::vector<uint32_t> hl(n);
-            PADO_HIP(copy_sync(hl.data(), len.p, 4ull * n, hipMemcpyDeviceToHost, st));
-            std::vector<uint64_t> no(n + 1, 0);
-            std::vector<uint32_t> nc(n);
-            for (uint32_t v = 0; v < n; ++v) {
-                nc[v] = hl[v] + (hl[v] >> 2) + 4;
-                no[v + 1] = no[v] + nc[v];
+    };
+    auto commit = [&](uint32_t b, uint32_t touched) {
+        const uint32_t rs = roots_start(b), rsz = roots_size(b);
+        hipLaunchKernelGGL(k_w_commit, dim3(touched_grid(touched)), dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, I.p,
+                           hmin.p, dcw.p, S, ctr.p);
+        hipLaunchKernelGGL(k_w_close, dim3(1), dim3(1), 0, st, ctr.p, roots_size(b + 1),
+                           static_cast<WClosed *>(ring_dev) + b % kWRing);
+    };
+    // Batches are enqueued whole, with as many rounds as the last three needed
+    // at most, and one ahead of the host's look at their records, so that the
+    // later ones (38 us of kernels each) do not wait for the host between
+    // their rounds and their filter.  A batch whose rounds turn out not to
+    // have ended, or whose labels might not fit the pool, holds everything
+    // behind it (k_w_filter); the host then ends it step by step and goes on
+    // from there.  Weighted R-MAT 20: 597 -> 576 ms; 200 K vertices: 80 -> 75.
+        constexpr uint32_t kRoundHistory = 3;
+    uint32_t hist[kRoundHistory] = {}, launched[kWRing] = {};
+    hist[0] = 6;
+    uint32_t next = 0, touched = n;  // batches enqueued; vertices the last batch touched
+    u64 rounds_seen = 0;
+    hipLaunchKernelGGL(k_w_close, dim3(1), dim3(1), 0, st, ctr.p, roots_size(0), (WClosed *)nullptr);
+    for (uint32_t b = 0; b < nb; ++b) {
+        // (the first few differ too much from each other to go ahead)
+        const uint32_t ahead = b < kWAheadFrom ? 1u : kWAhead;
+        for (; next < nb && next < b + ahead; ++next) {
+            const uint32_t rs = roots_start(next), rsz = roots_size(next);
+            // The hubs of the batch roots' labels are ids below the batch end, so
+            // that many table rows always suffice (no device round trip).  A
+            // batch that is held needs the table its rounds began with.
+            if (rs + rsz > dc_slots) {
+                if (next > b) break;
+                dc_slots = std::min<uint32_t>(n, std::max<uint32_t>(rs + rsz, dc_slots * 2));
+                PADO_TRY(dcw.alloc((uint64_t)dc_slots * kWB, wp));
+                hipLaunchKernelGGL(k_w_fill, dim3(fg), dim3(256), 0, st, dcw.p, (uint64_t)dc_slots * kWB, kWInf);
             }
-            const u64 nsize = std::max<u64>(pool_size * 2, 4 * no[n] + 2 * added + 8ull * h->n_touched + 1024);
-            DevBuf<u64> np;
-            DevBuf<uint64_t> dno;
-            PADO_TRY(np.alloc(nsize, wp));
-            PADO_TRY(dno.alloc((uint64_t)n + 1, wp));
-            PADO_HIP(copy_sync(dno.p, no.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st));
-            hipLaunchKernelGGL(k_w_move, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, pool.p,
-                               base.p, len.p, dno.p, np.p);
-            PADO_HIP(hipStreamSynchronize(st));
-            std::vector<u64> nb64(no.begin(), no.end() - 1);
-            PADO_HIP(copy_sync(base.p, nb64.data(), 8ull * n, hipMemcpyHostToDevice, st));
-            PADO_HIP(copy_sync(cap.p, nc.data(), 4ull * n, hipMemcpyHostToDevice, st));
-            pool.swap(np);
-            pool_size = nsize;
-            S.pool = pool.p;
-            S.pool_size = pool_size;
-            const u64 top = no[n];
-            PADO_HIP(copy_sync(&ctr.p->pool_top, &top, 8, hipMemcpyHostToDevice, st));
+            hipLaunchKernelGGL(k_w_init, dim3((rsz * 64 + 255) / 256), dim3(256 * (1 + kWInitFill)), 0, st, rs, rsz,
+                               next + 1, g->off.p, g->adj.p, T.p, tmark.p, tlist.p, alist.p, ag.p, amask.p, aend.p,
+                               chunks.p, hmin.p, dcw.p, S, ctr.p);
+            const uint32_t R = *std::max_element(hist, hist + kRoundHistory);
+            launched[next % kWRing] = R;
+            rounds(next, 0, R);
+            filter(next, touched, 1u, (R + 1) & 1u);
+            commit(next, touched);
+            PADO_HIP(hipEventRecord(ev[next % kWRing], st));
         }
-        hipLaunchKernelGGL(k_w_commit, dim3(2048), dim3(256), 0, st, rs, rsz, tlist.p, T.p, P.p, I.p, hmin.p, dcw.p,
-                           S, ctr.p);
+        PADO_HIP(hipEventSynchronize(ev[b % kWRing]));
+        PADO_HIP(hipGetLastError());
+        if (ring[b % kWRing].held) {
+            hipLaunchKernelGGL(k_w_unhold, dim3(1), dim3(1), 0, st, ctr.p);
+            uint32_t done = launched[b % kWRing], more = 1;
+            for (;;) {
+                PADO_HIP(hipMemcpyAsync(h, ctr.p, sizeof(WCounters), hipMemcpyDeviceToHost, st));
+                PADO_HIP(hipStreamSynchronize(st));
+                if (!h->n_act[(done + 1) & 1u]) break;  // no frontier for the next round
+                rounds(b, done, more);
+                done += more;
+                more = std::min(2 * more, 64u);
+            }
+            const u64 labels_before = h->labels;
+            filter(b, h->n_touched, 0u, 0u);
+            // The touched vertices are known once the rounds end: when even the
+            // reservation bound fits the pool, the commit needs no host check.
+            bool grow = h->pool_top + h->need_bound > pool_size;
+            if (grow) {
+                PADO_HIP(hipMemcpyAsync(h, ctr.p, sizeof(WCounters), hipMemcpyDeviceToHost, st));
+                PADO_HIP(hipStreamSynchronize(st));
+                grow = h->pool_top + h->need > pool_size;
+            }
+            if (grow) {
+                // Compact every list into a larger pool.  After compaction a list of
+                // length L has capacity L + L/4 + 4, so the commit can reserve at
+                // most 2.5 * live + new + 8 * touched words.
+                const u64 added = h->labels - labels_before;
+                std::vector<uint32_t> hl(n);
+                PADO_HIP(copy_sync(hl.data(), len.p, 4ull * n, hipMemcpyDeviceToHost, st));
+                std::vector<uint64_t> no(n + 1, 0);
+                std::vector<uint32_t> nc(n);
+                for (uint32_t v = 0; v < n; ++v) {
+                    nc[v] = hl[v] + (hl[v] >> 2) + 4;
+                    no[v + 1] = no[v] + nc[v];
+                }
+                const u64 nsize = std::max<u64>(pool_size * 2, 4 * no[n] + 2 * added + 8ull * h->n_touched + 1024);
+                DevBuf<u64> np;
+                DevBuf<uint64_t> dno;
+                PADO_TRY(np.alloc(nsize, wp));
+                PADO_TRY(dno.alloc((uint64_t)n + 1, wp));
+                PADO_HIP(copy_sync(dno.p, no.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st));
+                hipLaunchKernelGGL(k_w_move, dim3(grid_for((uint64_t)n * 64, 256, 8192)), dim3(256), 0, st, n, pool.p,
+                                   base.p, len.p, dno.p, np.p);
+                PADO_HIP(hipStreamSynchronize(st));
+                std::vector<u64> nb64(no.begin(), no.end() - 1);
+                PADO_HIP(copy_sync(base.p, nb64.data(), 8ull * n, hipMemcpyHostToDevice, st));
+                PADO_HIP(copy_sync(cap.p, nc.data(), 4ull * n, hipMemcpyHostToDevice, st));
+                pool.swap(np);
+                pool_size = nsize;
+                S.pool = pool.p;
+                S.pool_size = pool_size;
+                const u64 top = no[n];
+                PADO_HIP(copy_sync(&ctr.p->pool_top, &top, 8, hipMemcpyHostToDevice, st));
+            }
+            commit(b, h->n_touched);
+            PADO_HIP(hipStreamSynchronize(st));
+            next = b + 1;  // the ones behind it did nothing
+        }
+        const WClosed done{ring[b % kWRing].rounds, 0u, ring[b % kWRing].n_touched};
+        hist[b % kRoundHistory] = (uint32_t)(done.rounds - rounds_seen);
+        rounds_seen = done.rounds;
+        touched = done.n_touched;
     }
     hipLaunchKernelGGL(k_w_fold_stats, dim3(1), dim3(1024), 0, st, ctr.p);
     PADO_HIP(hipMemcpyAsync(h, ctr.p, sizeof(WCounters), hipMemcpyDeviceToHost, st));
