@@ -91,6 +91,12 @@ __device__ inline uint32_t lane_id() { return threadIdx.x & 63; }
 
 __device__ inline u64 *stat_rows(WCounters *C) { return reinterpret_cast<u64 *>(C + 1); }
 
+__device__ inline u64 readlane64(u64 x, uint32_t lane)
+{
+    return ((u64)__builtin_amdgcn_readlane((uint32_t)(x >> 32), lane) << 32) |
+           __builtin_amdgcn_readlane((uint32_t)x, lane);
+}
+
 __device__ inline uint32_t wave_max(uint32_t x)
 {
     x = max(x, dpp0<0x111, 0xF>(x));
@@ -127,32 +133,8 @@ __device__ inline uint32_t prefix_above(const uint64_t *off, const uint32_t *adj
     return a + (uint32_t)__popcll(__ballot(p));
 }
 
-__device__ inline u64 store_reserve(WStore S, WCounters *C, uint32_t v, uint32_t len, uint32_t add)
-{
-    const uint32_t lane = lane_id();
-    u64 base = S.base[v];
-    uint32_t cap = S.cap[v];
-    if (len + add <= cap) return base;
-    uint32_t ncap = cap * 2;
-    if (ncap < len + add) ncap = len + add;
-    if (ncap < 8) ncap = 8;
-    u64 nb = 0;
-    if (lane == 0) nb = atomicAdd(&C->pool_top, (u64)ncap);
-    nb = __shfl(nb, 0);
-    if (nb + ncap > S.pool_size) {
-        if (lane == 0) atomicOr(&C->overflow, 1u);
-        return ~0ull;
-    }
-    for (uint32_t j = lane; j < len; j += 64) S.pool[nb + j] = S.pool[base + j];
-    if (lane == 0) {
-        S.base[v] = nb;
-        S.cap[v] = ncap;
-    }
-    return nb;
-}
-
 // Pool words a commit of up to `add` new labels may reserve for a list of
-// length len and capacity cap (store_reserve's doubling rule).
+// length len and capacity cap (lists double).
 __device__ inline u64 reserve_words(uint32_t len, uint32_t cap, uint32_t add)
 {
     if (len + add <= cap) return 0;
@@ -325,6 +307,8 @@ constexpr uint32_t kWDense = 16, kWPushEdges = 4;
 
 // Touched vertices up to which k_w_filter reads the roots' entries in place.
 constexpr uint32_t kWDirectFilter = 4096;
+
+constexpr uint32_t kWWitness = 2;  // witnesses k_w_filter takes at a time (1 and 4 measure the same)
 
 // Batches in flight, from the kWAheadFrom-th on (weighted R-MAT 20: 2: 575
 // ms, 1: 585, 3: 584, 4: 585, 7: 599 -- a batch that is held costs the empty
@@ -757,7 +741,9 @@ __global__ __launch_bounds__(256) void k_w_roots_t(uint32_t rs, uint32_t rsz, co
 
 // filter_out_labels (WPARA:1100-1228): one wave per touched vertex; surviving
 // pairs (finite, not pruned) are dropped if an earlier batch root h witnesses
-// S(v,h) + S(r,h) <= S(v,r).  Reads T/P only, so every wave sees the same
+// S(v,h) + S(r,h) <= S(v,r).  The witnesses go through LDS, and a lane reads
+// of a witness's row only while it has a pair left that it could drop (650 K
+// vertices, 128 roots: 15.1 -> 9.8 ms).  Reads T/P only, so every wave sees the same
 // pre-filter state; the kept bitmap goes to I and the pool words the commit
 // may reserve are summed into C->need.  kDirect: the roots' entries come from
 // T/P rows directly (8 scattered reads per witness and lane, no transpose
@@ -779,7 +765,7 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
             return;
         }
     }
-    __shared__ uint8_t sv[4][64];
+    __shared__ uint2 s_wit[4][kWB];
     const uint32_t lane = lane_id();
     const uint32_t wib = threadIdx.x >> 6;
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
@@ -800,49 +786,62 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
             dv[q] = T[(uint64_t)v * kWB + lane * 8 + q];
             if (dv[q] != kWInf && !((pb >> q) & 1u)) surv |= 1u << q;
         }
-        sv[wib][lane] = (uint8_t)surv;
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        uint32_t drop = 0;
-        for (uint32_t w = 0; w < kWW; ++w) {
-            u64 word = 0;
+        // The vertex's surviving pairs, roots ascending: the witnesses.
+        const uint32_t cnt = __popc(surv);
+        const uint32_t incl = wave_incl_scan(cnt);
+        const uint32_t nwit = __builtin_amdgcn_readlane(incl, 63);
+        {
+            uint32_t at = incl - cnt;
 #pragma unroll
-            for (int bb = 0; bb < 8; ++bb) word |= (u64)sv[wib][w * 8 + bb] << (8 * bb);
-            while (word) {
-                const uint32_t h = w * 64 + __ffsll(word) - 1;  // witness root offset
-                word &= word - 1;
-                if (h >= lane * 8 + 7) break;  // only roots r > h of this lane can use h
-                const uint32_t dvh = T[(uint64_t)v * kWB + h];
-                // Column h of the roots' entries, 8 consecutive roots per lane.
-                uint32_t drh[8];
-                uint32_t prh = 0;
+            for (int q = 0; q < 8; ++q)
+                if ((surv >> q) & 1u) s_wit[wib][at++] = make_uint2(lane * 8 + q, dv[q]);
+        }
+        w_lds_sync();
+        uint32_t drop = 0;
+        for (uint32_t w = 0; w < nwit; w += kWWitness) {
+            // Column h of the roots' entries for four witnesses h, 8 consecutive
+            // roots per lane; only lanes that hold a root ranked below h and not
+            // yet dropped read.
+            uint32_t h[kWWitness], dvh[kWWitness], todo[kWWitness], drh[kWWitness][8], prh[kWWitness];
+#pragma unroll
+            for (uint32_t u = 0; u < kWWitness; ++u) {
+                const uint2 x = s_wit[wib][min(w + u, nwit - 1)];
+                h[u] = x.x;
+                dvh[u] = x.y;
+                const uint32_t below = lane * 8 > h[u] ? 0xFFu : lane * 8 + 7 <= h[u] ? 0u : 0xFFu & (0xFEu << (h[u] - lane * 8));
+                todo[u] = surv & ~drop & below;
+                prh[u] = 0;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) drh[u][q] = kWInf;
+                if (!todo[u]) continue;
                 if constexpr (kDirect) {
 #pragma unroll
                     for (int q = 0; q < 8; ++q) {
                         const uint32_t ro = lane * 8 + q;
-                        drh[q] = kWInf;
-                        if (((surv >> q) & 1u) && ro > h && ro < rsz) {
-                            drh[q] = T[(uint64_t)(rs + ro) * kWB + h];
-                            prh |= (uint32_t)((P[(uint64_t)(rs + ro) * kWW + h / 64] >> (h % 64)) & 1ull) << q;
+                        if ((todo[u] >> q) & 1u) {
+                            drh[u][q] = T[(uint64_t)(rs + ro) * kWB + h[u]];
+                            prh[u] |= (uint32_t)((P[(uint64_t)(rs + ro) * kWW + h[u] / 64] >> (h[u] % 64)) & 1ull) << q;
                         }
                     }
                 } else {
-                    const uint4 *rt = reinterpret_cast<const uint4 *>(RT + (uint64_t)h * kWB + lane * 8);
+                    const uint4 *rt = reinterpret_cast<const uint4 *>(RT + (uint64_t)h[u] * kWB + lane * 8);
                     const uint4 ra = rt[0], rb = rt[1];
-                    drh[0] = ra.x, drh[1] = ra.y, drh[2] = ra.z, drh[3] = ra.w;
-                    drh[4] = rb.x, drh[5] = rb.y, drh[6] = rb.z, drh[7] = rb.w;
-                    prh = reinterpret_cast<const uint8_t *>(PT + (uint64_t)h * kWW)[lane];
-                }
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const uint32_t ro = lane * 8 + q;
-                    if (!((surv >> q) & 1u) || ro <= h) continue;
-                    if (drh[q] == kWInf || ((prh >> q) & 1u)) continue;
-                    if ((uint64_t)dvh + drh[q] <= dv[q]) drop |= 1u << q;
+                    drh[u][0] = ra.x, drh[u][1] = ra.y, drh[u][2] = ra.z, drh[u][3] = ra.w;
+                    drh[u][4] = rb.x, drh[u][5] = rb.y, drh[u][6] = rb.z, drh[u][7] = rb.w;
+                    prh[u] = reinterpret_cast<const uint8_t *>(PT + (uint64_t)h[u] * kWW)[lane];
                 }
             }
+#pragma unroll
+            for (uint32_t u = 0; u < kWWitness; ++u) {
+                uint32_t by = 0;
+#pragma unroll
+                for (int q = 0; q < 8; ++q)
+                    by |= drh[u][q] != kWInf && (uint64_t)dvh[u] + drh[u][q] <= dv[q] ? 1u << q : 0u;
+                drop |= by & todo[u] & ~prh[u];
+            }
         }
-        __builtin_amdgcn_wave_barrier();
+        // (the next vertex's list must not overtake these reads)
+        w_lds_sync();
         const uint32_t keep = surv & ~drop;
         n_filt += __popc(drop);
         // The improved bitmap is all zero once the rounds end; it carries the
@@ -865,13 +864,14 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
     }
 }
 
-// update_index (WPARA:961-990): append the kept pairs of each touched vertex,
-// hubs ascending (batches are committed in root order and each lane's roots
-// follow the lower lanes'), then clear the carried bitmap.
 // update_index (WPARA:961-990) and reset_tables (WPARA:918-956) in one pass
-// over the touched vertices: each vertex's wave appends its kept pairs and
-// then empties its T / P rows; the batch roots (touched-list entries
-// 0..rsz-1) first clear the root-distance entries their labels wrote.
+// over the touched vertices: a wave appends a vertex's kept pairs, hubs
+// ascending (batches are committed in root order and each lane's roots follow
+// the lower lanes'), clears the carried bitmap and empties its T / P rows; the
+// batch roots (touched-list entries 0..rsz-1) first clear the root-distance
+// entries their labels wrote.  Waves take up to 64 vertices at a time and the
+// pool words for them with one atomic: one per vertex, all on one word, was
+// most of a large batch's commit (650 K vertices: 7.7 ms, now 0.9).
 __global__ __launch_bounds__(256) void k_w_commit(uint32_t rs, uint32_t rsz, const uint32_t *tlist, uint32_t *T, u64 *P,
                                                   u64 *I, uint32_t *hmin, uint32_t *dcw, WStore S, WCounters *C)
 {
@@ -880,40 +880,73 @@ __global__ __launch_bounds__(256) void k_w_commit(uint32_t rs, uint32_t rsz, con
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const uint32_t nwaves = (gridDim.x * blockDim.x) >> 6;
     const uint32_t nt = C->n_touched;
-    for (uint32_t i = wave; i < nt; i += nwaves) {
-        const uint32_t v = tlist[i];
-        if (i < rsz) {
-            // root offset i: its labels are those k_w_init entered
-            const uint32_t len = S.len[v];
-            const u64 base = S.base[v];
-            for (uint32_t j = lane; j < len; j += 64) {
-                const uint32_t h = (uint32_t)(S.pool[base + j] >> 32);
-                dcw[(uint64_t)h * kWB + i] = kWInf;
-                hmin[h] = kWInf;
+    const uint32_t group = min(64u, max(1u, nt / nwaves));
+    for (uint32_t i0 = wave * group; i0 < nt; i0 += nwaves * group) {
+        const uint32_t m = min(group, nt - i0);
+        // Lane i: the group's i-th vertex, its list and the words it moves to.
+        uint32_t v = 0, total = 0, len = 0, need = 0;
+        u64 base = 0;
+        if (lane < m) {
+            v = tlist[i0 + lane];
+            const ulonglong2 *kept = reinterpret_cast<const ulonglong2 *>(I + (uint64_t)v * kWW);
+#pragma unroll
+            for (uint32_t x = 0; x < kWW / 2; ++x) total += (uint32_t)(__popcll(kept[x].x) + __popcll(kept[x].y));
+            len = S.len[v];
+            base = S.base[v];
+            if (total) need = (uint32_t)reserve_words(len, S.cap[v], total);
+        }
+        const uint32_t incl = wave_incl_scan(need);
+        const uint32_t words = __builtin_amdgcn_readlane(incl, 63);
+        u64 nb = 0;
+        if (words) {
+            if (lane == 0) nb = atomicAdd(&C->pool_top, (u64)words);
+            nb = uniform64(nb);
+        }
+        const bool fits = words == 0 || nb + words <= S.pool_size;
+        if (!fits && lane == 0) atomicOr(&C->overflow, 1u);
+        const u64 to = need ? nb + (incl - need) : base;
+        if (lane < m && total && fits) {
+            S.len[v] = len + total;
+            if (need) {
+                S.base[v] = to;
+                S.cap[v] = need;
             }
         }
-        uint8_t *Kb = reinterpret_cast<uint8_t *>(I + (uint64_t)v * kWW);
-        const uint32_t keep = Kb[lane];
-        const uint32_t cnt = __popc(keep);
-        const uint32_t incl = wave_incl_scan(cnt);
-        const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-        if (total) {
-            if (keep) Kb[lane] = 0;
-            const uint32_t len = S.len[v];
-            const u64 nb = store_reserve(S, C, v, len, total);
-            if (nb != ~0ull) {
-                uint32_t pos = len + incl - cnt;
-                for (uint32_t kb = keep; kb; kb &= kb - 1) {
-                    const uint32_t q = __ffs(kb) - 1;
-                    S.pool[nb + pos++] = ((u64)(rs + lane * 8 + q) << 32) | T[(uint64_t)v * kWB + lane * 8 + q];
+        for (uint32_t s = 0; s < m; ++s) {
+            const uint32_t vs = __builtin_amdgcn_readlane(v, s), ls = __builtin_amdgcn_readlane(len, s);
+            const u64 from = readlane64(base, s);
+            if (i0 + s < rsz) {
+                // root offset i0 + s: its labels are those k_w_init entered
+                for (uint32_t j = lane; j < ls; j += 64) {
+                    const uint32_t h = (uint32_t)(S.pool[from + j] >> 32);
+                    dcw[(uint64_t)h * kWB + i0 + s] = kWInf;
+                    hmin[h] = kWInf;
                 }
-                if (lane == 0) S.len[v] = len + total;
             }
+            uint4 *row = reinterpret_cast<uint4 *>(T + (uint64_t)vs * kWB + lane * 8);
+            if (__builtin_amdgcn_readlane(total, s)) {
+                uint8_t *Kb = reinterpret_cast<uint8_t *>(I + (uint64_t)vs * kWW);
+                const uint32_t keep = Kb[lane];
+                uint4 r0 = make_uint4(0, 0, 0, 0), r1 = r0;
+                if (keep) {
+                    r0 = row[0];
+                    r1 = row[1];
+                    Kb[lane] = 0;
+                }
+                const u64 dst = readlane64(to, s);
+                if (__builtin_amdgcn_readlane(need, s) && fits)
+                    for (uint32_t j = lane; j < ls; j += 64) S.pool[dst + j] = S.pool[from + j];
+                const uint32_t cnt = __popc(keep);
+                u64 at = dst + ls + wave_incl_scan(cnt) - cnt;
+                const uint32_t d[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+                for (uint32_t q = 0; q < 8; ++q)
+                    if (fits && ((keep >> q) & 1u)) S.pool[at++] = ((u64)(rs + lane * 8 + q) << 32) | d[q];
+            }
+            // The row goes back to INF.
+            row[0] = row[1] = make_uint4(kWInf, kWInf, kWInf, kWInf);
+            if (lane < kWW) P[(uint64_t)vs * kWW + lane] = 0ull;
         }
-        // This lane's 8 entries were read above; the row goes back to INF.
-        uint4 *row = reinterpret_cast<uint4 *>(T + (uint64_t)v * kWB + lane * 8);
-        row[0] = row[1] = make_uint4(kWInf, kWInf, kWInf, kWInf);
-        if (lane < kWW) P[(uint64_t)v * kWW + lane] = 0ull;
     }
 }
 
