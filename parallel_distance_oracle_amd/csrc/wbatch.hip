@@ -489,6 +489,10 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
 // distance_query's first loop (WPARA:569-580) for every improved pair of an
 // improved tail: one wave per tail, lane l owns roots 8l..8l+7.  Pruned pairs
 // stop propagating; the others become the tail's next frontier bitmap.
+// Bound by instruction issue where a batch is large (4.1 G of them, 6.7 of
+// 9.8 ms, in the largest round of weighted R-MAT 20; the hubs' rows come from
+// L2): the sums through the hubs are kept as a saturated minimum per pair, two
+// instructions per hub where comparing each took seven (build 550 -> 504 ms).
 __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, const uint32_t *ilist, const uint64_t *off,
                                                  const uint32_t *adj, uint32_t *T, u64 *I, u64 *P, WStore S,
                                                  const uint32_t *hmin, const uint32_t *dcw,
@@ -511,12 +515,20 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
         const uint32_t imp = Ib[lane];
         // Clear after every lane has read (the store depends on the ballot).
         if (__ballot(imp != 0) != 0ull) Ib[lane] = 0;
-        uint32_t dv[8];
         uint32_t maxd = 0;
+        uint4 t0 = make_uint4(0, 0, 0, 0), t1 = t0;
+        if (imp) {
+            const uint4 *row = reinterpret_cast<const uint4 *>(T + (uint64_t)t * kWB + lane * 8);
+            t0 = row[0];
+            t1 = row[1];
+        }
+        // Tentative distances of the improved pairs, 0 for the others: a sum
+        // through an earlier hub is at least 2.
+        uint32_t dv[8] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w};
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            dv[q] = (imp >> q) & 1u ? T[(uint64_t)t * kWB + lane * 8 + q] : 0u;
-            if (((imp >> q) & 1u) && dv[q] > maxd) maxd = dv[q];
+            dv[q] = (imp >> q) & 1u ? dv[q] : 0u;
+            maxd = max(maxd, dv[q]);
         }
         const uint32_t wmax = wave_max(maxd);
         uint32_t prune = 0;
@@ -530,6 +542,9 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
         uint32_t j_gather = 0;
         if (wave_total(__popc(imp)) > kWGather) {
             j_gather = len;
+            uint32_t best[8];  // the least sums through the hubs so far
+#pragma unroll
+            for (int q = 0; q < 8; ++q) best[q] = kWInf;
             for (uint32_t j0 = 0; j0 < len; j0 += 64) {
                 const uint32_t j = j0 + lane;
                 uint32_t h = 0, d = kWInf;
@@ -539,41 +554,39 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
                     d = (uint32_t)lab;
                 }
                 // hmin is INF for hubs no batch root holds
-                const bool pass = j < len && (uint64_t)d + hmin[h] <= wmax;
+                const bool pass = j < len && __builtin_elementwise_add_sat(d, hmin[h]) <= wmax;
                 u64 m = __ballot(pass);
                 // Up to four passing hubs per step: their row loads go out
                 // together (32 B per lane each), and only lanes that still hold an
                 // unpruned improved pair load.
                 bool few = false;
                 while (m) {
-                    int src[4];
-                    bool ok[4];
+                    // (past the last one: that one again)
+                    uint32_t src[4];
 #pragma unroll
                     for (int u = 0; u < 4; ++u) {
-                        ok[u] = m != 0ull;
-                        src[u] = ok[u] ? __ffsll(m) - 1 : 0;
-                        if (ok[u]) m &= m - 1;
+                        src[u] = m ? (uint32_t)__ffsll(m) - 1 : src[u ? u - 1 : 0];
+                        m &= m - 1;
                     }
-                    const bool need = (imp & ~prune) != 0u;
-                    uint32_t dd[4];
-                    uint4 r0[4], r1[4];
+                    if (imp & ~prune) {
+                        uint4 r0[4], r1[4];
+                        uint32_t dd[4];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        dd[u] = __shfl(d, src[u]);
-                        const uint32_t sl = __shfl(h, src[u]);
-                        r0[u] = r1[u] = make_uint4(kWInf, kWInf, kWInf, kWInf);
-                        if (ok[u] && need) {
-                            const uint4 *row = reinterpret_cast<const uint4 *>(dcw + (uint64_t)sl * kWB + lane * 8);
-                            r0[u] = row[0];
-                            r1[u] = row[1];
+                        for (int u = 0; u < 4; ++u) {
+                            dd[u] = __builtin_amdgcn_readlane(d, src[u]);
+                            const uint32_t *hub = dcw + (uint64_t)__builtin_amdgcn_readlane(h, src[u]) * kWB;
+                            r0[u] = reinterpret_cast<const uint4 *>(hub)[lane * 2];
+                            r1[u] = reinterpret_cast<const uint4 *>(hub)[lane * 2 + 1];
                         }
-                    }
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        const uint32_t x[8] = {r0[u].x, r0[u].y, r0[u].z, r0[u].w, r1[u].x, r1[u].y, r1[u].z, r1[u].w};
+                        for (int u = 0; u < 4; ++u) {
+                            const uint32_t x[8] = {r0[u].x, r0[u].y, r0[u].z, r0[u].w, r1[u].x, r1[u].y, r1[u].z, r1[u].w};
 #pragma unroll
-                        for (int q = 0; q < 8; ++q)
-                            if (((imp >> q) & 1u) && x[q] != kWInf && (uint64_t)dd[u] + x[q] <= dv[q]) prune |= 1u << q;
+                            for (int q = 0; q < 8; ++q)
+                                best[q] = min(best[q], __builtin_elementwise_add_sat(x[q], dd[u]));
+                        }
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) prune |= best[q] <= dv[q] ? 1u << q : 0u;
                     }
                     if (wave_total(__popc(imp & ~prune)) <= kWGather) {
                         few = true;
@@ -622,15 +635,17 @@ __global__ __launch_bounds__(256) void k_w_check(uint32_t round, uint32_t rs, co
         if (ncand_t && j_gather < len) {
             auto gather_pass = [&](uint32_t d, uint32_t h, uint32_t hm) {
                 uint32_t x[kWGather];
+                const uint32_t least = __builtin_elementwise_add_sat(d, hm);
+                const uint32_t *row = dcw + (uint64_t)h * kWB;
 #pragma unroll
                 for (uint32_t k = 0; k < kWGather; ++k) {
                     x[k] = kWInf;
-                    if (k < ncand_t && !((cpr >> k) & 1u) && (uint64_t)d + hm <= cdv[k])
-                        x[k] = dcw[(uint64_t)h * kWB + croot[k]];
+                    if (k < ncand_t && !((cpr >> k) & 1u) && least <= cdv[k]) x[k] = row[croot[k]];
                 }
+                // (a tentative distance is below INF)
 #pragma unroll
                 for (uint32_t k = 0; k < kWGather; ++k)
-                    if (__ballot(x[k] != kWInf && (uint64_t)d + x[k] <= cdv[k]) != 0ull) cpr |= 1u << k;
+                    if (__ballot(__builtin_elementwise_add_sat(d, x[k]) <= cdv[k]) != 0ull) cpr |= 1u << k;
             };
             const u64 gb = base + j_gather;
             const uint32_t glen = len - j_gather;
@@ -833,10 +848,10 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
             }
 #pragma unroll
             for (uint32_t u = 0; u < kWWitness; ++u) {
-                uint32_t by = 0;
+                uint32_t by = 0;  // (a surviving pair's distance is below INF)
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
-                    by |= drh[u][q] != kWInf && (uint64_t)dvh[u] + drh[u][q] <= dv[q] ? 1u << q : 0u;
+                    by |= __builtin_elementwise_add_sat(drh[u][q], dvh[u]) <= dv[q] ? 1u << q : 0u;
                 drop |= by & todo[u] & ~prh[u];
             }
         }
