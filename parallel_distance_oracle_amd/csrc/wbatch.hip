@@ -1071,11 +1071,12 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     for (hipEvent_t &e : ev) PADO_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 
     WStore S{pool.p, base.p, len.p, cap.p, pool_size};
-    // The first batch takes a quarter of the roots: nothing prunes its
-    // searches, and its labels prune the next batch's (measured on weighted
-    // R-MAT 20 / 22: 1.04 -> 0.95 s / 6.5 -> 6.3 s).  Any split of the rank
-    // order into batches yields the same label set.
-    const uint32_t first = std::min(n, std::max<uint32_t>(1u, batch / 4));
+    // The first batch takes an eighth of the roots (one word of them, of 512):
+    // nothing prunes its searches, and its labels prune the next batch's.
+    // Any split of the rank order into batches yields the same label set.
+    // Weighted R-MAT 20: a quarter 503 ms, an eighth 491, a sixteenth 499, a
+    // 32nd 503; growing by doubling from either 498 to 511.
+    const uint32_t first = std::min(n, std::max<uint32_t>(1u, batch / 8));
     const uint32_t nb = 1 + (n - first + batch - 1) / batch;
     auto roots_start = [&](uint32_t b) { return b ? first + (b - 1) * batch : 0u; };
     auto roots_size = [&](uint32_t b) { return b >= nb ? 0u : std::min(b ? batch : first, n - roots_start(b)); };
