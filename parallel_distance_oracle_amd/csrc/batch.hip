@@ -465,37 +465,63 @@ __global__ void k_hub_info_init(HubInfo *p, uint64_t count)
     }
 }
 
-// Reserve room for `add` more labels of v (wave-uniform call).  Returns the
-// (possibly new) base; on pool exhaustion sets the overflow flag and returns
-// ~0ull.
-__device__ inline unsigned long long store_reserve_at(LabelStore S, BuildCounters *C, uint32_t v, uint32_t len,
-                                                      unsigned long long base, uint32_t cap, uint32_t add)
+// Pool words that a list of len labels and capacity cap takes for `add` more:
+// 0 if they fit.
+__device__ inline uint32_t store_words(uint32_t len, uint32_t cap, uint32_t add)
+{
+    if (len + add <= cap) return 0u;
+    const uint32_t ncap = max(cap * 4, len + add);  // few moves
+    return max(ncap, 32u);
+}
+
+// Moves v's list to `words` words at nb (wave-uniform call).  Past the pool's
+// end the overflow flag is set and nothing moves: false.
+__device__ inline bool store_move(LabelStore S, BuildCounters *C, uint32_t v, uint32_t len, unsigned long long base,
+                                  unsigned long long nb, uint32_t words)
 {
     const uint32_t lane = lane_id();
-    if (len + add <= cap) return base;
-    uint32_t ncap = cap * 4;  // few reallocations: each is an atomic on one shared counter
-    if (ncap < len + add) ncap = len + add;
-    if (ncap < 32) ncap = 32;
-    unsigned long long nb = 0;
-    if (lane == 0) nb = atomicAdd(&C->pool_top, (unsigned long long)ncap);
-    nb = __shfl(nb, 0);
-    if (nb + ncap > S.pool_size) {
+    if (nb + words > S.pool_size) {
         if (lane == 0) atomicOr(&C->overflow, 1u);
-        return ~0ull;
+        return false;
     }
     for (uint32_t j = lane; j < len; j += 64) S.pool[nb + j] = S.pool[base + j];
     if (lane == 0) {
         S.rec[v].base = nb;
-        S.rec[v].cap = ncap;
+        S.rec[v].cap = words;
     }
-    return nb;
+    return true;
 }
 
+// Pool words a wave has taken and not used yet.
+struct PoolGrab {
+    unsigned long long next = 0;
+    uint32_t left = 0;
+};
+
+// Room for `add` more labels of v (wave-uniform call): the possibly new base,
+// or ~0ull where the pool is exhausted.  Words come off the shared counter for
+// up to kPoolGrab at a time, as far as the wave's `rem` lists (this one
+// included) are likely to need them: an atomic per list, all on one word and
+// waited for, were 13 of the 44 ms of k_add in a build of R-MAT 20 (143 -> 132
+// ms).
+constexpr uint32_t kPoolGrab = 1024;
 __device__ inline unsigned long long store_reserve(LabelStore S, BuildCounters *C, uint32_t v, uint32_t len,
-                                                   uint32_t add)
+                                                   unsigned long long base, uint32_t cap, uint32_t add, PoolGrab &g,
+                                                   uint32_t rem)
 {
-    const LRec r = S.rec[v];
-    return store_reserve_at(S, C, v, len, r.base, r.cap, add);
+    const uint32_t words = store_words(len, cap, add);
+    if (words == 0) return base;
+    if (words > g.left) {
+        const uint32_t grab = max(words, (uint32_t)min((unsigned long long)words * rem, (unsigned long long)kPoolGrab));
+        unsigned long long nb = 0;
+        if (lane_id() == 0) nb = atomicAdd(&C->pool_top, (unsigned long long)grab);
+        g.next = uniform64(nb);
+        g.left = grab;
+    }
+    const unsigned long long nb = g.next;
+    g.next += words;
+    g.left -= words;
+    return store_move(S, C, v, len, base, nb, words) ? nb : ~0ull;
 }
 
 __global__ void k_fill_u32(uint32_t *p, uint64_t count, uint32_t val)
@@ -650,7 +676,8 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     uint32_t pdeg = 0;
     if (live) {
         const uint32_t len = rec0.len;
-        const unsigned long long base = store_reserve_at(S, C, r, len, rec0.base, rec0.cap, 1);
+        PoolGrab grab;
+        const unsigned long long base = store_reserve(S, C, r, len, rec0.base, rec0.cap, 1, grab, 1);
         if (base != ~0ull) {
             if (lane == 0) {
                 // the root-distance entry of the self label
@@ -1293,6 +1320,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
     // vertex; unused descriptor slots are padded.  The active count and the
     // frontier's push edges are added once per wave at the end.
     uint32_t c_next = 0, c_left = 0, my_act = 0, my_subs = 0;
+    PoolGrab grab;
     uint32_t my_pedge = 0;  // push edges of this wave's new frontier entries (flushed below 2^31)
     unsigned long long *nbits = abits + (uint64_t)(p ^ 1u) * C->abits_words;
     // The loop over this wave's candidates (grid-stride: i, i + nwaves, ...)
@@ -1571,7 +1599,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
         if (total == 0) continue;
         n_lab += total;
-        const unsigned long long nb = store_reserve_at(S, C, v, len, base, cap, total);
+        const unsigned long long nb = store_reserve(S, C, v, len, base, cap, total, grab, (ncand - 1 - i) / nwaves + 1);
         if (nb == ~0ull) continue;
         uint32_t pos = len + incl - cnt;
         for (Bits sb = surv; sb; sb &= sb - 1) {
