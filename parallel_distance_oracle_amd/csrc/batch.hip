@@ -957,6 +957,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
     __shared__ uint32_t s_cu[PW][64];              // a lane's running counts over its four words
     __shared__ uint32_t s_t[PW][64];               // each lane's tail
     __shared__ uint32_t s_w[PW][64];               // a lane's words of the step, one per byte
+    __shared__ uint32_t s_tl[PW][64], s_cl[PW][64];  // touched vertices and candidates on their way to the lists
     // set-phase scratch (bp_set_phase)
     __shared__ unsigned long long s_srem[PW][64], s_sone[PW][64];
     __shared__ uint32_t s_sro[PW][64], s_st[PW][64], s_sex[PW][64], s_shit[PW][64];
@@ -1013,6 +1014,7 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
             pull_step<W>(wave, nwaves, iter, p, rs, n, gen_iter, gen_batch, off, adj, abits + (uint64_t)p * nw, ag, ind,
                      cand, vmark, tlist, clist, bpd, lmask, rmask, bps, rset, C, bp_prune, s_nb[wv][0], s_keep[wv][0],
                      s_ex[wv], s_t[wv], sc, n_push, n_pass, n_bp, n_cand, n_edge, n_tail);
+    uint32_t held_t = 0, held_c = 0;
     for (uint32_t c0 = wave * DPS; !pull && c0 < nc; c0 += nwaves * DPS) {
         const uint32_t c = c0 + lane / CH;
         const unsigned long long desc = c < nc ? chunks[c] : kChunkPad;
@@ -1173,13 +1175,13 @@ __device__ __forceinline__ void push_body(uint32_t bid, uint32_t nblk, uint32_t 
                 new_c = got && prev < want;
             }
         }
-        const uint32_t ti = wave_append(&C->n_touched, new_t);
-        if (new_t) tlist[ti] = t;
-        const uint32_t ci = wave_append(&C->n_cand[p], new_c);
-        if (new_c) clist[ci] = t;
+        list_append(&C->n_touched, tlist, s_tl[wv], held_t, new_t, t);
+        list_append(&C->n_cand[p], clist, s_cl[wv], held_c, new_c, t);
         // s_t is rewritten by the next step.
         wave_lds_sync();
     }
+    list_flush(&C->n_touched, tlist, s_tl[wv], held_t);
+    list_flush(&C->n_cand[p], clist, s_cl[wv], held_c);
     if (__ballot(n_edge != 0u) != 0ull)
         add_stats<0>(stat_rows(C), wave, {n_edge, n_tail, n_push, n_pass, n_bp, n_cand});
 }

@@ -343,6 +343,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
 {
     __shared__ u64 s_g[kWPushWaves][64], s_imp[kWPushWaves][64];
     __shared__ uint32_t s_ex[kWPushWaves][64], s_u[kWPushWaves][64], s_t[kWPushWaves][64], s_w[kWPushWaves][64];
+    __shared__ uint32_t s_tl[kWPushWaves][64], s_il[kWPushWaves][64];  // entries on their way to the lists
     const uint32_t lane = lane_id(), wv = threadIdx.x >> 6;
     const uint32_t wave = blockIdx.x * kWPushWaves + wv;
     const uint32_t nwaves = gridDim.x * kWPushWaves;
@@ -358,6 +359,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         C->a_top[p ^ 1u] = 0;
         C->n_chunk[p ^ 1u] = 0;
     }
+    uint32_t held_t = 0, held_i = 0;
     uint32_t n_relax = 0, n_imp = 0, n_bound = 0;  // (a list's reservation fits 32 bits, and a lane's few do)
     for (uint32_t c0 = wave * 4; c0 < nc; c0 += nwaves * 4) {
         const uint32_t c = c0 + (lane >> 4);
@@ -466,19 +468,15 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         }
         const bool new_t = got && tmark[t] != gen_batch && atomicExch(&tmark[t], gen_batch) != gen_batch;
         const bool new_i = got && imark[t] != gen_round && atomicExch(&imark[t], gen_round) != gen_round;
-        const uint32_t ti = wave_append(&C->n_touched, new_t);
-        if (new_t) {
-            tlist[ti] = t;
-            n_bound += (uint32_t)reserve_words(S.len[t], S.cap[t], rsz);
-        }
-        const uint32_t ii = wave_append(&C->n_imp[p], new_i);
-        if (new_i) {
-            ilist[ii] = t;
-            ++n_imp;
-        }
+        list_append(&C->n_touched, tlist, s_tl[wv], held_t, new_t, t);
+        if (new_t) n_bound += (uint32_t)reserve_words(S.len[t], S.cap[t], rsz);
+        list_append(&C->n_imp[p], ilist, s_il[wv], held_i, new_i, t);
+        n_imp += new_i ? 1u : 0u;
         // s_u / s_t / s_w are rewritten by the next step.
         w_lds_sync();
     }
+    list_flush(&C->n_touched, tlist, s_tl[wv], held_t);
+    list_flush(&C->n_imp[p], ilist, s_il[wv], held_i);
     if (wave * 4 < nc) {
         const u64 t_bound = wave_total(n_bound & 0xFFFFu) + ((u64)wave_total(n_bound >> 16) << 16);
         if (lane == 0 && t_bound) atomicAdd(&C->need_bound, t_bound);
