@@ -20,11 +20,13 @@
 // schedule (the reference's own OpenMP order is arbitrary too).
 //
 // GPU layout (HBM):
-//   ind[n][16] u64   indicator bitmap, 1024 roots per vertex row (rows of the
-//                    vertices touched in a batch are cleared at its end)
-//   cand[n][16] u64  candidate bitmap of the current iteration
-//   ag[A][16] u64    last distance group of each active vertex, as a bitmap
-//   chunks[]         16-edge push work descriptors (active index, edge start)
+//   ind[n][RW] u64   indicator bitmap, a row of 64 RW roots per vertex (RW = 16,
+//                    or 64 where four batches of 1,024 run at once; rows of
+//                    the vertices touched in a batch are cleared at its end)
+//   cand[n][RW] u64  candidate bitmap of the current iteration
+//   ag[n][RW] u64    last distance group of each active vertex, as a bitmap
+//   chunks[]         push work descriptors (active vertex, edge start), eight
+//                    edges each
 //   pool[] u32       label store: per-vertex growable arrays of packed
 //                    (hub << 8 | dist) labels, grown fourfold (at least 32)
 //                    on overflow by a bump allocator (one wave owns one
@@ -36,11 +38,11 @@
 //                    vertex, raised by atomicMax); rmask / rset: the batch
 //                    roots' mask words and set pairs, word- / slot-major
 //   hinfo[n] 32 B    per hub: lane masks of the batch roots at distance 1, 2,
-//                    3 (bit l: roots [16l, 16l+16)) and 0xFFFFFF00 | min
+//                    3 (bit l: roots [RW l, RW l + RW)) and 0xFFFFFF00 | min
 //                    distance from any batch root
-//   dc[h][1024] u8   root-distance table: dc[h][r - rs] = dist(root r, hub h),
+//   dc[h][64 RW] u8  root-distance table: dc[h][r - rs] = dist(root r, hub h),
 //                    the transposed form of dist_matrix, rows by hub id
-// Kernels per iteration: k_push (edge-parallel, one edge per lane, 16-edge
+// Kernels per iteration: k_push (edge-parallel, one edge per lane, eight-edge
 // chunks) and k_add (wave per candidate vertex: distance query + label
 // append + next active entry).  The host enqueues blocks of iterations and
 // checks the frontier count once per block, running one batch ahead behind a
