@@ -131,7 +131,7 @@ __device__ inline u32x4 load4(const uint32_t *p, uint32_t j, uint32_t len)
     return v;
 }
 
-// The entries of load4 past the list as all-ones, which no hub is.  Apart from
+// The entries of load4 past the list as all-ones, which no label is.  Apart from
 // the load, so that a pair's loads are all in flight before the first is
 // waited for.
 __device__ inline u32x4 mask4(u32x4 v, uint32_t j, uint32_t len)
@@ -404,17 +404,18 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t r0, uint32_t njobs,
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     // x - key is the other distance if the hubs are equal,
-                    // else at least MASK + 1: a u8 answer it does not lower,
-                    // and neither do two entries past their lists (all-ones).
-                    const uint32_t u = tile_at(tile, pos[q]) - key[q];
-                    const uint32_t sum = __builtin_elementwise_add_sat(u, s[q] & MASK);
-                    d = min(d, W && u > MASK ? UNREACHED : sum);
+                    // else at least MASK + 1.  An entry past its list
+                    // (all-ones) has the last hub there can be, but distance
+                    // MASK, which no label of that hub has.  A u8 answer
+                    // starts at MASK, so neither lowers it.
+                    const uint32_t u = tile_at(tile, pos[q]) - key[q], e = s[q] & MASK;
+                    const uint32_t sum = __builtin_elementwise_add_sat(u, e);
+                    d = min(d, W && max(u, e) >= MASK ? UNREACHED : sum);
                 }
             }
             // The next copy must not overtake these reads.
             q_lds_sync();
         }
-        if (W && d >= 2 * MASK) d = UNREACHED;
         d = group_min<L>(d);
         if (first) {
             if (sa.x & sb.x)
