@@ -132,6 +132,22 @@ void pado_gpu_ctx_destroy(pado_gpu_ctx *ctx);
 void *pado_gpu_ctx_stream(pado_gpu_ctx *ctx);
 /* Wait for all work queued on the context's stream. */
 pado_gpu_status pado_gpu_ctx_sync(pado_gpu_ctx *ctx);
+
+/* Temporary device memory of a context's builds, ingest and ordering (no
+ * reference counterpart).  It stays with the context from one call for the
+ * next: idle blocks of at most 256 MiB, or of a sixteenth of the device's
+ * memory while a graph of the context lives, and of no more than that
+ * sixteenth over all contexts of the device.  They go back to the driver when
+ * the context is destroyed, when one of this library's own allocations fails,
+ * and with pado_gpu_ctx_trim, for programs whose other allocators need the
+ * memory. */
+pado_gpu_status pado_gpu_ctx_trim(pado_gpu_ctx *ctx);
+/* At most `bytes` of such memory in use at once (0 = any): a call that needs
+ * more ends with PADO_GPU_ERR_NOMEM.  Graphs and indexes do not count. */
+pado_gpu_status pado_gpu_ctx_set_work_limit(pado_gpu_ctx *ctx, uint64_t bytes);
+/* Bytes of it in use now, most in use since the last trim, and idle (each
+ * nullable). */
+pado_gpu_status pado_gpu_ctx_work_sizes(pado_gpu_ctx *ctx, uint64_t *in_use, uint64_t *peak, uint64_t *idle);
 /* Device-to-device copy of `bytes` bytes with a plain copy kernel on the
  * context's stream (16-byte aligned buffers; no reference counterpart: it is
  * the known-size kernel the HBM byte counters are calibrated with). */

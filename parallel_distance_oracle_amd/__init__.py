@@ -129,6 +129,10 @@ def lib():
         "pado_gpu_ctx_destroy": (None, [_vp]),
         "pado_gpu_ctx_stream": (_vp, [_vp]),
         "pado_gpu_ctx_sync": (ctypes.c_int, [_vp]),
+        "pado_gpu_ctx_trim": (ctypes.c_int, [_vp]),
+        "pado_gpu_ctx_set_work_limit": (ctypes.c_int, [_vp, _u64]),
+        "pado_gpu_ctx_work_sizes": (ctypes.c_int, [_vp, ctypes.POINTER(_u64), ctypes.POINTER(_u64),
+                                                   ctypes.POINTER(_u64)]),
         "pado_gpu_copy_bytes": (ctypes.c_int, [_vp, _vp, _vp, _u64]),
         "pado_gpu_graph_upload": (ctypes.c_int, [_vp, _u32, _u64, _vp, _vp, _vp, ctypes.POINTER(_vp)]),
         "pado_gpu_graph_free": (None, [_vp]),
@@ -445,6 +449,22 @@ class Context:
 
     def sync(self):
         _check(lib().pado_gpu_ctx_sync(self.h))
+
+    def trim(self):
+        """Gives idle temporary device memory back to the driver (for other
+        allocators of the program, torch's for instance)."""
+        _check(lib().pado_gpu_ctx_trim(self.h))
+
+    def set_work_limit(self, nbytes):
+        """At most nbytes of temporary device memory in use at once (0: any)."""
+        _check(lib().pado_gpu_ctx_set_work_limit(self.h, nbytes))
+
+    def work_sizes(self):
+        """Temporary device memory in bytes: in use, most in use since the last
+        trim, idle."""
+        x = _u64(), _u64(), _u64()
+        _check(lib().pado_gpu_ctx_work_sizes(self.h, *(ctypes.byref(v) for v in x)))
+        return tuple(v.value for v in x)
 
     def close(self):
         if self.h:

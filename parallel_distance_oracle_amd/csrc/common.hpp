@@ -112,11 +112,13 @@ constexpr uint32_t kListAlign = 32;  // label list alignment: one 128-byte line
 // stream only, so a block given back while that stream still works on it is
 // safe with the next taker.  What lies idle in it is bounded: a sixteenth of
 // the card while a graph of the context lives (it may be built again), else
-// kIdleWork; all of it goes back when the context is destroyed and whenever an
-// allocation fails.  Safe with several threads.
+// kIdleWork, and a sixteenth of the card for all contexts of a device
+// together.  All of it goes back when the context is destroyed, when its user
+// asks for it (pado_gpu_ctx_trim) and whenever an allocation fails.  Safe with
+// several threads.
 class WorkPool {
 public:
-    explicit WorkPool(size_t card_bytes);
+    WorkPool(int device, size_t card_bytes);
     ~WorkPool();
     // A block of at least `bytes` bytes (its size in *got), or null.
     void *take(size_t bytes, size_t *got);
@@ -126,7 +128,13 @@ public:
     void give_pinned(void *p);
     void hold(int graphs);  // graphs of the context that live, more or fewer
     void collect(size_t keep, std::vector<void *> *out);  // takes out idle blocks, oldest first
+    void trim();                                          // gives all idle blocks back
     void close();                                         // the context is gone
+    void set_limit(size_t bytes);                         // most bytes in use at once (0: any)
+    struct Sizes {
+        size_t in_use, peak, idle;  // peak: of in_use, since the last trim
+    };
+    Sizes sizes();
     static constexpr size_t kPinned = 131072;
 
 private:
@@ -137,10 +145,11 @@ private:
     std::mutex mu_;
     std::vector<Block> idle_;  // in the order they were given back
     std::vector<void *> pinned_;
-    size_t idle_bytes_ = 0, card_bytes_ = 0;
-    int graphs_ = 0;
+    size_t idle_bytes_ = 0, in_use_ = 0, peak_ = 0, max_use_ = 0, card_bytes_ = 0;
+    int device_ = 0, graphs_ = 0;
     bool closed_ = false;
-    size_t limit() const;
+    size_t shared_limit() const;  // idle bytes of all the device's pools
+    size_t limit() const;         // of this one
 };
 
 // hipMalloc under capture_mutex; where it fails, what the process's pools hold

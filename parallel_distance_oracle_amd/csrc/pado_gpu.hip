@@ -84,7 +84,7 @@ hipError_t device_alloc(void **p, size_t bytes)
     return e;
 }
 
-WorkPool::WorkPool(size_t card_bytes) : card_bytes_(card_bytes)
+WorkPool::WorkPool(int device, size_t card_bytes) : card_bytes_(card_bytes), device_(device)
 {
     std::lock_guard<std::mutex> g(pools().mu);
     pools().v.push_back(this);
@@ -100,9 +100,29 @@ WorkPool::~WorkPool()
     close();
 }
 
-size_t WorkPool::limit() const
+size_t WorkPool::shared_limit() const { return std::max(card_bytes_ / 16, kIdleWork); }
+
+size_t WorkPool::limit() const { return closed_ ? 0 : graphs_ > 0 ? shared_limit() : kIdleWork; }
+
+void WorkPool::trim()
 {
-    return closed_ ? 0 : graphs_ > 0 ? std::max(card_bytes_ / 16, kIdleWork) : kIdleWork;
+    std::vector<void *> out;
+    collect(0, &out);
+    free_blocks(out);
+    std::lock_guard<std::mutex> g(mu_);
+    peak_ = in_use_;
+}
+
+void WorkPool::set_limit(size_t bytes)
+{
+    std::lock_guard<std::mutex> g(mu_);
+    max_use_ = bytes;
+}
+
+WorkPool::Sizes WorkPool::sizes()
+{
+    std::lock_guard<std::mutex> g(mu_);
+    return {in_use_, peak_, idle_bytes_};
 }
 
 void WorkPool::close()
@@ -122,6 +142,7 @@ void WorkPool::close()
 void *WorkPool::take(size_t bytes, size_t *got)
 {
     bytes = block_size(bytes);
+    void *p = nullptr;
     {
         std::lock_guard<std::mutex> g(mu_);
         size_t best = idle_.size();
@@ -129,18 +150,21 @@ void *WorkPool::take(size_t bytes, size_t *got)
             if (idle_[i].bytes >= bytes && idle_[i].bytes <= bytes + bytes / 4 &&
                 (best == idle_.size() || idle_[i].bytes < idle_[best].bytes))
                 best = i;
+        const size_t size = best < idle_.size() ? idle_[best].bytes : bytes;
+        if (max_use_ && in_use_ + size > max_use_) return nullptr;
         if (best < idle_.size()) {
-            const Block b = idle_[best];
+            p = idle_[best].p;
             idle_.erase(idle_.begin() + (ptrdiff_t)best);
-            idle_bytes_ -= b.bytes;
-            *got = b.bytes;
-            return b.p;
+            idle_bytes_ -= size;
         }
+        in_use_ += size;
+        peak_ = std::max(peak_, in_use_);
+        *got = size;
     }
-    void *p = nullptr;
-    if (device_alloc(&p, bytes) != hipSuccess) return nullptr;
-    *got = bytes;
-    return p;
+    if (p || device_alloc(&p, bytes) == hipSuccess) return p;
+    std::lock_guard<std::mutex> g(mu_);
+    in_use_ -= bytes;
+    return nullptr;
 }
 
 void WorkPool::give(void *p, size_t bytes)
@@ -151,9 +175,18 @@ void WorkPool::give(void *p, size_t bytes)
         std::lock_guard<std::mutex> g(mu_);
         idle_.push_back({p, bytes});
         idle_bytes_ += bytes;
+        in_use_ -= bytes;
         keep = limit();
     }
-    collect(keep, &out);
+    {
+        // What the device's other pools hold idle leaves this one the less.
+        std::lock_guard<std::mutex> g(pools().mu);
+        size_t others = 0;
+        for (WorkPool *w : pools().v)
+            if (w != this && w->device_ == device_) others += w->sizes().idle;
+        const size_t all = shared_limit();
+        collect(std::min(keep, all - std::min(others, all)), &out);
+    }
     free_blocks(out);
 }
 
@@ -456,7 +489,7 @@ pado_gpu_status pado_gpu_ctx_create(int device, pado_gpu_ctx **out)
         c->num_cu = prop.multiProcessorCount;
         card = prop.totalGlobalMem;
     }
-    c->work = std::make_shared<WorkPool>(card);
+    c->work = std::make_shared<WorkPool>(device, card);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreateWithFlags(&c->side_ev, hipEventDisableTiming) != hipSuccess) {
@@ -488,6 +521,33 @@ pado_gpu_status pado_gpu_ctx_sync(pado_gpu_ctx *ctx)
     clear_error();
     PADO_TRY(check_ctx(ctx));
     PADO_HIP(hipStreamSynchronize(ctx->stream));
+    return PADO_GPU_OK;
+}
+
+pado_gpu_status pado_gpu_ctx_trim(pado_gpu_ctx *ctx)
+{
+    clear_error();
+    PADO_TRY(check_ctx(ctx));
+    ctx->work->trim();
+    return PADO_GPU_OK;
+}
+
+pado_gpu_status pado_gpu_ctx_set_work_limit(pado_gpu_ctx *ctx, uint64_t bytes)
+{
+    clear_error();
+    PADO_TRY(check_ctx(ctx));
+    ctx->work->set_limit(bytes);
+    return PADO_GPU_OK;
+}
+
+pado_gpu_status pado_gpu_ctx_work_sizes(pado_gpu_ctx *ctx, uint64_t *in_use, uint64_t *peak, uint64_t *idle)
+{
+    clear_error();
+    PADO_TRY(check_ctx(ctx));
+    const WorkPool::Sizes z = ctx->work->sizes();
+    if (in_use) *in_use = z.in_use;
+    if (peak) *peak = z.peak;
+    if (idle) *idle = z.idle;
     return PADO_GPU_OK;
 }
 
