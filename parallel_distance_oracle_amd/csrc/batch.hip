@@ -2535,7 +2535,7 @@ pado_gpu_status build_batches(pado_gpu_graph *g, pado_gpu_index *idx, const DevB
     // A pool that still runs dry inside a block (growth far above the recent
     // rate) costs one rerun of the batch phase from scratch with a larger
     // pool; no label is ever dropped.
-    unsigned long long exhausted = 0, pool_min = 0;
+    unsigned long long pool_min = 0;
     if ((cfg.flags & PADO_GPU_BUILD_DEVICE_LOOP) && !(cfg.flags & PADO_GPU_BUILD_STREAM)) {
         // One workgroup runs the whole batch phase; a pool that runs dry
         // there falls back to the launch schedule, which grows its pool.
@@ -2552,19 +2552,28 @@ pado_gpu_status build_batches(pado_gpu_graph *g, pado_gpu_index *idx, const DevB
     // one by one (any batch size gives the same labels, and `iterations` counts
     // the same either way): a batch costs its prologue and two launches per
     // iteration however little is in it.  Above kWideRowVertices the wider rows
-    // would take too much memory (5.6 KB more per vertex).
+    // would take too much memory (5.6 KB more per vertex); where they do not
+    // fit below it, the batches run one by one.
     const bool four = g->n > kBatch && g->n <= kWideRowVertices && (cfg.batch_size == 0 || cfg.batch_size == kBatch) &&
                       (cfg.flags & PADO_GPU_BUILD_STREAM) == 0 && (cfg.push_chunk == 0 || cfg.push_chunk == kPushChunk) &&
                       (cfg.push_waves == 0 || cfg.push_waves == kPushWaves) && cfg.pull_ratio == 0;
-    for (int attempt = 0;; ++attempt) {
-        exhausted = 0;
-        const auto build = idx->wide ? (four ? build_batches_t<true, kWideRow> : build_batches_t<true, kRow>)
-                                     : (four ? build_batches_t<false, kWideRow> : build_batches_t<false, kRow>);
-        const pado_gpu_status s = build(g, idx, d_used, cfg, pool_min, &exhausted);
-        if (s != PADO_GPU_ERR_NOMEM || !exhausted || attempt == 2) return s;
-        pool_min = exhausted * 4;
+    const auto run = [&](auto build) {
+        unsigned long long pool = pool_min, exhausted = 0;
+        for (int attempt = 0;; ++attempt) {
+            exhausted = 0;
+            const pado_gpu_status s = build(g, idx, d_used, cfg, pool, &exhausted);
+            if (s != PADO_GPU_ERR_NOMEM || !exhausted || attempt == 2) return s;
+            pool = exhausted * 4;
+            (void)hipStreamSynchronize(g->ctx->stream);
+        }
+    };
+    if (four) {
+        const pado_gpu_status s = run(idx->wide ? build_batches_t<true, kWideRow> : build_batches_t<false, kWideRow>);
+        if (s != PADO_GPU_ERR_NOMEM) return s;
         (void)hipStreamSynchronize(g->ctx->stream);
+        clear_error();
     }
+    return run(idx->wide ? build_batches_t<true, kRow> : build_batches_t<false, kRow>);
 }
 
 }  // namespace pado
