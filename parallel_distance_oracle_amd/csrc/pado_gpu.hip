@@ -279,7 +279,8 @@ __device__ inline uint32_t component(unsigned long long reached, const uint32_t 
 
 // One wave per vertex: its record, sets and padded label list.  slots: which
 // bit-parallel distances tell components (0 in a wide index whose BFS was cut
-// short); known: whether components are to be told at all.
+// short); known: whether components are to be told at all; qbps null: the sets
+// stay where they are.
 template <bool WEIGHTED>
 __global__ __launch_bounds__(256) void k_order_copy(uint32_t n, const uint32_t *rank, const uint8_t *bpd,
                                                     const ulonglong2 *bps, const uint64_t *loff, const uint32_t *lab,
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(256) void k_order_copy(uint32_t n, const uint32_t *
             unsigned long long f = 0;
             if (lane < kBP) {
                 const ulonglong2 set = bps[(uint64_t)v * kBP + lane];
-                qbps[(uint64_t)x * kBP + lane] = set;
+                if (qbps) qbps[(uint64_t)x * kBP + lane] = set;
                 f = set.x | (set.x >> 32);
                 f |= f >> 16;
                 f |= f >> 8;
@@ -357,8 +358,9 @@ pado_gpu_status check_ctx(pado_gpu_ctx *ctx)
     return PADO_GPU_OK;
 }
 
-// Builds the original-id query copy from the rank-space index (h_rank null:
-// the index is in original-id order already).
+// Builds the original-id query copy from the rank-space index.  h_rank null:
+// the index is in original-id order already, and its sets, most of its memory,
+// become the query copy's.
 pado_gpu_status order_index(pado_gpu_index *idx, const uint32_t *h_rank)
 {
     hipStream_t st = idx->ctx->stream;
@@ -398,11 +400,12 @@ pado_gpu_status order_index(pado_gpu_index *idx, const uint32_t *h_rank)
                            idx->qwdist.p);
     } else {
         PADO_TRY(idx->qrec.alloc((uint64_t)n * kQRecWords));
-        PADO_TRY(idx->qbps.alloc((uint64_t)n * kBP * 2));
+        if (h_rank) PADO_TRY(idx->qbps.alloc((uint64_t)n * kBP * 2));
         hipLaunchKernelGGL(k_order_copy<false>, grid, block, 0, st, n, rank.p, idx->bpd.p,
                            (const ulonglong2 *)idx->bps.p, idx->loff.p, idx->lab.p, nullptr, qoff.p, idx->built,
                            idx->bp_pass_through ? 0ull : ~0ull, idx->wide ? Hop<true>::kBits : Hop<false>::kBits,
                            idx->qrec.p, (ulonglong2 *)idx->qbps.p, idx->qlab.p, nullptr);
+        if (!h_rank) idx->qbps.swap(idx->bps);
     }
     PADO_HIP(hipGetLastError());
     PADO_HIP(hipStreamSynchronize(st));
@@ -1344,8 +1347,10 @@ pado_gpu_status pado_gpu_windex_load(pado_gpu_ctx *ctx, const char *filename, pa
         set_error("bad index file header");
         return PADO_GPU_ERR_IO;
     }
-    std::vector<uint64_t> off((uint64_t)n + 1, 0);
-    std::vector<uint32_t> hub, dist;
+    // As for the unweighted file, the query copy only: laid out as
+    // k_order_copy does, here, so that the labels are on the device once.
+    std::vector<uint32_t> rec((uint64_t)n * kWRecWords, 0), hub, dist;
+    uint64_t total = 0;
     for (uint32_t x = 0; x < n; ++x) {
         uint32_t sz = 0;
         f.read((char *)&sz, 4);
@@ -1353,6 +1358,9 @@ pado_gpu_status pado_gpu_windex_load(pado_gpu_ctx *ctx, const char *filename, pa
             set_error("truncated index file");
             return PADO_GPU_ERR_IO;
         }
+        const uint64_t packed = ((uint64_t)hub.size() << 24) | sz;
+        rec[(uint64_t)x * kWRecWords + 2] = (uint32_t)packed;
+        rec[(uint64_t)x * kWRecWords + 3] = (uint32_t)(packed >> 32);
         for (uint32_t i = 0; i < sz; ++i) {
             uint32_t h = 0;
             int16_t d = 0;
@@ -1365,7 +1373,11 @@ pado_gpu_status pado_gpu_windex_load(pado_gpu_ctx *ctx, const char *filename, pa
             hub.push_back(h);
             dist.push_back((uint32_t)d);
         }
-        off[x + 1] = hub.size();
+        total += sz;
+        while (hub.size() % kListAlign) {
+            hub.push_back(~0u);
+            dist.push_back(~0u);
+        }
     }
     if (!f.good()) {
         set_error("truncated index file");
@@ -1375,33 +1387,25 @@ pado_gpu_status pado_gpu_windex_load(pado_gpu_ctx *ctx, const char *filename, pa
     idx->ctx = ctx;
     idx->n = n;
     idx->weighted = 1;
-    idx->num_labels = hub.size();
+    idx->num_labels = total;
     const uint64_t L = hub.size();
     hipStream_t st = ctx->stream;
-    pado_gpu_status s = idx->loff.alloc((uint64_t)n + 1);
-    if (s == PADO_GPU_OK) s = idx->whub.alloc(L);
-    if (s == PADO_GPU_OK) s = idx->wdist.alloc(L);
+    pado_gpu_status s = idx->qrec.alloc(rec.size());
+    if (s == PADO_GPU_OK) s = idx->qlab.alloc(L);
+    if (s == PADO_GPU_OK) s = idx->qwdist.alloc(L);
     if (s != PADO_GPU_OK) {
         delete idx;
         return s;
     }
-    if (hipMemcpyAsync(idx->loff.p, off.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st) != hipSuccess ||
-        (L && hipMemcpyAsync(idx->whub.p, hub.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
-        (L && hipMemcpyAsync(idx->wdist.p, dist.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
+    if (hipMemcpyAsync(idx->qrec.p, rec.data(), 4ull * rec.size(), hipMemcpyHostToDevice, st) != hipSuccess ||
+        (L && hipMemcpyAsync(idx->qlab.p, hub.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
+        (L && hipMemcpyAsync(idx->qwdist.p, dist.data(), 4ull * L, hipMemcpyHostToDevice, st) != hipSuccess) ||
         hipStreamSynchronize(st) != hipSuccess) {
         delete idx;
         set_error("index upload failed");
         return PADO_GPU_ERR_HIP;
     }
-    // As for the unweighted file: the query copy only.
-    s = order_index(idx, nullptr);
-    if (s != PADO_GPU_OK) {
-        delete idx;
-        return s;
-    }
-    idx->loff.release();
-    idx->whub.release();
-    idx->wdist.release();
+    idx->ordered = 1;
     *out = idx;
     return PADO_GPU_OK;
 }
