@@ -390,6 +390,7 @@ pado_gpu_status order_index(pado_gpu_index *idx, const uint32_t *h_rank)
     PADO_TRY(scan_u32_to_u64(cnt.p, qoff.p, n, st, wp));
     uint64_t total = 0;
     PADO_HIP(copy_sync(&total, qoff.p + n, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+    idx->ordered = 0;  // (an earlier copy goes from here on)
     PADO_TRY(idx->qlab.alloc(total));
     const dim3 grid(grid_for((uint64_t)n * 64, 256, 8192)), block(256);
     if (idx->weighted) {
@@ -872,6 +873,10 @@ pado_gpu_status pado_gpu_index_order(pado_gpu_ctx *ctx, pado_gpu_index *idx, con
         set_error("rank must have num_v entries");
         return PADO_GPU_ERR_ARG;
     }
+    if (!idx->loff.p) {
+        set_error("index has no rank-space labels (loaded from an ordered file)");
+        return PADO_GPU_ERR_STATE;
+    }
     return order_index(idx, rank);
 }
 
@@ -1111,6 +1116,10 @@ pado_gpu_status pado_gpu_windex_export(pado_gpu_ctx *ctx, const pado_gpu_index *
         set_error("unweighted index: use pado_gpu_index_export");
         return PADO_GPU_ERR_STATE;
     }
+    if (!idx->loff.p) {
+        set_error("index has no rank-space labels (loaded from an ordered file)");
+        return PADO_GPU_ERR_STATE;
+    }
     hipStream_t st = ctx->stream;
     const uint64_t L = idx->num_labels;
     if (label_off)
@@ -1137,6 +1146,10 @@ pado_gpu_status pado_gpu_wquery(pado_gpu_ctx *ctx, pado_gpu_index *idx, const ui
     const bool rank_space = (flags & PADO_GPU_QUERY_RANK_SPACE) != 0;
     if (!rank_space && !idx->ordered) {
         set_error("query before order_labels: call pado_gpu_index_order or pass PADO_GPU_QUERY_RANK_SPACE");
+        return PADO_GPU_ERR_STATE;
+    }
+    if (rank_space && !idx->loff.p) {
+        set_error("index has no rank-space labels");
         return PADO_GPU_ERR_STATE;
     }
     if (k == 0) return PADO_GPU_OK;
