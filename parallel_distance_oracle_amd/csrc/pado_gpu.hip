@@ -1371,6 +1371,10 @@ pado_gpu_status pado_gpu_windex_load(pado_gpu_ctx *ctx, const char *filename, pa
             set_error("truncated index file");
             return PADO_GPU_ERR_IO;
         }
+        if (sz >= kMaxVertices) {  // (a record has 24 bits for it)
+            set_error("a label list longer than the vertices there can be");
+            return PADO_GPU_ERR_IO;
+        }
         const uint64_t packed = ((uint64_t)hub.size() << 24) | sz;
         rec[(uint64_t)x * kWRecWords + 2] = (uint32_t)packed;
         rec[(uint64_t)x * kWRecWords + 3] = (uint32_t)(packed >> 32);

@@ -1,6 +1,6 @@
 """A loaded index has the query copy only: calls that need rank-space labels
 are refused with a status (no kernel is launched), queries by original id are
-answered."""
+answered; files with lists that no record can hold are refused."""
 import ctypes
 import struct
 
@@ -12,7 +12,7 @@ import parallel_distance_oracle_amd as pado
 pytestmark = pytest.mark.gpu
 
 N = 4
-STATE = 5
+STATE, IO = 5, 6
 
 
 def _load(ctx, fn, path):
@@ -85,3 +85,20 @@ def test_ordering_that_fails_early_leaves_the_copy():
     idx.close()
     dg.close()
     ctx.close()
+
+
+def test_list_longer_than_a_record_holds(gpu_ctx, tmp_path):
+    """2^24 labels at one vertex (duplicate hubs, or they would not exist): the
+    record's 24-bit count would read as none, and move the list's start."""
+    path = tmp_path / "long"
+    with open(path, "wb") as f:
+        f.write(struct.pack("<II", 1, 1 << 24))
+        f.write(bytes(6 << 24))
+    assert _load(gpu_ctx, pado.lib().pado_gpu_windex_load, path)[0] == IO
+    with open(path, "wb") as f:
+        f.write(struct.pack("<II", 1, 1000) + bytes(6000))  # (duplicates alone are taken, as ever)
+    st, h = _load(gpu_ctx, pado.lib().pado_gpu_windex_load, path)
+    assert st == 0
+    idx = pado.Index(gpu_ctx, h)
+    assert idx.query([0], [0])[0] == 0
+    idx.close()
