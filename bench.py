@@ -21,7 +21,7 @@ build seconds over the K timed steps (lower is better).  The line also carries:
                 checks and the same serving measurement,
   multi      -- 1,024 graphs labeled as one job,
   roofline   -- the dominant build kernel's algorithmic bytes per launch over
-                its HIP-event launch time,
+                its HIP-event launch time, in a build of batches one by one,
   cpu_baseline -- the reference OpenMP build (oracle/_ref) on a bounded sample
                 (R-MAT 18, median of 3, physical cores) and its query_distance
                 single-threaded and OpenMP, with the GPU time for the same
@@ -418,6 +418,49 @@ def load_traffic():
         return json.load(f)
 
 
+ROOFLINE_SCHEDULE = "batches of 1,024 roots one by one"  # of a stream-mode build
+
+
+def build_roofline(st, timing, traffic, workload):
+    """The dominant labeling kernel's algorithmic bytes per launch over its
+    launch time.  st: the stats of ONE build, whose launches were timed; what
+    they scanned depends on the schedule, so times and counts of different
+    builds do not go together.  traffic: load_traffic()."""
+    push_bytes = 8 * st["actives"] + 4 * st["edges"] + BP_RECORD_BYTES * st["tails"]
+    add_bytes = 5 * st["dq_labels"] + 5 * st["labels_appended"]
+    kern = {
+        "k_push": (st["ms_push"], st["n_push"], push_bytes),
+        "k_add": (st["ms_add"], st["n_add"], add_bytes),
+    }
+    dom = max(kern, key=lambda k: kern[k][0])
+    ms_tot, n_launch, bytes_tot = kern[dom]
+    avg_ms = ms_tot / max(n_launch, 1)
+    achieved = (bytes_tot / max(n_launch, 1)) / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
+    roofline = {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
+                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": None,
+                "avg_launch_us": round(avg_ms * 1e3, 2), "launches": int(n_launch),
+                "alg_bytes_per_launch": round(bytes_tot / max(n_launch, 1), 1),
+                "kernel_ms": {k: round(v[0], 2) for k, v in kern.items()}, "schedule": ROOFLINE_SCHEDULE,
+                "timing": timing}
+    if traffic and traffic.get("workload") == workload and dom in traffic.get("kernels", {}):
+        roofline["traffic"] = traffic["kernels"][dom]["bytes_per_launch"]
+        roofline["traffic_source"] = traffic.get("source")
+    return roofline
+
+
+QUERY_RECORD_BYTES = 128  # a vertex's line of the query copy
+QUERY_TAIL_BYTES = 16     # its last four words: component, label list
+
+
+def query_bytes(connected, la, lb):
+    """Bytes that a batch of pairs cannot do without: ids and answers, the tail
+    of each end's record and, for a connected pair, the two records and label
+    lists (la, lb labels).  The set pairs that decide a slot come on top."""
+    connected = np.asarray(connected, bool)
+    own = 2 * QUERY_RECORD_BYTES + 4 * (np.asarray(la, np.int64) + np.asarray(lb, np.int64))
+    return int(np.where(connected, own, 2 * QUERY_TAIL_BYTES).sum()) + 9 * connected.size
+
+
 def main():
     global SERVE_MODE
     ap = argparse.ArgumentParser()
@@ -524,11 +567,12 @@ def main():
         parity["reference_build_s_container"] = meta.get("ref_build_s")
     del bp_d, bp_s, hub, dist
 
-    # Roofline of the dominant labeling kernel (push or add), per launch.  The
-    # stream-mode build brackets each push / add launch with HIP events on the
-    # build stream; a default build records none, so then one extra
-    # stream-mode build of the same graph (a batch at a time) times them.
+    # Roofline of the dominant labeling kernel (push or add), per launch, from
+    # one build of its own: a stream-mode build (a batch at a time) brackets
+    # each push / add launch with HIP events on the build stream, which a
+    # default build does not, and what it scans is what those launches did.
     timing_src = "timed builds (HIP events on the build stream)"
+    st_t = st
     if not args.stream:
         tcfg = pado.BuildCfg()
         tcfg.batch_size = pado.BATCH_SIZE
@@ -537,33 +581,11 @@ def main():
         ctx.sync()
         st_t = tb.stats()
         tb.close()
-        for k in ("ms_push", "ms_add", "n_push", "n_add"):
-            st[k] = st_t[k]
         timing_src = "one stream-mode build after the timed builds (HIP events on the build stream)"
-    push_bytes = 8 * st["actives"] + 4 * st["edges"] + BP_RECORD_BYTES * st["tails"]
-    add_bytes = 5 * st["dq_labels"] + 5 * st["labels_appended"]
-    kern = {
-        "k_push": (st["ms_push"], st["n_push"], push_bytes),
-        "k_add": (st["ms_add"], st["n_add"], add_bytes),
-    }
-    dom = max(kern, key=lambda k: kern[k][0])
-    ms_tot, n_launch, bytes_tot = kern[dom]
-    avg_ms = ms_tot / max(n_launch, 1)
-    achieved = (bytes_tot / max(n_launch, 1)) / (avg_ms * 1e-3) / 1e9 if avg_ms > 0 else 0.0
-    roofline = {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5), "traffic": None,
-                "avg_launch_us": round(avg_ms * 1e3, 2), "launches": int(n_launch),
-                "alg_bytes_per_launch": round(bytes_tot / max(n_launch, 1), 1),
-                "kernel_ms": {k: round(v[0], 2) for k, v in kern.items()}, "timing": timing_src}
-    tr = load_traffic()
-    wl = f"rmat{args.scale}_ef{args.edge_factor}"
-    if tr and tr.get("workload") == wl and dom in tr.get("kernels", {}):
-        t = tr["kernels"][dom]
-        roofline["traffic"] = t["bytes_per_launch"]
-        roofline["traffic_source"] = tr.get("source")
+    roofline = build_roofline(st_t, timing_src, load_traffic(), f"rmat{args.scale}_ef{args.edge_factor}")
     if args.build_only:
         print(json.dumps({"metric": "R-MAT build only (profiling run)", "value": round(build_s, 4), "unit": "s",
-                          "roofline": roofline, "parity": parity, "stats": st}), flush=True)
+                          "roofline": roofline, "parity": parity, "stats": st, "roofline_stats": st_t}), flush=True)
         return
 
     # Plain batch query: order by original id, k pairs on device, one launch.
@@ -601,8 +623,7 @@ def main():
                                                       digest(ref_mode) == meta["answers_sha256"])
     query["exact_vs_ref_compat_differ"] = int(np.count_nonzero(ref_mode != res[:k]))
     lab_per_v = np.diff(loff.astype(np.int64))
-    qbytes = 8 + 1 + 2 * BP_RECORD_BYTES + 5 * (lab_per_v[rank[qa]] + lab_per_v[rank[qb]])
-    query["alg_bytes"] = int(qbytes.sum())
+    query["alg_bytes"] = query_bytes(res != 255, lab_per_v[rank[qa]], lab_per_v[rank[qb]])
     query["achieved_GBps"] = round(query["alg_bytes"] / (q_ms * 1e-3) / 1e9, 1)
     # The drop-in's query_distance(a, b) loop (pado.cpp:114-119 calls it once
     # per pair): one-pair calls (pado_gpu_query_pair), and the same pairs as
