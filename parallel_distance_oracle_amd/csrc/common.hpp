@@ -451,6 +451,7 @@ struct pado_gpu_index {
     uint32_t wide = 0;  // labels in the wide hop domain (Hop<true>)
     uint32_t bp_pass_through = 0;  // wide build whose bit-parallel BFS was cut at level 254:
                                    // its bit-parallel vertices were labeled as ordinary hubs
+    uint64_t holds = 0, grows = 0;  // weighted build: batches held for the host, label pools grown
     // Bit-parallel labels, rank space: bpd[v*64 + i], bps[(v*50 + i)*2 + {0,1}];
     // the rest of a bpd line holds the nonempty-set bits (kBpNzByte).
     pado::DevBuf<uint8_t> bpd;

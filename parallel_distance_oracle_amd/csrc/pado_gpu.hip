@@ -727,6 +727,18 @@ pado_gpu_status pado_gpu_index_get_info(const pado_gpu_index *idx, pado_gpu_inde
     return PADO_GPU_OK;
 }
 
+pado_gpu_status pado_gpu_windex_holds(const pado_gpu_index *idx, uint64_t *holds, uint64_t *grows)
+{
+    clear_error();
+    if (!idx || !idx->weighted) {
+        set_error("bad argument (a weighted index is required)");
+        return PADO_GPU_ERR_ARG;
+    }
+    if (holds) *holds = idx->holds;
+    if (grows) *grows = idx->grows;
+    return PADO_GPU_OK;
+}
+
 }  // extern "C"
 
 namespace {

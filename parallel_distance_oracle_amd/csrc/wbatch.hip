@@ -1120,7 +1120,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
     // have ended, or whose labels might not fit the pool, holds everything
     // behind it (k_w_filter); the host then ends it step by step and goes on
     // from there.  Weighted R-MAT 20: 597 -> 576 ms; 200 K vertices: 80 -> 75.
-        constexpr uint32_t kRoundHistory = 3;
+    constexpr uint32_t kRoundHistory = 3;
     uint32_t hist[kRoundHistory] = {}, launched[kWRing] = {};
     hist[0] = 6;
     uint32_t next = 0, touched = n;  // batches enqueued; vertices the last batch touched
@@ -1153,6 +1153,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
         PADO_HIP(hipEventSynchronize(ev[b % kWRing]));
         PADO_HIP(hipGetLastError());
         if (ring[b % kWRing].held) {
+            idx->holds += 1;
             hipLaunchKernelGGL(k_w_unhold, dim3(1), dim3(1), 0, st, ctr.p);
             uint32_t done = launched[b % kWRing], more = 1;
             for (;;) {
@@ -1174,6 +1175,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
                 grow = h->pool_top + h->need > pool_size;
             }
             if (grow) {
+                idx->grows += 1;
                 // Compact every list into a larger pool.  After compaction a list of
                 // length L has capacity L + L/4 + 4, so the commit can reserve at
                 // most 2.5 * live + new + 8 * touched words.
