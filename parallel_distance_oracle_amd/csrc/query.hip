@@ -61,7 +61,7 @@ constexpr int kQOcc = 5;
 // takes the pair instead: it needs one or two, and the wave's other groups
 // would have waited for the longest (10 M pairs on R-MAT 20: 1,970 us at 3,
 // 2,060 at 2, 2,035 at 4, 2,610 without; weighted R-MAT 18: 364 us at 4, 378
-// at 3, 341 without: see kWMixedPairs).
+// at 3, 341 without: see kWMixedPairs and kLongMean).
 constexpr uint32_t kLongSteps = 3, kWLongSteps = 4;
 constexpr uint32_t kNoSlot = 0x7FFFu;         // sum of a slot that does not count
 
@@ -556,7 +556,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
 // once the counter passes k.
 constexpr uint32_t kGrab = 16;
 
-template <int K, class OT>
+template <int K, int M, class OT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) void k_query_ws(QIndex X, const uint32_t *qa,
                                                   const uint32_t *qb, uint64_t k, OT *out, int ref_compat,
                                                   unsigned long long *work)
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
         if (c0 >= k) break;
         const bool has = lane < kGrab && c0 + lane < k;
         const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
-        const uint32_t d = answer_pairs<K, true, K == kWeights ? kGrouped : kMixed>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
+        const uint32_t d = answer_pairs<K, true, M>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
         if (has) out[c0 + lane] = (OT)d;
         q_lds_sync();
     }
@@ -584,8 +584,8 @@ __global__ void k_zero_work(unsigned long long *work) { *work = 0ull; }
 uint32_t query_ws_blocks_per_cu(bool weighted)
 {
     int nb = 0;
-    const hipError_t e = weighted ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws<kWeights, uint32_t>, 256, 0)
-                                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws<kHops, uint8_t>, 256, 0);
+    const hipError_t e = weighted ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws<kWeights, kMixed, uint32_t>, 256, 0)
+                                  : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_query_ws<kHops, kMixed, uint8_t>, 256, 0);
     return (e == hipSuccess && nb > 0) ? (uint32_t)nb : 4u;
 }
 
@@ -847,43 +847,57 @@ pado_gpu_status launch_query_pair(const pado_gpu_index *idx, bool rank_space, ui
 
 namespace {
 
-// Up to here a whole wave takes each pair: the waves are on the chip together,
-// and a call takes as long as its longest lists, which the wave goes through
-// in fewer steps.  4,000 pairs, 900 K vertex R-MAT: 6.2 us, 22.2 in groups;
-// 200 K vertices weighted: 4.7 and 9.9; short lists 4.6 to 5.3 either way.
-// 8,000 pairs with short lists: 6.4 us, 4.5 in groups.
-constexpr uint64_t kAlonePairs = 4096;
+// How a call's pairs are shared out goes by the pairs and by the index's mean
+// list length: R-MAT graphs have 2 to 80 labels a vertex (weighted 20 to 220),
+// grids 30 to 170, sparse random graphs of 20 K to 200 K vertices 300 to 2,800.
+//
+// Up to so many pairs a whole wave takes each: the waves are on the chip
+// together, and a call takes as long as its longest lists, which the wave goes
+// through in fewer steps.  In us, alone against groups or the mix:
+//   mean 22-34,   6,000 pairs: 5.5-6.8 and 4.4-5.9 (3,000: equal)
+//   mean 80-170,  6,000: 5.8-7.1 and 9.2-10.1;  12,000: 8.1-10.9 and 9.8-14.9;
+//                 20,000: 14-18 and 11-18.5
+//   mean 300-2,800, 6,000: 10-142 and 15-388;  50,000: 53-918 and 52-4,391;
+//                 1,000,000: 0.94-16.8 ms and 0.73-15.3
+inline uint64_t alone_pairs(uint32_t mean) { return mean < 64 ? 4096 : mean < 256 ? 12288 : 65536; }
 
-// Weighted pairs go to groups only from here on: the whole wave's part costs
-// registers and scheduling (2 M pairs: 341 us, 362 mixed) and only a call's
-// last waves gain by it (16,000 pairs: 10.4 us, 9.3 mixed).
+// From this mean on nearly every pair is one for the whole wave, and a
+// weighted call takes the mix whatever its size (1 M pairs: 0.96-15.3 ms, in
+// groups 1.6-67).  Below it weighted pairs go to groups from kWMixedPairs on:
+// the whole wave's part costs registers and scheduling (2 M pairs: 341 us, 362
+// mixed) and only a call's last waves gain by it (16,000 pairs: 10.4 us, 9.3
+// mixed).
+constexpr uint32_t kLongMean = 256;
 constexpr uint64_t kWMixedPairs = 32768;
 
 // Consecutive pairs per wave otherwise: as many as leave 8,192 waves work, in
 // [4, 64].  A chunk's ids and records are two dependent reads before its first
 // pair, so long calls take 64 (1 M pairs: 87 us against 97 with 16 and 161
-// with 4); short ones spread over the chip.  Weighted pairs, whose distances
-// are one more dependent read, start at 2 (6,000 pairs, 200 K vertices: 7.3
-// us, 7.9 with 4; 12,000: 10.2 and 8.7).
-template <int K>
-uint32_t query_chunk(uint64_t k)
+// with 4); short ones spread over the chip.  Where the pairs come out one
+// after the other, 32,768 waves (100,000 pairs: 0.11-1.77 ms with 4, 0.14-2.3
+// with 16; 1 M: 0.96-15.3 with 16, 1.06-17.3 with 64).
+inline uint32_t query_chunk(uint64_t k, uint32_t mean)
 {
-    if (K == kWeights && k <= 2 * kAlonePairs) return 2;
+    const uint64_t waves = mean < kLongMean ? 8192 : 32768;
     uint32_t c = 64 / kQLanes;
-    while (c < 64 && (uint64_t)c * 2 * 8192 <= k) c *= 2;
+    while (c < 64 && (uint64_t)c * 2 * waves <= k) c *= 2;
     return c;
 }
 
+inline uint32_t mean_list(const pado_gpu_index *idx) { return (uint32_t)(idx->num_labels / idx->n); }
+
 template <int K, class OT>
-pado_gpu_status launch_batch(const QIndex &X, const uint32_t *qa, const uint32_t *qb, uint64_t k, OT *out, bool ref,
-                             hipStream_t st)
+pado_gpu_status launch_batch(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
+                             uint64_t k, OT *out, bool ref, hipStream_t st)
 {
     if (k == 0) return PADO_GPU_OK;
-    const bool alone = k <= kAlonePairs;
-    const uint32_t chunk = alone ? 1u : query_chunk<K>(k), grid = grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20);
+    const QIndex X = query_index(idx, rank_space);
+    const uint32_t mean = mean_list(idx);
+    const bool alone = k <= alone_pairs(mean);
+    const uint32_t chunk = alone ? 1u : query_chunk(k, mean), grid = grid_for((k + chunk - 1) / chunk * 64, 256, 1u << 20);
     auto kern = X.rec ? (alone ? k_query<K, true, kAlone, OT> : k_query<K, true, kMixed, OT>)
                       : (alone ? k_query<K, false, kAlone, OT> : k_query<K, false, kMixed, OT>);
-    if (K == kWeights && k > kWMixedPairs)
+    if (K == kWeights && k > kWMixedPairs && mean < kLongMean)
         kern = X.rec ? k_query<K, true, kGrouped, OT> : k_query<K, false, kGrouped, OT>;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, st, X, qa, qb, k, chunk, out, ref ? 1 : 0);
     PADO_HIP(hipGetLastError());
@@ -895,13 +909,13 @@ pado_gpu_status launch_batch(const QIndex &X, const uint32_t *qa, const uint32_t
 pado_gpu_status launch_wquery(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                               uint64_t k, uint32_t *out, bool ref_compat, hipStream_t st)
 {
-    return launch_batch<kWeights>(query_index(idx, rank_space), qa, qb, k, out, ref_compat, st);
+    return launch_batch<kWeights>(idx, rank_space, qa, qb, k, out, ref_compat, st);
 }
 
 pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                              uint64_t k, uint8_t *out, bool ref_compat, hipStream_t st)
 {
-    return launch_batch<kHops>(query_index(idx, rank_space), qa, qb, k, out, ref_compat, st);
+    return launch_batch<kHops>(idx, rank_space, qa, qb, k, out, ref_compat, st);
 }
 
 // u16 answers on device pairs: exact hops for a wide index, the reference's
@@ -909,9 +923,8 @@ pado_gpu_status launch_query(const pado_gpu_index *idx, bool rank_space, const u
 pado_gpu_status launch_query_wide(const pado_gpu_index *idx, bool rank_space, const uint32_t *qa, const uint32_t *qb,
                                   uint64_t k, uint16_t *out, bool ref_compat, hipStream_t st)
 {
-    const QIndex X = query_index(idx, rank_space);
-    if (idx->wide) return launch_batch<kWideHops>(X, qa, qb, k, out, false, st);
-    return launch_batch<kHops>(X, qa, qb, k, out, ref_compat, st);
+    if (idx->wide) return launch_batch<kWideHops>(idx, rank_space, qa, qb, k, out, false, st);
+    return launch_batch<kHops>(idx, rank_space, qa, qb, k, out, ref_compat, st);
 }
 
 // Query launch on device pairs for either index type, ordered ids: out holds
@@ -935,11 +948,12 @@ pado_gpu_status launch_query_any(const pado_gpu_index *idx, const uint32_t *qa, 
     const QIndex X = query_index(idx, false);
     hipLaunchKernelGGL(k_zero_work, dim3(1), dim3(1), 0, st, work);
     if (idx->weighted)
-        hipLaunchKernelGGL((k_query_ws<kWeights, uint32_t>), dim3(grid), dim3(256), 0, st, X, qa, qb, k,
-                           (uint32_t *)out, ref_compat ? 1 : 0, work);
+        hipLaunchKernelGGL((mean_list(idx) < kLongMean ? k_query_ws<kWeights, kGrouped, uint32_t>
+                                                       : k_query_ws<kWeights, kMixed, uint32_t>),
+                           dim3(grid), dim3(256), 0, st, X, qa, qb, k, (uint32_t *)out, ref_compat ? 1 : 0, work);
     else
-        hipLaunchKernelGGL((k_query_ws<kHops, uint8_t>), dim3(grid), dim3(256), 0, st, X, qa, qb, k, (uint8_t *)out,
-                           ref_compat ? 1 : 0, work);
+        hipLaunchKernelGGL((k_query_ws<kHops, kMixed, uint8_t>), dim3(grid), dim3(256), 0, st, X, qa, qb, k,
+                           (uint8_t *)out, ref_compat ? 1 : 0, work);
     PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
