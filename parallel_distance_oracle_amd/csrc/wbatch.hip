@@ -315,6 +315,12 @@ constexpr uint32_t kWWitness = 2;  // witnesses k_w_filter takes at a time (1 an
 // launches of those behind it).
 constexpr uint32_t kWAhead = 2, kWAheadFrom = 8;
 
+// Rounds that a batch is enqueued with at most.  Batches differ: after one of
+// 3,000 rounds the next ones of a path were given as many, at 7 us a round
+// that does nothing (weighted path of 3,000 vertices: 108 ms, with 16 to 128:
+// 38.3 to 39.9; 3,000 x 12 grid: 818 and 759-763; R-MAT 18: 86.5 either way).
+constexpr uint32_t kWRoundsAhead = 32;
+
 // Improved pairs of a tail up to which k_w_check reads single table entries.
 constexpr uint32_t kWGather = 8;
 
@@ -1114,12 +1120,13 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
                            static_cast<WClosed *>(ring_dev) + b % kWRing);
     };
     // Batches are enqueued whole, with as many rounds as the last three needed
-    // at most, and one ahead of the host's look at their records, so that the
-    // later ones (38 us of kernels each) do not wait for the host between
-    // their rounds and their filter.  A batch whose rounds turn out not to
-    // have ended, or whose labels might not fit the pool, holds everything
-    // behind it (k_w_filter); the host then ends it step by step and goes on
-    // from there.  Weighted R-MAT 20: 597 -> 576 ms; 200 K vertices: 80 -> 75.
+    // at most (up to kWRoundsAhead), and one ahead of the host's look at their
+    // records, so that the later ones (38 us of kernels each) do not wait for
+    // the host between their rounds and their filter.  A batch whose rounds
+    // turn out not to have ended, or whose labels might not fit the pool,
+    // holds everything behind it (k_w_filter); the host then ends it step by
+    // step and goes on from there.  Weighted R-MAT 20: 597 -> 576 ms; 200 K
+    // vertices: 80 -> 75.
     constexpr uint32_t kRoundHistory = 3;
     uint32_t hist[kRoundHistory] = {}, launched[kWRing] = {};
     hist[0] = 6;
@@ -1143,7 +1150,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
             hipLaunchKernelGGL(k_w_init, dim3((rsz * 64 + 255) / 256), dim3(256 * (1 + kWInitFill)), 0, st, rs, rsz,
                                next + 1, g->off.p, g->adj.p, T.p, tmark.p, tlist.p, alist.p, ag.p, amask.p, aend.p,
                                chunks.p, hmin.p, dcw.p, S, ctr.p);
-            const uint32_t R = *std::max_element(hist, hist + kRoundHistory);
+            const uint32_t R = std::min(kWRoundsAhead, *std::max_element(hist, hist + kRoundHistory));
             launched[next % kWRing] = R;
             rounds(next, 0, R);
             filter(next, touched, 1u, (R + 1) & 1u);
