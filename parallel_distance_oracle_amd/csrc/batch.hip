@@ -630,12 +630,15 @@ __device__ __forceinline__ void hub_rows(uint32_t fill, uint32_t ro, unsigned lo
 // root, kInitRoots roots per block of the launch schedule: the first wave of a
 // root sets it up while the other three enter its labels -- with one wave for
 // both, the root with the longest list (1,435 labels on R-MAT 20, six
-// dependent steps) set the kernel's time.  Root offset ro owns touched-list
+// dependent steps) set the kernel's time.  (PARTS = 1, the one-workgroup loop,
+// whose waves have roots enough: one wave for both; four per root took its
+// R-MAT 10 build from 1.3 to 2.1 ms.)  Root offset ro owns touched-list
 // slot ro (k_batch_begin sets the count and the frontier size), so the shared
 // counters left are the push-descriptor count, updated once per block, and
 // the frontier's push-edge count.
 constexpr uint32_t kRootWaves = 4, kInitRoots = 4;
-template <bool W, uint32_t CH, uint32_t RW>
+constexpr uint32_t kLoopWaves = 8;  // waves of a k_batch_loop workgroup, a root each
+template <bool W, uint32_t CH, uint32_t RW, uint32_t PARTS = kRootWaves>
 __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, const uint8_t *used, const uint64_t *off, const uint32_t *adj,
                                                      LabelStore S, HubInfo *hinfo, typename Hop<W>::Dist *dc,
                                                      unsigned long long *ind, unsigned long long *vmark,
@@ -645,12 +648,12 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
                                                      const unsigned long long *lmask, unsigned long long *rmask,
                                                      BuildCounters *C)
 {
-    __shared__ uint32_t s_nch[kInitRoots], s_pdeg[kInitRoots];
+    constexpr uint32_t ROOTS = PARTS == 1 ? kLoopWaves : kInitRoots;  // of a block
+    __shared__ uint32_t s_nch[ROOTS], s_pdeg[ROOTS];
     __shared__ uint32_t s_base;
     if (C->hold) return;
-    const uint32_t lane = lane_id(), part = (threadIdx.x >> 6) % kRootWaves, rb = threadIdx.x / (64 * kRootWaves);
-    const uint32_t roots = blockDim.x / (64 * kRootWaves);  // of this block
-    const uint32_t ro = bid * roots + rb;
+    const uint32_t lane = lane_id(), part = (threadIdx.x >> 6) % PARTS, rb = threadIdx.x / (64 * PARTS);
+    const uint32_t ro = bid * ROOTS + rb;
     const uint32_t rs = C->rs, rsz = C->rsz, gen_batch = C->gen_batch;
     const uint32_t r = rs + ro;
     // Every wave of a root reads its label record before the first one
@@ -660,7 +663,7 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     if (live) rec0 = S.rec[r];
     __syncthreads();
     if (part != 0) {
-        if (live) hub_rows<W, RW>(1u, ro, rec0.base, rec0.len, part - 1u, kRootWaves - 1u, S, hinfo, dc);
+        if (live) hub_rows<W, RW>(1u, ro, rec0.base, rec0.len, part - 1u, PARTS - 1u, S, hinfo, dc);
         __syncthreads();
         __syncthreads();
         return;
@@ -706,7 +709,7 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
     if (threadIdx.x == 0) {
         uint32_t tot = 0;
         unsigned long long tot_e = 0;
-        for (uint32_t w = 0; w < roots; ++w) {
+        for (uint32_t w = 0; w < ROOTS; ++w) {
             tot += s_nch[w];
             tot_e += s_pdeg[w];
         }
@@ -722,6 +725,7 @@ __device__ __forceinline__ void batch_init_body(uint32_t bid, uint32_t nblk, con
         for (uint32_t w = 0; w < rb; ++w) c0 += s_nch[w];
         for (uint32_t q = lane; q < nch; q += 64) chunks[c0 + q] = ((unsigned long long)(q * CH) << 32) | r;
     }
+    if (PARTS == 1 && live) hub_rows<W, RW>(1u, ro, rec0.base, rec0.len, 0u, 1u, S, hinfo, dc);
 }
 
 template <bool W, uint32_t CH, uint32_t RW>
@@ -740,19 +744,19 @@ __global__ __launch_bounds__(kInitRoots * kRootWaves * 64) void k_batch_init(con
 
 // The root-distance entries of the previous batch's roots (the labels they
 // held at its end, which include every entry written during it) are reset,
-// kRootWaves waves per root.
-template <bool W, uint32_t RW>
+// PARTS waves per root.
+template <bool W, uint32_t RW, uint32_t PARTS = kRootWaves>
 __device__ __forceinline__ void hub_reset_body(uint32_t bid, const uint8_t *used, LabelStore S, HubInfo *hinfo,
                                                typename Hop<W>::Dist *dc, const BuildCounters *C)
 {
     if (C->hold) return;
-    const uint32_t w = (bid * blockDim.x + threadIdx.x) >> 6, ro = w / kRootWaves;
+    const uint32_t w = (bid * blockDim.x + threadIdx.x) >> 6, ro = w / PARTS;
     const uint32_t rs = C->rs, rsz = C->rsz;
     if (ro >= rsz) return;
     const uint32_t r = rs + ro;
     if (used[r]) return;
     const LRec rec = S.rec[r];
-    hub_rows<W, RW>(0u, ro, rec.base, rec.len, w % kRootWaves, kRootWaves, S, hinfo, dc);
+    hub_rows<W, RW>(0u, ro, rec.base, rec.len, w % PARTS, PARTS, S, hinfo, dc);
 }
 
 
@@ -1798,7 +1802,6 @@ struct BatchPlan {
     BuildCounters *C;
 };
 
-constexpr uint32_t kLoopWaves = 8;  // waves of a k_batch_loop workgroup
 
 // Every phase ends at a workgroup barrier; the bodies' virtual blocks are
 // looped over (bid) with nblk = 1, so their grid-stride loops cover the work.
@@ -1815,8 +1818,8 @@ __global__ __launch_bounds__(kLoopWaves * 64) void k_batch_loop(const BatchPlan<
     for (uint32_t b = 0; b < nb; ++b) {
         // The previous batch's root-distance entries and indicator rows.
         const uint32_t prsz = C->rsz;
-        for (uint32_t vb = 0; vb * (kLoopWaves / kRootWaves) < prsz; ++vb)
-            hub_reset_body<W, kRow>(vb, P.used, P.S, P.hinfo, P.dc, C);
+        for (uint32_t vb = 0; vb * kLoopWaves < prsz; ++vb)
+            hub_reset_body<W, kRow, 1>(vb, P.used, P.S, P.hinfo, P.dc, C);
         batch_end_body<kRow>(0, 1, P.ind, P.tlist, P.abits, C);
         // Batch b: its non-bit-parallel roots are the first frontier.
         const uint32_t rs = b * P.batch, rsz = min(P.batch, P.n - rs);
@@ -1829,8 +1832,8 @@ __global__ __launch_bounds__(kLoopWaves * 64) void k_batch_loop(const BatchPlan<
         __syncthreads();
         if (threadIdx.x == 0) batch_begin_write(C, b, rs, rsz, {s_cnt, 0u, 0u, 0u});
         __syncthreads();
-        for (uint32_t vb = 0; vb * (kLoopWaves / kRootWaves) < rsz; ++vb)
-            batch_init_body<W, kChunk, kRow>(vb, 1, P.used, P.off, P.adj, P.S, P.hinfo, P.dc, P.ind, P.vmark, P.tlist,
+        for (uint32_t vb = 0; vb * kLoopWaves < rsz; ++vb)
+            batch_init_body<W, kChunk, kRow, 1>(vb, 1, P.used, P.off, P.adj, P.S, P.hinfo, P.dc, P.ind, P.vmark, P.tlist,
                                        P.abits, P.ag, P.amask, P.aend, P.chunks, P.bps, P.rset, P.lmask, P.rmask, C);
         __syncthreads();
         for (uint32_t iter = 1;; ++iter) {
