@@ -179,6 +179,11 @@ pado_gpu_status pado_gpu_graph_export(pado_gpu_ctx *ctx, const pado_gpu_graph *g
                                       uint8_t *w);
 pado_gpu_status pado_gpu_graph_get_info(const pado_gpu_graph *g, uint32_t *num_v, uint64_t *m_dir, int *weighted);
 
+/* Batches of 1,024 roots run four at a time (up to 2^22 vertices, where the
+ * memory for it is there) unless batch_size, push_chunk, push_waves,
+ * pull_ratio or PADO_GPU_BUILD_STREAM / _DEVICE_LOOP ask for anything but their
+ * defaults: those settings are for batches one by one, which take up to twice
+ * the time. */
 typedef struct {
     uint32_t batch_size;  /* roots per batch: 1..1024, 0 = 1024 (PARA:42); any value
                              gives the same labels, so it is a tuning knob */
@@ -199,9 +204,10 @@ typedef struct {
                              has more push edges than pull_ratio / 1000 of the
                              adjacency entries of the vertices >= roots_start runs
                              in pull form (each tail gathers the roots offered to
-                             it; same labels and counters).  0 = 0xFFFFFFFF =
-                             always push: on R-MAT 20 every threshold measured
-                             slower (400: +0.6%, 100: +11%) */
+                             it; same labels and counters).  0 and 0xFFFFFFFF:
+                             always push (0xFFFFFFFF in batches one by one): on
+                             R-MAT 20 every threshold measured slower (400:
+                             +0.6%, 100: +11%) */
 } pado_gpu_build_cfg;
 
 /* Bit-parallel labeling one BFS per slot (as the reference runs it) instead of
@@ -234,10 +240,9 @@ typedef struct {
 /* Run the whole batch phase inside one workgroup (no reference counterpart):
  * the same kernels' work back to back with workgroup barriers in place of
  * kernel launches and host checks.  Same labels.  It removes the launch and
- * host-check latency of every iteration but runs on one compute unit, so it
- * pays off only on small graphs (measured on MI355X: 7x faster on a
- * 1K-vertex R-MAT, 1.7x slower on a 1.6K-vertex grid, 20-40x slower on
- * 20K-60K-vertex grids); the autotuner tries it below 4K vertices.  Its label
+ * host-check latency of every iteration but runs on one compute unit (measured
+ * on MI355X: R-MAT 10 1.0 ms, 0.47 with launches enqueued ahead; 20-40x slower
+ * on 20K-60K-vertex grids); the autotuner tries it below 4K vertices.  Its label
  * pool is sized up front; if it runs dry the build falls back to the launch
  * schedule.  Ignored with PADO_GPU_BUILD_STREAM. */
 #define PADO_GPU_BUILD_DEVICE_LOOP 8u

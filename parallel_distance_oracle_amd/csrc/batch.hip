@@ -350,9 +350,10 @@ struct SetScratch {
 // pairs; the (pair, slot) tests left over, mostly those of pairs that pass,
 // are then spread over the wave 64 at a time, so a pair with dozens of
 // candidate slots costs a few wave steps instead of dozens.  Root set pairs
-// always come from the batch's slot-major table (800 KB, which stays in the
-// L2 cache), tail set pairs from the vertex-major table (in the spread steps
-// lanes hold slots of the same few tails, whose records they share).
+// always come from the batch's slot-major table (800 bytes per root: 0.8 MB
+// for 1,024 roots, 3.3 MB for 4,096, about an XCD's L2), tail set pairs from
+// the vertex-major table (in the spread steps lanes hold slots of the same few
+// tails, whose records they share).
 // Returns whether the lane's pair is pruned.
 template <uint32_t R>
 __device__ inline bool bp_set_phase(unsigned long long rem, unsigned long long one, const ulonglong2 *rset,
@@ -1510,7 +1511,7 @@ __device__ __forceinline__ void add_body(uint32_t bid, uint32_t nblk, uint32_t i
         // hubs.  There, a vertex with few candidate roots takes the distance
         // query hub-parallel: lanes hold labels, and each lane reads the one
         // root-distance entry per candidate root it needs, all of a step's
-        // reads in flight together.  Otherwise lanes hold roots (16 each) and
+        // reads in flight together.  Otherwise lanes hold roots (PER each) and
         // read row slices of the passing hubs (hub_pass).  croot: the
         // candidate root offsets (wave-uniform); cpr: which of them are
         // pruned.
@@ -1931,14 +1932,14 @@ struct BatchBuffers {
     DevBuf<unsigned long long> ind, cand, ag, chunks;
     DevBuf<unsigned long long> abits;  // frontier bitmaps, two slots of ceil(n / 64) words
     DevBuf<unsigned long long> lmask;  // bit-parallel mask rows, kLmWords words per vertex
-    DevBuf<unsigned long long> rmask;  // batch roots' mask words 0..kLmNz0, word-major [10][kBatch]
+    DevBuf<unsigned long long> rmask;  // batch roots' mask words 0..kLmNz0, word-major: kLmNz0 + 1 words, Rows::kRoots each
     DevBuf<uint64_t> amask;
     DevBuf<uint32_t> tlist, clist, aend, pool;
     DevBuf<HubInfo> hinfo;
     DevBuf<uint32_t> d1, d1len;  // distance-1 lists (HubList1): m slots, n counts
     DevBuf<LRec> lrec;
     DevBuf<typename Hop<W>::Dist> dc;
-    DevBuf<ulonglong2> rset;  // batch roots' bit-parallel sets, slot-major [kBP][kBatch]
+    DevBuf<ulonglong2> rset;  // batch roots' bit-parallel sets, slot-major: kBP slots, Rows::kRoots each
     DevBuf<BuildCounters> ctr;
     unsigned long long pool_size = 0;
     uint32_t dc_rows = 0;

@@ -55,9 +55,12 @@ constexpr uint32_t kAddGrid = 1024;
 // grid: 0.18 s vs 0.22 s with 1024), and concurrent builds share the chip.
 inline uint32_t default_grid(uint32_t n) { return n <= (1u << 17) ? 256u : 1024u; }
 // The batch labeling's push and add grids and push descriptor size by
-// default.  Measured on R-MAT 20 ef16 (median of 3 builds): push 768 blocks /
-// add 512 blocks / 8-edge descriptors 0.326 s; 1024 / 1024 / 16: 0.356 s;
-// 4-edge descriptors tie with 8; other grids within 1%.
+// default, chosen on single batches of an earlier build (R-MAT 20 ef16, median
+// of 3: push 768 blocks / add 512 blocks / 8-edge descriptors 0.326 s; 1024 /
+// 1024 / 16: 0.356 s; 4-edge descriptors tie with 8).  With batches four at a
+// time: 768 / 512 123.1 ms, 512 / 512 130.0, 768 / 256 133.7, 1024 / 512 121.5,
+// 768 / 1024 120.3, 1024 / 1024 118.5, 2048 / 2048 121.3; R-MAT 16, 256 / 256:
+// 3.50 ms, 768 / 512 3.31.
 inline uint32_t default_push_grid(uint32_t n) { return n <= (1u << 17) ? 256u : 768u; }
 inline uint32_t default_add_grid(uint32_t n) { return n <= (1u << 17) ? 256u : 512u; }
 constexpr uint32_t kPushChunk = 8;
@@ -464,7 +467,7 @@ struct pado_gpu_index {
     pado::DevBuf<uint32_t> whub;
     pado::DevBuf<uint32_t> wdist;
     // Query copy in original-id order (order_labels, PARA:2198-2281): records
-    // (QRec below), sets, and label lists that start at multiples of
+    // (kQRecWords above), sets, and label lists that start at multiples of
     // kListAlign entries and are padded to them with all-ones.
     int ordered = 0;
     int built = 0;  // labeled by this library (not imported): components are known

@@ -18,7 +18,8 @@
 // components are answered from those alone, the others become jobs in LDS and
 // are answered four at a time, sixteen lanes (one DPP row) each, so that the
 // first kind leaves no lanes idle.  Pairs with long lists are left to the end
-// and take the whole wave, one at a time; so do all pairs of a short call.
+// and take the whole wave, one at a time; so do all pairs of a short call (how
+// short goes by the index's mean list length: alone_pairs).
 //   Bit-parallel slots: a lane takes four slots as bytes of one word of the
 // record.  With m the smallest slot sum, only slots at m or m + 1 can lower
 // it, and only where the deciding sets can meet: the record has two bits per
@@ -34,8 +35,8 @@
 // Rank-space queries (many-graph jobs, checks) read the build's own arrays
 // through the same code (REC = false).
 //
-// What bounds it: on a large index the lines read at random (81 M of 128 B for
-// 10 M uniform pairs on R-MAT 20: 4.5 TB/s, a copy's rate), on a small one
+// What bounds it: on a large index the lines read at random (80 M of 128 B for
+// 10 M uniform pairs on R-MAT 20: 5.2 TB/s, a copy's rate), on a small one
 // instruction issue.  Against one wave per pair with the set pairs of every
 // slot within one of m read, in us:
 //                                      first   four pairs   records   long alone
@@ -449,7 +450,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t r0, uint32_t njobs,
 // Weighted query_distance (WPARA:2125-2243): min over common hubs of
 // La(h) + Lb(h).  Exact u32 answers, 0xFFFFFFFF when no hub is shared; with
 // ref_compat the reference's int16 domain (>= 32765 -> 32767, ids out of
-// range -> a == b ? 0 : 32767).  As answer_pairs, on the hub lists;
+// range -> a == b ? 0 : 32767).  As answer_jobs, on the hub lists;
 // distances of the shorter list come in with its hubs, those of the longer
 // list are read where a hub matches.
 template <bool REC, uint32_t L>
@@ -599,16 +600,16 @@ uint32_t query_ws_blocks_per_cu(bool weighted)
 // queue's device counter (queues are picked by workgroup, so the eight
 // counters and their traffic spread over the XCDs) and waits, sleeping, on
 // the mirrored count in L2.  A wave answers its descriptor's pairs with the
-// label merge of the batch kernel: one host read brings in the up-to-64
-// pairs' ids (lane j holds pair j), the lanes load their own pair's label
-// offsets together, and the pairs are then answered in turn from those
-// registers; the answers go back as one contiguous store into the mapped
-// answer ring.  The wave that completes a request's last descriptor writes
-// the request's sequence number into its slot's completion flag.  The poller
-// stops taking in new descriptors once asked to (host stop flag), after
-// max_ticks in any case, or after idle_ticks without work; when every
-// descriptor taken in is done it raises the exit flag, and every wave leaves.
-// The host relaunches the kernel when work arrives after an exit.
+// label merge of the batch kernel (answer_pairs): one host read brings in the
+// up-to-64 pairs' ids (lane j holds pair j), the lanes sort their own pairs
+// into jobs in LDS, and groups of lanes or the whole wave answer these; the
+// answers go back as one contiguous store into the mapped answer ring.  The
+// wave that completes a request's last descriptor writes the request's
+// sequence number into its slot's completion flag.  The poller stops taking in
+// new descriptors once asked to (host stop flag), after max_ticks in any case,
+// or after idle_ticks without work; when every descriptor taken in is done it
+// raises the exit flag, and every wave leaves.  The host relaunches the kernel
+// when work arrives after an exit.
 namespace {
 
 // Relaxed device-coherent load.  No acquire anywhere in the serving loop: an

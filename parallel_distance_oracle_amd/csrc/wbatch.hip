@@ -818,7 +818,7 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
         w_lds_sync();
         uint32_t drop = 0;
         for (uint32_t w = 0; w < nwit; w += kWWitness) {
-            // Column h of the roots' entries for four witnesses h, 8 consecutive
+            // Column h of the roots' entries for kWWitness witnesses h, 8 consecutive
             // roots per lane; only lanes that hold a root ranked below h and not
             // yet dropped read.
             uint32_t h[kWWitness], dvh[kWWitness], todo[kWWitness], drh[kWWitness][8], prh[kWWitness];
