@@ -28,8 +28,8 @@
 //   chunks[]         push work descriptors (active vertex, edge start), eight
 //                    edges each
 //   pool[] u32       label store: per-vertex growable arrays of packed
-//                    (hub << 8 | dist) labels, grown fourfold (at least 32)
-//                    on overflow by a bump allocator (one wave owns one
+//                    (hub << 8 | dist) labels, grown fourfold (at least 32;
+//                    twofold from 1,024) on overflow by a bump allocator (one wave owns one
 //                    vertex's array); rec[n] = (base, len, cap), 16 B each
 //   lmask[n][16] u64 bit-parallel level masks (bit i of word k < 8: slot i at
 //                    distance k), nonempty-set masks (words 8, 9: slots with
@@ -469,11 +469,14 @@ __global__ void k_hub_info_init(HubInfo *p, uint64_t count)
 }
 
 // Pool words that a list of len labels and capacity cap takes for `add` more:
-// 0 if they fit.
+// 0 if they fit.  Short lists grow fourfold, for few moves; from 1,024 words
+// on doubling costs no more time (R-MAT 20: 122.8 ms, 122.6), and graphs with
+// thousands of labels a vertex take half the pool (64,000 vertices of degree
+// 256, 624 M labels: 134 -> 69 GB).
 __device__ inline uint32_t store_words(uint32_t len, uint32_t cap, uint32_t add)
 {
     if (len + add <= cap) return 0u;
-    const uint32_t ncap = max(cap * 4, len + add);  // few moves
+    const uint32_t ncap = max(cap < 1024u ? cap * 4 : cap * 2, len + add);
     return max(ncap, 32u);
 }
 
@@ -2300,7 +2303,11 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
     // maximum), and the pool top at that check: the headroom kept before the
     // next blocks scales with it, so a fast-growing phase (labels-only
     // pruning, early batches) cannot run the pool dry inside a block.
-    double rate = 0.0;
+    // Iterations of one batch differ too much for the rate alone: once batches
+    // are complete, three times what the largest of the recent ones took is
+    // enough (two can run before the next check).
+    double rate = 0.0, batch_words = 0.0, recent_batch = 0.0;
+    bool unseen = false;  // words of this batch's first block went into a repack
     unsigned long long snap_top_prev = 0;
     for (uint32_t b = 0; b < nb; ++b) {
         const uint32_t batch_end = std::min<uint64_t>((uint64_t)(b + 1) * batch, n);
@@ -2371,16 +2378,18 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
                 return PADO_GPU_ERR_DOMAIN;
             }
             if (snap.pool_top >= snap_top_prev && cur_count) {
-                const double r = (double)(snap.pool_top - snap_top_prev) / cur_count;
-                rate = std::max(r, rate * 0.75);
+                const double words = (double)(snap.pool_top - snap_top_prev);
+                rate = std::max(words / cur_count, rate * 0.75);
+                batch_words += words;
             }
             snap_top_prev = snap.pool_top;
             // Keep at least 60% of the pool free, and room for four blocks of
             // the recent growth (two can run before the next check: this
-            // batch's next and the one ahead); a block ahead runs to
-            // completion first.
+            // batch's next and the one ahead) or for three batches; a block
+            // ahead runs to completion first.
             const double ahead_iters = std::max<uint32_t>(U, first_block(prev_batch_iters));
-            const double need = rate * 4.0 * ahead_iters;
+            double need = rate * 4.0 * ahead_iters;
+            if (recent_batch > 0.0) need = std::min(need, 3.0 * std::max(recent_batch, batch_words));
             if (snap.pool_top * 5 > pool_size * 2 || (double)snap.pool_top + need > 0.8 * (double)pool_size) {
                 PADO_HIP(hipStreamSynchronize(st));
                 unsigned long long top = 0;
@@ -2424,6 +2433,9 @@ static pado_gpu_status build_batches_t(pado_gpu_graph *g, pado_gpu_index *idx, c
         // alone takes 81 and 86.
         iters_hist[hist_pos++ % kIterHistory] = (uint32_t)(steps_seen - batch_first_step);
         prev_batch_iters = *std::max_element(iters_hist, iters_hist + kIterHistory);
+        if (!unseen) recent_batch = std::max(batch_words, recent_batch * 0.75);
+        unseen = repacked && spec;
+        batch_words = 0.0;
         // Pool growth of this batch (unknown across a repack, which blocks
         // running ahead until a batch has been measured again).
         if (repacked) {

@@ -51,3 +51,28 @@ def test_smaller_batches_where_the_wide_rows_do_not_fit(wide):
     assert np.array_equal(_build(ctx, dg, wide)[3], exp[3])
     dg.close()
     ctx.close()
+
+
+def test_label_pool_of_dense_label_sets():
+    """A random graph with 4,100 labels a vertex, most lists long enough to grow
+    by doubling.  A pool is made for twice the compacted lists (5/4 of the
+    labels) and three times what a batch took (up to 5/2 of the labels), and the
+    one before it is there while the lists move: 35 words a label at most.  By
+    the steepest iteration, for as long as a batch could last, it was some 80."""
+    rng = np.random.default_rng(1)
+    n = 32000
+    e = np.sort(rng.integers(0, n, (4_300_000, 2)), axis=1)
+    e = np.unique(e[e[:, 0] != e[:, 1]], axis=0).astype(np.uint32)
+    ctx = pado.Context(0)
+    dg, _, _ = pado.DeviceGraph.from_edges(ctx, e)
+    ctx.trim()
+    got = _build(ctx, dg, False)
+    peak, labels = ctx.work_sizes()[1], got[3].size
+    fixed = 5 * 64 * 8 * n + 4096 * n  # rows of 64 words, root-distance table
+    print(f"[gpu] {labels} labels, temporaries {peak >> 20} MiB", flush=True)
+    assert peak <= 2 * fixed + 4 * 35 * labels
+    ctx.trim()
+    exp = _build(ctx, dg, False, 0xFFFFFFFF)
+    assert all(np.array_equal(x, y) for x, y in zip(got, exp))
+    dg.close()
+    ctx.close()
