@@ -61,7 +61,8 @@ pado_gpu_status build_batches_loop(std::vector<LoopJob> &jobs, hipStream_t st);
 // Weighted labeling (WPARA).
 pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t batch_size);
 
-// Exclusive scan of n u32 values into n+1 u64 offsets (out[n] = total).
+// Exclusive scan of n u32 values into n+1 u64 offsets (out[n] = total),
+// enqueued on s, the stream of the pool's context.
 pado_gpu_status scan_u32_to_u64(const uint32_t *in, uint64_t *out, uint32_t n, hipStream_t s, WorkPool *wp);
 // Sort every CSR segment of u32 keys ascending in place, in vertex ranges of
 // at most max_items keys per hipCUB call (0 = kSortMaxItems; hipCUB counts

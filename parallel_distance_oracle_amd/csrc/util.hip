@@ -56,7 +56,8 @@ pado_gpu_status scan_u32_to_u64(const uint32_t *in, uint64_t *out, uint32_t n, h
     DevBuf<uint8_t> ws;
     PADO_TRY(ws.alloc(bytes, wp));
     PADO_HIP(hipcub::DeviceScan::ExclusiveSum(ws.p, bytes, tmp.p, out, (int)(n + 1), s));
-    PADO_HIP(hipStreamSynchronize(s));
+    // (the temporaries are the pool's: their next taker is behind on this stream)
+    PADO_HIP(hipGetLastError());
     return PADO_GPU_OK;
 }
 
