@@ -289,9 +289,11 @@ typedef struct {
 pado_gpu_status pado_gpu_index_get_info(const pado_gpu_index *idx, pado_gpu_index_info *info);
 /* How often a weighted build waited for the host: batches, enqueued whole and
  * ahead, that were held because their rounds had not ended or their labels
- * might not fit the pool, and how often the pool was then grown (each
- * nullable; 0 for a loaded index). */
-pado_gpu_status pado_gpu_windex_holds(const pado_gpu_index *idx, uint64_t *holds, uint64_t *grows);
+ * might not fit the pool, and how often the pool was then grown; and the most
+ * pool words (of one label each) that were handed out before a growth or the
+ * end (each nullable; 0 for a loaded index). */
+pado_gpu_status pado_gpu_windex_holds(const pado_gpu_index *idx, uint64_t *holds, uint64_t *grows,
+                                      uint64_t *pool_words);
 
 /* Canonical export in RANK space: bp_dist[n*50], bp_sets[n*50*2] (S^-1,
  * S^0\S^-1 per slot), label_off[n+1], hubs[num_labels] ascending per vertex,

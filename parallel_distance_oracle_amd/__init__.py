@@ -118,7 +118,7 @@ def lib():
         "pado_write_edge_binary": (ctypes.c_int, [ctypes.c_char_p, _vp, _u64]),
         "pado_free": (None, [_vp]),
         "pado_gpu_windex_export": (ctypes.c_int, [_vp, _vp, _vp, _vp, _vp]),
-        "pado_gpu_windex_holds": (ctypes.c_int, [_vp, ctypes.POINTER(_u64), ctypes.POINTER(_u64)]),
+        "pado_gpu_windex_holds": (ctypes.c_int, [_vp] + [ctypes.POINTER(_u64)] * 3),
         "pado_gpu_wquery": (ctypes.c_int, [_vp, _vp, _vp, _vp, _u64, _vp, _u32, _vp]),
         "pado_rmat_edges": (_u64, [_u32, _u32, ctypes.c_double, ctypes.c_double, ctypes.c_double, _u64, _vp, _u64]),
         "pado_grid_edges": (_u64, [_u32, ctypes.c_double, _u64, _vp, _u64]),
@@ -643,8 +643,9 @@ class Index:
         return loff, hub[:tot], dist[:tot]
 
     def holds(self):
-        """Weighted index: (batches its build held for the host, times its label pool was grown)."""
-        x = _u64(), _u64()
+        """Weighted index: (batches its build held for the host, times its label pool was grown, most
+        pool words taken)."""
+        x = _u64(), _u64(), _u64()
         _check(lib().pado_gpu_windex_holds(self.h, *(ctypes.byref(v) for v in x)))
         return tuple(v.value for v in x)
 

@@ -84,11 +84,7 @@ __device__ inline uint32_t ctz_any(uint64_t x) { return (uint32_t)__builtin_ctzl
 __device__ inline uint32_t popc_any(uint32_t x) { return (uint32_t)__popc(x); }
 __device__ inline uint32_t popc_any(uint64_t x) { return (uint32_t)__popcll(x); }
 __device__ inline uint32_t readlane_any(uint32_t x, uint32_t l) { return __builtin_amdgcn_readlane(x, l); }
-__device__ inline uint64_t readlane_any(uint64_t x, uint32_t l)
-{
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, l), hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), l);
-    return ((uint64_t)hi << 32) | lo;
-}
+__device__ inline uint64_t readlane_any(uint64_t x, uint32_t l) { return readlane64(x, l); }
 
 __device__ inline bool any_active(const uint32_t (&n_act)[4]) { return (n_act[0] | n_act[1] | n_act[2] | n_act[3]) != 0u; }
 

@@ -117,13 +117,6 @@ __global__ __launch_bounds__(256) void k_ms_seed(uint32_t nseeds, const uint32_t
     }
 }
 
-__device__ inline u64 readlane64(u64 x, uint32_t lane)
-{
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, lane);
-    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), lane);
-    return ((u64)hi << 32) | lo;
-}
-
 // For every lane j of `act`: f(vertex u of lane j, whether this lane's slot is
 // in its mask m), kMsAhead of them at a time.
 template <class F>

@@ -258,6 +258,15 @@ __device__ inline uint64_t uniform64(uint64_t x)
 
 __device__ inline uint32_t uniform32(uint32_t x) { return __builtin_amdgcn_readfirstlane(x); }
 
+// Lane `lane`'s 64 bits, in scalar registers.  (The builtin returns an int,
+// whose sign must not spread over the upper half.)
+__device__ inline unsigned long long readlane64(unsigned long long x, uint32_t lane)
+{
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, lane);
+    const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), lane);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
 template <int CTRL, int ROWS>
 __device__ inline uint32_t dpp0(uint32_t x)  // x moved by DPP, 0 where nothing moves in
 {
@@ -454,7 +463,8 @@ struct pado_gpu_index {
     uint32_t wide = 0;  // labels in the wide hop domain (Hop<true>)
     uint32_t bp_pass_through = 0;  // wide build whose bit-parallel BFS was cut at level 254:
                                    // its bit-parallel vertices were labeled as ordinary hubs
-    uint64_t holds = 0, grows = 0;  // weighted build: batches held for the host, label pools grown
+    // Weighted build: batches held for the host, label pools grown, most words taken of one.
+    uint64_t holds = 0, grows = 0, pool_words = 0;
     // Bit-parallel labels, rank space: bpd[v*64 + i], bps[(v*50 + i)*2 + {0,1}];
     // the rest of a bpd line holds the nonempty-set bits (kBpNzByte).
     pado::DevBuf<uint8_t> bpd;

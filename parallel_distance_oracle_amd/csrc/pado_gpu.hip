@@ -727,7 +727,8 @@ pado_gpu_status pado_gpu_index_get_info(const pado_gpu_index *idx, pado_gpu_inde
     return PADO_GPU_OK;
 }
 
-pado_gpu_status pado_gpu_windex_holds(const pado_gpu_index *idx, uint64_t *holds, uint64_t *grows)
+pado_gpu_status pado_gpu_windex_holds(const pado_gpu_index *idx, uint64_t *holds, uint64_t *grows,
+                                      uint64_t *pool_words)
 {
     clear_error();
     if (!idx || !idx->weighted) {
@@ -736,6 +737,7 @@ pado_gpu_status pado_gpu_windex_holds(const pado_gpu_index *idx, uint64_t *holds
     }
     if (holds) *holds = idx->holds;
     if (grows) *grows = idx->grows;
+    if (pool_words) *pool_words = idx->pool_words;
     return PADO_GPU_OK;
 }
 

@@ -91,12 +91,6 @@ __device__ inline uint32_t lane_id() { return threadIdx.x & 63; }
 
 __device__ inline u64 *stat_rows(WCounters *C) { return reinterpret_cast<u64 *>(C + 1); }
 
-__device__ inline u64 readlane64(u64 x, uint32_t lane)
-{
-    return ((u64)__builtin_amdgcn_readlane((uint32_t)(x >> 32), lane) << 32) |
-           __builtin_amdgcn_readlane((uint32_t)x, lane);
-}
-
 __device__ inline uint32_t wave_max(uint32_t x)
 {
     x = max(x, dpp0<0x111, 0xF>(x));
@@ -1183,6 +1177,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
             }
             if (grow) {
                 idx->grows += 1;
+                idx->pool_words = std::max<uint64_t>(idx->pool_words, h->pool_top);
                 // Compact every list into a larger pool.  After compaction a list of
                 // length L has capacity L + L/4 + 4, so the commit can reserve at
                 // most 2.5 * live + new + 8 * touched words.
@@ -1230,6 +1225,7 @@ pado_gpu_status build_weighted(pado_gpu_graph *g, pado_gpu_index *idx, uint32_t 
         set_error("weighted label pool exhausted");
         return PADO_GPU_ERR_NOMEM;
     }
+    idx->pool_words = std::max<uint64_t>(idx->pool_words, h->pool_top);
     idx->iterations = h->rounds;
     idx->counters.labels = h->labels;
     idx->counters.pushes = h->relax;

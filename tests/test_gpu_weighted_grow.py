@@ -32,7 +32,7 @@ def test_held_and_grown(gpu_ctx, kind, grows, batch):
     dg, rank, _ = pado.DeviceGraph.from_edges(gpu_ctx, edges, w)
     n = dg.num_v
     idx = pado.Index.build(gpu_ctx, dg, batch_size=batch)
-    held, grown = idx.holds()
+    held, grown, _ = idx.holds()
     print(f"[gpu] {kind} batch {batch}: {n} vertices, {idx.info.num_labels} labels, held {held}, grown {grown}",
           flush=True)
     assert held > 0 and (grown > 0) == grows
