@@ -397,8 +397,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
                 const uint32_t l0 = (uint32_t)__ffsll(todo) - 1;
                 u64 edges = todo & (0xFFFFull << (l0 & ~(kChunk - 1)));  // this chunk's
                 todo &= ~edges;
-                const u64 roots = ((u64)__builtin_amdgcn_readlane((uint32_t)(all >> 32), l0) << 32) |
-                                  __builtin_amdgcn_readlane((uint32_t)all, l0);
+                const u64 roots = readlane64(all, l0);
                 const uint32_t *from = T + (uint64_t)__builtin_amdgcn_readlane(u, l0) * kWB + wd * 64;
                 const uint32_t du = (roots >> lane) & 1ull ? from[lane] : kWInf;
                 while (edges) {
