@@ -268,15 +268,6 @@ __device__ inline bool bp_mask_scan(uint32_t iter, const unsigned long long *rm,
     }
 }
 
-// Orders LDS writes of some lanes of a wave before reads by other lanes of
-// the same wave.
-__device__ inline void wave_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // Position of the rank-th set bit of m (rank < popcount(m)).
 __device__ inline uint32_t nth_set_bit(unsigned long long m, uint32_t rank)
 {

@@ -267,6 +267,15 @@ __device__ inline unsigned long long readlane64(unsigned long long x, uint32_t l
     return ((unsigned long long)hi << 32) | lo;
 }
 
+// Orders LDS writes of some lanes of a wave before reads by other lanes of the
+// same wave.
+__device__ inline void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 template <int CTRL, int ROWS>
 __device__ inline uint32_t dpp0(uint32_t x)  // x moved by DPP, 0 where nothing moves in
 {
@@ -350,9 +359,7 @@ __device__ inline void list_flush(uint32_t *counter, uint32_t *list, const uint3
 {
     if (held == 0u) return;
     const uint32_t lane = threadIdx.x & 63;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    wave_lds_sync();
     uint32_t base = 0;
     if (lane == 0) base = atomicAdd(counter, held);
     base = uniform32(base);

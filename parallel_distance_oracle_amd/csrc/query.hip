@@ -81,14 +81,6 @@ struct Lanes {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef u32x4 u32x4_at4 __attribute__((aligned(4)));  // four words at any word address
 
-// Orders LDS writes of some lanes of a wave before reads by other lanes.
-__device__ inline void q_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 template <int N>
 __device__ inline uint32_t row_ror(uint32_t x)
 {
@@ -268,7 +260,7 @@ __device__ inline void make_jobs(const QIndex &X, bool has, uint32_t a, uint32_t
     ngroup = (uint32_t)__popcll(mg);
     njobs = ngroup + (uint32_t)__popcll(ma);
     if (job) buf.job[(alone ? ngroup : 0u) + (uint32_t)__popcll((alone ? ma : mg) & ((1ull << lane) - 1ull))] = j;
-    q_lds_sync();
+    wave_lds_sync();
 }
 
 // Answers jobs r0 to njobs, 64 / L at a time, each job's answer to
@@ -393,7 +385,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t r0, uint32_t njobs,
                 const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
                 tile_put(tile, u * G::kStep + 4 * l, REC ? v : mask4(v, j, lt));
             }
-            q_lds_sync();
+            wave_lds_sync();
             for (uint32_t i = 0; i < ms; i += G::kStep) {
                 const u32x4 v = i == 0 ? s0 : load4(S, i + 4 * l, ls);
                 const u32x4 s = REC ? v : mask4(v, i + 4 * l, ls);
@@ -415,7 +407,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t r0, uint32_t njobs,
                 }
             }
             // The next copy must not overtake these reads.
-            q_lds_sync();
+            wave_lds_sync();
         }
         d = group_min<L>(d);
         if (first) {
@@ -444,7 +436,7 @@ __device__ inline void answer_jobs(const QIndex &X, uint32_t r0, uint32_t njobs,
         if (!W && d >= 253u) d = 255u;
         if (has && l == 0) buf.ans[job.ls >> 24] = d;
     }
-    q_lds_sync();
+    wave_lds_sync();
 }
 
 // Weighted query_distance (WPARA:2125-2243): min over common hubs of
@@ -478,7 +470,7 @@ __device__ inline void answer_wjobs(const QIndex &X, uint32_t r0, uint32_t njobs
                 const u32x4 v = t0 == 0 && u < kQPre ? (u ? tv[1] : tv[0]) : load4(T, j, lt);
                 tile_put(tile, u * G::kStep + 4 * l, REC ? v : mask4(v, j, lt));
             }
-            q_lds_sync();
+            wave_lds_sync();
             for (uint32_t i = 0; i < ms; i += G::kStep) {
                 const u32x4 v = i == 0 ? s0 : load4(S, i + 4 * l, ls);
                 const u32x4 s = REC ? v : mask4(v, i + 4 * l, ls);
@@ -494,13 +486,13 @@ __device__ inline void answer_wjobs(const QIndex &X, uint32_t r0, uint32_t njobs
                 for (int q = 0; q < 4; ++q)  // (no hub, or a sum past 2^32: all-ones, which lowers nothing)
                     d = min(d, __builtin_elementwise_add_sat(x[q], e[q]));
             }
-            q_lds_sync();
+            wave_lds_sync();
         }
         d = group_min<L>(d);
         if (ref_compat && d >= 32765u) d = 32767u;
         if (has && l == 0) buf.ans[job.ls >> 24] = d;
     }
-    q_lds_sync();
+    wave_lds_sync();
 }
 
 // Kinds of index: u8 hops, the wide hop domain, weighted.
@@ -546,7 +538,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
         const uint32_t d = answer_pairs<K, REC, M>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
         if (has) out[c0 + lane] = (OT)d;
         // The next chunk's jobs and answers must not overtake these reads.
-        q_lds_sync();
+        wave_lds_sync();
     }
 }
 
@@ -573,7 +565,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
         const uint32_t a = has ? qa[c0 + lane] : 0u, b = has ? qb[c0 + lane] : 0u;
         const uint32_t d = answer_pairs<K, true, M>(X, has, a, b, ref_compat != 0, s_q[threadIdx.x >> 6]);
         if (has) out[c0 + lane] = (OT)d;
-        q_lds_sync();
+        wave_lds_sync();
     }
 }
 
@@ -727,7 +719,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kQOcc))) vo
         }
         const uint32_t mine = answer_pairs<K, true, kMixed>(X, lane < len, ia, ib, A.ref_compat != 0, s_q[wv]);
         // The next descriptor's writes must not overtake these reads.
-        q_lds_sync();
+        wave_lds_sync();
         if (lane < len) {
             if (K == kHops) st_sys(static_cast<uint8_t *>(A.out) + phys + lane, (uint8_t)mine);
             if (K == kWideHops) st_sys(static_cast<uint16_t *>(A.out) + phys + lane, (uint16_t)mine);

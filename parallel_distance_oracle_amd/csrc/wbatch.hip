@@ -285,14 +285,6 @@ __device__ inline uint32_t w_nth_set_bit(u64 m, uint32_t rank)
     return pos;
 }
 
-// Orders LDS writes of some lanes of a wave before reads by other lanes.
-__device__ inline void w_lds_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 constexpr uint32_t kWPushWaves = 4;  // waves per k_w_push block
 // Roots in a frontier word from which on k_w_push takes the word lane by lane,
 // kWPushEdges edges at a time (weighted R-MAT 20: 612 ms without, 597 at 16,
@@ -433,7 +425,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
                 s_g[wv][lane] = g;
                 s_ex[wv][lane] = incl - cnt;
                 s_imp[wv][lane] = 0ull;
-                w_lds_sync();
+                wave_lds_sync();
                 for (uint32_t x0 = 0; x0 < total; x0 += 64) {
                     const uint32_t x = x0 + lane;
                     if (x >= total) continue;
@@ -455,7 +447,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
                         if (cand < old) atomicOr(&s_imp[wv][o], 1ull << b);
                     }
                 }
-                w_lds_sync();
+                wave_lds_sync();
                 imp |= s_imp[wv][lane];
             }
             if (imp) {
@@ -463,7 +455,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
                 got = true;
             }
             // The next word's writes must not overtake this word's reads.
-            w_lds_sync();
+            wave_lds_sync();
         }
         const bool new_t = got && tmark[t] != gen_batch && atomicExch(&tmark[t], gen_batch) != gen_batch;
         const bool new_i = got && imark[t] != gen_round && atomicExch(&imark[t], gen_round) != gen_round;
@@ -472,7 +464,7 @@ __global__ __launch_bounds__(256) void k_w_push(uint32_t round, uint32_t rs, uin
         list_append(&C->n_imp[p], ilist, s_il[wv], held_i, new_i, t);
         n_imp += new_i ? 1u : 0u;
         // s_u / s_t / s_w are rewritten by the next step.
-        w_lds_sync();
+        wave_lds_sync();
     }
     list_flush(&C->n_touched, tlist, s_tl[wv], held_t);
     list_flush(&C->n_imp[p], ilist, s_il[wv], held_i);
@@ -808,7 +800,7 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
             for (int q = 0; q < 8; ++q)
                 if ((surv >> q) & 1u) s_wit[wib][at++] = make_uint2(lane * 8 + q, dv[q]);
         }
-        w_lds_sync();
+        wave_lds_sync();
         uint32_t drop = 0;
         for (uint32_t w = 0; w < nwit; w += kWWitness) {
             // Column h of the roots' entries for kWWitness witnesses h, 8 consecutive
@@ -853,7 +845,7 @@ __global__ __launch_bounds__(256) void k_w_filter(uint32_t rs, uint32_t rsz, con
             }
         }
         // (the next vertex's list must not overtake these reads)
-        w_lds_sync();
+        wave_lds_sync();
         const uint32_t keep = surv & ~drop;
         n_filt += __popc(drop);
         // The improved bitmap is all zero once the rounds end; it carries the
